@@ -2189,6 +2189,107 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
   store_epilogue<TrF32, C>(e, acc, mt, nt);
 }
 
+// Per-pair weight dots <V_j, G_i^T A_i> (V_j = G_j^T A_j of val sample j) from one sample's
+// K-major product per work item.  Each item forms one output tile of one sample's G^T A over
+// its T k-rows; with DOT = false (val samples) it stores the tile as V_j, with DOT = true
+// (train samples) it takes the tile's inner product with every V_j and stores one partial per
+// (val sample, tile, train sample): P[(j * tiles + tile) * n + i].  V_j is kept in the order of
+// the accumulators (both launches share tile and wave shape), packed to bf16 pairs: one
+// coalesced 16-byte load per lane for 8 accumulator entries, where a row-major V would touch 32
+// rows per load.  Work is n_val + n_train sample products, where one row-dot GEMM per val sample
+// takes n_val * n_train of them: 24 + 8 samples, T = 1024, 768 x 3072 took 1115-1146 us that
+// way and take 211 us this way (155 GFLOP).
+// What bounds it is the caches: an item reads T * 512 bytes of operands and n_val * 32 KiB of
+// V_j.  Order of the items: groups of `group` tiles (4 x 2 blocks), all samples of a group in
+// turn, the tiles of one sample adjacent, so that the items on one XCD share operand columns
+// and the group's V_j's (2 MiB at 8 val samples) in its L2.  Measured at the shape above /
+// at 40 + 2 samples, T = 1000, 2048 x 2048: tile by tile 294 / 665 us, groups of 4 229 / 430,
+// of 8 211 / 400, of 16 222 / 394, of 64 259 / 417.
+struct TpParams {
+  TnParams tn;       // L: G, R: A (K-row 0 of the sample set), gap: the skipped val block
+  int64_t T, n;      // k-rows per sample; samples (val: DOT = false, train: DOT = true)
+  int64_t n_val;     // V_j's the DOT launch reads
+  int64_t group;     // tiles of a group
+  uint4* V;          // [n_val][tiles][NW][MI * NI][2][64 lanes]
+  float* P;
+};
+template <class C, class D, bool DOT>
+__global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tn_pair_kernel(TpParams q) {
+  const TnParams& p = q.tn;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[D::STAGES * D::STAGE_BYTES];
+  constexpr int NW = C::WM * C::WN;
+  constexpr int64_t WAVE_V = C::MI * C::NI * 2 * 64;  // uint4 of one wave's tile share
+  const int64_t it = xcd_order(blockIdx.x, gridDim.x);
+  const int64_t tiles = p.m_tiles * p.n_tiles;
+  const int64_t grp = it / (q.group * q.n), rem = it - grp * q.group * q.n;
+  const int64_t gsize = tiles - grp * q.group < q.group ? tiles - grp * q.group : q.group;
+  const int64_t smp = rem / gsize, tile = grp * q.group + rem % gsize;
+  const bool m_inner = p.m_tiles <= p.n_tiles;
+  const int64_t inner = m_inner ? p.m_tiles : p.n_tiles;
+  const int64_t outer = m_inner ? p.n_tiles : p.m_tiles;
+  constexpr int64_t ROWS = 4;  // tiles of the longer side taken together
+  const int64_t sr = tile / (ROWS * inner), r = tile - sr * ROWS * inner;
+  const int64_t rows = outer - sr * ROWS < ROWS ? outer - sr * ROWS : ROWS;
+  const int64_t outer_i = sr * ROWS + r % rows, inner_i = r / rows;
+  const int64_t mt = m_inner ? inner_i : outer_i, nt = m_inner ? outer_i : inner_i;
+  f32x16_t acc[C::MI][C::NI];
+  zero_acc<TrBF16, C>(acc);
+  mainloop_tn<C, D>(p, mt, nt, smp * q.T, (smp + 1) * q.T, lds, acc);
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if constexpr (!DOT) {
+    uint4* dst = q.V + ((smp * tiles + tile) * NW + wid) * WAVE_V + lane;
+#pragma unroll
+    for (int i = 0; i < C::MI; ++i)
+#pragma unroll
+      for (int j = 0; j < C::NI; ++j)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          uint4 w;
+          w.x = pack_bf16x2(acc[i][j][8 * h], acc[i][j][8 * h + 1]);
+          w.y = pack_bf16x2(acc[i][j][8 * h + 2], acc[i][j][8 * h + 3]);
+          w.z = pack_bf16x2(acc[i][j][8 * h + 4], acc[i][j][8 * h + 5]);
+          w.w = pack_bf16x2(acc[i][j][8 * h + 6], acc[i][j][8 * h + 7]);
+          dst[((i * C::NI + j) * 2 + h) * 64] = w;
+        }
+  } else {
+    float* red = reinterpret_cast<float*>(lds);  // [NW][64]; the stages are free
+    for (int64_t j0 = 0; j0 < q.n_val; j0 += 64) {
+      const int nj = static_cast<int>(q.n_val - j0 < 64 ? q.n_val - j0 : 64);
+      float mine = 0.f;  // lane jj: this wave's share of val sample j0 + jj
+      for (int jj = 0; jj < nj; ++jj) {
+        const uint4* src = q.V + (((j0 + jj) * tiles + tile) * NW + wid) * WAVE_V + lane;
+        float d0 = 0.f, d1 = 0.f;
+#pragma unroll
+        for (int i = 0; i < C::MI; ++i)
+#pragma unroll
+          for (int j = 0; j < C::NI; ++j)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const uint4 w = src[((i * C::NI + j) * 2 + h) * 64];
+              const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                d0 += acc[i][j][8 * h + 2 * e] * __uint_as_float(u[e] << 16);
+                d1 += acc[i][j][8 * h + 2 * e + 1] * __uint_as_float(u[e] & 0xFFFF0000u);
+              }
+            }
+        const float d = wave_sum_dpp(d0 + d1);
+        mine = lane == jj ? d : mine;
+      }
+      __syncthreads();  // the previous 64 samples' sums have been read
+      red[wid * 64 + lane] = mine;
+      __syncthreads();
+      if (wid == 0 && lane < nj) {
+        float t = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) t += red[w * 64 + lane];
+        q.P[((j0 + lane) * tiles + tile) * q.n + smp] = t;
+      }
+    }
+  }
+}
+
 // out[i] = alpha * (sum over the splits of part[s][i]) in fixed order, rounded once to bf16
 // (or stored as fp32 with out_f32), 4 elements per thread.  With vsum ([vs_rows][vs_n]) its
 // rows are also summed into row 0, in place.
@@ -2352,6 +2453,7 @@ struct LinearPlan {
   int tile_reduce; // partials per tile instead of per train row
   int64_t p_ld;    // P row length: n-tiles (tile_reduce) or train rows
   int64_t cols;    // P entries per train sample in a P row
+  int pairs;       // VALGRAD pair matrix from per-sample products (tn_pair_kernel)
 };
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -2521,9 +2623,27 @@ bool rowdot_swap(int64_t d_in, int64_t d_out) {
   return std::is_same<Tr, TrBF16>::value && d_out > d_in && d_in % 8 == 0 &&
          d_out % 8 == 0;
 }
+// The pair matrix from per-sample products (tn_pair_kernel): bf16 operands the K-major GEMM
+// takes, and V_j's of at most 1 GiB (a small part of HBM).
+int64_t pair_tiles(int64_t d_in, int64_t d_out) {
+  return ceil_div(d_out, TnC::BM) * ceil_div(d_in, TnC::BN);
+}
+int64_t pair_v_bytes(int64_t n_val, int64_t d_in, int64_t d_out) {
+  return n_val * pair_tiles(d_in, d_out) * TnC::BM * TnC::BN * 2;
+}
+bool pair_products_ok(int dtype, int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
+                      int algo, int want_pair) {
+  return want_pair && algo != GS_ALGO_GHOST && dtype == GS_DTYPE_BF16 &&
+         tn_ok(nullptr, d_out, nullptr, d_in, N * T, d_out, d_in) &&
+         pair_v_bytes(n_val, d_in, d_out) <= (int64_t{1} << 30) &&
+         pair_tiles(d_in, d_out) * N <= INT32_MAX;
+}
+
+// `products`: the pair matrix may come from per-sample products (pair_products_ok, and at run
+// time 16-byte aligned operands).
 template <class Tr>
 LinearPlan plan_linear(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
-                       int semantics, int algo, int want_pair) {
+                       int semantics, int algo, int want_pair, bool products) {
   constexpr int64_t GBM = GhostCfg<Tr>::BM;
   const int64_t n_t = N - n_val;
   const bool swap = rowdot_swap<Tr>(d_in, d_out);
@@ -2541,6 +2661,30 @@ LinearPlan plan_linear(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_
   const double valgrad = vgemm + rowdot * (want_pair ? n_val : 1);
   pl.algo = algo;
   if (algo == GS_ALGO_AUTO) pl.algo = ghost <= valgrad ? GS_ALGO_GHOST : GS_ALGO_VALGRAD;
+  if (products) {
+    // Estimated times in us.  Sample products: whole 64-row stages of 128 x 128 tiles at
+    // 1 PF/s, the inner products at 0.13 ps per V_j entry and train sample, 12 us of launches
+    // and pipeline fill.  Ghost: rounds of 256 tiles of 256 x 256, each as long as its
+    // (d_in + d_out) / 64 stages however few tiles a round has.  Measured (products / ghost):
+    // 24 + 8 samples of 768 x 3072 at T = 64: 81 / 91, 256: 100 / 101, 512: 135 / 319, 1000:
+    // 211 / 1211; 2048 x 2048 at T = 64: 118 / 93, 512: 221 / 337; 8 + 2 of 512 x 512 at T = 16:
+    // 20 / 32.
+    const double area = static_cast<double>(pair_tiles(d_in, d_out)) * TnC::BM * TnC::BN;
+    const double prod = 12.0 + 2e-9 * N * ceil_div(T, TnD::KB) * TnD::KB * area +
+                        1.3e-7 * n_val * n_t * area;
+    const double tiles = static_cast<double>(nv_eff * ceil_div(T, GBM)) *
+                         ceil_div(n_t * T, static_cast<int64_t>(StashCfg::BN));
+    const double gtime = 6.0 + std::ceil(tiles / 256.0) * 0.024 * (d_in + d_out);
+    pl.pairs = algo == GS_ALGO_VALGRAD || prod <= gtime ? 1 : 0;
+    if (pl.pairs) {
+      pl.algo = GS_ALGO_VALGRAD;
+      pl.groups = n_val;
+      pl.p_rows = n_val * pair_tiles(d_in, d_out);
+      pl.p_ld = n_t;
+      pl.cols = 1;
+      return pl;
+    }
+  }
   int64_t bn;
   if (pl.algo == GS_ALGO_GHOST) {
     pl.ghost_flat = flat ? 1 : 0;
@@ -2563,11 +2707,29 @@ LinearPlan plan_linear(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_
   return pl;
 }
 
+// `products` false: without the per-sample-product form of the pair matrix (operands that are
+// not 16-byte aligned, or no scratch for the V_j's).
 LinearPlan plan_any(int dtype, int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
-                    int semantics, int algo, int want_pair) {
+                    int semantics, int algo, int want_pair, bool products = true) {
   if (dtype == GS_DTYPE_F32)
-    return plan_linear<TrF32>(N, n_val, T, d_in, d_out, semantics, algo, want_pair);
-  return plan_linear<TrBF16>(N, n_val, T, d_in, d_out, semantics, algo, want_pair);
+    return plan_linear<TrF32>(N, n_val, T, d_in, d_out, semantics, algo, want_pair, false);
+  products = products && pair_products_ok(dtype, N, n_val, T, d_in, d_out, algo, want_pair);
+  return plan_linear<TrBF16>(N, n_val, T, d_in, d_out, semantics, algo, want_pair, products);
+}
+// The plan of a call on known operands, with at most `cap` bytes of scratch for the V_j's form.
+// AUTO with the reference's rounding keeps to the forms whose ghost side honours it.
+size_t linear_bytes(int dtype, const LinearPlan& pl, int64_t n_val, int64_t T, int64_t d_in,
+                    int64_t d_out, int semantics, const void* A, const void* G);
+LinearPlan plan_call(int dtype, int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
+                     int semantics, int algo, int want_pair, int rounding, const void* A,
+                     const void* G, size_t cap = SIZE_MAX) {
+  const bool products = aligned16(A) && aligned16(G) &&
+                        !(algo == GS_ALGO_AUTO && rounding == GS_ROUND_REF_BF16);
+  const LinearPlan pl = plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair,
+                                 products);
+  if (pl.pairs && linear_bytes(dtype, pl, n_val, T, d_in, d_out, semantics, A, G) > cap)
+    return plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair, false);
+  return pl;
 }
 
 // Workspace of run_linear, in the order it carves.  `tn`: VALGRAD forms V by the K-major
@@ -2577,7 +2739,10 @@ template <class S>
 void carve_linear(S& c, const LinearPlan& pl, int dtype, int64_t T, int64_t d_in,
                   int64_t d_out, int semantics, bool tn) {
   const size_t esz = elem_size(dtype);
-  if (pl.algo == GS_ALGO_GHOST) {
+  if (pl.pairs) {
+    c.template take<char>(pair_v_bytes(pl.groups, d_in, d_out));
+    c.template take<float>(pl.p_rows * pl.p_ld);
+  } else if (pl.algo == GS_ALGO_GHOST) {
     if (semantics == GS_SEM_PRESUM) {
       c.template take<char>(T * d_in * esz);
       c.template take<char>(T * d_out * esz);
@@ -2730,6 +2895,44 @@ int run_linear(const void* A, const void* G, int64_t N, int64_t n_val, int64_t v
   const int64_t a_bytes = N * T * d_in * static_cast<int64_t>(esz);
   const int64_t g_bytes = N * T * d_out * static_cast<int64_t>(esz);
 
+  if constexpr (std::is_same<Tr, TrBF16>::value) {
+    if (pl.pairs) {
+      TpParams q{};
+      q.V = reinterpret_cast<uint4*>(cv.take<char>(pair_v_bytes(n_val, d_in, d_out)));
+      q.P = cv.take<float>(pl.p_rows * pl.p_ld);
+      q.T = T;
+      q.n = q.n_val = n_val;
+      TnParams& p = q.tn;
+      p.ldl = p.M = d_out;
+      p.ldr = p.N = d_in;
+      p.m_tiles = ceil_div(d_out, TnC::BM);
+      p.n_tiles = ceil_div(d_in, TnC::BN);
+      p.L = static_cast<const E*>(G) + val_start * T * d_out;
+      p.R = static_cast<const E*>(A) + val_start * T * d_in;
+      p.l_nbytes = n_val * T * d_out * 2;
+      p.r_nbytes = n_val * T * d_in * 2;
+      p.gap_at = INT64_MAX;
+      const int64_t tiles = p.m_tiles * p.n_tiles;
+      q.group = tiles;  // sample by sample
+      hipLaunchKernelGGL((tn_pair_kernel<TnC, TnD, false>),
+                         dim3(static_cast<unsigned>(tiles * n_val)), dim3(TnC::NT), 0, s, q);
+      p.L = G;
+      p.R = A;
+      p.l_nbytes = g_bytes;
+      p.r_nbytes = a_bytes;
+      p.gap_at = val_start * T < n_t * T ? val_start * T : INT64_MAX;
+      p.gap = p.gap_at < n_t * T ? n_val * T : 0;
+      q.n = n_t;
+      q.group = 8;
+      hipLaunchKernelGGL((tn_pair_kernel<TnC, TnD, true>),
+                         dim3(static_cast<unsigned>(tiles * n_t)), dim3(TnC::NT), 0, s, q);
+      int rc = check_launch("tn_pair_kernel");
+      if (rc) return rc;
+      hipLaunchKernelGGL(reduce_partials_kernel, dim3(static_cast<unsigned>(n_t)), dim3(256), 0,
+                         s, q.P, pl.groups, tiles, pl.p_ld, pl.cols, n_t, out_pair, out_dot);
+      return check_launch("reduce_partials_kernel");
+    }
+  }
   if (pl.algo == GS_ALGO_GHOST) {
     const void* La = A;
     const void* Lg = G;
@@ -2880,7 +3083,14 @@ extern "C" size_t gs_linear_dot_workspace(int dtype, int64_t N, int64_t n_val, i
                                           int want_pair) {
   if (!linear_args_ok(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair)) return 0;
   const LinearPlan pl = plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair);
-  return linear_bytes(dtype, pl, n_val, T, d_in, d_out, semantics, nullptr, nullptr) + 256;
+  size_t need = linear_bytes(dtype, pl, n_val, T, d_in, d_out, semantics, nullptr, nullptr);
+  if (pl.pairs) {  // the operands may turn out not to be 16-byte aligned
+    const LinearPlan other = plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo,
+                                      want_pair, false);
+    need = std::max(need, linear_bytes(dtype, other, n_val, T, d_in, d_out, semantics, nullptr,
+                                       nullptr));
+  }
+  return need + 256;
 }
 
 extern "C" int gs_linear_dot_algo(int dtype, int64_t N, int64_t n_val, int64_t T, int64_t d_in,
@@ -2931,7 +3141,8 @@ extern "C" int gs_linear_dot(const void* A, const void* G, int dtype, int64_t N,
   int rc = check_linear_args("gs_linear_dot", A, G, dtype, N, n_val, val_start, T, d_in, d_out,
                              semantics, algo, rounding, out_dot, want_pair);
   if (rc) return rc;
-  const LinearPlan pl = plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair);
+  const LinearPlan pl = plan_call(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair,
+                                  rounding, A, G);
   if (workspace == nullptr ||
       workspace_bytes < linear_bytes(dtype, pl, n_val, T, d_in, d_out, semantics, A, G))
     return fail(GS_ERR_WORKSPACE, "gs_linear_dot: workspace too small");
@@ -2948,7 +3159,8 @@ extern "C" size_t gs_linear_dot_noalloc_bytes(const void* A, const void* G, int 
                                               int64_t d_out, int semantics, int algo,
                                               int want_pair) {
   if (!linear_args_ok(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair)) return 0;
-  const LinearPlan pl = plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair);
+  const LinearPlan pl = plan_call(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair,
+                                  GS_ROUND_FP32, A, G, GS_LINEAR_NOALLOC_SCRATCH_BYTES);
   return linear_bytes(dtype, pl, n_val, T, d_in, d_out, semantics, A, G);
 }
 
@@ -2960,7 +3172,8 @@ extern "C" int gs_linear_dot_noalloc(const void* A, const void* G, int dtype, in
   int rc = check_linear_args("gs_linear_dot_noalloc", A, G, dtype, N, n_val, val_start, T,
                              d_in, d_out, semantics, algo, rounding, out_dot, want_pair);
   if (rc) return rc;
-  const LinearPlan pl = plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair);
+  const LinearPlan pl = plan_call(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair,
+                                  rounding, A, G, GS_LINEAR_NOALLOC_SCRATCH_BYTES);
   const size_t need = linear_bytes(dtype, pl, n_val, T, d_in, d_out, semantics, A, G);
   if (need > GS_LINEAR_NOALLOC_SCRATCH_BYTES)
     return fail(GS_ERR_UNSUPPORTED,

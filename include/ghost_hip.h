@@ -55,8 +55,11 @@ typedef enum { GS_SEM_PAIRWISE_SUM = 0, GS_SEM_PRESUM = 1 } gs_semantics;
 /* Algorithm used to evaluate a given semantics (the result is the same quantity).
  *   GHOST:   fused dual-Gram MFMA kernel; the T x T Gram blocks live only in registers.
  *   VALGRAD: V = sum_val B^T A (one GEMM), then dot_i = sum_t <b_it, V a_it> fused into
- *            the epilogue of a second GEMM; per-sample gradients are never stored.
- *   AUTO:    the one with fewer MFMA flops for the shape. */
+ *            the epilogue of a second GEMM; per-sample gradients are never stored.  With a
+ *            pair matrix and aligned bf16 operands: one V_j per val row, and each train row's
+ *            gradient tile times every V_j as it leaves the accumulators.
+ *   AUTO:    the one with fewer MFMA flops for the shape; where a pair matrix can come from the
+ *            sample products above, the one with the shorter estimated time. */
 typedef enum { GS_ALGO_AUTO = 0, GS_ALGO_GHOST = 1, GS_ALGO_VALGRAD = 2 } gs_algo;
 
 /* Rounding of the ghost Gram blocks.

@@ -66,6 +66,44 @@ def test_linear_pairs_and_val_first_layout(gpu, shape, algo):
         assert_close(pair.cpu().double().sum(0), dot.cpu().double(), 1e-5, "pair-sum")
 
 
+@pytest.mark.parametrize("case", [
+    # N, n_val, val_start, T, d_in, d_out: one partial tile; ragged T and tiles, val first; whole
+    # tiles, val in the middle; one token; more val samples than a wave has lanes
+    (5, 2, 3, 5, 24, 40), (9, 3, 0, 100, 136, 264), (8, 2, 4, 128, 256, 128),
+    (80, 16, 64, 1, 512, 104), (72, 67, 0, 9, 16, 136), (6, 5, 1, 65, 392, 8)])
+def test_pair_matrix_from_sample_products(gpu, case):
+    """The bf16 pair matrix from per-sample products, against <V_j, G_i^T A_i> in float64 with
+    V_j rounded to bf16 as the kernel holds it.  Beyond that rounding the kernel's sums are fp32;
+    an entry of V_j whose fp32 sum falls on the other side of a rounding tie moves by 2^-8, a
+    share of at most ~2^-8 of the entries, independent in sign: 1e-3 of the rms bounds both."""
+    N, n_val, vs, T, d_in, d_out = case
+    print(f"pair products case={case}", flush=True)
+    A, G = _inputs(N, T, d_in, d_out, 310 + T, torch.bfloat16)
+    dot, pair = _native.ops().linear_dot(A.to(gpu), G.to(gpu), n_val, val_start=vs,
+                                         algo=_native.ALGO_VALGRAD, want_pair=True)
+    M = torch.einsum("nto,nti->noi", G.double(), A.double())
+    V = M[vs:vs + n_val].bfloat16().double()
+    want = torch.einsum("joi,noi->jn", V, torch.cat([M[:vs], M[vs + n_val:]]))
+    assert_close(pair.cpu(), want, 1e-3, "pair")
+    assert_close(pair.cpu().double().sum(0), dot.cpu().double(), 1e-5, "pair-sum")
+
+
+def test_pair_matrix_unaligned_operands_take_the_general_path(gpu):
+    """Operands two bytes off a 16-byte boundary: the products' loads do not apply, and the call
+    runs as it does for them without the products."""
+    N, n_val, T, d_in, d_out = 7, 2, 40, 64, 96
+    A, G = _inputs(N, T, d_in, d_out, 330, torch.bfloat16)
+    buf = torch.zeros(A.numel() + 1, dtype=torch.bfloat16, device=gpu)
+    off = buf[1:].view(A.shape)
+    off.copy_(A)
+    assert off.data_ptr() % 16 and off.is_contiguous()
+    for algo in (_native.ALGO_AUTO, _native.ALGO_VALGRAD):
+        dot, pair = _native.ops().linear_dot(off, G.to(gpu), n_val, algo=algo, want_pair=True)
+        want = R.linear_dot_exact(A, G, n_val, "pairwise", pair=True)
+        assert_close(pair.cpu(), want, BF16_TOL, f"pair {algo}")
+        assert_close(pair.cpu().double().sum(0), dot.cpu().double(), 1e-5, "pair-sum")
+
+
 @pytest.mark.parametrize("shape", [(10, 3, 64, 128, 96), (6, 2, 40, 64, 72)])
 def test_ghost_reference_rounding_matches_reference_sequence(gpu, shape):
     N, n_val, T, d_in, d_out = shape
