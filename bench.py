@@ -104,6 +104,14 @@ class TimedOps:
         return out
 
     def linear_dot_train_grad(self, A, G, n_val, **k):
+        return self._dot_train_grad(self.inner.linear_dot_train_grad, k.get("bias"), A, G, n_val,
+                                    **k)
+
+    def linear_layer_pass(self, A, G, n_val, **k):
+        return self._dot_train_grad(self.inner.linear_layer_pass,
+                                    k.get("bias_grad_dtype") is not None, A, G, n_val, **k)
+
+    def _dot_train_grad(self, fn, bias, A, G, n_val, **k):
         # The op's work is the dots by the cheapest same-semantics algorithm,
         # 2 (n_v' + n_t) T d_in d_out (the V GEMM over the val rows, then one GEMM over the
         # train rows), which is also what it executes: the weight train gradient is the
@@ -115,11 +123,10 @@ class TimedOps:
         nv = n_val if k.get("semantics", 0) == _native.SEM_PAIRWISE_SUM else 1
         dot = 2.0 * (nv * T + (N - n_val) * T) * d_in * d_out
         grad = 2.0 * (N - n_val) * T * d_in * d_out if k.get("grad_scale") is not None else 0.0
-        tag = "+bias" if k.get("bias") else ""
+        tag = "+bias" if bias else ""
         kind = "conv1d" if k.get("conv1d") else "linear"
         out = self._run(f"{kind}_valgrad{tag}+train_grad[{d_in}x{d_out}]",
-                        ("mfma", dot, dot + grad),
-                        self.inner.linear_dot_train_grad, A, G, n_val, **k)
+                        ("mfma", dot, dot + grad), fn, A, G, n_val, **k)
         if out is None and self.enabled:
             self.records.pop()   # not supported for this shape: nothing ran
         return out

@@ -81,6 +81,10 @@ _SIGNATURES = {
     "gs_conv1d_dot_train_grad_workspace": (_SZ, [_I, _I64, _I64, _I64, _I64, _I64, _I, _I]),
     "gs_conv1d_dot_train_grad": (_I, [_P, _P, _I, _I64, _I64, _I64, _I64, _I64, _I64, _I, _P,
                                       _P, _I, _F, _P, _P, _I, _F, _P, _SZ, _P]),
+    "gs_linear_layer_pass_workspace": (_SZ, [_I, _I64, _I64, _I64, _I64, _I64, _I, _I, _I, _I,
+                                             _I]),
+    "gs_linear_layer_pass": (_I, [_P, _P, _I, _I64, _I64, _I64, _I64, _I64, _I64, _I, _I, _P, _I,
+                                  _P, _I, _F, _P, _I, _P, _I, _F, _P, _SZ, _P]),
     "gs_linear_train_grad_workspace": (_SZ, [_I, _I64, _I64, _I64, _I64, _I64]),
     "gs_linear_train_grad": (_I, [_P, _P, _I, _I64, _I64, _I64, _I64, _I64, _I64, _F, _P, _I,
                                   _I, _P, _SZ, _P]),
@@ -325,6 +329,53 @@ class HipOps:
         if rc == ERR_UNSUPPORTED:
             return None
         _check(rc, name)
+        return dot, grad, bdot, bgrad
+
+    def linear_layer_pass(self, A: torch.Tensor, G: torch.Tensor, n_val: int, *, semantics: int,
+                          algo: int, rounding: int, conv1d: bool, grad_scale: float,
+                          grad_dtype: torch.dtype, dot_dtype: torch.dtype,
+                          bias_grad_dtype: Optional[torch.dtype] = None,
+                          bias_dot_dtype: Optional[torch.dtype] = None, val_start=None):
+        """A Linear / Conv1D layer's dots and train gradients in one pass (gs_linear_layer_pass):
+        any T, the dots in the dtypes asked for; the bias terms when bias_grad_dtype is given.
+        Returns (dot, grad, bias_dot, bias_grad), or None where the separate passes must run or
+        are faster for `algo`."""
+        dev = _require_device(A, G)
+        if A.dtype != G.dtype:
+            raise GhostHipError(f"A and G dtypes differ: {A.dtype} vs {G.dtype}")
+        A = A.contiguous()
+        G = G.contiguous()
+        N = A.shape[0]
+        d_in, d_out = A.shape[-1], G.shape[-1]
+        T = _tokens(A, N, d_in)
+        if _tokens(G, N, d_out) != T:
+            raise GhostHipError(f"A {tuple(A.shape)} and G {tuple(G.shape)} token counts differ")
+        n_t = N - n_val
+        vs = n_t if val_start is None else int(val_start)
+        bias = bias_grad_dtype is not None
+        dt = _gs_dtype(A)
+        lib = load_library()
+        ws_bytes = lib.gs_linear_layer_pass_workspace(dt, N, n_val, T, d_in, d_out, semantics,
+                                                      int(conv1d), int(bias), algo, rounding)
+        if ws_bytes == 0:
+            return None
+        ws = _workspace(ws_bytes, dev)
+        dot = torch.empty(n_t, dtype=dot_dtype, device=dev)
+        grad = torch.empty((d_in, d_out) if conv1d else (d_out, d_in), dtype=grad_dtype,
+                           device=dev)
+        bdot = bgrad = None
+        if bias:
+            bdot = torch.empty(n_t, dtype=bias_dot_dtype, device=dev)
+            bgrad = torch.empty(d_out, dtype=bias_grad_dtype, device=dev)
+        rc = lib.gs_linear_layer_pass(
+            A.data_ptr(), G.data_ptr(), dt, N, n_val, vs, T, d_in, d_out, semantics, int(conv1d),
+            dot.data_ptr(), _gs_dtype(dot), grad.data_ptr(), _gs_dtype(grad), float(grad_scale),
+            _ptr(bdot), _gs_dtype(bdot) if bias else DTYPE_F32, _ptr(bgrad),
+            _gs_dtype(bgrad) if bias else DTYPE_F32, float(grad_scale), ws.data_ptr(), ws_bytes,
+            _stream(dev))
+        if rc == ERR_UNSUPPORTED:
+            return None
+        _check(rc, "gs_linear_layer_pass")
         return dot, grad, bdot, bgrad
 
     def linear_train_grad(self, A: torch.Tensor, G: torch.Tensor, n_val: int, scale: float, *,

@@ -1382,9 +1382,10 @@ __device__ __forceinline__ float4 split_sum4(const float* __restrict__ part, int
 template <class GE>
 __global__ void __launch_bounds__(256) tgdot_finish_kernel(
     const float* __restrict__ pdot, int64_t shares, int64_t n_t, const float* __restrict__ pbias,
-    int64_t bshares, const float* __restrict__ csum, int64_t cs_rows, int64_t M, float* out_dot,
-    float* out_bdot, GE* bgrad, float bscale, int64_t gblocks, const float* __restrict__ part,
-    int64_t count, int sp, void* grad, float gscale, int grad_f32) {
+    int64_t bshares, const float* __restrict__ csum, int64_t cs_rows, int64_t M, void* out_dot,
+    int dot_f32, void* out_bdot, int bdot_f32, GE* bgrad, float bscale, int64_t gblocks,
+    const float* __restrict__ part, int64_t count, int sp, void* grad, float gscale,
+    int grad_f32) {
   __shared__ float red[4];
   int64_t b = blockIdx.x;
   if (b < n_t) {
@@ -1396,7 +1397,13 @@ __global__ void __launch_bounds__(256) tgdot_finish_kernel(
     }
     if (r < shares) s0 += pdot[r * n_t + b];
     const float s = block_sum(s0 + s1, red);
-    if (threadIdx.x == 0) out_dot[b] = s;
+    auto put = [](void* out, int f32, int64_t at, float v) {
+      if (f32)
+        static_cast<float*>(out)[at] = v;
+      else
+        static_cast<uint16_t*>(out)[at] = f32_to_bf16(v);
+    };
+    if (threadIdx.x == 0) put(out_dot, dot_f32, b, s);
     if (pbias == nullptr) return;
     const float* pb = pbias + b * bshares;
     float t0 = 0.f, t1 = 0.f;
@@ -1407,7 +1414,7 @@ __global__ void __launch_bounds__(256) tgdot_finish_kernel(
     }
     if (r < bshares) t0 += pb[r];
     const float t = block_sum(t0 + t1, red);
-    if (threadIdx.x == 0) out_bdot[b] = t;
+    if (threadIdx.x == 0) put(out_bdot, bdot_f32, b, t);
     return;
   }
   b -= n_t;
@@ -1728,6 +1735,23 @@ struct TnStreamer {
     for (int q = 0; q < D::QR; ++q)
       dma16_at(rr, offr[q] + br, stage + D::L_BYTES + wb + D::NW * q * 1024);
   }
+  // Physical k-rows [row0, row0 + KB), rows at or past row_end as zeros: the buffers end there
+  // (a row's chunks lie wholly before the next row), so the cut costs no per-lane work.
+  __device__ __forceinline__ void issue_rows(const TnParams& p, unsigned stage, int row0,
+                                             int row_end) {
+    const unsigned wb = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) *
+                        1024u;
+    const unsigned l2 = static_cast<unsigned>(ldl2), r2 = static_cast<unsigned>(ldr2);
+    const __amdgpu_buffer_rsrc_t el = make_rsrc(p.L, static_cast<unsigned>(row_end) * l2);
+    const __amdgpu_buffer_rsrc_t er = make_rsrc(p.R, static_cast<unsigned>(row_end) * r2);
+    const unsigned bl = static_cast<unsigned>(row0) * l2, br = static_cast<unsigned>(row0) * r2;
+#pragma unroll
+    for (int q = 0; q < D::QL; ++q)
+      dma16_at(el, offl[q] + bl, stage + wb + D::NW * q * 1024);
+#pragma unroll
+    for (int q = 0; q < D::QR; ++q)
+      dma16_at(er, offr[q] + br, stage + D::L_BYTES + wb + D::NW * q * 1024);
+  }
   // `stage`: the LDS byte address of the stage (wave-uniform).
   __device__ __forceinline__ void issue(unsigned stage, int64_t k0, int64_t k_end) {
     const unsigned wb = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) *
@@ -1927,6 +1951,64 @@ __device__ __forceinline__ void mainloop_tn(const TnParams& p, int64_t mt, int64
   raw_barrier();
 }
 
+// mainloop_tn over samples of T rows, T any number, each padded to whole stages: k counts the
+// padded rows (Tp per sample), and a stage never crosses a sample's end.
+template <class C, class D, class Hook, class Cmp>
+__device__ __forceinline__ void mainloop_tn_samples(const TnParams& p, int64_t mt, int64_t nt,
+                                                    int64_t k_begin, int64_t k_end, int64_t Tp,
+                                                    int T, unsigned char* lds,
+                                                    f32x16_t (&acc)[C::MI][C::NI], Hook hook,
+                                                    Cmp cmp) {
+  constexpr int NQ = D::QL + D::QR;
+  constexpr int AHEAD = D::STAGES - 1;
+  TnStreamer<C, D> st;
+  st.init(p, mt, nt);
+  const int nk = static_cast<int>((k_end - k_begin) / D::KB);
+  const int sps = static_cast<int>(Tp / D::KB);
+  const unsigned lds0 = lds_addr(lds);
+  auto slot = [&](int k) { return lds + (k % D::STAGES) * D::STAGE_BYTES; };
+  auto slot_at = [&](int k) {
+    return lds0 + static_cast<unsigned>((k % D::STAGES) * D::STAGE_BYTES);
+  };
+  // The next stage to load: its first physical row, its sample's end and the stages left in it
+  // (wave-uniform; all row numbers fit 31 bits: the operands are below 2 GiB).
+  const int gap_at = p.gap != 0 ? static_cast<int>(p.gap_at) : -1;
+  const int gap = static_cast<int>(p.gap);
+  const int s0 = static_cast<int>(k_begin / Tp);
+  const int ss0 = static_cast<int>((k_begin - s0 * Tp) / D::KB);
+  int first = s0 * T;
+  if (p.gap != 0 && first >= gap_at) first += gap;
+  int row = first + ss0 * D::KB, end = first + T, left = sps - ss0;
+  auto load = [&](int k) {
+    st.issue_rows(p, slot_at(k), row, end);
+    row += D::KB;
+    if (--left == 0) {
+      left = sps;
+      row = end == gap_at ? end + gap : end;
+      end = row + T;
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s)
+    if (s < nk) load(s);
+  int kt = 0;
+  for (; kt + AHEAD < nk; ++kt) {
+    wait_vmcnt<(AHEAD - 1) * NQ>();
+    raw_barrier();
+    load(kt + AHEAD);
+    cmp(slot(kt), acc);
+    hook(kt, slot(kt));
+  }
+  for (; kt < nk; ++kt) {
+    wait_stages<NQ, AHEAD - 1>(nk - 1 - kt);
+    raw_barrier();
+    cmp(slot(kt), acc);
+    hook(kt, slot(kt));
+  }
+  wait_vmcnt<0>();
+  raw_barrier();
+}
+
 // Work item of this workgroup: (split, mt, nt).  The items are ordered split-major, then by
 // blocks of the side with more tiles, the other side innermost, and each XCD takes a
 // contiguous run of them (workgroup w runs on XCD w mod 8): the workgroups resident on one
@@ -2030,13 +2112,15 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tn_gemm_kernel(TnParams p
 // boundary (T k-rows, a multiple of the stage height) and at a split's end inside a sample,
 // each wave forms <acc, V tile> against the V tile it holds in registers and stores the
 // growth since the previous boundary as its share of that sample; acc runs on and ends as
-// the split's train-gradient partial.  With CS the column sums of the L tile (G: the bias
+// the split's train-gradient partial.  RAG: T is not a multiple of the stage height, and every
+// sample's rows are padded with zeros to whole stages (nothing is read for them).  With CS the column sums of the L tile (G: the bias
 // terms) are taken per stage as well, after the stage's MFMAs, spread over the workgroups.
 struct TgParams {
   TnParams tn;          // k-rows per split (kper) a multiple of the stage height, >= T;
                         // out: fp32 partials
   const uint16_t* Vt;   // V^T: [N][M] bf16
   int64_t T, n_t;       // k-rows per sample (a multiple of the stage height), train samples
+  int64_t T_rows;       // with RAG: the rows a sample has (T counts them padded to whole stages)
   float* pdot;          // [m_tiles * n_tiles][NW][2 slots][n_t] wave shares of the weight dots
   float* csum;          // with CS: [n_t][2 T / stage height][M] column sums of L (CS 1; of R,
                         // [..][N], with CS 2), two rows (halves of the stage's k-rows) per stage
@@ -2046,7 +2130,7 @@ struct TgParams {
                         //   dotted with vb
 };
 
-template <class C, class D, int CS>
+template <class C, class D, int CS, bool RAG = false>
 __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) {
   const TnParams& p = q.tn;
   __shared__ __attribute__((aligned(16))) unsigned char lds[D::STAGES * D::STAGE_BYTES];
@@ -2176,9 +2260,17 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
     auto cmp = [&](const unsigned char* stage, f32x16_t (&a)[C::MI][C::NI]) {
       tn_compute<C, D, CS>(stage, a, keep);
     };
-    mainloop_tn<C, D>(p, mt, nt, k_begin, k_end, lds, acc, hook, cmp);
+    if constexpr (RAG)
+      mainloop_tn_samples<C, D>(p, mt, nt, k_begin, k_end, q.T, static_cast<int>(q.T_rows), lds,
+                                acc, hook, cmp);
+    else
+      mainloop_tn<C, D>(p, mt, nt, k_begin, k_end, lds, acc, hook, cmp);
   } else {
-    mainloop_tn<C, D>(p, mt, nt, k_begin, k_end, lds, acc, hook);
+    if constexpr (RAG)
+      mainloop_tn_samples<C, D>(p, mt, nt, k_begin, k_end, q.T, static_cast<int>(q.T_rows), lds,
+                                acc, hook, TnPlainCompute<C, D>{});
+    else
+      mainloop_tn<C, D>(p, mt, nt, k_begin, k_end, lds, acc, hook);
   }
   if (k_end < (sample + 1) * q.T && k_end > sample * q.T) flush(false);  // ends inside a sample
   GemmParams e{};
@@ -3432,12 +3524,13 @@ struct TgPlan {
   int64_t m_tiles, n_tiles, bias;  // bias: the bias terms are wanted
   int bias_a;                // the bias terms are A's column sums (d_in wide), not G's
   int64_t bias_d;            // features of the bias side
+  int64_t Tp;                // T padded to whole stages
   int wide;                  // train rows in 256 x 256 tiles (TnCW), else 128 x 128 (TnC)
   int wm, wn;                // waves of a tile along M and N
 };
 bool tg_ok(int dtype, int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
            int semantics) {
-  if (dtype != GS_DTYPE_BF16 || n_val <= 0 || n_val >= N || T % TnD::KB != 0) return false;
+  if (dtype != GS_DTYPE_BF16 || n_val <= 0 || n_val >= N) return false;
   if (semantics != GS_SEM_PAIRWISE_SUM && semantics != GS_SEM_PRESUM) return false;
   if (!val_tn(dtype, n_val, T, d_in, d_out, semantics == GS_SEM_PRESUM)) return false;
   return tn_ok(nullptr, d_out, nullptr, d_in, N * T, d_out, d_in);
@@ -3452,7 +3545,8 @@ TgPlan plan_tg(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
   t.vk = (t.presum ? 1 : n_val) * T;
   t.n_val = n_val;
   t.n_t = N - n_val;
-  t.K = t.n_t * T;
+  t.Tp = ceil_div(T, static_cast<int64_t>(TnD::KB)) * TnD::KB;
+  t.K = t.n_t * t.Tp;
   // The train rows' GEMM in 256 x 256 tiles of 8 waves of 128 x 64 (a quarter fewer LDS
   // fragment bytes per flop than 64 x 64 wave tiles, half the stage bytes; one workgroup per
   // CU), unsplit, when those tiles alone cover 7/8 of the CUs or more (the Pythia-1B MLP and
@@ -3475,10 +3569,33 @@ TgPlan plan_tg(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
     t.kper = tn_kper(t.K, tn_splits(t.K, d_out, d_in));
   }
   // Splits at least one sample long (a sample then meets at most two splits).
-  if (t.kper < T) t.kper = T;
+  if (t.kper < t.Tp) t.kper = t.Tp;
   t.sp = ceil_div(t.K, t.kper);
   t.bias = bias ? 1 : 0;
   return t;
+}
+// Whether the fused pass (V GEMM, the train rows' GEMM with each sample padded to whole stages)
+// beats the dots by `algo` and the train gradient apart.  Estimated times in us.  Measured, one
+// layer's hook with a bias, fused / apart: 16 + 4 samples of 768 x 3072 at T = 1: 57 / 106, 32:
+// 56 / 127, 129: 57 / 149, 500: 94 / 203; 200 + 16 samples of 1024 x 1024 at T = 1: 64 / 97 (64
+// padded rows to every real one); 13 + 3 of 768 x 2304 at T = 777: 86 / 162.
+bool layer_pass_pays(int algo, int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
+                     int semantics, int with_bias) {
+  const int64_t n_t = N - n_val, nv = semantics == GS_SEM_PRESUM ? 1 : n_val;
+  const double area = static_cast<double>(pair_tiles(d_in, d_out)) * TnC::BM * TnC::BN;
+  const int64_t Tp = ceil_div(T, static_cast<int64_t>(TnD::KB)) * TnD::KB;
+  auto gemm = [&](double rows) { return 2e-6 * rows * area / 0.8e9; };
+  const double fused = 25.0 + gemm(static_cast<double>(nv) * T) + gemm(static_cast<double>(n_t) * Tp);
+  const double grad = 10.0 + gemm(static_cast<double>(n_t) * T) + (with_bias ? 15.0 : 0.0);
+  double dots;
+  if (algo == GS_ALGO_GHOST) {
+    const double tiles = static_cast<double>(ceil_div(nv * T, int64_t{StashCfg::BM})) *
+                         ceil_div(n_t * T, int64_t{StashCfg::BN});
+    dots = 6.0 + std::ceil(tiles / 256.0) * 0.024 * (d_in + d_out);
+  } else {
+    dots = 15.0 + gemm(static_cast<double>(nv) * T) + gemm(static_cast<double>(n_t) * T);
+  }
+  return fused <= dots + grad;
 }
 struct TgBufs {
   uint16_t *abar, *gbar, *V;
@@ -3501,9 +3618,9 @@ TgBufs carve_tg(S& c, const TgPlan& t, int64_t T, int64_t d_in, int64_t d_out) {
       t.presum ? presum_rows(T) : tn_vsum_rows(t.vk, d_in, d_out, !t.bias_a);
   b.vp = t.bias ? c.template take<float>(vp_rows * t.bias_d) : nullptr;
   b.pdot = c.template take<float>(t.m_tiles * t.n_tiles * (t.wm * t.wn) * 2 * t.n_t);
-  b.csum = t.bias ? c.template take<float>(t.n_t * 2 * (T / TnD::KB) * t.bias_d) : nullptr;
+  b.csum = t.bias ? c.template take<float>(t.n_t * 2 * (t.Tp / TnD::KB) * t.bias_d) : nullptr;
   const int64_t bw = t.bias_a ? t.n_tiles * t.wn : t.m_tiles * t.wm;
-  b.pbias = t.bias ? c.template take<float>(t.n_t * (T / TnD::KB) * bw) : nullptr;
+  b.pbias = t.bias ? c.template take<float>(t.n_t * (t.Tp / TnD::KB) * bw) : nullptr;
   b.tgpart = c.template take<float>(t.sp * d_out * d_in);
   return b;
 }
@@ -3513,8 +3630,9 @@ TgBufs carve_tg(S& c, const TgPlan& t, int64_t T, int64_t d_in, int64_t d_out) {
 namespace gs {
 namespace {
 size_t tg_workspace(int dtype, int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
-                    int semantics, bool bias, bool bias_a) {
+                    int semantics, bool bias, bool bias_a, bool any_T = false) {
   if (N <= 0 || T <= 0 || d_in <= 0 || d_out <= 0) return 0;
+  if (T % TnD::KB != 0 && !any_T) return 0;
   if (!tg_ok(dtype, N, n_val, T, d_in, d_out, semantics)) return 0;
   const TgPlan t = plan_tg(N, n_val, T, d_in, d_out, semantics, bias, bias_a);
   Sizer sz;
@@ -3541,14 +3659,16 @@ extern "C" size_t gs_conv1d_dot_train_grad_workspace(int dtype, int64_t N, int64
 
 namespace gs {
 namespace {
-// The fused pass (gs_linear_dot_train_grad); bias_a: the bias terms are A's column sums.
-int dot_train_grad(bool bias_a, const void* A, const void* G, int dtype, int64_t N,
-                   int64_t n_val, int64_t val_start, int64_t T, int64_t d_in, int64_t d_out,
-                   int semantics, float* out_dot, void* out_grad, int grad_dtype,
-                   float grad_scale, float* out_bias_dot, void* out_bias_grad,
-                   int bias_grad_dtype, float bias_grad_scale, void* workspace,
-                   size_t workspace_bytes, void* stream) {
-  const std::string who = bias_a ? "gs_conv1d_dot_train_grad" : "gs_linear_dot_train_grad";
+// The fused pass; bias_a: the bias terms are A's column sums; any_T: T need not be a multiple
+// of the stage height.
+int dot_train_grad(const char* name, bool bias_a, bool any_T, const void* A, const void* G,
+                   int dtype, int64_t N, int64_t n_val, int64_t val_start, int64_t T,
+                   int64_t d_in, int64_t d_out, int semantics, void* out_dot, int dot_dtype,
+                   void* out_grad, int grad_dtype, float grad_scale, void* out_bias_dot,
+                   int bias_dot_dtype, void* out_bias_grad, int bias_grad_dtype,
+                   float bias_grad_scale, void* workspace, size_t workspace_bytes,
+                   void* stream) {
+  const std::string who = name;
   if (N <= 0 || T <= 0 || d_in <= 0 || d_out <= 0 || n_val <= 0 || n_val >= N)
     return fail(GS_ERR_INVALID, who + ": invalid shape");
   if (val_start < 0 || val_start + n_val > N)
@@ -3557,19 +3677,25 @@ int dot_train_grad(bool bias_a, const void* A, const void* G, int dtype, int64_t
     return fail(GS_ERR_INVALID, who + ": null pointer");
   if (semantics != GS_SEM_PAIRWISE_SUM && semantics != GS_SEM_PRESUM)
     return fail(GS_ERR_INVALID, who + ": invalid semantics");
-  if ((out_grad != nullptr && grad_dtype != GS_DTYPE_BF16 && grad_dtype != GS_DTYPE_F32) ||
-      (out_bias_grad != nullptr && bias_grad_dtype != GS_DTYPE_BF16 &&
-       bias_grad_dtype != GS_DTYPE_F32))
+  auto grad_ok = [](const void* out, int dt) {
+    return out == nullptr || dt == GS_DTYPE_BF16 || dt == GS_DTYPE_F32;
+  };
+  if (!grad_ok(out_grad, grad_dtype) || !grad_ok(out_bias_grad, bias_grad_dtype))
     return fail(GS_ERR_DTYPE, who + ": gradient dtypes must be bf16 or fp32");
-  if (!tg_ok(dtype, N, n_val, T, d_in, d_out, semantics) || !aligned16(A) || !aligned16(G))
+  if (!grad_ok(out_dot, dot_dtype) || !grad_ok(out_bias_dot, bias_dot_dtype))
+    return fail(GS_ERR_DTYPE, who + ": dot dtypes must be bf16 or fp32");
+  const bool rag = T % TnD::KB != 0;
+  if ((rag && !any_T) || !tg_ok(dtype, N, n_val, T, d_in, d_out, semantics) || !aligned16(A) ||
+      !aligned16(G))
     return fail(GS_ERR_UNSUPPORTED,
-                who + ": needs bf16, 16-byte aligned operands below 2 GiB, "
-                "T a multiple of 64 and feature counts that are multiples of 8");
+                who + ": needs bf16, 16-byte aligned operands below 2 GiB, " +
+                (any_T ? "" : "T a multiple of 64 ") +
+                "and feature counts that are multiples of 8");
   const bool bias = out_bias_dot != nullptr || out_bias_grad != nullptr;
   const TgPlan t = plan_tg(N, n_val, T, d_in, d_out, semantics, bias, bias_a);
   if (workspace == nullptr ||
-      workspace_bytes < tg_workspace(dtype, N, n_val, T, d_in, d_out, semantics, bias, bias_a) -
-                            256)
+      workspace_bytes < tg_workspace(dtype, N, n_val, T, d_in, d_out, semantics, bias, bias_a,
+                                     any_T) - 256)
     return fail(GS_ERR_WORKSPACE, who + ": workspace too small");
   Carver cv(workspace, workspace_bytes);
   const TgBufs b = carve_tg(cv, t, T, d_in, d_out);
@@ -3615,8 +3741,8 @@ int dot_train_grad(bool bias_a, const void* A, const void* G, int dtype, int64_t
   p.ldr = d_in;
   p.l_nbytes = N * T * d_out * 2;
   p.r_nbytes = N * T * d_in * 2;
-  p.gap_at = val_start * T < t.K ? val_start * T : INT64_MAX;
-  p.gap = p.gap_at < t.K ? n_val * T : 0;
+  p.gap_at = val_start < t.n_t ? val_start * T : INT64_MAX;
+  p.gap = val_start < t.n_t ? n_val * T : 0;
   p.K = t.K;
   p.kper = t.kper;
   p.M = d_out;
@@ -3627,7 +3753,8 @@ int dot_train_grad(bool bias_a, const void* A, const void* G, int dtype, int64_t
   p.part_out = 1;
   p.alpha = 1.f;
   q.Vt = b.V;
-  q.T = T;
+  q.T = t.Tp;
+  q.T_rows = T;
   q.n_t = t.n_t;
   q.pdot = b.pdot;
   q.csum = b.csum;
@@ -3637,26 +3764,30 @@ int dot_train_grad(bool bias_a, const void* A, const void* G, int dtype, int64_t
   if (items > INT32_MAX) return fail(GS_ERR_UNSUPPORTED, "GEMM grid too large");
   const dim3 tg_grid(static_cast<unsigned>(items));
   const int cs = q.csum == nullptr ? 0 : (t.bias_a ? 2 : 1);
-  if (t.wide) {
+  auto go = [&](auto wide, auto csk, auto ragged) {
+    constexpr bool W = decltype(wide)::value;
+    using C = std::conditional_t<W, TnCW, TnC>;
+    using D = std::conditional_t<W, TnDW, TnD>;
+    hipLaunchKernelGGL((tgdot_kernel<C, D, decltype(csk)::value, decltype(ragged)::value>),
+                       tg_grid, dim3(C::NT), 0, s, q);
+  };
+  auto go_cs = [&](auto wide, auto ragged) {
     if (cs == 0)
-      hipLaunchKernelGGL((tgdot_kernel<TnCW, TnDW, 0>), tg_grid, dim3(TnCW::NT), 0, s, q);
+      go(wide, std::integral_constant<int, 0>{}, ragged);
     else if (cs == 1)
-      hipLaunchKernelGGL((tgdot_kernel<TnCW, TnDW, 1>), tg_grid, dim3(TnCW::NT), 0, s, q);
+      go(wide, std::integral_constant<int, 1>{}, ragged);
     else
-      hipLaunchKernelGGL((tgdot_kernel<TnCW, TnDW, 2>), tg_grid, dim3(TnCW::NT), 0, s, q);
-  } else {
-    if (cs == 0)
-      hipLaunchKernelGGL((tgdot_kernel<TnC, TnD, 0>), tg_grid, dim3(TnC::NT), 0, s, q);
-    else if (cs == 1)
-      hipLaunchKernelGGL((tgdot_kernel<TnC, TnD, 1>), tg_grid, dim3(TnC::NT), 0, s, q);
-    else
-      hipLaunchKernelGGL((tgdot_kernel<TnC, TnD, 2>), tg_grid, dim3(TnC::NT), 0, s, q);
-  }
+      go(wide, std::integral_constant<int, 2>{}, ragged);
+  };
+  if (t.wide)
+    rag ? go_cs(std::true_type{}, std::true_type{}) : go_cs(std::true_type{}, std::false_type{});
+  else
+    rag ? go_cs(std::false_type{}, std::true_type{}) : go_cs(std::false_type{}, std::false_type{});
   rc = check_launch("tgdot_kernel");
   if (rc) return rc;
   // One launch: the dots, the bias train gradient and the train-gradient reduction.
   const int64_t shares = t.m_tiles * t.n_tiles * (t.wm * t.wn) * 2;
-  const int64_t sps = T / TnD::KB;
+  const int64_t sps = t.Tp / TnD::KB;
   const int64_t bshares = sps * (t.bias_a ? t.n_tiles * t.wn : t.m_tiles * t.wm);
   const float* pbias = out_bias_dot != nullptr ? b.pbias : nullptr;
   const int64_t gblocks =
@@ -3664,16 +3795,17 @@ int dot_train_grad(bool bias_a, const void* A, const void* G, int dtype, int64_t
   const int64_t count = out_grad != nullptr ? d_out * d_in : 0;  // a multiple of 8
   const dim3 grid(static_cast<unsigned>(t.n_t + gblocks + ceil_div(count / 4, int64_t{256})));
   const int gf32 = grad_dtype == GS_DTYPE_F32 ? 1 : 0;
+  const int df32 = dot_dtype == GS_DTYPE_F32 ? 1 : 0, bf32 = bias_dot_dtype == GS_DTYPE_F32 ? 1 : 0;
   if (bias_grad_dtype == GS_DTYPE_F32)
     hipLaunchKernelGGL(tgdot_finish_kernel<float>, grid, dim3(256), 0, s, b.pdot, shares, t.n_t,
-                       pbias, bshares, b.csum, 2 * sps, t.bias_d, out_dot, out_bias_dot,
+                       pbias, bshares, b.csum, 2 * sps, t.bias_d, out_dot, df32, out_bias_dot, bf32,
                        static_cast<float*>(out_bias_grad), bias_grad_scale, gblocks, b.tgpart,
                        count, static_cast<int>(t.sp), out_grad, grad_scale, gf32);
   else
     hipLaunchKernelGGL(tgdot_finish_kernel<uint16_t>, grid, dim3(256), 0, s, b.pdot, shares,
-                       t.n_t, pbias, bshares, b.csum, 2 * sps, t.bias_d, out_dot, out_bias_dot,
-                       static_cast<uint16_t*>(out_bias_grad), bias_grad_scale, gblocks,
-                       b.tgpart, count, static_cast<int>(t.sp), out_grad, grad_scale, gf32);
+                       t.n_t, pbias, bshares, b.csum, 2 * sps, t.bias_d, out_dot, df32,
+                       out_bias_dot, bf32, static_cast<uint16_t*>(out_bias_grad),
+                       bias_grad_scale, gblocks, b.tgpart, count, static_cast<int>(t.sp), out_grad, grad_scale, gf32);
   return check_launch("tgdot_finish_kernel");
 }
 }  // namespace
@@ -3687,8 +3819,9 @@ extern "C" int gs_linear_dot_train_grad(const void* A, const void* G, int dtype,
                                         void* out_bias_grad, int bias_grad_dtype,
                                         float bias_grad_scale, void* workspace,
                                         size_t workspace_bytes, void* stream) {
-  return dot_train_grad(false, A, G, dtype, N, n_val, val_start, T, d_in, d_out, semantics,
-                        out_dot, out_grad, grad_dtype, grad_scale, out_bias_dot, out_bias_grad,
+  return dot_train_grad("gs_linear_dot_train_grad", false, false, A, G, dtype, N, n_val,
+                        val_start, T, d_in, d_out, semantics, out_dot, GS_DTYPE_F32, out_grad,
+                        grad_dtype, grad_scale, out_bias_dot, GS_DTYPE_F32, out_bias_grad,
                         bias_grad_dtype, bias_grad_scale, workspace, workspace_bytes, stream);
 }
 
@@ -3700,9 +3833,42 @@ extern "C" int gs_conv1d_dot_train_grad(const void* A, const void* G, int dtype,
                                         void* out_bias_grad, int bias_grad_dtype,
                                         float bias_grad_scale, void* workspace,
                                         size_t workspace_bytes, void* stream) {
-  return dot_train_grad(true, G, A, dtype, N, n_val, val_start, T, d_out, d_in, semantics,
-                        out_dot, out_grad, grad_dtype, grad_scale, out_bias_dot, out_bias_grad,
-                        bias_grad_dtype, bias_grad_scale, workspace, workspace_bytes, stream);
+  return dot_train_grad("gs_conv1d_dot_train_grad", true, false, G, A, dtype, N, n_val, val_start,
+                        T, d_out, d_in, semantics, out_dot, GS_DTYPE_F32, out_grad, grad_dtype,
+                        grad_scale, out_bias_dot, GS_DTYPE_F32, out_bias_grad, bias_grad_dtype,
+                        bias_grad_scale, workspace, workspace_bytes, stream);
+}
+
+// The whole layer: any T, either weight layout, the dots in the dtypes asked for.
+extern "C" size_t gs_linear_layer_pass_workspace(int dtype, int64_t N, int64_t n_val, int64_t T,
+                                                 int64_t d_in, int64_t d_out, int semantics,
+                                                 int conv1d, int with_bias, int algo,
+                                                 int rounding) {
+  if (!linear_args_ok(dtype, N, n_val, T, d_in, d_out, semantics, algo, 0)) return 0;
+  if (algo == GS_ALGO_GHOST || !tg_ok(dtype, N, n_val, T, d_in, d_out, semantics)) return 0;
+  const LinearPlan pl = plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, 0);
+  if (pl.algo == GS_ALGO_GHOST && rounding == GS_ROUND_REF_BF16) return 0;
+  if (!layer_pass_pays(pl.algo, N, n_val, T, d_in, d_out, semantics, with_bias)) return 0;
+  return conv1d ? tg_workspace(dtype, N, n_val, T, d_out, d_in, semantics, with_bias != 0, true,
+                               true)
+                : tg_workspace(dtype, N, n_val, T, d_in, d_out, semantics, with_bias != 0, false,
+                               true);
+}
+
+extern "C" int gs_linear_layer_pass(const void* A, const void* G, int dtype, int64_t N,
+                                    int64_t n_val, int64_t val_start, int64_t T, int64_t d_in,
+                                    int64_t d_out, int semantics, int conv1d, void* out_dot,
+                                    int dot_dtype, void* out_grad, int grad_dtype,
+                                    float grad_scale, void* out_bias_dot, int bias_dot_dtype,
+                                    void* out_bias_grad, int bias_grad_dtype,
+                                    float bias_grad_scale, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+  const bool cv = conv1d != 0;
+  return dot_train_grad("gs_linear_layer_pass", cv, true, cv ? G : A, cv ? A : G, dtype, N, n_val,
+                        val_start, T, cv ? d_out : d_in, cv ? d_in : d_out, semantics, out_dot,
+                        dot_dtype, out_grad, grad_dtype, grad_scale, out_bias_dot,
+                        bias_dot_dtype, out_bias_grad, bias_grad_dtype, bias_grad_scale,
+                        workspace, workspace_bytes, stream);
 }
 
 extern "C" size_t gs_linear_rowdot_workspace(int dtype, int64_t N, int64_t n_val, int64_t T,

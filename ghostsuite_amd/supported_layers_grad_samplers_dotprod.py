@@ -119,7 +119,7 @@ def _dot_dtype(x: torch.Tensor, pairwise: bool) -> torch.dtype:
 def _reference_dtypes(layer: nn.Module, weight_dtype: Optional[torch.dtype],
                       bias_dtype: Optional[torch.dtype]) -> None:
     """Casts the dots the sampler set to the dtypes the reference's sampler returns (a None
-    dtype: left fp32).  Its materialised branches and bias dots are einsums over operands in
+    dtype: left fp32; nothing where the kernels already wrote them so).  Its materialised branches and bias dots are einsums over operands in
     the layer's dtype (Linear :131-146 in the original dtype, Conv1D :445-471 and Conv2d
     :552-559 in bf16); its ghost branches sum in fp32 (:129-130, :437, :550)."""
     if options["dot_dtypes"] != "reference" or options["precision"] == "fp32":
@@ -130,6 +130,16 @@ def _reference_dtypes(layer: nn.Module, weight_dtype: Optional[torch.dtype],
         dot = param.__dict__.get("grad_dot_prod")
         if dot is not None and dot.dtype != dt:
             param.grad_dot_prod = dot.to(dt)
+
+
+def _dot_result_dtypes(layer: nn.Module, A: torch.Tensor, B: torch.Tensor, conv1d: bool):
+    """The dtypes _reference_dtypes gives a Linear (Conv1D) layer's weight and bias dots, for
+    kernels that write them directly."""
+    if options["dot_dtypes"] != "reference" or options["precision"] == "fp32":
+        return torch.float32, torch.float32
+    weight = torch.float32 if layer.use_ghost_computation else \
+        torch.bfloat16 if conv1d else A.dtype
+    return weight, torch.bfloat16 if conv1d else B.dtype
 
 
 def _overwritten_later(layer: nn.Module) -> bool:
@@ -225,12 +235,12 @@ def _fused_dot_train_grad(layer: nn.Module, A: torch.Tensor, B: torch.Tensor,
                           conv1d: bool = False) -> bool:
     """Weight dot and weight train gradient (and with a bias its dot and train gradient) from
     one K-major pass over the train rows: per train row, sum_t g^T V a = <V, G_i^T A_i>, and
-    the train gradient is the sum of the same G_i^T A_i (gs_linear_dot_train_grad).  Taken
-    for bf16 layers on the val-gradient algorithm whose weight trains; the train gradients
-    are parked for _apply_train_grad.  Returns False when the other paths must run.
+    the train gradient is the sum of the same G_i^T A_i (gs_linear_layer_pass).  Taken for
+    bf16 layers whose weight trains, unless linear_algo is 'ghost' or the separate passes are
+    estimated to be faster; the train gradients are parked for _apply_train_grad.  Returns
+    False when the other paths must run.
 
-    With ``conv1d`` (HF Conv1D, weight [d_in, d_out]) the Conv1D entry point runs the same
-    pass with the operands swapped: the dot <G_i^T A_i, V> equals <A_i^T G_i, V^T>, the train
+    With ``conv1d`` (HF Conv1D, weight [d_in, d_out]) the kernels run the same pass with the operands swapped: the dot <G_i^T A_i, V> equals <A_i^T G_i, V^T>, the train
     gradient comes out as the sum of A_i^T G_i (the Conv1D layout), and the bias terms come
     from the column sums of G as for a Linear layer."""
     scale = getattr(layer, "_gs_bias_grad_scale", None)
@@ -244,17 +254,27 @@ def _fused_dot_train_grad(layer: nn.Module, A: torch.Tensor, B: torch.Tensor,
                        not getattr(layer.bias, "initially_requires_grad", False))):
         return False
     Bc = B.to(dtype) if B.dtype != dtype else B
-    N, d_in, d_out = A.shape[0], A.shape[-1], Bc.shape[-1]
-    T = A.numel() // (N * d_in)
     sem = _native.SEM_PAIRWISE_SUM if pairwise else _native.SEM_PRESUM
-    if ops().linear_algo(dtype, N, val_batch_size, T, d_in, d_out, sem,
-                         _ALGOS[options["linear_algo"]], False) != _native.ALGO_VALGRAD:
-        return False
-    res = ops().linear_dot_train_grad(A, Bc, val_batch_size, semantics=sem, grad_scale=scale,
-                                      grad_dtype=layer.weight.dtype, bias=bias,
-                                      bias_grad_scale=scale,
-                                      bias_grad_dtype=layer.bias.dtype if bias else None,
-                                      conv1d=conv1d)
+    algo = _ALGOS[options["linear_algo"]]
+    layer_pass = getattr(ops(), "linear_layer_pass", None)
+    if layer_pass is not None:
+        weight_dt, bias_dt = _dot_result_dtypes(layer, A, B, conv1d)
+        res = layer_pass(A, Bc, val_batch_size, semantics=sem, algo=algo,
+                         rounding=_ROUNDINGS[options["rounding"]], conv1d=conv1d,
+                         grad_scale=scale, grad_dtype=layer.weight.dtype, dot_dtype=weight_dt,
+                         bias_grad_dtype=layer.bias.dtype if bias else None,
+                         bias_dot_dtype=bias_dt)
+    else:   # a kernel layer without the whole-layer pass
+        N, d_in, d_out = A.shape[0], A.shape[-1], Bc.shape[-1]
+        T = A.numel() // (N * d_in)
+        if ops().linear_algo(dtype, N, val_batch_size, T, d_in, d_out, sem, algo,
+                             False) != _native.ALGO_VALGRAD:
+            return False
+        res = ops().linear_dot_train_grad(A, Bc, val_batch_size, semantics=sem,
+                                          grad_scale=scale, grad_dtype=layer.weight.dtype,
+                                          bias=bias, bias_grad_scale=scale,
+                                          bias_grad_dtype=layer.bias.dtype if bias else None,
+                                          conv1d=conv1d)
     if res is None:
         return False
     dot, grad, bias_dot, bias_grad = res

@@ -507,6 +507,93 @@ def test_linear_dot_train_grad_declines(gpu):
 
 
 @pytest.mark.parametrize("case", [
+    # N, n_val, T, d_in, d_out, semantics, val position, bias, conv1d: T on both sides of the
+    # 64-row stage, the val block first, inside and last, one train sample, splits inside
+    # samples, and 256 x 256 tiles
+    (6, 2, 63, 40, 24, "pairwise", "last", True, False),
+    (6, 2, 65, 40, 24, "presum", "mid", True, False),
+    (5, 1, 1, 136, 264, "pairwise", "first", True, False),
+    (3, 2, 100, 16, 8, "pairwise", "mid", False, False),
+    (16, 3, 777, 768, 264, "presum", "first", True, False),
+    (16, 3, 129, 264, 768, "presum", "mid", True, True),
+    (9, 2, 200, 512, 512, "pairwise", "mid", True, False),
+    (4, 1, 70, 2000, 7176, "pairwise", "mid", True, False),
+    (4, 1, 70, 2000, 7176, "presum", "first", True, True),
+    (6, 2, 128, 136, 264, "presum", "last", True, True),   # whole stages
+])
+def test_linear_layer_pass_any_length(gpu, case):
+    """gs_linear_layer_pass at any T, both weight layouts, fp32 and bf16 dots, against float64:
+    the dots through the val-term form at the kernel's rounding points (beyond them the sums
+    are fp32), the train gradients as closed forms; a bf16 dot is the fp32 one rounded once.
+    A NaN in one train sample stays in its own dot, though its rows follow another sample's
+    padded end."""
+    N, n_val, T, d_in, d_out, sem, pos, bias, conv1d = case
+    vs = {"last": N - n_val, "first": 0, "mid": 1}[pos]
+    n_t = N - n_val
+    print(f"layer pass case={case}", flush=True)
+    A = randn((N, T, d_in), 210 + T, 1.0, torch.bfloat16)
+    G = randn((N, T, d_out), 211 + T, 1e-3, torch.bfloat16)
+    semantics = _native.SEM_PAIRWISE_SUM if sem == "pairwise" else _native.SEM_PRESUM
+
+    def run(a, dot_dtype):
+        return _native.ops().linear_layer_pass(
+            a.to(gpu), G.to(gpu), n_val, semantics=semantics, algo=_native.ALGO_VALGRAD,
+            rounding=_native.ROUND_FP32, conv1d=conv1d, grad_scale=1.5 / n_t,
+            grad_dtype=torch.float32, dot_dtype=dot_dtype,
+            bias_grad_dtype=torch.float32 if bias else None, bias_dot_dtype=dot_dtype,
+            val_start=vs)
+    res = run(A, torch.float32)
+    if res is None:      # padding to whole stages costs more than the separate passes
+        assert T < 64
+        return
+    dot, grad, bdot, bgrad = res
+    Ad, Gd = A.to(gpu), G.to(gpu)
+    want = R.linear_dot_valterm_exact(Ad, Gd, n_val, sem, val_start=vs,
+                                      round_dtype=torch.bfloat16).cpu()
+    # entries of V (and of the presums) on the other side of a rounding tie: 2^-8 of a share of
+    # the entries, independent in sign; 5e-3 of the rms bounds them for the smallest case
+    assert_close(dot.cpu(), want, 5e-3, "weight dot")
+    assert_close(grad.cpu(), _train_grad_want(A, G, n_val, vs, 1.5 / n_t, conv1d, gpu),
+                 FP32_TOL, "weight train grad")
+    if bias:
+        assert_close(bdot.cpu(), R.bias_dot_exact(G, n_val, vs), FP32_TOL, "bias dot")
+        tr, _ = R.split_rows(G.double(), n_val, vs)
+        assert_close(bgrad.cpu(), tr.sum((0, 1)) * (1.5 / n_t), FP32_TOL, "bias train grad")
+    low = run(A, torch.bfloat16)
+    assert torch.equal(low[0], dot.bfloat16()) and torch.equal(low[1], grad)
+    if bias:
+        assert torch.equal(low[2], bdot.bfloat16())
+    # one train sample's NaN stays in its own dot (its first row follows another's last row)
+    if n_t > 1 and T > 1:
+        bad = A.clone()
+        rows = [i for i in range(N) if not vs <= i < vs + n_val]
+        bad[rows[1], 0] = float("nan")
+        dn = run(bad, torch.float32)[0].cpu()
+        assert torch.isnan(dn[1]) and torch.equal(dn[0], dot.cpu()[0])
+
+
+def test_linear_layer_pass_declines(gpu):
+    """Unaligned feature counts, fp32 operands, the ghost algorithm, and the automatic choice of
+    the ghost kernel with the reference's rounding keep the separate passes."""
+    def taken(A, G, algo=_native.ALGO_AUTO, rounding=_native.ROUND_FP32):
+        return _native.ops().linear_layer_pass(
+            A.to(gpu), G.to(gpu), 2, semantics=_native.SEM_PAIRWISE_SUM, algo=algo,
+            rounding=rounding, conv1d=False, grad_scale=1.0, grad_dtype=torch.float32,
+            dot_dtype=torch.float32) is not None
+    A, G = _inputs(6, 100, 64, 256, 5, torch.bfloat16)
+    assert taken(A, G) and taken(A, G, _native.ALGO_VALGRAD)
+    assert not taken(A, G, _native.ALGO_GHOST)
+    A, G = _inputs(6, 100, 12, 256, 6, torch.bfloat16)
+    assert not taken(A, G)
+    A, G = _inputs(6, 64, 64, 256, 7, torch.float32)
+    assert not taken(A, G)
+    A, G = _inputs(6, 64, 2048, 2048, 8, torch.bfloat16)
+    assert _native.ops().linear_algo(torch.bfloat16, 6, 2, 64, 2048, 2048, 0, 0,
+                                     False) == _native.ALGO_GHOST
+    assert not taken(A, G, rounding=_native.ROUND_REF_BF16)
+
+
+@pytest.mark.parametrize("case", [
     # N, n_val, T, d_in, d_out
     (6, 2, 128, 136, 264),
     (20, 4, 1024, 768, 3072),    # GPT-2-small mlp.c_fc
