@@ -5,14 +5,16 @@
 // Projections with more than 64 rows on a side run as several launches over 64-row slices of
 // the projection matrices, each writing its block of the [kL, kR] partials.
 //
-// One workgroup takes one sample and a chunk of 64 tokens; its 8 waves take interleaved
-// 32-feature pieces of all 64 token rows (so the workgroup reads 256 contiguous features of
-// every row at a time).  A wave streams its pieces of the G and A rows straight from HBM
-// into MFMA operands (v_mfma_f32_16x16x32_bf16 / v_mfma_f32_16x16x4f32) against the
-// projection rows (small, L2-resident), each projection fragment serving the 4 sixteen-row
-// groups, so G and A are read exactly once.  The wave shares (fp32) are summed in LDS, the
-// 64-token outer-product sum is formed there, and the per-chunk partials are reduced per
-// sample in a fixed order.
+// One workgroup takes one sample and a chunk of 32 tokens; its 8 waves take interleaved
+// pieces of 128 bytes of every token row.  A wave streams its pieces of the G and A rows straight
+// from HBM into MFMA operands (v_mfma_f32_16x16x32_bf16 / v_mfma_f32_16x16x4f32) against the
+// projection rows (small, L2-resident), the next piece's rows in flight while the current one is
+// multiplied, so G and A are read exactly once.  The wave shares (fp32) are summed in LDS, the
+// chunk's outer-product sum is formed there with fp32 MFMAs, and the per-chunk partials are
+// reduced per sample in a fixed order.  Bound by HBM: 32 x 1024 tokens of 1024 + 4096
+// bf16 features at 16 x 16 projection rows take 67 us (5.0 TB/s, a 1 GiB copy 5.1; 75 us when
+// all waves loaded, multiplied and waited in step), of 1024 + 3072 at 39 x 13 54 us (113 us with
+// both sides padded to 64 rows and 133 KiB of LDS).
 //
 // 16x16 MFMA layout: lane l supplies row (l % 16) of A and column (l % 16) of B with its
 // k-slice chosen by l / 16; result element e of lane l is C[4*(l/16) + e][l % 16].
@@ -29,8 +31,10 @@ namespace gs {
 typedef __bf16 bf16x8p_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int PJ_TOK = 64;  // tokens per workgroup
+constexpr int PJ_TOK = 32;      // tokens per workgroup
+constexpr int PJ_TG = PJ_TOK / 16;  // its 16-token MFMA row groups
 constexpr int PJ_THREADS = 512;
+constexpr int PJ_WAVES = PJ_THREADS / 64;
 constexpr int PJ_KMAX = 64;     // projection rows per side of one launch
 
 struct PjBF16 {
@@ -58,64 +62,102 @@ struct PjF32 {
   }
 };
 
-// Loads 16 bytes of row `row` starting at element k (zero beyond n or for a null row).
-template <class Tr>
-__device__ __forceinline__ uint4 lane_load(const typename Tr::E* row, int64_t k, int64_t n,
-                                           int vec_ok) {
-  using E = typename Tr::E;
-  union { uint4 v; E e[Tr::VEC]; } u;
-  if (row != nullptr && vec_ok && k + Tr::VEC <= n) {
-    u.v = *reinterpret_cast<const uint4*>(row + k);
-  } else {
-#pragma unroll
-    for (int v = 0; v < Tr::VEC; ++v) u.e[v] = (row != nullptr && k + v < n) ? row[k + v] : E(0);
-  }
-  return u.v;
-}
-
-constexpr int PJ_WAVES = PJ_THREADS / 64;
-constexpr int PJ_TG = PJ_TOK / 16;  // 16-token MFMA row groups per workgroup
-
-// Partial projections over this wave's share of the features of the workgroup's PJ_TOK
-// token rows:
-// acc[tg][nb][e] = sum_f P[16*nb + l%16][f] * row(16*tg + 4*(l/16) + e)[f].  Every projection
-// fragment loaded is used by the PJ_TG row groups (one MFMA each).
-template <class Tr, int NB>
+// One side's partial projections over this wave's share of the features of the chunk's
+// PJ_TOK token rows: acc[tg][nb][e] = sum_f P[16 nb + l%16][f] * row(16 tg + 4 (l/16) + e)[f].
+// A wave takes pieces of 2 KSTEP features (128 bytes of a row), lane group g the g-th 32 bytes
+// of them, in two loads, so that a wave uses whole cache lines; every projection fragment
+// serves the PJ_TG row groups.  `rows` point at valid rows (a token past the end reads another
+// row and is dropped by the caller: an operand row reaches only its own result row), and rows of
+// P past kP repeat its last row (columns nobody reads).  VEC false: rows or projections are
+// not 16-byte aligned, elements are loaded one by one.
+template <class Tr, int NB, bool VEC>
 __device__ __forceinline__ void project_rows(const typename Tr::E* const (&rows)[PJ_TG],
                                              const typename Tr::E* P, int64_t n, int64_t kP,
-                                             int vec_ok, int vec_p, f32x4_t (&acc)[PJ_TG][NB]) {
+                                             f32x4_t (&acc)[PJ_TG][NB]) {
   using E = typename Tr::E;
-  const int lane = threadIdx.x & 63;
-  const int kg = lane >> 4;  // lane group: k-slice selector
-  const E* prow[NB];         // this lane's projection row in each 16-row block
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int64_t koff = (lane >> 4) * 2 * Tr::VEC;  // this lane group's 32 bytes of a piece
+  const E* prow[NB];  // this lane's projection row in each 16-row block
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
-    prow[nb] = 16 * nb + (lane & 15) < kP ? P + static_cast<int64_t>(16 * nb + (lane & 15)) * n
-                                          : nullptr;
-  constexpr int U = 1;  // k-steps of loads in flight (x PJ_TG rows)
-  // The waves interleave in pieces of U k-steps, so a workgroup reads one contiguous run
-  // of PJ_WAVES pieces of every row at a time.
-  const int64_t f_step = static_cast<int64_t>(PJ_WAVES) * U * Tr::KSTEP;
-  for (int64_t f0 = (threadIdx.x >> 6) * U * Tr::KSTEP; f0 < n; f0 += f_step) {
-    uint4 a[U][PJ_TG];
+  for (int nb = 0; nb < NB; ++nb) {
+    const int64_t r = 16 * nb + (lane & 15);
+    prow[nb] = P + (r < kP ? r : kP - 1) * n;
+  }
+  constexpr int64_t PIECE = 2 * Tr::KSTEP, STEP = PJ_WAVES * PIECE;
+  auto fetch = [&](const E* row, int64_t k, bool whole) -> uint4 {
+    if constexpr (VEC) {
+      // Past the end (VEC divides n, so a chunk is wholly inside or outside): a valid address,
+      // then zeros.
+      uint4 v = *reinterpret_cast<const uint4*>(row + (whole || k < n ? k : 0));
+      if (!whole && k >= n) v = make_uint4(0u, 0u, 0u, 0u);
+      return v;
+    } else {
+      union { uint4 v; E e[Tr::VEC]; } u;
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+      for (int i = 0; i < Tr::VEC; ++i) u.e[i] = k + i < n ? row[k + i] : E(0);
+      return u.v;
+    }
+  };
+  auto load_rows = [&](uint4 (&a)[2][PJ_TG], int64_t f0, bool whole) {
 #pragma unroll
-      for (int tg = 0; tg < PJ_TG; ++tg)
-        a[u][tg] = lane_load<Tr>(rows[tg], f0 + u * Tr::KSTEP + kg * Tr::VEC, n, vec_ok);
+    for (int tg = 0; tg < PJ_TG; ++tg)
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t k = f0 + u * Tr::KSTEP + kg * Tr::VEC;
+      for (int u = 0; u < 2; ++u) a[u][tg] = fetch(rows[tg], f0 + koff + u * Tr::VEC, whole);
+  };
+  auto compute = [&](const uint4 (&a)[2][PJ_TG], int64_t f0, bool whole) {
+    uint4 b[2][NB];
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        const uint4 bq = lane_load<Tr>(prow[nb], k, n, vec_p);
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) b[u][nb] = fetch(prow[nb], f0 + koff + u * Tr::VEC, whole);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int tg = 0; tg < PJ_TG; ++tg)
 #pragma unroll
-          for (int s = 0; s < Tr::SUB; ++s) Tr::mma(acc[tg][nb], a[u][tg], bq, s);
-      }
-    }
+          for (int s = 0; s < Tr::SUB; ++s) Tr::mma(acc[tg][nb], a[u][tg], b[u][nb], s);
+  };
+  // Whole steps first, then the wave's piece of the last, partial one; each piece is loaded
+  // before its predecessor is used.  The whole steps start at a different one in every
+  // workgroup: in step, all of them would read the same columns of rows a power of two apart,
+  // which few HBM channels serve (1024 + 4096 features: 75 us
+  // in step, 67 us so).
+  const int64_t whole = n / STEP, f0 = wid * PIECE, tail = f0 + whole * STEP;
+  const bool has_tail = tail < n;
+  const int64_t rot = whole > 0 ? (blockIdx.x + blockIdx.y) % whole : 0;
+  auto at = [&](int64_t i) {
+    const int64_t j = i + rot;
+    return f0 + (j < whole ? j : j - whole) * STEP;
+  };
+  uint4 a0[2][PJ_TG], a1[2][PJ_TG];
+  auto advance = [&]() {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int tg = 0; tg < PJ_TG; ++tg) a0[u][tg] = a1[u][tg];
+  };
+  if (whole > 0)
+    load_rows(a0, at(0), true);
+  else if (has_tail)
+    load_rows(a0, tail, false);
+  int64_t i = 0;
+  for (; i + 2 < whole; i += 2) {
+    load_rows(a1, at(i + 1), true);
+    compute(a0, at(i), true);
+    load_rows(a0, at(i + 2), true);
+    compute(a1, at(i + 1), true);
   }
+  for (; i < whole; ++i) {  // the last one or two
+    if (i + 1 < whole)
+      load_rows(a1, at(i + 1), true);
+    else if (has_tail)
+      load_rows(a1, tail, false);
+    compute(a0, at(i), true);
+    advance();
+  }
+  if (has_tail) compute(a0, tail, false);
 }
 
 // Where a launch writes: its [kL, kR] block of the per-(sample, chunk) partials
@@ -126,92 +168,94 @@ struct PjSlice {
 
 // GATHER: the input side is an embedding, whose "projected input" for token id x is column
 // x of P_i, i.e. row x of R = P_i^T ([vocab, ldr], this launch's kR columns); `ids` replaces A.
-// Workgroup = one sample x PJ_TOK tokens; wave w projects all PJ_TOK token rows over its
-// share of the features, the wave shares are summed in LDS (fixed order), then the
-// PJ_TOK-token outer-product sum is formed.  NB: 16-row projection blocks per side
-// (kL, kR <= 16 * NB).
-template <class Tr, bool GATHER, int NB>
-__global__ void __launch_bounds__(PJ_THREADS) kron_proj_kernel(
+// NL, NR: 16-row projection blocks of the two sides (kL <= 16 NL, kR <= 16 NR); VL, VR:
+// 16-byte aligned rows and projections of the G and A sides (element-wise loads need the
+// registers of two waves per SIMD).
+template <class Tr, bool GATHER, int NL, int NR, bool VL, bool VR>
+__global__ void __launch_bounds__(PJ_THREADS, VL && VR ? 4 : 2) kron_proj_kernel(
     const typename Tr::E* __restrict__ A, const int64_t* __restrict__ ids, int64_t vocab,
     const typename Tr::E* __restrict__ G, int64_t T, int64_t n_a, int64_t n_g,
     const typename Tr::E* __restrict__ R, const typename Tr::E* __restrict__ L, int64_t kR,
-    int64_t kL, int64_t ldr, int vec_a, int vec_g, int vec_r, int vec_l, int64_t chunks,
-    PjSlice sl, float* __restrict__ part) {
+    int64_t kL, int64_t ldr, int64_t chunks, PjSlice sl, float* __restrict__ part) {
   using E = typename Tr::E;
-  constexpr int KM = 16 * NB;  // LDS width: projection rows per side
-  // Wave slices combine in two steps through [PJ_WAVES / 2] slices of LDS.
-  constexpr int HW = PJ_WAVES / 2;
-  __shared__ float sg[HW][PJ_TOK][KM + 1];
-  __shared__ float sa[HW][PJ_TOK][KM + 1];
+  constexpr int TOK = PJ_TOK, TG = PJ_TG, LD = TOK + 4;  // LDS rows: one projection row, its tokens
+  __shared__ __attribute__((aligned(16))) float slice[PJ_WAVES][16][LD];  // one 16-row block
+  __shared__ float fin[(NL + NR) * 16][LD];   // the sums: L's projections, then R's
   const int64_t b = blockIdx.y, c = blockIdx.x;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const E* grows[PJ_TG];
-  const E* arows[PJ_TG];
+  const int64_t t0 = c * TOK;
+  const int nvalid = static_cast<int>(T - t0 < TOK ? T - t0 : TOK);
+  // Sums a block's wave shares in wave order into fin[row0 + 0..15]; tokens past the end get 0.
+  auto combine = [&](const f32x4_t (&acc)[TG], int row0) {
 #pragma unroll
-  for (int tg = 0; tg < PJ_TG; ++tg) {
-    const int64_t t = c * PJ_TOK + tg * 16 + (lane & 15);  // this lane's operand row
-    grows[tg] = t < T ? G + (b * T + t) * n_g : nullptr;
-    arows[tg] = (!GATHER && t < T) ? A + (b * T + t) * n_a : nullptr;
-  }
-  f32x4_t accg[PJ_TG][NB], acca[PJ_TG][NB];
+    for (int tg = 0; tg < TG; ++tg)
+      *reinterpret_cast<f32x4_t*>(&slice[wid][lane & 15][tg * 16 + 4 * (lane >> 4)]) = acc[tg];
+    __syncthreads();
+    for (int x = threadIdx.x; x < 16 * TOK; x += PJ_THREADS) {
+      const int k = x / TOK, tok = x % TOK;
+      float v = slice[0][k][tok];
 #pragma unroll
-  for (int tg = 0; tg < PJ_TG; ++tg)
+      for (int w = 1; w < PJ_WAVES; ++w) v += slice[w][k][tok];
+      fin[row0 + k][tok] = tok < nvalid ? v : 0.f;
+    }
+    __syncthreads();
+  };
+  auto side = [&](const E* X, int64_t n, const E* P, int64_t kP, int row0, auto nbc, auto vec) {
+    constexpr int NB = decltype(nbc)::value;
+    const E* rows[TG];
 #pragma unroll
-    for (int i = 0; i < NB; ++i)
+    for (int tg = 0; tg < TG; ++tg) {
+      const int t = tg * 16 + (lane & 15);  // this lane's operand row
+      rows[tg] = X + (b * T + t0 + (t < nvalid ? t : 0)) * n;
+    }
+    f32x4_t acc[TG][NB];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) accg[tg][i][e] = acca[tg][i][e] = 0.f;
-  project_rows<Tr, NB>(grows, L, n_g, kL, vec_g, vec_l, accg);
-  if constexpr (!GATHER) project_rows<Tr, NB>(arows, R, n_a, kR, vec_a, vec_r, acca);
-  // Waves HW.. park their slices, waves 0..HW-1 add their own, then slice 0 takes the sum
-  // of the HW slices (fixed order); the gather fills slice 0 of sa.
-  auto put = [&](bool add) {
-    const int ws = wid % HW;
-#pragma unroll
-    for (int tg = 0; tg < PJ_TG; ++tg)
+    for (int tg = 0; tg < TG; ++tg)
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int tok = tg * 16 + 4 * (lane >> 4) + e;
-          const int k = nb * 16 + (lane & 15);
-          sg[ws][tok][k] = (add ? sg[ws][tok][k] : 0.f) + accg[tg][nb][e];
-          if constexpr (!GATHER) sa[ws][tok][k] = (add ? sa[ws][tok][k] : 0.f) + acca[tg][nb][e];
-        }
-  };
-  if (wid >= HW) put(false);
-  __syncthreads();
-  if (wid < HW) put(true);
-  __syncthreads();
-  for (int x = threadIdx.x; x < PJ_TOK * KM; x += PJ_THREADS) {
-    const int tok = x / KM, q = x % KM;
-    float g = sg[0][tok][q];
+        for (int e = 0; e < 4; ++e) acc[tg][nb][e] = 0.f;
+    project_rows<Tr, NB, decltype(vec)::value>(rows, P, n, kP, acc);
 #pragma unroll
-    for (int w = 1; w < HW; ++w) g += sg[w][tok][q];
-    sg[0][tok][q] = g;
-    if constexpr (GATHER) {
-      const int64_t tt = c * PJ_TOK + tok;
+    for (int nb = 0; nb < NB; ++nb) {
+      f32x4_t one[TG];
+#pragma unroll
+      for (int tg = 0; tg < TG; ++tg) one[tg] = acc[tg][nb];
+      combine(one, row0 + 16 * nb);
+    }
+  };
+  side(G, n_g, L, kL, 0, std::integral_constant<int, NL>{}, std::integral_constant<bool, VL>{});
+  if constexpr (GATHER) {
+    for (int x = threadIdx.x; x < 16 * NR * TOK; x += PJ_THREADS) {
+      const int q = x % (16 * NR), tok = x / (16 * NR);
       float v = 0.f;
-      if (tt < T && q < kR) {
-        const int64_t id = ids[b * T + tt];
+      if (tok < nvalid && q < kR) {
+        const int64_t id = ids[b * T + t0 + tok];
         if (id >= 0 && id < vocab) v = to_f32<E>(R[id * ldr + q]);
       }
-      sa[0][tok][q] = v;
-    } else {
-      float a = sa[0][tok][q];
-#pragma unroll
-      for (int w = 1; w < HW; ++w) a += sa[w][tok][q];
-      sa[0][tok][q] = a;
+      fin[16 * NL + q][tok] = v;
     }
+    __syncthreads();
+  } else {
+    side(A, n_a, R, kR, 16 * NL, std::integral_constant<int, NR>{},
+         std::integral_constant<bool, VR>{});
   }
-  __syncthreads();
-  const int64_t nvalid = std::min<int64_t>(PJ_TOK, T - c * PJ_TOK);
-  const int64_t nout = kL * kR;
+  // part[p][q] = sum over the tokens of fin[p][tok] fin[16 NL + q][tok]: 16 x 16 blocks by fp32
+  // MFMAs, four tokens each.
   float* dst = part + (b * chunks + c) * sl.kl_tot * sl.kr_tot + sl.l0 * sl.kr_tot + sl.r0;
-  for (int64_t o = threadIdx.x; o < nout; o += PJ_THREADS) {
-    const int p = static_cast<int>(o / kR), q = static_cast<int>(o % kR);
-    float s = 0.f;
-    for (int64_t tk = 0; tk < nvalid; ++tk) s += sg[0][tk][p] * sa[0][tk][q];
-    dst[p * sl.kr_tot + q] = s;
+  for (int blk = wid; blk < NL * NR; blk += PJ_WAVES) {
+    const int p0 = blk / NR * 16, q0 = blk % NR * 16;
+    const float* lp = &fin[p0 + (lane & 15)][lane >> 4];
+    const float* rp = &fin[16 * NL + q0 + (lane & 15)][lane >> 4];
+    f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < TOK; t += 4)
+      o = __builtin_amdgcn_mfma_f32_16x16x4f32(lp[t], rp[t], o, 0, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int64_t p = p0 + 4 * (lane >> 4) + e, q = q0 + (lane & 15);
+      if (p < kL && q < kR) dst[p * sl.kr_tot + q] = o[e];
+    }
   }
 }
 
@@ -221,9 +265,18 @@ __global__ void kron_reduce_kernel(const float* __restrict__ part, int64_t chunk
   const int64_t b = blockIdx.y;
   const int64_t o = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (o >= nout) return;
-  float s = 0.f;
-  for (int64_t c = 0; c < chunks; ++c) s += part[(b * chunks + c) * nout + o];
-  s *= scale;
+  // Four running sums over whole groups of eight chunks keep the loads in flight together.
+  const float* src = part + b * chunks * nout + o;
+  float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+  int64_t c = 0;
+  for (; c + 8 <= chunks; c += 8, src += 8 * nout) {
+    a0 += src[0] + src[4 * nout];
+    a1 += src[nout] + src[5 * nout];
+    a2 += src[2 * nout] + src[6 * nout];
+    a3 += src[3 * nout] + src[7 * nout];
+  }
+  for (; c < chunks; ++c, src += nout) a0 += *src;
+  const float s = ((a0 + a1) + (a2 + a3)) * scale;
   if constexpr (std::is_same<OE, float>::value) {
     out[b * nout + o] = s;
   } else if constexpr (std::is_same<OE, __half>::value) {
@@ -242,15 +295,40 @@ template <class Tr, bool GATHER>
 int launch_pj_slice(const typename Tr::E* A, const int64_t* ids, int64_t vocab,
                     const typename Tr::E* G, int64_t B, int64_t T, int64_t n_a, int64_t n_g,
                     const typename Tr::E* R, const typename Tr::E* L, int64_t kr, int64_t kl,
-                    int64_t ldr, int va, int vg, int vr, int vl, int64_t chunks, PjSlice sl,
-                    float* part, hipStream_t s) {
+                    int64_t ldr, int va, int vg, int vr, int vl, int64_t chunks,
+                    PjSlice sl, float* part, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(chunks), static_cast<unsigned>(B));
-  const int64_t km = std::max(kl, kr);  // LDS width (a gathered side occupies it too)
-  auto k = km > 32   ? kron_proj_kernel<Tr, GATHER, 4>
-           : km > 16 ? kron_proj_kernel<Tr, GATHER, 2>
-                     : kron_proj_kernel<Tr, GATHER, 1>;
-  hipLaunchKernelGGL(k, grid, dim3(PJ_THREADS), 0, s, A, ids, vocab, G, T, n_a, n_g, R, L, kr,
-                     kl, ldr, va, vg, vr, vl, chunks, sl, part);
+  const bool vec_l = vg && vl, vec_r = GATHER || (va && vr);
+  auto go = [&](auto nl, auto nr, auto vecl, auto vecr) {
+    auto k = kron_proj_kernel<Tr, GATHER, decltype(nl)::value, decltype(nr)::value,
+                              decltype(vecl)::value, decltype(vecr)::value>;
+    hipLaunchKernelGGL(k, grid, dim3(PJ_THREADS), 0, s, A, ids, vocab, G, T, n_a, n_g, R, L, kr,
+                       kl, ldr, chunks, sl, part);
+  };
+  auto blocks = [](int64_t k, auto f) {  // f(the number of 16-row blocks of k rows)
+    if (k <= 16) return f(std::integral_constant<int, 1>{});
+    if (k <= 32) return f(std::integral_constant<int, 2>{});
+    if (k <= 48) return f(std::integral_constant<int, 3>{});
+    return f(std::integral_constant<int, 4>{});
+  };
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  if (vec_l && vec_r) {
+    blocks(kl, [&](auto nl) { blocks(kr, [&](auto nr) { go(nl, nr, yes, yes); }); });
+  } else {  // element-wise loads bound these: one or four blocks a side
+    auto some = [&](auto nb) {
+      if (vec_l)
+        go(nb, nb, yes, no);
+      else if (vec_r)
+        go(nb, nb, no, yes);
+      else
+        go(nb, nb, no, no);
+    };
+    if (std::max(kl, kr) <= 16)
+      some(std::integral_constant<int, 1>{});
+    else
+      some(std::integral_constant<int, 4>{});
+  }
   return check_launch(GATHER ? "kron_proj_kernel(gather)" : "kron_proj_kernel");
 }
 
@@ -259,8 +337,8 @@ int launch_pj_slice(const typename Tr::E* A, const int64_t* ids, int64_t vocab,
 template <class Tr, bool GATHER>
 int launch_pj(const void* A, const int64_t* ids, int64_t vocab, const void* G, int64_t B,
               int64_t T, int64_t n_a, int64_t n_g, const void* R, const void* L, int64_t kR,
-              int64_t kL, int va, int vg, int vr, int vl, int64_t chunks, float* part,
-              hipStream_t s) {
+              int64_t kL, int va, int vg, int vr, int vl, int64_t chunks,
+              float* part, hipStream_t s) {
   using E = typename Tr::E;
   for (int64_t l0 = 0; l0 < kL; l0 += PJ_KMAX) {
     for (int64_t r0 = 0; r0 < kR; r0 += PJ_KMAX) {
@@ -330,7 +408,7 @@ extern "C" int gs_kron_proj(const void* A, const void* G, int dtype, int64_t B, 
   const int64_t chunks = pj_cdiv(T, PJ_TOK);
   if (workspace == nullptr || workspace_bytes < gs_kron_proj_workspace(B, T, k_i, k_o) - 256)
     return fail(GS_ERR_WORKSPACE, "gs_kron_proj: workspace too small");
-  if (chunks > 65535 || B > 65535) return fail(GS_ERR_UNSUPPORTED, "gs_kron_proj: grid too large");
+  if (chunks > 2 * 65535 || B > 65535) return fail(GS_ERR_UNSUPPORTED, "gs_kron_proj: grid too large");
   Carver cv(workspace, workspace_bytes);
   float* part = cv.take<float>(B * chunks * kL * kR);
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -365,7 +443,7 @@ extern "C" int gs_kron_embed_proj(const int64_t* ids, const void* G, int dtype, 
   const int64_t chunks = pj_cdiv(T, PJ_TOK);
   if (workspace == nullptr || workspace_bytes < gs_kron_proj_workspace(B, T, k_i, k_o) - 256)
     return fail(GS_ERR_WORKSPACE, "gs_kron_embed_proj: workspace too small");
-  if (chunks > 65535 || B > 65535)
+  if (chunks > 2 * 65535 || B > 65535)
     return fail(GS_ERR_UNSUPPORTED, "gs_kron_embed_proj: grid too large");
   Carver cv(workspace, workspace_bytes);
   float* part = cv.take<float>(B * chunks * k_o * k_i);

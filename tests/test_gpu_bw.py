@@ -219,6 +219,37 @@ def test_layernorm_dots_and_grads(gpu, dtype, shape, mid):
     assert_close(gb.cpu(), gb_ref, tol, "ln bias grad")
 
 
+@pytest.mark.parametrize("conf", [
+    # B, T, n_i, n_o, k_i, k_o: a chunk's last token missing / whole / one token over; features
+    # one vector around a whole step of the waves, several steps, less than a wave's piece; rank
+    # blocks of 16, 32, 48, 64 rows from both sides; one side or both not 16-byte aligned
+    (2, 31, 512, 520, 16, 17), (3, 32, 504, 1032, 32, 33), (2, 33, 2056, 24, 48, 49),
+    (1, 1, 8, 1544, 64, 65), (2, 65, 511, 1024, 15, 3), (2, 40, 1024, 10, 40, 8),
+    (2, 40, 13, 513, 20, 13)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_kron_projection_edges(gpu, dtype, conf):
+    """The chunk, piece and rank-block edges against float64 (fp32 sums of at most 2056 features
+    and 65 tokens: 1e-5 of the rms).  A token row of NaN reaches its own sample only, though the
+    next chunk's padded tokens read valid rows in its place."""
+    B, T, n_i, n_o, k_i, k_o = conf
+    print(f"kron edges conf={conf} {dtype}", flush=True)
+    A = randn((B, T, n_i), 51 + T, 1.0, dtype)
+    G = randn((B, T, n_o), 52 + T, 1e-3, dtype)
+    P_i = randn((k_i, n_i), 53, k_i ** -0.5, dtype)
+    P_o = randn((k_o, n_o), 54, k_o ** -0.5, dtype)
+
+    def run(a):
+        return _native.ops().kron_proj(a.to(gpu), G.to(gpu), P_i.to(gpu), P_o.to(gpu), 2.0).cpu()
+    got = run(A)
+    want = R.kron_proj_exact(A, G, P_i, P_o, 2.0)
+    assert_close(got, want, 1e-5, "projection")
+    if B > 1:
+        bad = A.clone()
+        bad[1, 0] = float("nan")
+        out = run(bad)
+        assert torch.equal(out[0], got[0]) and torch.isnan(out[1]).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("conf", [
     # B, T, n_i, n_o, k_i, k_o
