@@ -2382,6 +2382,251 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tn_pair_kernel(TpParams q
   }
 }
 
+// ------------------------------------------------------------------ fp32 K-major pass
+// The fused layer pass for fp32 operands: the val term V = sum_val g a^T (VAL) and the train
+// rows' product with its per-sample dots and column sums, on v_mfma_f32_32x32x2f32.  With one k
+// per lane the K-major rows are the fragments' own layout: stages of TF_KB rows go to LDS as they
+// lie by wave-level DMA, and a fragment is one ds_read_b32 per lane (32 consecutive columns of
+// one row per half-wave, no bank conflicts).  Bound by the fp32 matrix rate (a 128 x 128 tile's
+// 8-row stage is 1024 MFMA cycles per wave against 64 reads).  16 + 4 samples, T = 256, 768 x 768,
+// one layer's hook with a bias: 229 us as a transposed val GEMM on 64 x 64 tiles without splits,
+// row-dot, bias passes and hipBLASLt, 84 us so (6.0 GFLOP; the train launch 56 us, 79% MFMA busy
+// while its CUs are; a ring of 8 stages gives no more).  Measured against the separate passes at
+// T = 1 to 500 and 64 to 5120 features it is never behind (64 + 16 samples of a 1024 x 1024 2-D
+// layer 184 -> 53 us, 12 + 2 of 1280 x 5120 at T = 55 656 -> 147), so nothing else is estimated.
+//
+// Samples are padded with zero rows to whole stages (the buffer ends at the sample's last row).
+// At each sample's end the accumulators hold that sample's G_i^T A_i: its inner product with V
+// is the dot, and it is added to the running train gradient and reset, so that a dot is no
+// difference of larger sums.  V and its split partials are kept in the accumulators' order
+// ([tile][wave][16 MI NI / 4][lane] float4), which the train launch reads coalesced.  The column
+// sums of the bias side (CS 1: L, 2: R) come from the fragments, one wave per 64 columns, summed
+// per stage and then per sample.
+constexpr int TF_KB = 8, TF_NS = 4;
+using TfC = Cfg<TrF32, 2, 2, 2, 2>;
+struct TfParams {
+  const float *L, *R;      // k-row 0 of the operands (M, N columns, contiguous rows)
+  int64_t M, N, m_tiles, n_tiles;
+  int64_t K, kper;         // padded k-rows in all, per split (whole stages)
+  int64_t Tp, T, n;        // padded and real k-rows per sample, samples (VAL: one sample)
+  int64_t gap_at, gap;     // physical row where the skipped block starts, its rows (0: none)
+  float4* V;               // VAL: [split][...] out; else [...] in
+  float* vsum;             // VAL, CS: [split][ext] column sums
+  float* part;             // train: [split][M][N]
+  float* pdot;             // train: [tiles][NW][2 slots][n] as TgParams
+  float* csum;             // train, CS: [n][2 slots][ext]
+  const float* vb;         // train, CS: [ext]
+  float* pbias;            // train, CS: [n][2 slots][ext / 64-column waves]
+};
+template <bool VAL, int CS>
+__global__ void __launch_bounds__(TfC::NT, 2) tnf_kernel(TfParams p) {
+  using C = TfC;
+  constexpr int NW = C::WM * C::WN, ROWB = 512, PART = TF_KB * ROWB, STAGE = 2 * PART;
+  static_assert(C::BM == 128 && C::BN == 128 && PART == NW * 1024, "one DMA per wave and side");
+  __shared__ __attribute__((aligned(16))) unsigned char lds[TF_NS * STAGE];
+  const int64_t it = xcd_order(blockIdx.x, gridDim.x), tiles = p.m_tiles * p.n_tiles;
+  const int64_t split = it / tiles, tile = it - split * tiles;
+  const bool m_inner = p.m_tiles <= p.n_tiles;
+  const int64_t inner = m_inner ? p.m_tiles : p.n_tiles;
+  const int64_t outer_i = tile / inner, inner_i = tile - outer_i * inner;
+  const int64_t mt = m_inner ? inner_i : outer_i, nt = m_inner ? outer_i : inner_i;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wid / C::WN, wn = wid % C::WN;
+
+  // Loads: wave w brings k-rows 2 w, 2 w + 1 of each side's stage, 16 bytes per lane.
+  const unsigned l4 = static_cast<unsigned>(p.M * 4), r4 = static_cast<unsigned>(p.N * 4);
+  const int krow = 2 * wid + (lane >> 5), chunk = (lane & 31) * 4;
+  const unsigned offl = mt * C::BM + chunk < p.M
+                            ? krow * l4 + static_cast<unsigned>((mt * C::BM + chunk) * 4)
+                            : DMA_OOB_ROW;
+  const unsigned offr = nt * C::BN + chunk < p.N
+                            ? krow * r4 + static_cast<unsigned>((nt * C::BN + chunk) * 4)
+                            : DMA_OOB_ROW;
+  const unsigned lds0 = lds_addr(lds);
+  const int64_t k_begin = split * p.kper;
+  const int64_t k_end = k_begin + p.kper < p.K ? k_begin + p.kper : p.K;
+  const int nk = static_cast<int>((k_end - k_begin) / TF_KB);
+  const int sps = static_cast<int>(p.Tp / TF_KB), T = static_cast<int>(p.T);
+  const int s0 = static_cast<int>(k_begin / p.Tp);
+  const int ss0 = static_cast<int>((k_begin - s0 * p.Tp) / TF_KB);
+  const int gap_at = p.gap != 0 ? static_cast<int>(p.gap_at) : -1, gap = static_cast<int>(p.gap);
+  int first = s0 * T;
+  if (p.gap != 0 && first >= gap_at) first += gap;
+  int row = first + ss0 * TF_KB, end = first + T, toload = sps - ss0;
+  auto load = [&](int k) {
+    const unsigned at = lds0 + (k % TF_NS) * STAGE + wid * 1024;
+    dma16_at(make_rsrc(p.L, static_cast<unsigned>(end) * l4),
+             offl + static_cast<unsigned>(row) * l4, at);
+    dma16_at(make_rsrc(p.R, static_cast<unsigned>(end) * r4),
+             offr + static_cast<unsigned>(row) * r4, at + PART);
+    row += TF_KB;
+    if (--toload == 0) {
+      toload = sps;
+      row = end == gap_at ? end + gap : end;
+      end = row + T;
+    }
+  };
+
+  f32x16_t acc[C::MI][C::NI], tot[VAL ? 1 : C::MI][VAL ? 1 : C::NI];
+  zero_acc<TrF32, C>(acc);
+  float4 vr[VAL ? 1 : C::MI][VAL ? 1 : C::NI][4];
+  if constexpr (!VAL) {
+    zero_acc<TrF32, C>(tot);
+    const float4* v = p.V + (tile * NW + wid) * (C::MI * C::NI * 4 * 64) + lane;
+#pragma unroll
+    for (int i = 0; i < C::MI; ++i)
+#pragma unroll
+      for (int j = 0; j < C::NI; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) vr[i][j][g] = v[((i * C::NI + j) * 4 + g) * 64];
+  }
+  // Column sums: the waves of tile 0 along the other side, one per 64 columns.
+  const bool summing = CS == 1 ? nt == 0 && wn == 0 : CS == 2 && mt == 0 && wm == 0;
+  const int64_t ext = CS == 2 ? p.N : p.M;
+  const int64_t col0 = (CS == 2 ? nt * C::BN + wn * 64 : mt * C::BM + wm * 64) + (lane & 31);
+  float rc[2] = {0.f, 0.f}, vbr[2] = {0.f, 0.f};
+  if constexpr (!VAL && CS != 0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) vbr[i] = col0 + 32 * i < ext ? p.vb[col0 + 32 * i] : 0.f;
+  }
+  int sample = s0, left = sps - ss0;
+  bool started = ss0 == 0;
+  auto flush = [&](bool ended) __attribute__((always_inline)) {
+    float d0 = 0.f, d1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < C::MI; ++i)
+#pragma unroll
+      for (int j = 0; j < C::NI; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 w = vr[VAL ? 0 : i][VAL ? 0 : j][g];
+          d0 += acc[i][j][4 * g] * w.x + acc[i][j][4 * g + 1] * w.y;
+          d1 += acc[i][j][4 * g + 2] * w.z + acc[i][j][4 * g + 3] * w.w;
+        }
+    const float d = wave_sum_dpp(d0 + d1);
+    const int slot = started ? 0 : 1;
+    const bool whole = started && ended;
+    float* pd = p.pdot + (tile * NW + wid) * 2 * p.n + sample;
+    if (lane == 0) {
+      pd[slot * p.n] = d;
+      if (whole) pd[p.n] = 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < C::MI; ++i)
+#pragma unroll
+      for (int j = 0; j < C::NI; ++j) tot[VAL ? 0 : i][VAL ? 0 : j] += acc[i][j];
+    zero_acc<TrF32, C>(acc);
+    if (CS != 0 && summing) {
+      float bd = 0.f;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float t = rc[i] + __shfl_xor(rc[i], 32, 64);
+        const int64_t col = col0 + 32 * i;
+        if (lane < 32 && col < ext) {
+          p.csum[(2 * static_cast<int64_t>(sample) + slot) * ext + col] = t;
+          if (whole) p.csum[(2 * static_cast<int64_t>(sample) + 1) * ext + col] = 0.f;
+          bd += t * vbr[i];
+        }
+        rc[i] = 0.f;
+      }
+      bd = wave_sum_dpp(bd);
+      if (lane == 0) {
+        const int64_t waves = CS == 2 ? p.n_tiles * C::WN : p.m_tiles * C::WM;
+        const int64_t w = CS == 2 ? nt * C::WN + wn : mt * C::WM + wm;
+        p.pbias[(2 * static_cast<int64_t>(sample) + slot) * waves + w] = bd;
+        if (whole) p.pbias[(2 * static_cast<int64_t>(sample) + 1) * waves + w] = 0.f;
+      }
+    }
+  };
+  const float* fa = reinterpret_cast<const float*>(lds) + (lane >> 5) * 128 + wm * 64 + (lane & 31);
+  const float* fb = reinterpret_cast<const float*>(lds + PART) + (lane >> 5) * 128 + wn * 64 +
+                    (lane & 31);
+  auto stage = [&](int kt) {
+    const float* a = fa + (kt % TF_NS) * (STAGE / 4);
+    const float* b = fb + (kt % TF_NS) * (STAGE / 4);
+    float st[2] = {0.f, 0.f};
+    // All of the stage's fragments first (one LDS latency per stage), then the MFMAs.
+    float av[TF_KB / 2][C::MI], bv[TF_KB / 2][C::NI];
+#pragma unroll
+    for (int ks = 0; ks < TF_KB / 2; ++ks) {
+#pragma unroll
+      for (int i = 0; i < C::MI; ++i) av[ks][i] = a[ks * 256 + 32 * i];
+#pragma unroll
+      for (int j = 0; j < C::NI; ++j) bv[ks][j] = b[ks * 256 + 32 * j];
+    }
+#pragma unroll
+    for (int ks = 0; ks < TF_KB / 2; ++ks) {
+#pragma unroll
+      for (int i = 0; i < C::MI; ++i)
+#pragma unroll
+        for (int j = 0; j < C::NI; ++j) TrF32::mma(acc[i][j], av[ks][i], bv[ks][j]);
+      if constexpr (CS != 0) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) st[i] += CS == 2 ? bv[ks][i] : av[ks][i];
+      }
+    }
+    // (each pair of fragments 32 columns apart is one ds_read2_b32)
+    __builtin_amdgcn_sched_group_barrier(0x100, TF_KB / 2 * (C::MI + C::NI) / 2, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, TF_KB / 2 * C::MI * C::NI, 0);
+    if constexpr (CS != 0) {
+      rc[0] += st[0];
+      rc[1] += st[1];
+    }
+    if constexpr (!VAL) {
+      if (--left == 0) {
+        flush(true);
+        left = sps;
+        started = true;
+        ++sample;
+      }
+    }
+  };
+  constexpr int AHEAD = TF_NS - 1;
+#pragma unroll
+  for (int k = 0; k < AHEAD; ++k)
+    if (k < nk) load(k);
+  int kt = 0;
+  for (; kt + AHEAD < nk; ++kt) {
+    wait_vmcnt<(AHEAD - 1) * 2>();
+    raw_barrier();
+    load(kt + AHEAD);
+    stage(kt);
+  }
+  for (; kt < nk; ++kt) {
+    wait_stages<2, AHEAD - 1>(nk - 1 - kt);
+    raw_barrier();
+    stage(kt);
+  }
+  if constexpr (VAL) {
+    float4* v = p.V + ((split * tiles + tile) * NW + wid) * (C::MI * C::NI * 4 * 64) + lane;
+#pragma unroll
+    for (int i = 0; i < C::MI; ++i)
+#pragma unroll
+      for (int j = 0; j < C::NI; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          v[((i * C::NI + j) * 4 + g) * 64] =
+              make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2],
+                          acc[i][j][4 * g + 3]);
+    if (CS != 0 && summing) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float t = rc[i] + __shfl_xor(rc[i], 32, 64);
+        if (lane < 32 && col0 + 32 * i < ext) p.vsum[split * ext + col0 + 32 * i] = t;
+      }
+    }
+  } else {
+    if (left != sps) flush(false);  // the split ends inside a sample
+    GemmParams e{};
+    e.m_rows = p.M;
+    e.n_cols = p.N;
+    e.c_ld = p.N;
+    e.C = p.part + split * p.M * p.N;
+    store_epilogue<TrF32, C>(e, tot, mt, nt);
+  }
+}
+
 // out[i] = alpha * (sum over the splits of part[s][i]) in fixed order, rounded once to bf16
 // (or stored as fp32 with out_f32), 4 elements per thread.  With vsum ([vs_rows][vs_n]) its
 // rows are also summed into row 0, in place.
@@ -3659,6 +3904,32 @@ extern "C" size_t gs_conv1d_dot_train_grad_workspace(int dtype, int64_t N, int64
 
 namespace gs {
 namespace {
+// One launch: the dots, the bias train gradient and the train-gradient reduction (count 0: no
+// weight gradient wanted; else a multiple of 4).
+int launch_tgdot_finish(const float* pdot, int64_t shares, int64_t n_t, const float* pbias,
+                        int64_t bshares, const float* csum, int64_t cs_rows, int64_t bias_d,
+                        void* out_dot, int dot_dtype, void* out_bias_dot, int bias_dot_dtype,
+                        void* out_bias_grad, int bias_grad_dtype, float bias_grad_scale,
+                        const float* part, int64_t count, int64_t sp, void* out_grad,
+                        int grad_dtype, float grad_scale, hipStream_t s) {
+  const int64_t gblocks =
+      out_bias_grad != nullptr ? ceil_div(bias_d, int64_t{FINISH_GF}) : 0;
+  const dim3 grid(static_cast<unsigned>(n_t + gblocks + ceil_div(count / 4, int64_t{256})));
+  const int gf32 = grad_dtype == GS_DTYPE_F32 ? 1 : 0;
+  const int df32 = dot_dtype == GS_DTYPE_F32 ? 1 : 0, bf32 = bias_dot_dtype == GS_DTYPE_F32 ? 1 : 0;
+  if (bias_grad_dtype == GS_DTYPE_F32)
+    hipLaunchKernelGGL(tgdot_finish_kernel<float>, grid, dim3(256), 0, s, pdot, shares, n_t, pbias,
+                       bshares, csum, cs_rows, bias_d, out_dot, df32, out_bias_dot, bf32,
+                       static_cast<float*>(out_bias_grad), bias_grad_scale, gblocks, part, count,
+                       static_cast<int>(sp), out_grad, grad_scale, gf32);
+  else
+    hipLaunchKernelGGL(tgdot_finish_kernel<uint16_t>, grid, dim3(256), 0, s, pdot, shares, n_t,
+                       pbias, bshares, csum, cs_rows, bias_d, out_dot, df32, out_bias_dot, bf32,
+                       static_cast<uint16_t*>(out_bias_grad), bias_grad_scale, gblocks, part,
+                       count, static_cast<int>(sp), out_grad, grad_scale, gf32);
+  return check_launch("tgdot_finish_kernel");
+}
+
 // The fused pass; bias_a: the bias terms are A's column sums; any_T: T need not be a multiple
 // of the stage height.
 int dot_train_grad(const char* name, bool bias_a, bool any_T, const void* A, const void* G,
@@ -3785,28 +4056,188 @@ int dot_train_grad(const char* name, bool bias_a, bool any_T, const void* A, con
     rag ? go_cs(std::false_type{}, std::true_type{}) : go_cs(std::false_type{}, std::false_type{});
   rc = check_launch("tgdot_kernel");
   if (rc) return rc;
-  // One launch: the dots, the bias train gradient and the train-gradient reduction.
   const int64_t shares = t.m_tiles * t.n_tiles * (t.wm * t.wn) * 2;
   const int64_t sps = t.Tp / TnD::KB;
   const int64_t bshares = sps * (t.bias_a ? t.n_tiles * t.wn : t.m_tiles * t.wm);
-  const float* pbias = out_bias_dot != nullptr ? b.pbias : nullptr;
-  const int64_t gblocks =
-      out_bias_grad != nullptr ? ceil_div(t.bias_d, int64_t{FINISH_GF}) : 0;
-  const int64_t count = out_grad != nullptr ? d_out * d_in : 0;  // a multiple of 8
-  const dim3 grid(static_cast<unsigned>(t.n_t + gblocks + ceil_div(count / 4, int64_t{256})));
-  const int gf32 = grad_dtype == GS_DTYPE_F32 ? 1 : 0;
-  const int df32 = dot_dtype == GS_DTYPE_F32 ? 1 : 0, bf32 = bias_dot_dtype == GS_DTYPE_F32 ? 1 : 0;
-  if (bias_grad_dtype == GS_DTYPE_F32)
-    hipLaunchKernelGGL(tgdot_finish_kernel<float>, grid, dim3(256), 0, s, b.pdot, shares, t.n_t,
-                       pbias, bshares, b.csum, 2 * sps, t.bias_d, out_dot, df32, out_bias_dot, bf32,
-                       static_cast<float*>(out_bias_grad), bias_grad_scale, gblocks, b.tgpart,
-                       count, static_cast<int>(t.sp), out_grad, grad_scale, gf32);
+  return launch_tgdot_finish(b.pdot, shares, t.n_t, out_bias_dot != nullptr ? b.pbias : nullptr,
+                             bshares, b.csum, 2 * sps, t.bias_d, out_dot, dot_dtype,
+                             out_bias_dot, bias_dot_dtype, out_bias_grad, bias_grad_dtype,
+                             bias_grad_scale, b.tgpart, out_grad != nullptr ? d_out * d_in : 0,
+                             t.sp, out_grad, grad_dtype, grad_scale, s);
+}
+}  // namespace
+}  // namespace gs
+
+// ------------------------------------------------------------------ fp32 layer pass, host side
+namespace gs {
+namespace {
+struct TfPlan {
+  int presum, bias;
+  int64_t vrows, vK, vkper, vsp;   // val k-rows, padded, per split, splits
+  int64_t Tp, n_t, K, kper, sp;    // train
+  int64_t M, N, m_tiles, n_tiles, bias_d, waves;  // waves: 64-column waves of the bias side
+};
+// Splits of K padded k-rows over `tiles` tiles, each at least `unit` rows long: two workgroups
+// on a CU share its fp32 matrix rate (0.27 TF/s each, 0.33 alone), the fp32 partials cost a write
+// and a read at 4 TB/s.
+int64_t tf_kper(int64_t K, int64_t tiles, int64_t count, int64_t unit) {
+  int64_t best = K;
+  double best_t = 1e30;
+  for (int64_t sp = 1; sp <= 16; ++sp) {
+    const int64_t kper = std::max(ceil_div(ceil_div(K, sp), int64_t{TF_KB}) * TF_KB, unit);
+    const int64_t n = ceil_div(K, kper), items = tiles * n;
+    const double rounds = std::ceil(static_cast<double>(items) / 512.0);
+    const double t = rounds * 2.0 * TfC::BM * TfC::BN * kper / (items <= 256 ? 0.33e12 : 0.27e12) +
+                     8.0 * n * count / 4e12;
+    if (t < best_t) {
+      best_t = t;
+      best = kper;
+    }
+  }
+  return best;
+}
+bool tf_ok(int dtype, int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
+           int semantics) {
+  if (dtype != GS_DTYPE_F32 || n_val <= 0 || n_val >= N || T <= 0) return false;
+  if (semantics != GS_SEM_PAIRWISE_SUM && semantics != GS_SEM_PRESUM) return false;
+  if (d_in <= 0 || d_out <= 0 || d_in % 4 || d_out % 4) return false;
+  return N * T * d_in * 4 < INT32_MAX && N * T * d_out * 4 < INT32_MAX;
+}
+TfPlan plan_tf(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out, int semantics,
+               bool bias, bool conv1d) {
+  TfPlan t{};
+  t.presum = semantics == GS_SEM_PRESUM ? 1 : 0;
+  t.bias = bias ? 1 : 0;
+  t.M = conv1d ? d_in : d_out;
+  t.N = conv1d ? d_out : d_in;
+  t.m_tiles = ceil_div(t.M, TfC::BM);
+  t.n_tiles = ceil_div(t.N, TfC::BN);
+  t.bias_d = d_out;
+  t.waves = conv1d ? t.n_tiles * TfC::WN : t.m_tiles * TfC::WM;
+  const int64_t tiles = t.m_tiles * t.n_tiles, area = tiles * TfC::BM * TfC::BN;
+  t.vrows = (t.presum ? 1 : n_val) * T;
+  t.vK = ceil_div(t.vrows, int64_t{TF_KB}) * TF_KB;
+  t.vkper = tf_kper(t.vK, tiles, area, TF_KB);
+  t.vsp = ceil_div(t.vK, t.vkper);
+  t.n_t = N - n_val;
+  t.Tp = ceil_div(T, int64_t{TF_KB}) * TF_KB;
+  t.K = t.n_t * t.Tp;
+  t.kper = tf_kper(t.K, tiles, t.M * t.N, t.Tp);  // a sample meets at most two splits
+  t.sp = ceil_div(t.K, t.kper);
+  return t;
+}
+struct TfBufs {
+  float *abar, *gbar, *V, *vpart, *vp, *pdot, *csum, *pbias, *part;
+};
+template <class S>
+TfBufs carve_tf(S& c, const TfPlan& t, int64_t T, int64_t d_in, int64_t d_out) {
+  TfBufs b{};
+  const int64_t tiles = t.m_tiles * t.n_tiles, area = tiles * TfC::BM * TfC::BN;
+  b.abar = t.presum ? c.template take<float>(T * d_in) : nullptr;
+  b.gbar = t.presum ? c.template take<float>(T * d_out) : nullptr;
+  b.V = c.template take<float>(area);
+  b.vpart = t.vsp > 1 ? c.template take<float>(t.vsp * area) : nullptr;
+  // the reduction reads the sums in fours
+  b.vp = t.bias ? c.template take<float>(t.vsp * t.bias_d) : nullptr;
+  b.pdot = c.template take<float>(tiles * TfC::WM * TfC::WN * 2 * t.n_t);
+  b.csum = t.bias ? c.template take<float>(t.n_t * 2 * t.bias_d) : nullptr;
+  b.pbias = t.bias ? c.template take<float>(t.n_t * 2 * t.waves) : nullptr;
+  b.part = c.template take<float>(t.sp * t.M * t.N);
+  return b;
+}
+size_t tf_workspace(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
+                    int semantics, bool bias, bool conv1d) {
+  Sizer sz;
+  carve_tf(sz, plan_tf(N, n_val, T, d_in, d_out, semantics, bias, conv1d), T, d_in, d_out);
+  return sz.used + 256;
+}
+template <bool VAL>
+void launch_tnf(const TfParams& p, int64_t items, int cs, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(items)), block(TfC::NT);
+  if (cs == 0)
+    hipLaunchKernelGGL((tnf_kernel<VAL, 0>), grid, block, 0, s, p);
+  else if (cs == 1)
+    hipLaunchKernelGGL((tnf_kernel<VAL, 1>), grid, block, 0, s, p);
   else
-    hipLaunchKernelGGL(tgdot_finish_kernel<uint16_t>, grid, dim3(256), 0, s, b.pdot, shares,
-                       t.n_t, pbias, bshares, b.csum, 2 * sps, t.bias_d, out_dot, df32,
-                       out_bias_dot, bf32, static_cast<uint16_t*>(out_bias_grad),
-                       bias_grad_scale, gblocks, b.tgpart, count, static_cast<int>(t.sp), out_grad, grad_scale, gf32);
-  return check_launch("tgdot_finish_kernel");
+    hipLaunchKernelGGL((tnf_kernel<VAL, 2>), grid, block, 0, s, p);
+}
+// The fp32 layer pass; the caller has checked the arguments.
+int layer_pass_f32(bool conv1d, const float* A, const float* G, int64_t N, int64_t n_val,
+                   int64_t val_start, int64_t T, int64_t d_in, int64_t d_out, int semantics,
+                   void* out_dot, int dot_dtype, void* out_grad, int grad_dtype,
+                   float grad_scale, void* out_bias_dot, int bias_dot_dtype,
+                   void* out_bias_grad, int bias_grad_dtype, float bias_grad_scale,
+                   void* workspace, size_t workspace_bytes, hipStream_t s) {
+  const bool bias = out_bias_dot != nullptr || out_bias_grad != nullptr;
+  const TfPlan t = plan_tf(N, n_val, T, d_in, d_out, semantics, bias, conv1d);
+  Carver cv(workspace, workspace_bytes);
+  const TfBufs b = carve_tf(cv, t, T, d_in, d_out);
+  const float* va = A + val_start * T * d_in;
+  const float* vg = G + val_start * T * d_out;
+  if (t.presum) {
+    const RowMap map = val_rows(n_val, val_start, T);
+    auto sum = [&](const float* in, int64_t d, float* out) {
+      const int64_t blocks = std::min<int64_t>(ceil_div(T * d, 256), 65536);
+      hipLaunchKernelGGL(presum_rows_kernel<float>, dim3(static_cast<unsigned>(blocks)),
+                         dim3(256), 0, s, in, d, map, d, out);
+    };
+    sum(A, d_in, b.abar);
+    sum(G, d_out, b.gbar);
+    va = b.abar;
+    vg = b.gbar;
+  }
+  const int64_t tiles = t.m_tiles * t.n_tiles, area = tiles * TfC::BM * TfC::BN;
+  const int cs = !bias ? 0 : conv1d ? 2 : 1;
+  if (tiles * std::max(t.vsp, t.sp) > INT32_MAX)
+    return fail(GS_ERR_UNSUPPORTED, "GEMM grid too large");
+  TfParams p{};
+  p.M = t.M;
+  p.N = t.N;
+  p.m_tiles = t.m_tiles;
+  p.n_tiles = t.n_tiles;
+  p.L = conv1d ? va : vg;
+  p.R = conv1d ? vg : va;
+  p.K = p.Tp = t.vK;
+  p.kper = t.vkper;
+  p.T = t.vrows;
+  p.n = 1;
+  p.V = reinterpret_cast<float4*>(t.vsp > 1 ? b.vpart : b.V);
+  p.vsum = b.vp;
+  launch_tnf<true>(p, tiles * t.vsp, cs, s);
+  int rc = check_launch("tnf_kernel (val)");
+  if (rc) return rc;
+  if (t.vsp > 1) {  // V and the val column sums, summed over the splits
+    hipLaunchKernelGGL(tn_reduce_kernel,
+                       dim3(static_cast<unsigned>(ceil_div(std::max(area, t.bias_d) / 4, 256))),
+                       dim3(256), 0, s, b.vpart, area, static_cast<int>(t.vsp), b.V, 1.f, 1,
+                       b.vp, t.bias_d, t.vsp);
+    rc = check_launch("tn_reduce_kernel");
+    if (rc) return rc;
+  }
+  p.L = conv1d ? A : G;
+  p.R = conv1d ? G : A;
+  p.K = t.K;
+  p.kper = t.kper;
+  p.Tp = t.Tp;
+  p.T = T;
+  p.n = t.n_t;
+  p.gap = val_start < t.n_t ? n_val * T : 0;
+  p.gap_at = val_start * T;
+  p.V = reinterpret_cast<float4*>(b.V);
+  p.part = b.part;
+  p.pdot = b.pdot;
+  p.csum = b.csum;
+  p.vb = b.vp;
+  p.pbias = b.pbias;
+  launch_tnf<false>(p, tiles * t.sp, cs, s);
+  rc = check_launch("tnf_kernel (train)");
+  if (rc) return rc;
+  return launch_tgdot_finish(b.pdot, tiles * TfC::WM * TfC::WN * 2, t.n_t,
+                             out_bias_dot != nullptr ? b.pbias : nullptr, 2 * t.waves, b.csum, 2,
+                             t.bias_d, out_dot, dot_dtype, out_bias_dot, bias_dot_dtype,
+                             out_bias_grad, bias_grad_dtype, bias_grad_scale, b.part,
+                             out_grad != nullptr ? t.M * t.N : 0, t.sp, out_grad, grad_dtype,
+                             grad_scale, s);
 }
 }  // namespace
 }  // namespace gs
@@ -3845,6 +4276,10 @@ extern "C" size_t gs_linear_layer_pass_workspace(int dtype, int64_t N, int64_t n
                                                  int conv1d, int with_bias, int algo,
                                                  int rounding) {
   if (!linear_args_ok(dtype, N, n_val, T, d_in, d_out, semantics, algo, 0)) return 0;
+  if (algo != GS_ALGO_GHOST && dtype == GS_DTYPE_F32)
+    return tf_ok(dtype, N, n_val, T, d_in, d_out, semantics)
+               ? tf_workspace(N, n_val, T, d_in, d_out, semantics, with_bias != 0, conv1d != 0)
+               : 0;
   if (algo == GS_ALGO_GHOST || !tg_ok(dtype, N, n_val, T, d_in, d_out, semantics)) return 0;
   const LinearPlan pl = plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, 0);
   if (pl.algo == GS_ALGO_GHOST && rounding == GS_ROUND_REF_BF16) return 0;
@@ -3864,6 +4299,34 @@ extern "C" int gs_linear_layer_pass(const void* A, const void* G, int dtype, int
                                     float bias_grad_scale, void* workspace,
                                     size_t workspace_bytes, void* stream) {
   const bool cv = conv1d != 0;
+  if (dtype == GS_DTYPE_F32) {
+    const std::string who = "gs_linear_layer_pass";
+    if (N <= 0 || T <= 0 || d_in <= 0 || d_out <= 0 || n_val <= 0 || n_val >= N ||
+        val_start < 0 || val_start + n_val > N)
+      return fail(GS_ERR_INVALID, who + ": invalid shape");
+    if (A == nullptr || G == nullptr || out_dot == nullptr)
+      return fail(GS_ERR_INVALID, who + ": null pointer");
+    if (semantics != GS_SEM_PAIRWISE_SUM && semantics != GS_SEM_PRESUM)
+      return fail(GS_ERR_INVALID, who + ": invalid semantics");
+    auto ok = [](const void* out, int dt) {
+      return out == nullptr || dt == GS_DTYPE_BF16 || dt == GS_DTYPE_F32;
+    };
+    if (!ok(out_dot, dot_dtype) || !ok(out_grad, grad_dtype) ||
+        !ok(out_bias_dot, bias_dot_dtype) || !ok(out_bias_grad, bias_grad_dtype))
+      return fail(GS_ERR_DTYPE, who + ": output dtypes must be bf16 or fp32");
+    if (!tf_ok(dtype, N, n_val, T, d_in, d_out, semantics) || !aligned16(A) || !aligned16(G))
+      return fail(GS_ERR_UNSUPPORTED, who + ": fp32 operands need 16-byte alignment, feature "
+                                            "counts that are multiples of 4 and less than 2 GiB");
+    const bool bias = out_bias_dot != nullptr || out_bias_grad != nullptr;
+    if (workspace == nullptr ||
+        workspace_bytes < tf_workspace(N, n_val, T, d_in, d_out, semantics, bias, cv) - 256)
+      return fail(GS_ERR_WORKSPACE, who + ": workspace too small");
+    return layer_pass_f32(cv, static_cast<const float*>(A), static_cast<const float*>(G), N,
+                          n_val, val_start, T, d_in, d_out, semantics, out_dot, dot_dtype,
+                          out_grad, grad_dtype, grad_scale, out_bias_dot, bias_dot_dtype,
+                          out_bias_grad, bias_grad_dtype, bias_grad_scale, workspace,
+                          workspace_bytes, static_cast<hipStream_t>(stream));
+  }
   return dot_train_grad("gs_linear_layer_pass", cv, true, cv ? G : A, cv ? A : G, dtype, N, n_val,
                         val_start, T, cv ? d_out : d_in, cv ? d_in : d_out, semantics, out_dot,
                         dot_dtype, out_grad, grad_dtype, grad_scale, out_bias_dot,

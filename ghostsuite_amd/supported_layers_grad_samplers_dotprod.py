@@ -236,7 +236,7 @@ def _fused_dot_train_grad(layer: nn.Module, A: torch.Tensor, B: torch.Tensor,
     """Weight dot and weight train gradient (and with a bias its dot and train gradient) from
     one K-major pass over the train rows: per train row, sum_t g^T V a = <V, G_i^T A_i>, and
     the train gradient is the sum of the same G_i^T A_i (gs_linear_layer_pass).  Taken for
-    bf16 layers whose weight trains, unless linear_algo is 'ghost' or the separate passes are
+    bf16 and fp32 layers whose weight trains, unless linear_algo is 'ghost' or the separate passes are
     estimated to be faster; the train gradients are parked for _apply_train_grad.  Returns
     False when the other paths must run.
 
@@ -246,8 +246,8 @@ def _fused_dot_train_grad(layer: nn.Module, A: torch.Tensor, B: torch.Tensor,
     scale = getattr(layer, "_gs_bias_grad_scale", None)
     bias = layer.bias is not None
     grad_dtypes = (torch.bfloat16, torch.float32)   # train gradients in the parameters' dtype
-    if scale is None or dtype != torch.bfloat16 or A.dtype != torch.bfloat16 or \
-            (pairwise and options["store_pairs"]) or \
+    if scale is None or dtype not in (torch.bfloat16, torch.float32) or A.dtype != dtype or \
+            (dtype == torch.float32 and B.dtype != dtype) or (pairwise and options["store_pairs"]) or \
             layer.weight.dtype not in grad_dtypes or \
             not getattr(layer.weight, "initially_requires_grad", False) or \
             (bias and (layer.bias.dtype not in grad_dtypes or
@@ -264,6 +264,8 @@ def _fused_dot_train_grad(layer: nn.Module, A: torch.Tensor, B: torch.Tensor,
                          grad_scale=scale, grad_dtype=layer.weight.dtype, dot_dtype=weight_dt,
                          bias_grad_dtype=layer.bias.dtype if bias else None,
                          bias_dot_dtype=bias_dt)
+    elif dtype != torch.bfloat16:
+        return False
     else:   # a kernel layer without the whole-layer pass
         N, d_in, d_out = A.shape[0], A.shape[-1], Bc.shape[-1]
         T = A.numel() // (N * d_in)

@@ -178,12 +178,13 @@ int gs_conv1d_dot_train_grad(const void* A, const void* G, int dtype, int64_t N,
                              int bias_grad_dtype, float bias_grad_scale, void* workspace,
                              size_t workspace_bytes, void* stream);
 
-/* The same pass for a layer's backward hook: any T, the weight layout by `conv1d` (0: out_grad
+/* The same pass for a layer's backward hook: bf16 operands as above or fp32 ones (16-byte
+ * aligned, feature counts multiples of 4, below 2 GiB; fp32 products throughout), any T, the weight layout by `conv1d` (0: out_grad
  * [d_out, d_in], gs_linear_dot_train_grad; 1: [d_in, d_out], gs_conv1d_dot_train_grad), and the
  * dots rounded once from fp32 to dot_dtype / bias_dot_dtype (GS_DTYPE_BF16 or GS_DTYPE_F32).
- * With T not a multiple of 64 each train sample is padded with zero rows inside the kernel
+ * Where T is not a whole number of the kernel's stages each train sample is padded with zero rows inside the kernel
  * (nothing is read for them).  The workspace query returns 0 where the pass does not apply
- * (operands as for gs_linear_dot_train_grad, algo GHOST, or AUTO choosing GHOST with the
+ * (algo GHOST, or AUTO choosing GHOST with the
  * reference's rounding) and where, for `algo`, the dots and the train gradient apart are
  * estimated to be faster.  Reference: as for the two entry points above. */
 size_t gs_linear_layer_pass_workspace(int dtype, int64_t N, int64_t n_val, int64_t T,

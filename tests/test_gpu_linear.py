@@ -572,8 +572,53 @@ def test_linear_layer_pass_any_length(gpu, case):
         assert torch.isnan(dn[1]) and torch.equal(dn[0], dot.cpu()[0])
 
 
+@pytest.mark.parametrize("case", [
+    # N, n_val, T, d_in, d_out, semantics, val position, bias, conv1d: T around the 8-row stage,
+    # a 2-D layer's single token, ragged tiles, one train sample, splits inside samples
+    (6, 2, 7, 40, 24, "pairwise", "last", True, False),
+    (6, 2, 9, 132, 4, "presum", "mid", True, False),
+    (80, 16, 1, 512, 264, "pairwise", "last", True, False),
+    (3, 2, 100, 16, 8, "pairwise", "mid", False, False),
+    (16, 3, 77, 768, 264, "presum", "first", True, True),
+    (9, 2, 200, 260, 512, "pairwise", "mid", True, True),
+    (20, 4, 256, 768, 768, "pairwise", "last", True, False),
+])
+def test_linear_layer_pass_fp32(gpu, case):
+    """The fp32 layer pass against float64.  Its products and sums are fp32 in blocks of a sample:
+    a relative error of 2^-24 times the square root of the longest chain (4096 rows) at most,
+    1e-5 of the rms with the constant; a NaN stays in its own sample's dot."""
+    N, n_val, T, d_in, d_out, sem, pos, bias, conv1d = case
+    vs = {"last": N - n_val, "first": 0, "mid": 1}[pos]
+    n_t = N - n_val
+    print(f"fp32 layer pass case={case}", flush=True)
+    A, G = _inputs(N, T, d_in, d_out, 250 + T, torch.float32)
+
+    def run(a):
+        return _native.ops().linear_layer_pass(
+            a.to(gpu), G.to(gpu), n_val, algo=_native.ALGO_VALGRAD, rounding=_native.ROUND_FP32,
+            semantics=_native.SEM_PAIRWISE_SUM if sem == "pairwise" else _native.SEM_PRESUM,
+            conv1d=conv1d, grad_scale=1.5 / n_t, grad_dtype=torch.float32,
+            dot_dtype=torch.float32, bias_grad_dtype=torch.float32 if bias else None,
+            bias_dot_dtype=torch.float32, val_start=vs)
+    dot, grad, bdot, bgrad = run(A)
+    assert_close(dot.cpu(), R.linear_dot_exact(A, G, n_val, sem, val_start=vs), 1e-5, "dot")
+    assert_close(grad.cpu(), _train_grad_want(A, G, n_val, vs, 1.5 / n_t, conv1d, gpu), 1e-5,
+                 "weight train grad")
+    if bias:
+        assert_close(bdot.cpu(), R.bias_dot_exact(G, n_val, vs), 1e-5, "bias dot")
+        tr, _ = R.split_rows(G.double(), n_val, vs)
+        assert_close(bgrad.cpu(), tr.sum((0, 1)) * (1.5 / n_t), 1e-5, "bias train grad")
+    if n_t > 1:
+        bad = A.clone()
+        rows = [i for i in range(N) if not vs <= i < vs + n_val]
+        bad[rows[1], 0] = float("nan")
+        dn = run(bad)[0].cpu()
+        others = [i for i in range(n_t) if i != 1]
+        assert torch.isnan(dn[1]) and torch.equal(dn[others], dot.cpu()[others])
+
+
 def test_linear_layer_pass_declines(gpu):
-    """Unaligned feature counts, fp32 operands, the ghost algorithm, and the automatic choice of
+    """Unaligned feature counts, the ghost algorithm, and the automatic choice of
     the ghost kernel with the reference's rounding keep the separate passes."""
     def taken(A, G, algo=_native.ALGO_AUTO, rounding=_native.ROUND_FP32):
         return _native.ops().linear_layer_pass(
@@ -585,7 +630,7 @@ def test_linear_layer_pass_declines(gpu):
     assert not taken(A, G, _native.ALGO_GHOST)
     A, G = _inputs(6, 100, 12, 256, 6, torch.bfloat16)
     assert not taken(A, G)
-    A, G = _inputs(6, 64, 64, 256, 7, torch.float32)
+    A, G = _inputs(6, 64, 64, 10, 7, torch.float32)
     assert not taken(A, G)
     A, G = _inputs(6, 64, 2048, 2048, 8, torch.bfloat16)
     assert _native.ops().linear_algo(torch.bfloat16, 6, 2, 64, 2048, 2048, 0, 0,
