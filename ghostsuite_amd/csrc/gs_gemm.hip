@@ -1677,6 +1677,7 @@ struct TnParams {
   int vparts;       // the first vparts tiles along the other side (N, or M with vsum_r)
                     //   share the column sums
   int64_t gap_at, gap;  // logical k-rows >= gap_at lie gap rows further on (a skipped block)
+  int acc_order;    // out (or the partials) in accumulator order, whole tiles: acc_store
 };
 
 template <class C, class D>
@@ -2028,6 +2029,54 @@ __device__ __forceinline__ void tn_item(const TnParams& p, int64_t& mt, int64_t&
   nt = m_inner ? outer_i : inner_i;
 }
 
+// Accumulator order of a tile set: [tile][wave][MI * NI blocks][2 halves][64 lanes][8 entries], the
+// order the accumulators hold them, so that a kernel of the same tile and wave shape reads its own
+// tile's entries (a V to take inner products with) by coalesced 16-byte loads.
+template <class C>
+__device__ __forceinline__ int64_t acc_base(int64_t tile, int wid) {
+  return (tile * (C::WM * C::WN) + wid) * (C::MI * C::NI * 2 * 64) + (threadIdx.x & 63);
+}
+__device__ __forceinline__ uint4 acc_pack(const f32x16_t& a, int h) {
+  uint4 w;
+  w.x = pack_bf16x2(a[8 * h], a[8 * h + 1]);
+  w.y = pack_bf16x2(a[8 * h + 2], a[8 * h + 3]);
+  w.z = pack_bf16x2(a[8 * h + 4], a[8 * h + 5]);
+  w.w = pack_bf16x2(a[8 * h + 6], a[8 * h + 7]);
+  return w;
+}
+// The tile as bf16 pairs (out: uint4 per lane and half), or with F32 as fp32.
+template <class C, bool F32>
+__device__ __forceinline__ void acc_store(void* out, int64_t tile, int wid,
+                                          const f32x16_t (&acc)[C::MI][C::NI]) {
+  const int64_t base = acc_base<C>(tile, wid);
+#pragma unroll
+  for (int i = 0; i < C::MI; ++i)
+#pragma unroll
+    for (int j = 0; j < C::NI; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int64_t at = base + ((i * C::NI + j) * 2 + h) * 64;
+        const f32x16_t& a = acc[i][j];
+        if constexpr (F32) {
+          float4* o = static_cast<float4*>(out) + at * 2;
+          o[0] = make_float4(a[8 * h], a[8 * h + 1], a[8 * h + 2], a[8 * h + 3]);
+          o[1] = make_float4(a[8 * h + 4], a[8 * h + 5], a[8 * h + 6], a[8 * h + 7]);
+        } else {
+          static_cast<uint4*>(out)[at] = acc_pack(a, h);
+        }
+      }
+}
+// d0 + d1 += <one half block of acc, its packed counterpart>.
+__device__ __forceinline__ void acc_dot(const f32x16_t& a, int h, const uint4& w, float& d0,
+                                        float& d1) {
+  const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    d0 += a[8 * h + 2 * e] * __uint_as_float(u[e] << 16);
+    d1 += a[8 * h + 2 * e + 1] * __uint_as_float(u[e] & 0xFFFF0000u);
+  }
+}
+
 // One output tile per work item: bf16 out, or fp32 partials (several splits or an output
 // option) reduced by tn_reduce_kernel.
 template <class C, class D, int CSM>
@@ -2089,6 +2138,15 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tn_gemm_kernel(TnParams p
       }
     }
   }
+  if (p.acc_order) {
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t tiles = p.m_tiles * p.n_tiles, tile = mt * p.n_tiles + nt;
+    if (p.part_out)
+      acc_store<C, true>(p.out, split * tiles + tile, wid, acc);
+    else
+      acc_store<C, false>(p.out, tile, wid, acc);
+    return;
+  }
   GemmParams e{};
   e.m_rows = p.M;
   e.n_cols = p.N;
@@ -2117,14 +2175,15 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tn_gemm_kernel(TnParams p
 // terms) are taken per stage as well, after the stage's MFMAs, spread over the workgroups.
 struct TgParams {
   TnParams tn;          // k-rows per split (kper) a multiple of the stage height, >= T;
-                        // out: fp32 partials
-  const uint16_t* Vt;   // V^T: [N][M] bf16
+                        // out: fp32 partials, or with one split the gradient (part_out 0)
+  const uint4* V;       // V (bf16) in accumulator order of the same tiles (acc_store)
   int64_t T, n_t;       // k-rows per sample (a multiple of the stage height), train samples
   int64_t T_rows;       // with RAG: the rows a sample has (T counts them padded to whole stages)
   float* pdot;          // [m_tiles * n_tiles][NW][2 slots][n_t] wave shares of the weight dots
   float* csum;          // with CS: [n_t][2 T / stage height][M] column sums of L (CS 1; of R,
                         // [..][N], with CS 2), two rows (halves of the stage's k-rows) per stage
-  const float* vb;      // with CS: [M] ([N]) the val rows' column sums of the same side
+  const float* vb;      // with CS: [vb_rows][M] ([N]) the val rows' column sums of the same side
+  int vb_rows;          //   (at most 4 rows, added here)
   float* pbias;         // with CS: [n_t][T / stage height][m_tiles][WM] ([..][n_tiles][WN])
                         //   bias-dot shares: a stage's column sums of one wave's columns
                         //   dotted with vb
@@ -2144,30 +2203,18 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
   f32x16_t acc[C::MI][C::NI];
   zero_acc<TrBF16, C>(acc);
   float s_prev = 0.f;  // <acc, V tile> of this wave at the previous boundary
-  // This lane's V elements: for block (i, j) and row group g, the 4 consecutive rows
-  // m(i, g) .. m(i, g) + 3 of column n(j), one 8-byte load of V^T row n (M and N are
-  // multiples of 8, so a group is wholly inside or outside the matrix).  With 64 x 64 wave
-  // tiles they are loaded once and held for the work item (32 registers); wider wave tiles
-  // have no registers to spare beside their accumulators, and load them again from V^T (in
-  // L2) at each boundary, a few per sample.
+  // This lane's V entries: 16 bytes per half block.  With 64 x 64 wave tiles they are loaded
+  // once and held for the work item (32 registers); wider wave tiles have no registers to spare
+  // beside their accumulators, and load them again (from L2) at each boundary, a few per sample.
+  // (In accumulator order: from a row-major V^T, 8 bytes of 32 rows per load, the eight boundaries
+  // of a 2048 x 8192 gradient cost 52 of the hook's 663 us.)
   constexpr bool VHELD = C::MI * C::NI <= 4;
-  const int64_t m_lane = mt * C::BM + wm * 32 * C::MI + 4 * (lane >> 5);
-  const int64_t n_lane = nt * C::BN + wn * 32 * C::NI + (lane & 31);
-  // (captures by value: a reference to the kernel-argument struct from inside the stage
-  // loop makes the compiler copy the struct to private memory)
-  auto vload = [Vt = q.Vt, M = p.M, N = p.N, m_lane, n_lane](int i, int j, int g) {
-    const int64_t n = n_lane + j * 32, m = m_lane + i * 32 + 8 * g;
-    return (n < N && m < M) ? *reinterpret_cast<const uint2*>(Vt + n * M + m)
-                            : make_uint2(0u, 0u);
-  };
-  uint2 vr[VHELD ? C::MI : 1][VHELD ? C::NI : 1][4];
+  const int64_t tile = mt * p.n_tiles + nt;
+  const uint4* vsrc = q.V + acc_base<C>(tile, wid);
+  uint4 vr[VHELD ? C::MI * C::NI * 2 : 1];
   if constexpr (VHELD) {
 #pragma unroll
-    for (int j = 0; j < C::NI; ++j)
-#pragma unroll
-      for (int i = 0; i < C::MI; ++i)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) vr[i][j][g] = vload(i, j, g);
+    for (int k = 0; k < C::MI * C::NI * 2; ++k) vr[k] = vsrc[k * 64];
   }
   // Column sums of L (G's train rows: the bias terms), with CS: every workgroup along N
   // takes a share, so no work item runs longer than the others.  After the MFMAs of the
@@ -2187,9 +2234,16 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
 #pragma unroll
   for (int i = 0; i < F; ++i) {
     const int64_t col = col0 + i * 32;
-    vbr[i] = CS && col < ext ? q.vb[col] : 0.f;
+    vbr[i] = 0.f;
+    if constexpr (CS != 0) {
+      const int64_t c = col < ext ? col : 0;
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = q.vb[(r < q.vb_rows ? r : 0) * ext + c];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) vbr[i] += r < q.vb_rows && col < ext ? v[r] : 0.f;
+    }
   }
-  const int64_t tile = mt * p.n_tiles + nt;
   // Stages left in the current sample (wave-uniform; no division in the stage loop).  A
   // split may start or end inside a sample (kper >= T, so a sample meets at most two
   // splits): the share of the part before a split's end goes to slot 0, the part after a
@@ -2200,20 +2254,17 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
   int left = static_cast<int>(((sample + 1) * q.T - k_begin) / D::KB);
   bool started = sample * q.T == k_begin;  // the current sample starts inside this split
   auto flush = [&](bool ended) __attribute__((always_inline)) {
-    float d = 0.f;
+    float d0 = 0.f, d1 = 0.f;
 #pragma unroll
     for (int i = 0; i < C::MI; ++i)
 #pragma unroll
       for (int j = 0; j < C::NI; ++j)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const uint2 w = VHELD ? vr[VHELD ? i : 0][VHELD ? j : 0][g] : vload(i, j, g);
-          d += acc[i][j][4 * g] * __uint_as_float(w.x << 16) +
-               acc[i][j][4 * g + 1] * __uint_as_float(w.x & 0xFFFF0000u) +
-               acc[i][j][4 * g + 2] * __uint_as_float(w.y << 16) +
-               acc[i][j][4 * g + 3] * __uint_as_float(w.y & 0xFFFF0000u);
+        for (int h = 0; h < 2; ++h) {
+          const int k = (i * C::NI + j) * 2 + h;
+          acc_dot(acc[i][j], h, VHELD ? vr[VHELD ? k : 0] : vsrc[k * 64], d0, d1);
         }
-    d = wave_sum_dpp(d);
+    const float d = wave_sum_dpp(d0 + d1);
     const int slot = started ? 0 : 1;
     const bool whole = started && ended;
     float* pd = q.pdot + (tile * (C::WM * C::WN) + wid) * 2 * q.n_t + sample;
@@ -2277,8 +2328,16 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
   e.m_rows = p.M;
   e.n_cols = p.N;
   e.c_ld = p.N;
-  e.C = static_cast<float*>(p.out) + split * p.M * p.N;
-  store_epilogue<TrF32, C>(e, acc, mt, nt);
+  if (p.part_out) {
+    e.C = static_cast<float*>(p.out) + split * p.M * p.N;
+    store_epilogue<TrF32, C>(e, acc, mt, nt);
+  } else if (p.out != nullptr) {  // one split: the gradient itself
+    e.C = p.out;
+    if (p.out_f32)
+      store_epilogue<TrF32, C>(e, acc, mt, nt, p.alpha);
+    else
+      store_epilogue<TrBF16, C>(e, acc, mt, nt, p.alpha);
+  }
 }
 
 // Per-pair weight dots <V_j, G_i^T A_i> (V_j = G_j^T A_j of val sample j) from one sample's
@@ -2310,7 +2369,6 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tn_pair_kernel(TpParams q
   const TnParams& p = q.tn;
   __shared__ __attribute__((aligned(16))) unsigned char lds[D::STAGES * D::STAGE_BYTES];
   constexpr int NW = C::WM * C::WN;
-  constexpr int64_t WAVE_V = C::MI * C::NI * 2 * 64;  // uint4 of one wave's tile share
   const int64_t it = xcd_order(blockIdx.x, gridDim.x);
   const int64_t tiles = p.m_tiles * p.n_tiles;
   const int64_t grp = it / (q.group * q.n), rem = it - grp * q.group * q.n;
@@ -2330,42 +2388,22 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tn_pair_kernel(TpParams q
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if constexpr (!DOT) {
-    uint4* dst = q.V + ((smp * tiles + tile) * NW + wid) * WAVE_V + lane;
-#pragma unroll
-    for (int i = 0; i < C::MI; ++i)
-#pragma unroll
-      for (int j = 0; j < C::NI; ++j)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          uint4 w;
-          w.x = pack_bf16x2(acc[i][j][8 * h], acc[i][j][8 * h + 1]);
-          w.y = pack_bf16x2(acc[i][j][8 * h + 2], acc[i][j][8 * h + 3]);
-          w.z = pack_bf16x2(acc[i][j][8 * h + 4], acc[i][j][8 * h + 5]);
-          w.w = pack_bf16x2(acc[i][j][8 * h + 6], acc[i][j][8 * h + 7]);
-          dst[((i * C::NI + j) * 2 + h) * 64] = w;
-        }
+    acc_store<C, false>(q.V, smp * tiles + tile, wid, acc);
   } else {
     float* red = reinterpret_cast<float*>(lds);  // [NW][64]; the stages are free
     for (int64_t j0 = 0; j0 < q.n_val; j0 += 64) {
       const int nj = static_cast<int>(q.n_val - j0 < 64 ? q.n_val - j0 : 64);
       float mine = 0.f;  // lane jj: this wave's share of val sample j0 + jj
       for (int jj = 0; jj < nj; ++jj) {
-        const uint4* src = q.V + (((j0 + jj) * tiles + tile) * NW + wid) * WAVE_V + lane;
+        const uint4* src = q.V + acc_base<C>((j0 + jj) * tiles + tile, wid);
         float d0 = 0.f, d1 = 0.f;
 #pragma unroll
         for (int i = 0; i < C::MI; ++i)
 #pragma unroll
           for (int j = 0; j < C::NI; ++j)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              const uint4 w = src[((i * C::NI + j) * 2 + h) * 64];
-              const uint32_t u[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                d0 += acc[i][j][8 * h + 2 * e] * __uint_as_float(u[e] << 16);
-                d1 += acc[i][j][8 * h + 2 * e + 1] * __uint_as_float(u[e] & 0xFFFF0000u);
-              }
-            }
+            for (int h = 0; h < 2; ++h)
+              acc_dot(acc[i][j], h, src[((i * C::NI + j) * 2 + h) * 64], d0, d1);
         const float d = wave_sum_dpp(d0 + d1);
         mine = lane == jj ? d : mine;
       }
@@ -2868,8 +2906,8 @@ int tn_splits_raw(int64_t K, int64_t M, int64_t N, bool reduce_free = false) {
 int tn_splits(int64_t K, int64_t M, int64_t N, bool reduce_free = false) {
   return static_cast<int>(ceil_div(K, tn_kper(K, tn_splits_raw(K, M, N, reduce_free))));
 }
-int64_t tn_part_elems(int64_t K, int64_t M, int64_t N, bool reduce_free = false) {
-  const int sp = tn_splits(K, M, N, reduce_free);
+int64_t tn_part_elems(int64_t K, int64_t M, int64_t N) {
+  const int sp = tn_splits(K, M, N);
   return sp > 1 ? sp * M * N : 0;
 }
 
@@ -2896,8 +2934,6 @@ struct TnOut {
   float alpha = 1.f;
   int out_f32 = 0;
   int64_t gap_at = INT64_MAX, gap = 0;
-  float* vrows = nullptr;  // column-sum rows written before the launch (no vsum): the
-  int64_t vrows_n = 0;     //   reduction also folds these vrows_n rows into row 0
 };
 int launch_tn(const void* L, int64_t ldl, const void* R, int64_t ldr, int64_t K, int64_t M,
               int64_t N, void* out, float* part, hipStream_t s, float* vsum = nullptr,
@@ -2917,9 +2953,8 @@ int launch_tn(const void* L, int64_t ldl, const void* R, int64_t ldr, int64_t K,
   p.N = N;
   p.m_tiles = ceil_div(M, TnC::BM);
   p.n_tiles = ceil_div(N, TnC::BN);
-  const bool rf = o.vrows != nullptr && o.vrows_n > 1;  // the reduction runs anyway
-  p.kper = tn_kper(K, tn_splits_raw(K, M, N, rf));
-  const int sp = tn_splits(K, M, N, rf);
+  p.kper = tn_kper(K, tn_splits_raw(K, M, N));
+  const int sp = tn_splits(K, M, N);
   p.vsum = vsum;
   p.vsum_r = vsum_r ? 1 : 0;
   p.vparts = static_cast<int>(tn_vparts(M, N, vsum_r));
@@ -2939,15 +2974,13 @@ int launch_tn(const void* L, int64_t ldl, const void* R, int64_t ldr, int64_t K,
   else
     hipLaunchKernelGGL((tn_gemm_kernel<TnC, TnD, 2>), grid, dim3(TnC::NT), 0, s, p);
   int rc = check_launch("tn_gemm_kernel");
-  float* vs = vsum != nullptr ? vsum : o.vrows;
-  const int64_t vs_rows = vsum != nullptr ? tn_vsum_rows(K, M, N, vsum_r)
-                                          : (o.vrows != nullptr ? o.vrows_n : 1);
+  const int64_t vs_rows = vsum != nullptr ? tn_vsum_rows(K, M, N, vsum_r) : 1;
   if (rc || (!via_part && vs_rows <= 1)) return rc;
   const int64_t count = via_part ? M * N : 0;  // a multiple of 8 (N % 8 == 0)
   const int64_t vs_n = vsum_r ? N : M;
   hipLaunchKernelGGL(tn_reduce_kernel,
                      dim3(static_cast<unsigned>(ceil_div(std::max(count, vs_n) / 4, 256))),
-                     dim3(256), 0, s, part, count, sp, out, o.alpha, o.out_f32, vs, vs_n,
+                     dim3(256), 0, s, part, count, sp, out, o.alpha, o.out_f32, vsum, vs_n,
                      vs_rows);
   return check_launch("tn_reduce_kernel");
 }
@@ -3843,30 +3876,40 @@ bool layer_pass_pays(int algo, int64_t N, int64_t n_val, int64_t T, int64_t d_in
   return fused <= dots + grad;
 }
 struct TgBufs {
-  uint16_t *abar, *gbar, *V;
+  uint16_t *abar, *gbar;
+  uint4* V;
   float *vpart, *vp, *pdot, *csum, *pbias, *tgpart;
 };
+// The V GEMM of the pass: the train GEMM's orientation and tiles; wide tiles unsplit, narrow ones
+// by the split estimate.  With the presum and a bias its reduction launch also folds the presum
+// kernel's column-sum rows (more than one when T > PS_T) whatever the splits.
+int64_t tg_area(const TgPlan& t) {
+  return t.m_tiles * t.n_tiles * (t.wide ? TnCW::BM * TnCW::BN : TnC::BM * TnC::BN);
+}
+int64_t tg_vsplits(const TgPlan& t, int64_t T, int64_t d_in, int64_t d_out) {
+  return t.wide ? 1 : tn_splits(t.vk, d_out, d_in, t.presum && t.bias && presum_rows(T) > 1);
+}
+int64_t tg_vparts(const TgPlan& t) {
+  return std::min<int64_t>(4, t.bias_a ? t.m_tiles : t.n_tiles);
+}
 template <class S>
 TgBufs carve_tg(S& c, const TgPlan& t, int64_t T, int64_t d_in, int64_t d_out) {
   TgBufs b{};
   b.abar = t.presum ? c.template take<uint16_t>(T * d_in) : nullptr;
   b.gbar = t.presum ? c.template take<uint16_t>(T * d_out) : nullptr;
-  b.V = c.template take<uint16_t>(d_out * d_in);  // V^T, [d_in][d_out]
-  // Presum with a bias: the V GEMM's reduction also folds the presum kernel's column-sum rows
-  // (more than one when T > PS_T), as launch_tn sizes it.
-  b.vpart = c.template take<float>(
-      tn_part_elems(t.vk, d_out, d_in, t.presum && t.bias && presum_rows(T) > 1));
+  b.V = c.template take<uint4>(tg_area(t) / 8);
+  const int64_t vsp = tg_vsplits(t, T, d_in, d_out);
+  b.vpart = vsp > 1 ? c.template take<float>(vsp * tg_area(t)) : nullptr;
   // Val column sums of G: the V GEMM's own partials for the pairwise semantics (its operands
   // are the val rows as they lie); for the presum, whose V operands are rounded to bf16, the
   // presum kernel's fp32 sums.
-  const int64_t vp_rows =
-      t.presum ? presum_rows(T) : tn_vsum_rows(t.vk, d_in, d_out, !t.bias_a);
+  const int64_t vp_rows = t.presum ? presum_rows(T) : vsp * tg_vparts(t);
   b.vp = t.bias ? c.template take<float>(vp_rows * t.bias_d) : nullptr;
   b.pdot = c.template take<float>(t.m_tiles * t.n_tiles * (t.wm * t.wn) * 2 * t.n_t);
   b.csum = t.bias ? c.template take<float>(t.n_t * 2 * (t.Tp / TnD::KB) * t.bias_d) : nullptr;
   const int64_t bw = t.bias_a ? t.n_tiles * t.wn : t.m_tiles * t.wm;
   b.pbias = t.bias ? c.template take<float>(t.n_t * (t.Tp / TnD::KB) * bw) : nullptr;
-  b.tgpart = c.template take<float>(t.sp * d_out * d_in);
+  b.tgpart = t.sp > 1 ? c.template take<float>(t.sp * d_out * d_in) : nullptr;
   return b;
 }
 }  // namespace
@@ -3976,11 +4019,9 @@ int dot_train_grad(const char* name, bool bias_a, bool any_T, const void* A, con
   const E* Gp = static_cast<const E*>(G);
   const E* La = Ap + val_start * T * d_in;
   const E* Lg = Gp + val_start * T * d_out;
-  // V^T = A_val^T G_val (or the product of the val rows presummed per position); with a bias,
-  // the val rows' column sums of G in fp32 from the rows as they lie: from the V GEMM's
-  // workgroups (pairwise) or the presum kernel (presum), as partial rows the V GEMM's
-  // reduction folds into row 0.
-  TnOut vo;
+  // V = G_val^T A_val (or the product of the val rows presummed per position); with a bias, the
+  // val rows' column sums of G in fp32 from the rows as they lie: from the V GEMM's workgroups
+  // (pairwise) or the presum kernel (presum), as partial rows the reduction folds into row 0.
   if (t.presum) {
     PresumPair pp{};
     pp.in[0] = Ap;
@@ -3995,14 +4036,58 @@ int dot_train_grad(const char* name, bool bias_a, bool any_T, const void* A, con
     if (rc) return rc;
     La = b.abar;
     Lg = b.gbar;
-    if (b.vp != nullptr) {
-      vo.vrows = b.vp;
-      vo.vrows_n = presum_rows(T);
-    }
   }
-  int rc = launch_tn(La, d_in, Lg, d_out, t.vk, d_in, d_out, b.V, b.vpart, s,
-                     t.presum ? nullptr : b.vp, !t.bias_a, vo);
+  const int64_t vsp = tg_vsplits(t, T, d_in, d_out);
+  TnParams v{};
+  v.L = Lg;
+  v.R = La;
+  v.ldl = v.M = d_out;
+  v.ldr = v.N = d_in;
+  v.l_nbytes = t.vk * d_out * 2;
+  v.r_nbytes = t.vk * d_in * 2;
+  v.K = t.vk;
+  v.kper = vsp > 1 ? tn_kper(t.vk, static_cast<int>(vsp)) : t.vk;
+  v.m_tiles = t.m_tiles;
+  v.n_tiles = t.n_tiles;
+  v.out = vsp > 1 ? static_cast<void*>(b.vpart) : b.V;
+  v.part_out = vsp > 1 ? 1 : 0;
+  v.acc_order = 1;
+  v.alpha = 1.f;
+  v.vsum = t.presum ? nullptr : b.vp;
+  v.vparts = static_cast<int>(tg_vparts(t));
+  v.gap_at = INT64_MAX;
+  const int vcs = v.vsum == nullptr ? 0 : (t.bias_a ? 2 : 1);
+  const int64_t vitems = t.m_tiles * t.n_tiles * vsp;
+  if (vitems > INT32_MAX) return fail(GS_ERR_UNSUPPORTED, "GEMM grid too large");
+  auto go_v = [&](auto wide, auto csk) {
+    constexpr bool W = decltype(wide)::value;
+    using C = std::conditional_t<W, TnCW, TnC>;
+    using D = std::conditional_t<W, TnDW, TnD>;
+    hipLaunchKernelGGL((tn_gemm_kernel<C, D, decltype(csk)::value>),
+                       dim3(static_cast<unsigned>(vitems)), dim3(C::NT), 0, s, v);
+  };
+  auto go_vcs = [&](auto wide) {
+    if (vcs == 0)
+      go_v(wide, std::integral_constant<int, 0>{});
+    else if (vcs == 1)
+      go_v(wide, std::integral_constant<int, 1>{});
+    else
+      go_v(wide, std::integral_constant<int, 2>{});
+  };
+  t.wide ? go_vcs(std::true_type{}) : go_vcs(std::false_type{});
+  int rc = check_launch("tn_gemm_kernel (V)");
   if (rc) return rc;
+  const int64_t vs_rows = b.vp == nullptr ? 1 : t.presum ? presum_rows(T) : vsp * v.vparts;
+  // Four column-sum rows or fewer are added by the train launch itself (a launch of 4-6 us less).
+  if (vsp > 1 || vs_rows > 4) {
+    const int64_t count = vsp > 1 ? tg_area(t) : 0;
+    hipLaunchKernelGGL(tn_reduce_kernel,
+                       dim3(static_cast<unsigned>(ceil_div(std::max(count, t.bias_d) / 4, 256))),
+                       dim3(256), 0, s, b.vpart, count, static_cast<int>(vsp), b.V, 1.f, 0, b.vp,
+                       t.bias_d, vs_rows);
+    rc = check_launch("tn_reduce_kernel");
+    if (rc) return rc;
+  }
   // The train rows: dots at every sample boundary, train-gradient partials per split.
   TgParams q{};
   TnParams& p = q.tn;
@@ -4020,16 +4105,19 @@ int dot_train_grad(const char* name, bool bias_a, bool any_T, const void* A, con
   p.N = d_in;
   p.m_tiles = t.m_tiles;
   p.n_tiles = t.n_tiles;
-  p.out = b.tgpart;
-  p.part_out = 1;
-  p.alpha = 1.f;
-  q.Vt = b.V;
+  const bool direct = t.sp == 1;  // unsplit: the gradient is written here, scaled and rounded
+  p.out = direct ? out_grad : static_cast<void*>(b.tgpart);
+  p.part_out = direct ? 0 : 1;
+  p.alpha = grad_scale;
+  p.out_f32 = grad_dtype == GS_DTYPE_F32 ? 1 : 0;
+  q.V = b.V;
   q.T = t.Tp;
   q.T_rows = T;
   q.n_t = t.n_t;
   q.pdot = b.pdot;
   q.csum = b.csum;
   q.vb = b.vp;
+  q.vb_rows = vsp > 1 || vs_rows > 4 ? 1 : static_cast<int>(vs_rows);
   q.pbias = b.pbias;
   const int64_t items = t.m_tiles * t.n_tiles * t.sp;
   if (items > INT32_MAX) return fail(GS_ERR_UNSUPPORTED, "GEMM grid too large");
@@ -4062,8 +4150,8 @@ int dot_train_grad(const char* name, bool bias_a, bool any_T, const void* A, con
   return launch_tgdot_finish(b.pdot, shares, t.n_t, out_bias_dot != nullptr ? b.pbias : nullptr,
                              bshares, b.csum, 2 * sps, t.bias_d, out_dot, dot_dtype,
                              out_bias_dot, bias_dot_dtype, out_bias_grad, bias_grad_dtype,
-                             bias_grad_scale, b.tgpart, out_grad != nullptr ? d_out * d_in : 0,
-                             t.sp, out_grad, grad_dtype, grad_scale, s);
+                             bias_grad_scale, b.tgpart,
+                             out_grad != nullptr && !direct ? d_out * d_in : 0, t.sp, out_grad, grad_dtype, grad_scale, s);
 }
 }  // namespace
 }  // namespace gs
