@@ -11,6 +11,7 @@ samplers call ``ops()``); product code never does.
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from typing import Optional, Tuple
 
@@ -103,6 +104,8 @@ _SIGNATURES = {
 def load_library() -> ctypes.CDLL:
     """Loads libghost_hip.so (built in-tree by ghostsuite_amd.build) once per process."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib
@@ -156,8 +159,16 @@ def _require_device(*ts: torch.Tensor) -> torch.device:
     return dev
 
 
-def _stream(dev: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+def _stream(dev: torch.device) -> int:
+    """The current stream's handle (without the stream object torch.cuda.current_stream makes)."""
+    idx = dev.index if dev.index is not None else torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(idx)
+
+
+@functools.lru_cache(maxsize=4096)
+def _size(query: str, *args: int) -> int:
+    """A workspace query's answer: the host plan of the call, which depends on its sizes alone."""
+    return getattr(load_library(), query)(*args)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -355,8 +366,8 @@ class HipOps:
         bias = bias_grad_dtype is not None
         dt = _gs_dtype(A)
         lib = load_library()
-        ws_bytes = lib.gs_linear_layer_pass_workspace(dt, N, n_val, T, d_in, d_out, semantics,
-                                                      int(conv1d), int(bias), algo, rounding)
+        ws_bytes = _size("gs_linear_layer_pass_workspace", dt, N, n_val, T, d_in, d_out,
+                         semantics, int(conv1d), int(bias), algo, rounding)
         if ws_bytes == 0:
             return None
         ws = _workspace(ws_bytes, dev)
@@ -531,7 +542,7 @@ class HipOps:
         T = _tokens(G, N, d)
         vs = N - n_val if val_start is None else int(val_start)
         lib = load_library()
-        ws_bytes = lib.gs_bias_dot_workspace(N, T, d)
+        ws_bytes = _size("gs_bias_dot_workspace", N, T, d)
         ws = _workspace(ws_bytes, dev)
         out = torch.empty(N - n_val, dtype=torch.float32, device=dev)
         grad = None
@@ -555,7 +566,7 @@ class HipOps:
             raise GhostHipError(f"ids {tuple(ids.shape)} and G {tuple(G.shape)} disagree")
         vs = N - n_val if val_start is None else int(val_start)
         lib = load_library()
-        ws_bytes = lib.gs_embedding_dot_workspace(N, n_val, T, d, vocab)
+        ws_bytes = _size("gs_embedding_dot_workspace", N, n_val, T, d, vocab)
         if ws_bytes == 0:
             raise GhostHipError(f"gs_embedding_dot: invalid arguments N={N} n_val={n_val}")
         ws = _workspace(ws_bytes, dev)
@@ -582,7 +593,7 @@ class HipOps:
         vocab = out.shape[0]
         vs = N - n_val if val_start is None else int(val_start)
         lib = load_library()
-        ws_bytes = lib.gs_embedding_train_grad_workspace(N, n_val, T, d, vocab)
+        ws_bytes = _size("gs_embedding_train_grad_workspace", N, n_val, T, d, vocab)
         if ws_bytes == 0:
             raise GhostHipError(f"gs_embedding_train_grad: invalid arguments N={N} n_val={n_val}")
         ws = _workspace(ws_bytes, dev)
@@ -606,7 +617,7 @@ class HipOps:
         T = _tokens(X, N, F)
         vs = N - n_val if val_start is None else int(val_start)
         lib = load_library()
-        ws_bytes = lib.gs_layernorm_dot_workspace(N, T, F)
+        ws_bytes = _size("gs_layernorm_dot_workspace", N, T, F)
         ws = _workspace(ws_bytes, dev)
         n_t = N - n_val
         dw = torch.empty(n_t, dtype=torch.float32, device=dev) if want_dot else None
@@ -648,7 +659,7 @@ class HipOps:
                 raise GhostHipError("projection widths do not match the layer (Conv1D roles)")
             shape = (B, k_i, k_o)
         lib = load_library()
-        ws_bytes = lib.gs_kron_proj_workspace(B, T, k_i, k_o)
+        ws_bytes = _size("gs_kron_proj_workspace", B, T, k_i, k_o)
         ws = _workspace(ws_bytes, dev)
         out = torch.empty(shape, dtype=out_dtype, device=dev)
         rc = lib.gs_kron_proj(A.data_ptr(), G.data_ptr(), _gs_dtype(A), B, T, n_a, n_g,

@@ -1,10 +1,11 @@
 """Side-stream execution of the per-layer dot-product kernels, overlapped with the rest of
 the backward pass.
 
-A backward hook enqueues its layer's dot kernels on a second HIP stream (default priority)
-after that stream has waited for everything the autograd stream enqueued so far.  The
-hook's input tensors are marked as in use by the side stream, so the caching allocator
-does not hand their memory back to the autograd stream before the side kernels finish.
+The backward hook of a layer with enough work to overlap enqueues its kernels on a second
+HIP stream (default priority) after that stream has waited for everything the autograd
+stream enqueued so far.  The hook's input tensors are marked as in use by the side stream, so
+the caching allocator does not hand their memory back to the autograd stream before the side
+kernels finish.
 At the end of the backward pass an autograd-engine callback makes the autograd stream wait
 for the side stream, so the optimizer, the engines' aggregation and any host copy see
 finished results.  ``join(device)`` does the same wait explicitly (the engines call it
@@ -12,10 +13,12 @@ before reading results, which also covers a backward pass that raised).
 
 Memory written on the side stream and later read on the autograd stream needs no extra
 bookkeeping: every later side-stream launch is preceded by a wait on the autograd stream.
+A train gradient that one layer stored on the autograd stream and another adds to on the side
+stream (or the other way round) is kept by its parameter until after that wait, and the adding
+layer joins first.
 """
 from __future__ import annotations
 
-import contextlib
 import threading
 from typing import Dict
 
@@ -24,6 +27,7 @@ import torch
 _lock = threading.Lock()
 _streams: Dict[int, torch.cuda.Stream] = {}
 _join_queued: Dict[int, bool] = {}
+_events = threading.local()   # per thread: {device index: the event of _wait}
 
 enabled = True
 
@@ -36,6 +40,21 @@ def side_stream(device: torch.device) -> torch.cuda.Stream:
             s = torch.cuda.Stream(device=idx)   # default priority
             _streams[idx] = s
     return s
+
+
+def _wait(idx: int, waiter: torch.cuda.Stream, on: torch.cuda.Stream) -> None:
+    """`waiter` waits for what `on` holds so far, through one event kept per thread and device (a
+    wait refers to the record before it; recording again does not reach earlier waits).  Under
+    graph capture the event belongs to the graph, so each wait takes its own."""
+    if torch.cuda.is_current_stream_capturing():
+        waiter.wait_stream(on)
+        return
+    events = _events.__dict__.setdefault("by_device", {})
+    ev = events.get(idx)
+    if ev is None:
+        ev = events[idx] = torch.cuda.Event()
+    ev.record(on)
+    ev.wait(waiter)
 
 
 def join(device=None) -> None:
@@ -71,30 +90,46 @@ def _queue_join(idx: int, cur: torch.cuda.Stream, side: torch.cuda.Stream) -> No
         _join_queued.pop(idx, None)
 
 
-@contextlib.contextmanager
-def on_side_stream(*tensors):
-    """Runs the body on the side stream of the tensors' device (no-op on CPU or when
-    disabled).  The tensors are the body's inputs produced on the current stream."""
-    ts = [t for t in tensors if isinstance(t, torch.Tensor)]
-    if not enabled or not ts or ts[0].device.type != "cuda":
-        yield
-        return
-    dev = ts[0].device
-    idx = dev.index if dev.index is not None else torch.cuda.current_device()
-    side = side_stream(dev)
-    cur = torch.cuda.current_stream(idx)
-    side.wait_stream(cur)
-    for t in ts:
-        t.record_stream(side)
-    if torch.cuda.current_device() == idx:
-        # Same device: switch the current stream only (the stream context manager also
-        # saves and restores the current device, several times the cost per hook).
-        torch.cuda.set_stream(side)
-        try:
-            yield
-        finally:
-            torch.cuda.set_stream(cur)
-    else:
-        with torch.cuda.stream(side):
-            yield
-    _queue_join(idx, cur, side)
+class on_side_stream:
+    """``with on_side_stream(*tensors):`` runs the body on the side stream of the tensors' device
+    (no-op on CPU or when disabled).  The tensors are the body's inputs produced on the current
+    stream."""
+
+    __slots__ = ("_tensors", "_idx", "_cur", "_side", "_ctx")
+
+    def __init__(self, *tensors):
+        self._tensors = tensors
+        self._side = self._ctx = None
+
+    def __enter__(self):
+        ts = [t for t in self._tensors if isinstance(t, torch.Tensor)]
+        if not enabled or not ts or ts[0].device.type != "cuda":
+            return self
+        dev = ts[0].device
+        here = torch.cuda.current_device()
+        self._idx = idx = dev.index if dev.index is not None else here
+        side = side_stream(dev)
+        self._cur = torch.cuda.current_stream(idx)
+        _wait(idx, side, self._cur)
+        for t in ts:
+            t.record_stream(side)
+        if here == idx:
+            # Same device: switch the current stream only (the stream context manager also
+            # saves and restores the current device, several times the cost per hook).
+            torch.cuda.set_stream(side)
+        else:
+            self._ctx = torch.cuda.stream(side)
+            self._ctx.__enter__()
+        self._side = side
+        return self
+
+    def __exit__(self, exc_type, exc, tb):
+        if self._side is None:
+            return False
+        if self._ctx is not None:
+            self._ctx.__exit__(exc_type, exc, tb)
+        else:
+            torch.cuda.set_stream(self._cur)
+        if exc_type is None:
+            _queue_join(self._idx, self._cur, self._side)
+        return False

@@ -64,6 +64,40 @@ def to_host_async(t: torch.Tensor) -> Tuple[torch.Tensor, Optional[torch.cuda.Ev
     return host, ev
 
 
+def trees_to_host_async(datas: List[Any], events: List[torch.cuda.Event]) -> List[Any]:
+    """``tree_to_host_async`` of several trees with one stream wait and one event for all of their
+    CUDA tensors of a device."""
+    jobs: Dict[int, list] = {}
+
+    def host(x):
+        if isinstance(x, dict):
+            return {k: host(v) for k, v in x.items()}
+        if not isinstance(x, torch.Tensor):
+            return x
+        if x.device.type != "cuda":
+            return x.detach().clone()
+        idx = x.device.index if x.device.index is not None else torch.cuda.current_device()
+        out = torch.empty(x.shape, dtype=x.dtype, pin_memory=True)
+        with torch.cuda.device(idx):
+            src = x.detach().clone()   # ordered before anything the caller enqueues on x later
+        jobs.setdefault(idx, []).append((out, src))
+        return out
+
+    outs = [host(x) for x in datas]
+    for idx, pairs in jobs.items():
+        cs = _copy_stream(idx)
+        cs.wait_stream(torch.cuda.current_stream(idx))
+        with torch.cuda.stream(cs):
+            for out, src in pairs:
+                out.copy_(src, non_blocking=True)
+            ev = torch.cuda.Event()
+            ev.record(cs)
+        for _, src in pairs:
+            src.record_stream(cs)
+        events.append(ev)
+    return outs
+
+
 def tree_to_host_async(data: Any, events: List[torch.cuda.Event]) -> Any:
     """``to_host_async`` over a tensor or a dict of tensors (the shapes the engines log)."""
     if isinstance(data, dict):

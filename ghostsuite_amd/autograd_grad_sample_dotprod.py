@@ -21,6 +21,7 @@ import torch.nn as nn
 from . import _overlap
 from .supported_layers_grad_samplers_dotprod import (
     APPLIED,
+    _param,
     _supported_layers_dotprod,
     _create_or_accumulate_train_grad,
     options,
@@ -93,16 +94,17 @@ def _new_step(module, inputs):
 
 def _capture_activations(layer: nn.Module, inputs: Tuple, outputs: Tuple):
     """Forward hook: caches the (detached) layer input (reference :92-94)."""
-    layer.activations = inputs[0].detach()
-    layer._gs_fwd_seq = (_current_step[0], next(_fwd_counter))
+    d = layer.__dict__   # plain attributes, without nn.Module.__setattr__'s searches
+    d["activations"] = inputs[0].detach()
+    d["_gs_fwd_seq"] = (_current_step[0], next(_fwd_counter))
 
 
 def _prepare_sample_grad_or_dotprod(layer: nn.Module, grad_output: Tuple[torch.Tensor],
                                     val_batch_size: int, loss_reduction: str = 'mean'):
     """Backward-hook stage 1: the layer's dot products (reference :97-137)."""
     backprops = grad_output[0].detach()
-    if not hasattr(layer, 'activations'):
-        layer.activations = None
+    d = layer.__dict__
+    d.setdefault("activations", None)
     compute_layer_dotprod, _ = _supported_layers_dotprod.get(type(layer))
 
     scale = float(backprops.shape[0]) if loss_reduction == 'mean' else 1.0
@@ -110,12 +112,13 @@ def _prepare_sample_grad_or_dotprod(layer: nn.Module, grad_output: Tuple[torch.T
     if n_train > 0:
         # Train-gradient scales for the fused bias / LayerNorm passes.  The bias path always
         # divides by n_train (_apply_train_grad is called without loss_reduction, :67).
-        layer._gs_bias_grad_scale = scale / n_train
-        layer._gs_ln_grad_scale = scale / n_train
+        d["_gs_bias_grad_scale"] = scale / n_train
+        d["_gs_ln_grad_scale"] = scale / n_train
 
-    acts = layer.activations
+    acts = d["activations"]
     # The dot kernels run on a side stream, overlapped with the rest of backward.
-    side = _overlap.on_side_stream(acts, backprops) if options["overlap"] else \
+    side = _overlap.on_side_stream(acts, backprops) \
+        if options["overlap"] and _worth_overlapping(layer, acts, backprops) else \
         contextlib.nullcontext()
     with side:
         if acts is not None and acts.dtype != backprops.dtype and acts.is_floating_point():
@@ -132,8 +135,8 @@ def _prepare_sample_grad_or_dotprod(layer: nn.Module, grad_output: Tuple[torch.T
         else:
             compute_layer_dotprod(layer, acts, backprops, val_batch_size=val_batch_size)
 
-    layer.backprops = backprops
-    layer.backprops_scale = scale
+    d["backprops"] = backprops
+    d["backprops_scale"] = scale
 
 
 def _apply_train_grad(layer: nn.Module, val_batch_size: int, loss_reduction: str = 'mean'):
@@ -143,15 +146,16 @@ def _apply_train_grad(layer: nn.Module, val_batch_size: int, loss_reduction: str
         raise ValueError(
             f"Layer {layer.__class__.__name__} is not supported for training gradient "
             "computation. Ensure it is included in the _supported_layers_dotprod dictionary.")
-    scale = getattr(layer, "backprops_scale", 1.0)
+    scale = layer.__dict__.get("backprops_scale", 1.0)
     # The train-gradient kernels join the layer's dot kernels on the side stream: both read
     # only this layer's activations and backprops, and the end-of-backward join orders
     # param.train_grad before the optimizer reads it.  When the dot stage already formed
     # every train gradient, nothing is enqueued here but an add_ into an existing train_grad
     # (after a join), so the side stream is left alone.
-    side = _overlap.on_side_stream(layer.__dict__.get("activations"),
-                                   layer.__dict__.get("backprops")) \
-        if options["overlap"] and not _train_grads_parked(layer) else contextlib.nullcontext()
+    acts, backprops = layer.__dict__.get("activations"), layer.__dict__.get("backprops")
+    side = _overlap.on_side_stream(acts, backprops) \
+        if options["overlap"] and not _train_grads_parked(layer) and \
+        _worth_overlapping(layer, acts, backprops) else contextlib.nullcontext()
     try:
         with side:
             _apply_train_grad_body(layer, compute_layer_train_grad, val_batch_size, scale,
@@ -163,16 +167,35 @@ def _apply_train_grad(layer: nn.Module, val_batch_size: int, loss_reduction: str
             layer.__dict__.pop(attr, None)
 
 
+# Below this much work a layer's kernels run on the autograd stream: entering the side stream
+# costs the host 29 us a hook (an event recorded, waited for, and the stream switched; MI355X, one
+# hook), while such kernels take about 10 us and leave little to overlap.  Measured with everything
+# on the side stream / with this rule: an engine step of a 512-1024-1024-10 fp32 MLP of 80 rows
+# 1420 / 1160 us, of a four-layer GPT-2 of 10 rows x 512 tokens (its LayerNorms and embeddings are
+# below, its Linears above) 7113 / 6755 us.
+_INLINE_ELEMENTS = 8 << 20     # of the layer's input and output gradient together
+_INLINE_FLOPS = 1e9            # of one product of the two
+
+
+def _worth_overlapping(layer: nn.Module, acts, backprops) -> bool:
+    if not isinstance(acts, torch.Tensor) or not isinstance(backprops, torch.Tensor):
+        return True
+    if acts.numel() + backprops.numel() > _INLINE_ELEMENTS:
+        return True
+    return not isinstance(layer, (nn.LayerNorm, nn.Embedding)) and \
+        2.0 * acts.numel() * backprops.shape[-1] > _INLINE_FLOPS
+
+
 def _train_grads_parked(layer: nn.Module) -> bool:
     """True when the dot stage parked every train gradient this layer applies."""
     d = layer.__dict__
     if isinstance(layer, nn.LayerNorm):
         return "_gs_ln_train_grads" in d
-    w = getattr(layer, "weight", None)
+    w = _param(layer, "weight")
     if w is None or not getattr(w, "initially_requires_grad", False) or \
             "_gs_weight_train_grad" not in d:
         return False
-    b = getattr(layer, "bias", None)
+    b = _param(layer, "bias")
     return b is None or not getattr(b, "initially_requires_grad", False) or \
         "_gs_bias_train_grad" in d
 
@@ -184,26 +207,26 @@ def _apply_train_grad_body(layer: nn.Module, compute_layer_train_grad, val_batch
         compute_layer_train_grad(layer, layer.activations, layer.backprops, val_batch_size,
                                  scale=scale)
     else:
-        if hasattr(layer, 'weight') and layer.weight.initially_requires_grad:
+        weight, bias = _param(layer, "weight"), _param(layer, "bias")
+        if weight is not None and weight.initially_requires_grad:
             grad_weight = compute_layer_train_grad(layer, layer.activations, layer.backprops,
                                                    val_batch_size, scale=scale)
             if grad_weight is APPLIED:
                 pass   # the sampler added into param.train_grad itself
             elif grad_weight is not None:
-                _create_or_accumulate_train_grad(layer.weight, grad_weight)
+                _create_or_accumulate_train_grad(weight, grad_weight)
             else:
                 raise ValueError(
                     f"Layer {layer.__class__.__name__} returned None for weight gradient. "
                     "Ensure the compute_layer_train_grad function is implemented correctly.")
-        if hasattr(layer, 'bias') and layer.bias is not None and \
-                layer.bias.initially_requires_grad:
+        if bias is not None and bias.initially_requires_grad:
             grad_bias = layer.__dict__.pop("_gs_bias_train_grad", None)
             if grad_bias is None:
                 grad_bias = _compute_train_grad_bias(layer.backprops, val_batch_size,
                                                      loss_reduction=loss_reduction)
                 if scale != 1.0:
                     grad_bias = grad_bias * scale
-            _create_or_accumulate_train_grad(layer.bias, grad_bias)
+            _create_or_accumulate_train_grad(bias, grad_bias)
 
 
 def _compute_train_grad_bias(B: torch.Tensor, val_batch_size: int,

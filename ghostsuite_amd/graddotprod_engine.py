@@ -169,10 +169,12 @@ class GradDotProdEngine:
             # Same record as the reference, but the host copies are asynchronous (pinned
             # memory, copy stream): the step does not wait for the GPU here.
             events = []
+            dots, x_host, y_host = async_io.trees_to_host_async(
+                [total, self.X_train, self.Y_train], events)
             self.dot_product_log.append_pending({
-                'dot_product': async_io.tree_to_host_async(total, events),
-                'X_train': async_io.tree_to_host_async(self.X_train, events),
-                'Y_train': async_io.tree_to_host_async(self.Y_train, events),
+                'dot_product': dots,
+                'X_train': x_host,
+                'Y_train': y_host,
                 'iter_num': self.iter_num,
                 'batch_idx': self.batch_idx,
             }, events)

@@ -82,7 +82,7 @@ def _should_use_ghost_computation(layer: nn.Module, A: torch.Tensor, B: torch.Te
                                   conv: bool = False):
     """Caches ``layer.use_ghost_computation = 2*T^2 <= weight.numel()`` on the first call
     (reference :7-41; never reset)."""
-    if hasattr(layer, "use_ghost_computation"):
+    if "use_ghost_computation" in layer.__dict__ or hasattr(layer, "use_ghost_computation"):
         return
     if not conv:
         T = math.prod(A.shape[1:-1]) if A.dim() > 2 else 1
@@ -101,6 +101,15 @@ def _create_or_accumulate_train_grad(param: torch.Tensor, grad: torch.Tensor) ->
         param.train_grad.add_(new_grad)
     else:
         param.train_grad = new_grad
+
+
+def _param(layer: nn.Module, name: str) -> Optional[torch.Tensor]:
+    """layer.<name>, None where there is none: straight from the module's parameters (an attribute
+    that is no plain one costs nn.Module.__getattr__'s searches at every access)."""
+    params = layer.__dict__.get("_parameters")
+    if params is not None and name in params:
+        return params[name]
+    return getattr(layer, name, None)
 
 
 def _train_split(A: torch.Tensor, val_batch_size: int):
@@ -124,7 +133,8 @@ def _reference_dtypes(layer: nn.Module, weight_dtype: Optional[torch.dtype],
     :552-559 in bf16); its ghost branches sum in fp32 (:129-130, :437, :550)."""
     if options["dot_dtypes"] != "reference" or options["precision"] == "fp32":
         return
-    for param, dt in ((layer.weight, weight_dtype), (getattr(layer, "bias", None), bias_dtype)):
+    for param, dt in ((_param(layer, "weight"), weight_dtype),
+                      (_param(layer, "bias"), bias_dtype)):
         if param is None or dt is None:
             continue
         dot = param.__dict__.get("grad_dot_prod")
@@ -148,10 +158,10 @@ def _overwritten_later(layer: nn.Module) -> bool:
     assignment of ``grad_dot_prod`` replaces this layer's."""
     if not options["skip_overwritten_tied_dots"]:
         return False
-    emb = getattr(layer, "_gs_tied_embedding", None)
+    emb = layer.__dict__.get("_gs_tied_embedding")
     if emb is None:
         return False
-    mine, theirs = getattr(layer, "_gs_fwd_seq", None), getattr(emb, "_gs_fwd_seq", None)
+    mine, theirs = layer.__dict__.get("_gs_fwd_seq"), emb.__dict__.get("_gs_fwd_seq")
     return mine is not None and theirs is not None and theirs[0] == mine[0] and theirs[1] < mine[1]
 
 
@@ -222,11 +232,11 @@ def _linear_dots(layer: nn.Linear, A: torch.Tensor, B: torch.Tensor, val_batch_s
         dt = _dot_dtype(A, pairwise)
         if _fused_dot_train_grad(layer, A, B, val_batch_size, pairwise, dt):
             return
-        if layer.bias is not None and _fused_bias_dot(layer, A, B, val_batch_size, pairwise, dt,
-                                                      _dot_dtype(B, False)):
+        if _param(layer, "bias") is not None and \
+                _fused_bias_dot(layer, A, B, val_batch_size, pairwise, dt, _dot_dtype(B, False)):
             return
         _linear_like_dot(layer, A, B, val_batch_size, pairwise, dt)
-    if layer.bias is not None:
+    if _param(layer, "bias") is not None:
         _bias_dot_and_grad(layer, B, val_batch_size, _dot_dtype(B, False))
 
 
@@ -243,15 +253,17 @@ def _fused_dot_train_grad(layer: nn.Module, A: torch.Tensor, B: torch.Tensor,
     With ``conv1d`` (HF Conv1D, weight [d_in, d_out]) the kernels run the same pass with the operands swapped: the dot <G_i^T A_i, V> equals <A_i^T G_i, V^T>, the train
     gradient comes out as the sum of A_i^T G_i (the Conv1D layout), and the bias terms come
     from the column sums of G as for a Linear layer."""
-    scale = getattr(layer, "_gs_bias_grad_scale", None)
-    bias = layer.bias is not None
+    d = layer.__dict__
+    scale = d.get("_gs_bias_grad_scale")
+    weight, bias_p = _param(layer, "weight"), _param(layer, "bias")
+    bias = bias_p is not None
     grad_dtypes = (torch.bfloat16, torch.float32)   # train gradients in the parameters' dtype
     if scale is None or dtype not in (torch.bfloat16, torch.float32) or A.dtype != dtype or \
             (dtype == torch.float32 and B.dtype != dtype) or (pairwise and options["store_pairs"]) or \
-            layer.weight.dtype not in grad_dtypes or \
-            not getattr(layer.weight, "initially_requires_grad", False) or \
-            (bias and (layer.bias.dtype not in grad_dtypes or
-                       not getattr(layer.bias, "initially_requires_grad", False))):
+            weight.dtype not in grad_dtypes or \
+            not getattr(weight, "initially_requires_grad", False) or \
+            (bias and (bias_p.dtype not in grad_dtypes or
+                       not getattr(bias_p, "initially_requires_grad", False))):
         return False
     Bc = B.to(dtype) if B.dtype != dtype else B
     sem = _native.SEM_PAIRWISE_SUM if pairwise else _native.SEM_PRESUM
@@ -261,8 +273,8 @@ def _fused_dot_train_grad(layer: nn.Module, A: torch.Tensor, B: torch.Tensor,
         weight_dt, bias_dt = _dot_result_dtypes(layer, A, B, conv1d)
         res = layer_pass(A, Bc, val_batch_size, semantics=sem, algo=algo,
                          rounding=_ROUNDINGS[options["rounding"]], conv1d=conv1d,
-                         grad_scale=scale, grad_dtype=layer.weight.dtype, dot_dtype=weight_dt,
-                         bias_grad_dtype=layer.bias.dtype if bias else None,
+                         grad_scale=scale, grad_dtype=weight.dtype, dot_dtype=weight_dt,
+                         bias_grad_dtype=bias_p.dtype if bias else None,
                          bias_dot_dtype=bias_dt)
     elif dtype != torch.bfloat16:
         return False
@@ -273,18 +285,18 @@ def _fused_dot_train_grad(layer: nn.Module, A: torch.Tensor, B: torch.Tensor,
                              False) != _native.ALGO_VALGRAD:
             return False
         res = ops().linear_dot_train_grad(A, Bc, val_batch_size, semantics=sem,
-                                          grad_scale=scale, grad_dtype=layer.weight.dtype,
+                                          grad_scale=scale, grad_dtype=weight.dtype,
                                           bias=bias, bias_grad_scale=scale,
-                                          bias_grad_dtype=layer.bias.dtype if bias else None,
+                                          bias_grad_dtype=bias_p.dtype if bias else None,
                                           conv1d=conv1d)
     if res is None:
         return False
     dot, grad, bias_dot, bias_grad = res
-    layer.weight.grad_dot_prod = dot
-    layer._gs_weight_train_grad = grad
+    weight.grad_dot_prod = dot
+    d["_gs_weight_train_grad"] = grad
     if bias:
-        layer.bias.grad_dot_prod = bias_dot
-        layer._gs_bias_train_grad = bias_grad
+        bias_p.grad_dot_prod = bias_dot
+        d["_gs_bias_train_grad"] = bias_grad
     if options["record_algorithms"]:
         ALGO_LOG[getattr(layer, "name", id(layer))] = ("pairwise" if pairwise else "presum",
                                                        "valgrad+train_grad")
@@ -403,15 +415,15 @@ def _compute_embedding_dot_product(layer: nn.Embedding, A: torch.Tensor, B: torc
     # With the train-grad scale announced, the train gradient is formed here as well (same
     # stream as the dot, no second hook-stage launch sequence) and parked for
     # _compute_embedding_train_grad.
-    scale = getattr(layer, "_gs_bias_grad_scale", None)
+    scale = layer.__dict__.get("_gs_bias_grad_scale")
     if scale is not None and getattr(layer.weight, "initially_requires_grad", False):
         # The train gradient is built from the ids the layer saw: the reference's gradient
         # stage reads layer.activations (autograd_grad_sample_dotprod.py:166-181), not the ids
         # its dot stage promoted to the backprops' dtype (:116-123), which may have rounded.
         ids = layer.__dict__.get("activations")
         ids = A if ids is None or ids.is_floating_point() else ids.detach()
-        layer._gs_weight_train_grad = _embedding_train_grad(layer, ids, B, val_batch_size,
-                                                            scale, join=False)
+        layer.__dict__["_gs_weight_train_grad"] = _embedding_train_grad(
+            layer, ids, B, val_batch_size, scale)
 
 
 # Returned by a train-grad sampler that has already added its gradient into
@@ -433,21 +445,19 @@ def _compute_embedding_train_grad(layer: nn.Embedding, A: torch.Tensor, B: torch
     parked = layer.__dict__.pop("_gs_weight_train_grad", None)
     if parked is not None:   # formed with the dot, same scale
         return parked
-    return _embedding_train_grad(layer, A, B, val_batch_size, scale / n_t, join=True)
+    return _embedding_train_grad(layer, A, B, val_batch_size, scale / n_t)
 
 
 def _embedding_train_grad(layer: nn.Embedding, A: torch.Tensor, B: torch.Tensor,
-                          val_batch_size: int, alpha: float, join: bool):
+                          val_batch_size: int, alpha: float):
     """alpha * (sum of the train rows of B per token id) as a fresh gradient, or added into
-    the weight's existing train gradient (then APPLIED).  ``join``: order the current stream
-    after the side stream first (not needed on the side stream itself)."""
+    the weight's existing train gradient (then APPLIED)."""
     B = B.detach()
     if B.dtype not in (torch.bfloat16, torch.float32):
         B = B.float()
     prev = getattr(layer.weight, "train_grad", None)
     if prev is not None and prev.shape == layer.weight.shape:
-        if join:
-            _overlap.join(prev.device)   # prev may come from the side stream
+        _overlap.join(prev.device)   # prev may come from the other stream
         ops().embedding_train_grad(A.detach(), B, val_batch_size, alpha, prev, accumulate=True)
         return APPLIED
     grad = torch.empty_like(layer.weight)
@@ -477,15 +487,16 @@ def _compute_layernorm_dot_product(layer: nn.LayerNorm, A: torch.Tensor, B: torc
         A.dtype if A.dtype in (torch.bfloat16, torch.float32) else torch.float32)
     Ac = A.to(dt) if A.dtype != dt else A
     Bc = B.to(dt) if B.dtype != dt else B
-    scale = getattr(layer, "_gs_ln_grad_scale", None)
+    scale = layer.__dict__.get("_gs_ln_grad_scale")
+    weight, bias = _param(layer, "weight"), _param(layer, "bias")
     dw, db, gw, gb = ops().layernorm_dot(
-        Ac, Bc, val_batch_size, layer.eps, want_dot=True, want_bias=layer.bias is not None,
-        grad_scale=scale, grad_dtype=layer.weight.dtype)
-    layer.weight.grad_dot_prod = dw
-    if layer.bias is not None:
-        layer.bias.grad_dot_prod = db
+        Ac, Bc, val_batch_size, layer.eps, want_dot=True, want_bias=bias is not None,
+        grad_scale=scale, grad_dtype=weight.dtype)
+    weight.grad_dot_prod = dw
+    if bias is not None:
+        bias.grad_dot_prod = db
     if gw is not None:
-        layer._gs_ln_train_grads = (gw, gb)
+        layer.__dict__["_gs_ln_train_grads"] = (gw, gb)
 
 
 def _compute_layernorm_train_grad(layer: nn.LayerNorm, A: torch.Tensor, B: torch.Tensor,
@@ -504,9 +515,9 @@ def _compute_layernorm_train_grad(layer: nn.LayerNorm, A: torch.Tensor, B: torch
             grad_dtype=layer.weight.dtype)
     else:
         gw, gb = stash
-    _create_or_accumulate_train_grad(layer.weight, gw)
-    if layer.bias is not None:
-        _create_or_accumulate_train_grad(layer.bias, gb)
+    _create_or_accumulate_train_grad(_param(layer, "weight"), gw)
+    if _param(layer, "bias") is not None:
+        _create_or_accumulate_train_grad(_param(layer, "bias"), gb)
     return None
 
 

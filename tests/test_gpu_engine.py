@@ -848,3 +848,50 @@ def test_ordered_sum_matches_sequential_in_place_adds(gpu, first, n):
     rev = [s.to(gpu) for s in srcs[:1] + srcs[:0:-1]]
     assert not torch.equal(_native.ops().ordered_sum_(rev), want)
 
+
+
+def test_side_stream_with_layers_on_both_sides_of_its_line(gpu):
+    """One weight shared by a Linear call small enough for the autograd stream, one that runs on
+    the side stream and an embedding: the same bits as without overlap, whichever comes first."""
+    from ghostsuite_amd import autograd_grad_sample_dotprod as hooks
+    d, T = 512, 256
+
+    class Net(nn.Module):
+        def __init__(self, small_first):
+            super().__init__()
+            self.small_first = small_first
+            self.emb = nn.Embedding(d, d)
+            self.big, self.small = nn.Linear(d, d), nn.Linear(d, d)
+            self.big.weight = self.small.weight = self.emb.weight
+
+        def forward(self, x):
+            h = self.emb(x)
+            if self.small_first:
+                return self.big(h + self.small(h[:, :2]).mean(1, keepdim=True)).float()
+            return self.small(torch.tanh(self.big(h))[:, :2]).float()
+
+    x = torch.randint(0, d, (12, T), generator=gen(33)).to(gpu)
+    big = torch.empty(12, T, d, device="meta")
+    assert hooks._worth_overlapping(nn.Linear(1, 1), big, big)
+    assert not hooks._worth_overlapping(nn.Linear(1, 1), big[:, :2], big[:, :2])
+    for small_first in (False, True):
+        res = []
+        for overlap in (True, False):
+            torch.manual_seed(34)
+            model = Net(small_first).to(gpu).bfloat16()
+            opt = torch.optim.SGD(model.parameters(), lr=1e-2)
+            eng = GradDotProdEngine(model, val_batch_size=2, use_dummy_bias=False,
+                                    precision="reference", overlap=overlap)
+            eng.attach(opt)
+            for step in range(3):
+                eng.attach_train_batch(x[:10], x[:10], step, 0)
+                model(x).square().mean().backward()
+                eng.prepare_gradients()
+                opt.step()
+                eng.aggregate_and_log()
+                eng.clear_gradients()
+            eng.detach()
+            res.append([r["dot_product"] for r in eng.dot_product_log] +
+                       [p.detach().float().cpu() for p in model.parameters()])
+        for a, b in zip(*res):
+            assert torch.isfinite(a).all() and torch.equal(a, b)
