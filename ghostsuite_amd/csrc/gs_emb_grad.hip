@@ -2,11 +2,13 @@
 //
 //   grad[v] = scale * sum over the train tokens t with id_t = v of g_t        grad: [vocab, d]
 //
-// The train tokens are sorted by the key (id << 32 | token index), so every id's tokens form
-// one run, in index order, of a sorted token list; sums run over that list in a fixed order,
-// so the result is the same bits on every run, and every step's work is linear in the number
-// of tokens however often an id repeats.  Four launches:
-//   1. eg_sort_kernel    -- chunks of EG_CHUNK tokens sorted in registers and LDS (bitonic);
+// The train tokens are listed by id, so every id's tokens form one run, in index order, of a
+// sorted token list; sums run over that list in a fixed order, so the result is the same bits on
+// every run, and every step's work is linear in the number of tokens however often an id repeats.
+// Launches:
+//   1. eg_bucket_kernel  -- the list, its length and the presence bitmap of the ids, for up to
+//                           131072 tokens and 131072 ids; beyond that in two launches:
+//      eg_sort_kernel    -- chunks of EG_CHUNK tokens sorted in registers and LDS (bitonic);
 //                           per-chunk counts of in-range ids; the id-presence bitmap cleared.
 //   2. eg_merge_kernel   -- every key's place in the whole list = its place in its chunk plus
 //                           the number of smaller keys in each other chunk (binary search);
@@ -22,9 +24,9 @@
 //                           the workgroups whose windows it covers, a share of the features
 //                           each, for a run of hundreds of tokens or more.
 // Token ids outside [0, vocab) take no part.  Measured on MI355X (GPT-2 wte, 16 train rows of
-// 1024 tokens, d = 768, bf16): sort 15 us, merge 14, windows 19-21, combine 6-8; a padded
-// batch of 65536 train tokens with one id on 59k of them: sort 15, merge 52, windows 41-47,
-// combine 36 (the same case took 0.59 ms with each long run summed by one workgroup).
+// 1024 tokens, d = 768, bf16): list 11 us, windows 19.5 (102 MB written and read: the rate of a
+// copy), combine 6; a padded batch of 65536 train tokens with one id on 59k of them, d = 256:
+// list 52, windows 26, combine 33.
 
 #include <algorithm>
 
@@ -48,11 +50,32 @@ __device__ __forceinline__ int64_t key_tok(unsigned long long k) {
   return static_cast<int64_t>(k & 0xffffffffull);
 }
 
-// Physical row of train token q (tokens numbered in train-row order).
-__device__ __forceinline__ int64_t eg_row(const RowMap& tr, int64_t q) {
-  const int64_t seg = q / tr.seglen;
-  return tr.phys_row(seg, q - seg * tr.seglen);
+// Physical row of token q of a row set (tokens numbered in row order): the set is contiguous but
+// for the samples it skips, so one compare, not a division by the row length.
+struct EgRows {
+  int64_t M, off, cut, skip;   // tokens; row of token 0; first token past the skip; rows skipped
+  __device__ int64_t operator()(int64_t q) const { return q + off + (q >= cut ? skip : 0); }
+};
+EgRows eg_rows(const RowMap& m) {
+  const int64_t M = m.total();
+  return EgRows{M, m.seg_offset * m.seglen, m.skip_at >= m.nseg ? M : m.skip_at * m.seglen,
+                m.skip_n * m.seglen};
 }
+
+// An id's order in the token list.  Bucketed (shift >= 0): the list is ordered by (id % 256, id /
+// 256), whose number `(id % 256) << shift | id / 256` takes the id's place in the keys; presence
+// bits lie in whole words per bucket.  Otherwise (shift < 0): by the id itself.
+struct EgOrder {
+  int shift;
+  __device__ int64_t id(int64_t o) const {
+    return shift < 0 ? o : ((o & ((int64_t{1} << shift) - 1)) << 8) | (o >> shift);
+  }
+  __host__ __device__ int64_t bucket_words() const { return ((int64_t{1} << shift) + 31) / 32; }
+  __device__ bool present(const uint32_t* __restrict__ bits, int64_t v) const {
+    if (shift < 0) return (bits[v >> 5] >> (v & 31)) & 1u;
+    return (bits[(v & 255) * bucket_words() + (v >> 13)] >> ((v >> 8) & 31)) & 1u;
+  }
+};
 
 // Lane l's value of v, as a wave-uniform value (l a compile-time or uniform lane index).
 __device__ __forceinline__ unsigned long long readlane_u64(unsigned long long v, int l) {
@@ -124,12 +147,12 @@ __device__ __forceinline__ unsigned long long shfl_xor_key(unsigned long long v,
 // through LDS; sixteen waves per workgroup hide each other's shuffle and LDS latency.
 template <class K>
 __global__ void __launch_bounds__(EG_SORT_THREADS) eg_sort_kernel(
-    const int64_t* __restrict__ ids, RowMap tr, int64_t vocab, K* __restrict__ ck,
+    const int64_t* __restrict__ ids, EgRows tr, int64_t vocab, K* __restrict__ ck,
     int32_t* __restrict__ cnt, uint32_t* __restrict__ present, int64_t present_words) {
   __shared__ K xs[EG_CHUNK];
   __shared__ int32_t wcount[EG_SORT_THREADS / 64];
   const int t = threadIdx.x, lane = t & 63;
-  const int64_t M = tr.total();
+  const int64_t M = tr.M;
   const int64_t q0 = static_cast<int64_t>(blockIdx.x) * EG_CHUNK;
   for (int64_t w = static_cast<int64_t>(blockIdx.x) * EG_SORT_THREADS + t; w < present_words;
        w += static_cast<int64_t>(gridDim.x) * EG_SORT_THREADS)
@@ -141,7 +164,7 @@ __global__ void __launch_bounds__(EG_SORT_THREADS) eg_sort_kernel(
     const int64_t q = q0 + t + EG_SORT_THREADS * u;
     K k = EgKey<K>::NONE;
     if (q < M) {
-      const int64_t id = ids[eg_row(tr, q)];
+      const int64_t id = ids[tr(q)];
       if (id >= 0 && id < vocab) {
         k = EgKey<K>::make(id, q, q0);
         ++valid;
@@ -353,6 +376,161 @@ __global__ void __launch_bounds__(EG_THREADS) eg_merge_kernel(
   }
 }
 
+// The token list of one row set in one launch (vocab of up to 256 << EG_BUCKET_SHIFT ids): bucket
+// b = blockIdx % 256 holds the ids congruent to b, and its workgroup reads every id of the set.
+// The tokens of lower buckets, counted in passing, are where the bucket's part of the list
+// begins, so no workgroup waits for another; taking ids modulo 256 spreads the frequent low ids
+// of a real vocabulary over the buckets.  Each of the 16 waves takes a contiguous share of the
+// tokens and keeps the bucket's in LDS (a wave in whose share the bucket has more than
+// EG_BUCKET_KEEP, a padded batch, reads its ids a second time instead).  Counts per (wave, id) in
+// LDS, where tokens of one id among 64 are found by a ballot per bit of the id, become places by
+// a scan over (id, wave); the keys (order << 32 | token) are written in the order (bucket, id,
+// token).  Also writes the bucket's presence bits and the length of the list (cnt[0], by the last
+// bucket).  Bound by the latency of its two or three trips to L2 for small batches and by the
+// 256-fold reading of the ids for large ones.  Measured on MI355X against the sort and merge below
+// (whole gradient call, us): 16384 tokens of 50257 ids 53.9 -> 35.2 (11 in this kernel, 29 in
+// those two), with 90% of them one id 70.8 -> 53.9; 65536 tokens 101 -> 52.7, 90% one id 125 ->
+// 108; 131072 tokens 225 -> 86, 90% one id 240 -> 177; 192 tokens 40 -> 27.
+constexpr int EG_BUCKET_THREADS = 1024, EG_BUCKET_SHIFT = 9, EG_BUCKET_KEEP = 384;
+constexpr int64_t EG_BUCKET_TOKENS = int64_t{1} << 17;
+struct EgList {
+  EgRows rows;
+  unsigned long long* sk;
+  int32_t* cnt;
+  uint32_t* present;
+};
+
+__global__ void __launch_bounds__(EG_BUCKET_THREADS) eg_bucket_kernel(
+    const int64_t* __restrict__ ids, EgList list, int64_t vocab, EgOrder order) {
+  constexpr int NW = EG_BUCKET_THREADS / 64, U = 8, SHARE_BITS = 13;
+  static_assert(EG_BUCKET_TOKENS / NW <= 1 << SHARE_BITS, "a token's place in its share");
+  extern __shared__ int eg_counts[];   // [NW][R]
+  __shared__ uint32_t eg_kept[NW][EG_BUCKET_KEEP];   // id of the bucket << SHARE_BITS | place
+  __shared__ int wbase[NW], wtot[NW];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int b = blockIdx.x, R = 1 << order.shift;
+  const int M = static_cast<int>(list.rows.M);
+  const int share = ((M + NW - 1) / NW + 63) & ~63;
+  const int q_begin = std::min(M, wv * share), q_end = std::min(M, q_begin + share);
+  const unsigned nv = static_cast<unsigned>(vocab);
+  int* const mine = eg_counts + wv * R;
+  uint32_t* const kept = eg_kept[wv];
+  for (int x = lane; x < R; x += 64) mine[x] = 0;
+  // f(v, q) for the wave's tokens, 64 at a time: v is the id of the lane's token q, or a number
+  // past the vocabulary.  The loads of the next U groups are in flight meanwhile.
+  const auto scan = [&](auto&& f) {
+    int64_t next[U];
+    const auto load = [&](int q) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int x = q + 64 * u + lane;
+        next[u] = x < q_end ? ids[list.rows(x)] : -1;
+      }
+    };
+    load(q_begin);
+    for (int q = q_begin; q < q_end; q += 64 * U) {
+      unsigned v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        v[u] = next[u] >= 0 && next[u] < vocab ? static_cast<unsigned>(next[u]) : ~0u;
+      load(q + 64 * U);
+#pragma unroll
+      for (int u = 0; u < U; ++u) f(v[u], q + 64 * u + lane);
+    }
+  };
+  // The lanes of `in` whose token has this lane's id of the bucket.
+  const auto same_id = [&](unsigned long long in, int lid) {
+    const int one = __builtin_amdgcn_readlane(lid, __builtin_ctzll(in));
+    if ((__ballot(lid == one) & in) == in) return in;
+    for (int bit = 0; bit < order.shift; ++bit) {
+      const unsigned long long set = __ballot((lid >> bit) & 1);
+      in &= ((lid >> bit) & 1) ? set : ~set;
+    }
+    return in;
+  };
+  const auto count = [&](bool hit, int lid) {
+    const unsigned long long same = same_id(__ballot(hit), lid);
+    if (hit && __builtin_ctzll(same) == lane) atomicAdd(mine + lid, __popcll(same));
+  };
+  int below = 0, n = 0;
+  scan([&](unsigned v, int q) {
+    below += __popcll(__ballot(v < nv && static_cast<int>(v & 255u) < b));
+    const bool hit = v < nv && static_cast<int>(v & 255u) == b;
+    const unsigned long long hits = __ballot(hit);
+    if (hits == 0) return;
+    const int lid = static_cast<int>(v >> 8), n0 = n;
+    n += __popcll(hits);
+    if (n <= EG_BUCKET_KEEP) {
+      if (hit)
+        kept[n0 + __popcll(hits & ((1ull << lane) - 1ull))] =
+            static_cast<uint32_t>(lid) << SHARE_BITS | static_cast<uint32_t>(q - q_begin);
+    } else {
+      if (n0 <= EG_BUCKET_KEEP)   // count what was kept, once
+        for (int x = lane; x - lane < n0; x += 64)
+          count(x < n0, x < n0 ? static_cast<int>(kept[x] >> SHARE_BITS) : 0);
+      count(hit, lid);
+    }
+  });
+  if (n <= EG_BUCKET_KEEP)
+    for (int x = lane; x - lane < n; x += 64)
+      count(x < n, x < n ? static_cast<int>(kept[x] >> SHARE_BITS) : 0);
+  if (lane == 0) wbase[wv] = below;
+  __syncthreads();
+  // Counts to places: thread t owns id t of the bucket.
+  int total = 0;
+  if (t < R)
+    for (int w = 0; w < NW; ++w) total += eg_counts[w * R + t];
+  int incl = total;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int x = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += x;
+  }
+  if (lane == 63) wtot[wv] = incl;
+  __syncthreads();
+  int place = incl - total, all = 0;
+  for (int w = 0; w < NW; ++w) {
+    place += wbase[w] + (w < wv ? wtot[w] : 0);
+    all += wbase[w] + wtot[w];
+  }
+  if (b == 255 && t == 0) list.cnt[0] = all;
+  const unsigned long long present = __ballot(total > 0);
+  const int words = static_cast<int>(order.bucket_words());
+  if ((lane & 31) == 0 && (t >> 5) < words)
+    list.present[b * words + (t >> 5)] = static_cast<uint32_t>(present >> lane);
+  if (t < R)
+    for (int w = 0; w < NW; ++w) {
+      const int x = eg_counts[w * R + t];
+      eg_counts[w * R + t] = place;
+      place += x;
+    }
+  __syncthreads();
+  const uint32_t o = static_cast<uint32_t>(b) << order.shift;
+  const auto write = [&](bool hit, int lid, int q) {
+    const unsigned long long same = same_id(__ballot(hit), lid);
+    const int lead = hit ? __builtin_ctzll(same) : lane;
+    int first = 0;
+    if (hit && lead == lane) first = atomicAdd(mine + lid, __popcll(same));
+    first = __shfl(first, lead, 64);
+    if (hit)
+      list.sk[first + __popcll(same & ((1ull << lane) - 1ull))] =
+          static_cast<unsigned long long>(o | static_cast<uint32_t>(lid)) << 32 |
+          static_cast<unsigned long long>(q);
+  };
+  if (n <= EG_BUCKET_KEEP) {
+    for (int x = lane; x - lane < n; x += 64) {
+      const uint32_t k = x < n ? kept[x] : 0u;
+      write(x < n, static_cast<int>(k >> SHARE_BITS),
+            q_begin + static_cast<int>(k & ((1u << SHARE_BITS) - 1u)));
+    }
+  } else {
+    scan([&](unsigned v, int q) {
+      const bool hit = v < nv && static_cast<int>(v & 255u) == b;
+      if (__ballot(hit) != 0) write(hit, hit ? static_cast<int>(v >> 8) : 0, q);
+    });
+  }
+}
+
 // Sum of cnt[0, chunks): the number of in-range keys, the length of the sorted list.
 __device__ __forceinline__ int64_t list_length(const int32_t* __restrict__ cnt, int64_t chunks) {
   const int lane = threadIdx.x & 63;
@@ -427,7 +605,7 @@ __device__ __forceinline__ void eg_store(GE* __restrict__ out, int64_t f0, int64
 // absent from the list are written as zeros.
 template <class E, class GE>
 __global__ void __launch_bounds__(EG_THREADS) eg_window_kernel(
-    const E* __restrict__ G, RowMap tr, int64_t d, int64_t vocab,
+    const E* __restrict__ G, EgRows tr, EgOrder order, int64_t d, int64_t vocab,
     const unsigned long long* __restrict__ sk, const int32_t* __restrict__ cnt, int64_t chunks,
     const uint32_t* __restrict__ present, int64_t windows, float scale, int accumulate, int vec,
     float* __restrict__ part, GE* __restrict__ grad) {
@@ -439,7 +617,8 @@ __global__ void __launch_bounds__(EG_THREADS) eg_window_kernel(
     // both modes): 16 rows, lanes over chunks
     const int64_t v0 = (w - windows) * 16;
     if (accumulate || v0 >= vocab) return;
-    const uint32_t bits = present[v0 >> 5] >> (v0 & 31);   // v0 is a multiple of 16
+    const unsigned long long bits =
+        __ballot(lane < 16 && v0 + lane < vocab && order.present(present, v0 + lane));
     for (int r = 0; r < 16 && v0 + r < vocab; ++r) {
       if ((bits >> r) & 1u) continue;
       GE* out = grad + (v0 + r) * d;
@@ -459,7 +638,7 @@ __global__ void __launch_bounds__(EG_THREADS) eg_window_kernel(
   // lane i < n: the key at place r0 + i, its id and G row; read as wave-uniform values below
   const unsigned long long k = lane < n ? sk[r0 + lane] : EG_NONE;
   const int64_t my_id = key_id(k);
-  const int64_t my_row = lane < n ? eg_row(tr, key_tok(k)) : 0;
+  const int64_t my_row = lane < n ? tr(key_tok(k)) : 0;
   const bool from_before = r0 > 0 && key_id(sk[r0 - 1]) == readlane_i64(my_id, 0);
   const bool into_next = r0 + n < n_list && key_id(sk[r0 + n]) == readlane_i64(my_id, n - 1);
   // two feature passes per round (lanes own chunks f0 and f0 + 64 VE); the window's rows in
@@ -515,7 +694,7 @@ __global__ void __launch_bounds__(EG_THREADS) eg_window_kernel(
                   for (int e = 0; e < VE; ++e)
                     if (f0 + e < d) pp[f0 + e] = acc[h][e];
                 } else {
-                  eg_store<GE, VE>(grad + id_p * d, f0, d, acc[h], scale, accumulate,
+                  eg_store<GE, VE>(grad + order.id(id_p) * d, f0, d, acc[h], scale, accumulate,
                                    vec && f0 + VE <= d);
                 }
               }
@@ -623,8 +802,8 @@ __device__ void eg_spread_sum(const float* __restrict__ part, int64_t ws, int64_
 template <class GE>
 __global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
     const unsigned long long* __restrict__ sk, const int32_t* __restrict__ cnt, int64_t chunks,
-    const float* __restrict__ part, int64_t windows, int64_t d, float scale, int accumulate,
-    GE* __restrict__ grad) {
+    const float* __restrict__ part, int64_t windows, EgOrder order, int64_t d, float scale,
+    int accumulate, GE* __restrict__ grad) {
   constexpr int NW = EG_COMBINE_WAVES, CB = 1024;   // waves; features per block
   static_assert(NW * 64 == CB, "one feature of a block per thread");
   __shared__ __attribute__((aligned(16))) float red[NW][CB];
@@ -658,7 +837,7 @@ __global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
         const int64_t ws = first / EG_WIN, w_end = (lo - 1) / EG_WIN;
         const int64_t b_lo = ws / NW + 1, nb = w_end / NW - 1 - b_lo + 1;
         if (nb >= EG_SPREAD)
-          eg_spread_sum<GE>(part, ws, w_end - ws + 1, d, id0, blockIdx.x - b_lo, nb, scale,
+          eg_spread_sum<GE>(part, ws, w_end - ws + 1, d, order.id(id0), blockIdx.x - b_lo, nb, scale,
                             accumulate, &red[0][0], grad);
         return;
       }
@@ -702,7 +881,7 @@ __global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
   // summed by the whole workgroup.
   const int64_t parts_found = found ? (end - 1) / EG_WIN - w + 1 : 0;
   if (found && parts_found <= EG_LIGHT) {
-    GE* out = grad + id * d;
+    GE* out = grad + order.id(id) * d;
     for (int64_t f = static_cast<int64_t>(lane) * 4; f < d; f += 256) {
       float4 x[EG_LIGHT];
 #pragma unroll
@@ -748,7 +927,7 @@ __global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
     for (int v = 0; v < wid; ++v) slot += flags[v];
     run_w[slot] = w;
     run_end[slot] = end;
-    run_id[slot] = id;
+    run_id[slot] = order.id(id);
     atomicAdd(&n_runs, 1);
   }
   __syncthreads();
@@ -811,21 +990,29 @@ int64_t eg_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 struct EgPlan {
   int64_t M, chunks, windows, present_words;
+  EgOrder order;
 };
 
+// The bucketed list where its counters and a wave's places fit (131072 tokens, 131072 ids): there it
+// was the faster one at every size measured (figures at eg_bucket_kernel).  Sort and merge beyond.
 EgPlan eg_plan(int64_t M, int64_t vocab) {
   EgPlan p;
   p.M = M;
-  p.chunks = eg_cdiv(M, EG_CHUNK);
   p.windows = eg_cdiv(M, EG_WIN);
-  p.present_words = eg_cdiv(vocab, 32);
+  p.order.shift = -1;
+  if (M <= EG_BUCKET_TOKENS && vocab <= (int64_t{256} << EG_BUCKET_SHIFT)) {
+    p.order.shift = 0;
+    while ((int64_t{256} << p.order.shift) < vocab) ++p.order.shift;
+  }
+  p.chunks = p.order.shift < 0 ? eg_cdiv(M, EG_CHUNK) : 1;
+  p.present_words = p.order.shift < 0 ? eg_cdiv(vocab, 32) : 256 * p.order.bucket_words();
   return p;
 }
 
 template <class S>
 void carve_emb_grad(S& c, const EgPlan& p, int64_t d, unsigned long long** ck,
                     unsigned long long** sk, int32_t** cnt, uint32_t** present, float** part) {
-  *ck = c.template take<unsigned long long>(p.chunks * EG_CHUNK);
+  *ck = c.template take<unsigned long long>(p.order.shift < 0 ? p.chunks * EG_CHUNK : 0);
   *sk = c.template take<unsigned long long>(p.M);
   *cnt = c.template take<int32_t>(p.chunks);
   *present = c.template take<uint32_t>(p.present_words);
@@ -833,20 +1020,20 @@ void carve_emb_grad(S& c, const EgPlan& p, int64_t d, unsigned long long** ck,
 }
 
 template <class E, class GE>
-int launch_rows(const void* G, const RowMap& tr, int64_t d, int64_t vocab, const EgPlan& pl,
+int launch_rows(const void* G, const EgRows& tr, int64_t d, int64_t vocab, const EgPlan& pl,
                 const unsigned long long* sk, const int32_t* cnt, const uint32_t* present,
                 float* part, float scale, int accumulate, int vec, void* grad, hipStream_t s) {
   const int64_t zero_waves = accumulate ? 0 : eg_cdiv(vocab, 16);
   const int64_t waves = pl.windows + zero_waves;
   hipLaunchKernelGGL((eg_window_kernel<E, GE>),
                      dim3(static_cast<unsigned>(eg_cdiv(waves, EG_THREADS / 64))),
-                     dim3(EG_THREADS), 0, s, static_cast<const E*>(G), tr, d, vocab, sk, cnt,
+                     dim3(EG_THREADS), 0, s, static_cast<const E*>(G), tr, pl.order, d, vocab, sk, cnt,
                      pl.chunks, present, pl.windows, scale, accumulate, vec, part,
                      static_cast<GE*>(grad));
   hipLaunchKernelGGL((eg_combine_kernel<GE>),
                      dim3(static_cast<unsigned>(eg_cdiv(pl.windows, EG_COMBINE_WAVES))),
-                     dim3(EG_COMBINE_WAVES * 64), 0, s, sk, cnt, pl.chunks, part, pl.windows, d,
-                     scale, accumulate, static_cast<GE*>(grad));
+                     dim3(EG_COMBINE_WAVES * 64), 0, s, sk, cnt, pl.chunks, part, pl.windows,
+                     pl.order, d, scale, accumulate, static_cast<GE*>(grad));
   return check_launch("eg_window_kernel / eg_combine_kernel");
 }
 
@@ -895,9 +1082,14 @@ extern "C" int gs_embedding_train_grad(const int64_t* ids, const void* G, int dt
   Carver cv(workspace, workspace_bytes);
   carve_emb_grad(cv, pl, d, &ck, &sk, &cnt, &present, &part);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const RowMap tr = train_rows(N, n_val, val_start, T);
+  const EgRows tr = eg_rows(train_rows(N, n_val, val_start, T));
   const dim3 mgrid(static_cast<unsigned>(eg_cdiv(pl.chunks * EG_CHUNK, EG_THREADS)));
-  if (vocab <= EG_KEY32_VOCAB) {
+  if (pl.order.shift >= 0) {
+    const EgList list{tr, sk, cnt, present};
+    hipLaunchKernelGGL(eg_bucket_kernel, dim3(256), dim3(EG_BUCKET_THREADS),
+                       (EG_BUCKET_THREADS / 64) * sizeof(int) << pl.order.shift, s, ids, list,
+                       vocab, pl.order);
+  } else if (vocab <= EG_KEY32_VOCAB) {
     uint32_t* ck32 = reinterpret_cast<uint32_t*>(ck);
     hipLaunchKernelGGL(eg_sort_kernel<uint32_t>, dim3(static_cast<unsigned>(pl.chunks)),
                        dim3(EG_SORT_THREADS), 0, s, ids, tr, vocab, ck32, cnt, present,
@@ -916,7 +1108,7 @@ extern "C" int gs_embedding_train_grad(const int64_t* ids, const void* G, int dt
     hipLaunchKernelGGL((eg_merge_kernel<unsigned long long, false>), mgrid, dim3(EG_THREADS),
                        0, s, ck, pl.chunks, sk, present);
   }
-  int rc = check_launch("eg_sort_kernel / eg_merge_kernel");
+  int rc = check_launch("eg_bucket_kernel / eg_sort_kernel / eg_merge_kernel");
   if (rc) return rc;
   const size_t esz = elem_size(dtype), gsz = elem_size(grad_dtype);
   const int vec = (reinterpret_cast<uintptr_t>(G) % 16 == 0) &&

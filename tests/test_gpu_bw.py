@@ -187,6 +187,33 @@ def test_embedding_train_grad_heavy_ids(gpu, shape, pad_frac):
     assert_close(got, prev.double() + want, 1e-2, "heavy ids, accumulate")
 
 
+@pytest.mark.parametrize("shape,pad_frac", [
+    # N, n_val, T, d, vocab
+    ((3, 1, 500, 8, 256), 0.0),          # one id a bucket
+    ((3, 1, 1025, 8, 257), 0.5),         # two; a token past the waves' even shares
+    ((4, 1, 2100, 8, 131072), 0.93),     # most ids; shares that keep 384 tokens of a bucket or more
+    ((4, 1, 2100, 8, 131073), 0.93),     # one id too many: sorted chunks
+    ((65, 1, 2048, 8, 1000), 0.1),       # most tokens
+    ((66, 2, 2049, 8, 1000), 0.1),       # sorted chunks
+])
+def test_embedding_train_grad_list_edges(gpu, shape, pad_frac):
+    """The token list at the edges of its two forms: float64 index_add within fp32 rounding of a
+    sum in a fixed order, absent ids zero, out-of-range ids left out."""
+    N, n_val, T, d, vocab = shape
+    ids = torch.randint(-2, vocab + 2, (N, T), generator=gen(190 + T))
+    ids[torch.rand(N, T, generator=gen(191 + T)) < pad_frac] = vocab - 1
+    G = randn((N, T, d), 192 + T, 1e-2, torch.float32)
+    out = torch.full((vocab, d), float("nan"), device=gpu)
+    _native.ops().embedding_train_grad(ids.to(gpu), G.to(gpu), n_val, 2.0, out, val_start=1)
+    ok = (ids >= 0) & (ids < vocab)
+    want, touched = _emb_grad_exact(ids, G, n_val, 1, vocab, 2.0)
+    assert torch.equal(touched.nonzero()[:, 0],
+                       torch.unique(torch.cat([ids[:1], ids[1 + n_val:]])[
+                           torch.cat([ok[:1], ok[1 + n_val:]])]))
+    assert_close(out.cpu(), want, FP32_TOL, "list edges")
+    assert torch.all(out.cpu()[~touched] == 0)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("shape", [(6, 2, 5, 24), (20, 4, 70, 768), (5, 1, 3, 2048), (4, 1, 2, 100),
                                    (3, 1, 130, 1024), (4, 2, 64, 1600), (20, 4, 1024, 768),
