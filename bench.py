@@ -75,6 +75,15 @@ class TimedOps:
         return self._run("embedding_train_grad", ("hbm", nbytes),
                          self.inner.embedding_train_grad, ids, G, n_val, scale, out, **k)
 
+    def embedding_layer_pass(self, ids, G, n_val, scale, out, **k):
+        # the train gradient's traffic; the dots read what it reads, and the val rows
+        n_tok = (G.shape[0] - n_val) * (ids.numel() // G.shape[0])
+        row = out.shape[-1] * out.element_size()
+        rows = 2 * min(out.shape[0], n_tok) if k.get("accumulate") else out.shape[0]
+        nbytes = G.numel() * G.element_size() + ids.numel() * 8 + rows * row
+        return self._run("embedding_layer_pass", ("hbm", nbytes),
+                         self.inner.embedding_layer_pass, ids, G, n_val, scale, out, **k)
+
     def linear_dot(self, A, G, n_val, **k):
         from ghostsuite_amd import _native
         N, d_in, d_out = A.shape[0], A.shape[-1], G.shape[-1]

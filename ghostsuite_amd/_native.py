@@ -62,6 +62,9 @@ _SIGNATURES = {
     "gs_embedding_dot": (_I, [_P, _P, _I, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _SZ,
                               _P]),
     "gs_embedding_train_grad_workspace": (_SZ, [_I64, _I64, _I64, _I64, _I64]),
+    "gs_embedding_layer_pass_workspace": (_SZ, [_I64, _I64, _I64, _I64, _I64]),
+    "gs_embedding_layer_pass": (_I, [_P, _P, _I, _I64, _I64, _I64, _I64, _I64, _I64, _P, _F, _P,
+                                     _I, _I, _P, _SZ, _P]),
     "gs_embedding_train_grad": (_I, [_P, _P, _I, _I64, _I64, _I64, _I64, _I64, _I64, _F, _P,
                                      _I, _I, _P, _SZ, _P]),
     "gs_layernorm_dot_workspace": (_SZ, [_I64, _I64, _I64]),
@@ -602,6 +605,36 @@ class HipOps:
                                          _gs_dtype(out), int(accumulate), ws.data_ptr(),
                                          ws_bytes, _stream(dev))
         _check(rc, "gs_embedding_train_grad")
+
+    def embedding_layer_pass(self, ids: torch.Tensor, G: torch.Tensor, n_val: int, scale: float,
+                             out: torch.Tensor, *, accumulate: bool = False,
+                             val_start=None) -> Optional[torch.Tensor]:
+        """embedding_dot and embedding_train_grad (into out) of one layer in shared launches
+        (gs_embedding_layer_pass): the dots, or None, with nothing done, for sizes it leaves to
+        the two calls."""
+        dev = _require_device(ids, G, out)
+        ids = ids.to(torch.int64).contiguous()
+        G = G.contiguous()
+        N, d = G.shape[0], G.shape[-1]
+        T = ids.numel() // N
+        if _tokens(G, N, d) != T or out.dim() != 2 or out.shape[1] != d or \
+                not out.is_contiguous():
+            raise GhostHipError(f"embedding_layer_pass: ids {tuple(ids.shape)}, G "
+                                f"{tuple(G.shape)} and out {tuple(out.shape)} disagree")
+        vocab = out.shape[0]
+        vs = N - n_val if val_start is None else int(val_start)
+        lib = load_library()
+        ws_bytes = _size("gs_embedding_layer_pass_workspace", N, n_val, T, d, vocab)
+        if ws_bytes == 0:
+            return None
+        ws = _workspace(ws_bytes, dev)
+        dot = torch.empty(N - n_val, dtype=torch.float32, device=dev)
+        rc = lib.gs_embedding_layer_pass(ids.data_ptr(), G.data_ptr(), _gs_dtype(G), N, n_val, vs,
+                                         T, d, vocab, dot.data_ptr(), float(scale),
+                                         out.data_ptr(), _gs_dtype(out), int(accumulate),
+                                         ws.data_ptr(), ws_bytes, _stream(dev))
+        _check(rc, "gs_embedding_layer_pass")
+        return dot
 
     def layernorm_dot(self, X: torch.Tensor, G: torch.Tensor, n_val: int, eps: float, *,
                       val_start=None, want_dot: bool = True, want_bias: bool = True,

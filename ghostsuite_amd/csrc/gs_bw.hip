@@ -472,7 +472,8 @@ __global__ void __launch_bounds__(BW_THREADS) feature_finish_kernel(
 // (table[id] = min index, an order-independent integer atomicMin).  Segment sums are
 // accumulated in 64-bit fixed point with integer atomics (order-independent, hence
 // deterministic) under one power-of-two scale taken from max |g| over the val rows; each
-// train token finds its segment through table[id] and takes a dot with that row.
+// train token finds its segment through table[id] and takes a dot with that row.  (More than
+// 8192 val tokens, or ids of 2^19 and above; the others go through the val tokens' list.)
 constexpr int EMB_SLOTS = 256;  // max |g| is gathered in 256 slots to avoid one hot atomic
 
 // table[0, vocab) = INT32_MAX, slots = 0, fixed-point rows = 0.
@@ -574,196 +575,6 @@ __global__ void emb_dot_kernel(const int64_t* __restrict__ ids, const E* __restr
   }
   const float sf = static_cast<float>(s * inv);
   const float tot = block_sum(sf, red);
-  if (threadIdx.x == 0) part[i * chunks + c] = tot;
-}
-
-// ---- sorted-segment path (at most EMB_SORT_MAX val tokens, ids below 2^19) --------------
-// The val tokens are ordered by the distinct keys (id << EMB_QBITS | index): a token's sorted
-// position is the number of smaller keys (every workgroup counts against all keys in LDS).  A
-// run of equal ids is a segment and table[id] = the run's first sorted position.  Each run's
-// rows are summed in index order (fp32, no atomics, nothing to zero-fill), and each train
-// token dots its row with its id's run sum.
-constexpr int EMB_SORT_MAX = 8192, EMB_QBITS = 13;
-// A val token whose id is out of range gets the key EMB_NOKEY | index: above every valid key
-// (ids below 2^19 - 1), distinct, and in index order, so every key has its own rank.
-// EMB_PAD (above all of them) pads the key array.
-constexpr uint32_t EMB_NOKEY = 0xFFFFE000u, EMB_PAD = 0xFFFFFFFFu;
-__device__ __forceinline__ bool emb_nokey(uint32_t k) { return k >= EMB_NOKEY; }
-
-// keys[rank(i)] = key(i) for the n val tokens (the keys are distinct, so a key's rank is the
-// number of smaller keys); val tokens whose id is out of range go last, in index order.  Each
-// workgroup forms all n keys in LDS from the ids and ranks EMB_RK of them, each counted
-// against all keys by EMB_RP threads (one interleaved slice of the keys each) with the slice
-// counts combined through LDS; it also resets its grid-stride share of table[0, vocab) to -1.
-constexpr int EMB_RK = 8, EMB_RP = BW_THREADS / EMB_RK;
-__global__ void __launch_bounds__(BW_THREADS) emb_rank_kernel(
-    const int64_t* __restrict__ ids, RowMap val, int64_t vocab, int32_t* __restrict__ table,
-    uint32_t* __restrict__ keys) {
-  __shared__ __attribute__((aligned(16))) uint32_t sk[EMB_SORT_MAX];
-  __shared__ int cnt[EMB_RP][EMB_RK];
-  const int n = static_cast<int>(val.total()), n4 = (n + 3) / 4 * 4;
-  const int64_t gstride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t x = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; x < vocab;
-       x += gstride)
-    table[x] = -1;
-  // The val rows are one contiguous block, so val token j is ids[first + j]; a thread's
-  // loads are all issued before the first key is formed.
-  const int64_t* vids = ids + val.phys_row(0, 0);
-  constexpr int PER = EMB_SORT_MAX / BW_THREADS;
-  int64_t idr[PER];
-#pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    const int j = threadIdx.x + q * BW_THREADS;
-    idr[q] = j < n ? vids[j] : -1;
-  }
-#pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    const int j = threadIdx.x + q * BW_THREADS;
-    if (j < n4)
-      sk[j] = j >= n ? EMB_PAD
-                     : (idr[q] >= 0 && idr[q] < vocab)
-                           ? (static_cast<uint32_t>(idr[q]) << EMB_QBITS) | static_cast<uint32_t>(j)
-                           : EMB_NOKEY | static_cast<uint32_t>(j);
-  }
-  __syncthreads();
-  const int kk = threadIdx.x % EMB_RK, part = threadIdx.x / EMB_RK;
-  const int i = blockIdx.x * EMB_RK + kk;
-  const uint32_t k = i < n ? sk[i] : EMB_PAD;
-  // Slice `part` is every EMB_RP-th group of four keys, so the parts of a wave read
-  // consecutive 16-byte words (no LDS bank conflicts).
-  int lt = 0;
-  for (int j = part * 4; j < n4; j += EMB_RP * 4) {
-    const uint4 w = *reinterpret_cast<const uint4*>(sk + j);
-    lt += (w.x < k) + (w.y < k) + (w.z < k) + (w.w < k);
-  }
-  cnt[part][kk] = lt;
-  __syncthreads();
-  if (part == 0 && i < n) {
-    int a = 0;
-    for (int q = 0; q < EMB_RP; ++q) a += cnt[q][kk];
-    keys[a] = k;
-  }
-}
-
-// S[p][:] = sum of the val rows of the run starting at sorted position p (index order) when the
-// run has two or more tokens, and table[id] = p for every run.
-template <class E>
-__global__ void __launch_bounds__(BW_THREADS) emb_segsum_kernel(
-    const E* __restrict__ G, RowMap val, int64_t d, const uint32_t* __restrict__ keys,
-    int32_t* __restrict__ table, float* __restrict__ S) {
-  constexpr int VE = Vec<E>::VE;
-  const int64_t p = blockIdx.x, n_vt = val.total();
-  const uint32_t kprev = p > 0 ? keys[p - 1] : EMB_PAD;
-  const uint32_t k0 = keys[p];
-  const uint32_t knext = p + 1 < n_vt ? keys[p + 1] : EMB_PAD;
-  if (emb_nokey(k0) || (p > 0 && (kprev >> EMB_QBITS) == (k0 >> EMB_QBITS))) return;
-  const uint32_t id = k0 >> EMB_QBITS;
-  if (threadIdx.x == 0) table[id] = static_cast<int32_t>(p);
-  // A one-token run needs no sum: the train tokens read that val row itself.
-  if (emb_nokey(knext) || (knext >> EMB_QBITS) != id) return;
-  const int vec = (d * static_cast<int64_t>(sizeof(E))) % 16 == 0 &&
-                  (reinterpret_cast<uintptr_t>(G) % 16 == 0);
-  for (int64_t f = static_cast<int64_t>(threadIdx.x) * VE; f < d;
-       f += static_cast<int64_t>(blockDim.x) * VE) {
-    float a[VE];
-#pragma unroll
-    for (int e = 0; e < VE; ++e) a[e] = 0.f;
-    for (int64_t r = p; r < n_vt; ++r) {
-      const uint32_t k = r == p ? k0 : r == p + 1 ? knext : keys[r];
-      if (emb_nokey(k) || (k >> EMB_QBITS) != id) break;
-      const int64_t q = k & ((1u << EMB_QBITS) - 1);
-      const int64_t seg = q / val.seglen;
-      Vec<E> x;
-      x.load(G + val.phys_row(seg, q - seg * val.seglen) * d + f, vec && f + VE <= d, d - f);
-#pragma unroll
-      for (int e = 0; e < VE; ++e) a[e] += x.v[e];
-    }
-#pragma unroll
-    for (int e = 0; e < VE; ++e)
-      if (f + e < d) S[p * d + f + e] = a[e];
-  }
-}
-
-// part[i * chunks + c] = sum over train row i's tokens in chunk c of <g_it, run sum of x_it>:
-// the chunk's runs are looked up first (one token per thread): a run of two or more tokens is
-// read from S, a one-token run straight from that val token's row of G.  Then one token per
-// half-wave at a time with lanes over 16-byte feature chunks; fixed-order block sum.
-template <class E>
-__global__ void __launch_bounds__(BW_THREADS) emb_segdot_kernel(
-    const int64_t* __restrict__ ids, const E* __restrict__ G, RowMap train, RowMap val, int64_t d,
-    int64_t vocab, const uint32_t* __restrict__ keys, const int32_t* __restrict__ table,
-    const float* __restrict__ S, int64_t chunks, float* __restrict__ part) {
-  constexpr int VE = Vec<E>::VE;
-  static_assert(TOK_CHUNK <= BW_THREADS, "one lookup per thread");
-  __shared__ float red[BW_THREADS / 64];
-  __shared__ int64_t src[TOK_CHUNK];  // >= 0: row of S; < 0: -1 - (row of G); INT64_MIN: none
-  const int64_t i = blockIdx.y, c = blockIdx.x;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int64_t T = train.seglen, n_vt = val.total();
-  const int64_t t0 = c * TOK_CHUNK, t1 = std::min<int64_t>(T, t0 + TOK_CHUNK);
-  if (threadIdx.x < TOK_CHUNK) {
-    int64_t sr = INT64_MIN;
-    const int64_t t = t0 + threadIdx.x;
-    if (t < t1) {
-      const int64_t id = ids[train.phys_row(i, t)];
-      const int32_t r = (id >= 0 && id < vocab) ? table[id] : -1;
-      if (r >= 0) {
-        const uint32_t k = keys[r];
-        const uint32_t kn = r + 1 < n_vt ? keys[r + 1] : EMB_PAD;
-        if (!emb_nokey(kn) && (kn >> EMB_QBITS) == (k >> EMB_QBITS)) {
-          sr = r;
-        } else {
-          const int64_t q = k & ((1u << EMB_QBITS) - 1);
-          const int64_t seg = q / val.seglen;
-          sr = -1 - val.phys_row(seg, q - seg * val.seglen);
-        }
-      }
-    }
-    src[threadIdx.x] = sr;
-  }
-  __syncthreads();
-  const int vec = (d * static_cast<int64_t>(sizeof(E))) % 16 == 0 &&
-                  (reinterpret_cast<uintptr_t>(G) % 16 == 0) && d % 4 == 0;
-  float s = 0.f;
-  const int half = lane >> 5, hl = lane & 31;  // two tokens per wave, 32 lanes each
-  for (int64_t tb = t0 + 2 * wid; tb < t1; tb += 2 * (BW_THREADS / 64)) {
-    const int64_t t = tb + half;
-    const int64_t sr = t < t1 ? src[t - t0] : INT64_MIN;
-    if (sr == INT64_MIN) continue;
-    const E* gr = G + train.phys_row(i, t) * d;
-    if (sr >= 0) {
-      const float* srow = S + sr * d;
-#pragma unroll 4
-      for (int64_t f = static_cast<int64_t>(hl) * VE; f < d; f += 32 * VE) {
-        Vec<E> x;
-        const bool full = vec && f + VE <= d;
-        x.load(gr + f, full, d - f);
-        if (full) {
-#pragma unroll
-          for (int e = 0; e < VE; e += 4) {
-            const float4 w = *reinterpret_cast<const float4*>(srow + f + e);
-            s += x.v[e] * w.x + x.v[e + 1] * w.y + x.v[e + 2] * w.z + x.v[e + 3] * w.w;
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < VE; ++e)
-            if (f + e < d) s += x.v[e] * srow[f + e];
-        }
-      }
-    } else {
-      const E* vrow = G + (-1 - sr) * d;
-#pragma unroll 4
-      for (int64_t f = static_cast<int64_t>(hl) * VE; f < d; f += 32 * VE) {
-        Vec<E> x, y;
-        const bool full = vec && f + VE <= d;
-        x.load(gr + f, full, d - f);
-        y.load(vrow + f, full, d - f);
-#pragma unroll
-        for (int e = 0; e < VE; ++e) s += x.v[e] * y.v[e];
-      }
-    }
-  }
-  const float tot = block_sum(s, red);
   if (threadIdx.x == 0) part[i * chunks + c] = tot;
 }
 
@@ -1114,23 +925,12 @@ extern "C" int gs_layernorm_dot(const void* X, const void* G, int dtype, int64_t
 
 // ------------------------------------------------------------------------------ embedding
 namespace {
-// The sorted-segment path when the val tokens fit one sorting workgroup, else the
-// fixed-point path.
-bool emb_sorted(int64_t n_val, int64_t T, int64_t vocab) {
-  // (id << EMB_QBITS | index) must stay below the no-keys: ids below 2^19 - 1.
-  return n_val * T <= EMB_SORT_MAX && vocab < (int64_t{1} << (32 - EMB_QBITS));
-}
 template <class S>
 void carve_embedding(S& c, int64_t N, int64_t n_val, int64_t T, int64_t d, int64_t vocab) {
   const int64_t n_vt = n_val * T, n_t = N - n_val, chunks = cdiv(T, TOK_CHUNK);
   c.template take<int32_t>(vocab);
-  if (emb_sorted(n_val, T, vocab)) {
-    c.template take<uint32_t>(n_vt);
-    c.template take<float>(n_vt * d);
-  } else {
-    c.template take<unsigned>(EMB_SLOTS);
-    c.template take<unsigned long long>(n_vt * d);
-  }
+  c.template take<unsigned>(EMB_SLOTS);
+  c.template take<unsigned long long>(n_vt * d);
   c.template take<float>(n_t * chunks);
 }
 }  // namespace
@@ -1138,6 +938,8 @@ void carve_embedding(S& c, int64_t N, int64_t n_val, int64_t T, int64_t d, int64
 extern "C" size_t gs_embedding_dot_workspace(int64_t N, int64_t n_val, int64_t T, int64_t d,
                                              int64_t vocab) {
   if (N <= 0 || n_val <= 0 || n_val >= N || T <= 0 || d <= 0 || vocab <= 0) return 0;
+  if (embedding_dot_is_listed(n_val, T, vocab))
+    return embedding_dot_listed_workspace(N, n_val, T, d, vocab);
   Sizer sz;
   carve_embedding(sz, N, n_val, T, d, vocab);
   return sz.used + 256;
@@ -1154,6 +956,9 @@ extern "C" int gs_embedding_dot(const int64_t* ids, const void* G, int dtype, in
     return fail(GS_ERR_INVALID, "gs_embedding_dot: invalid arguments");
   if (n_val * T >= INT32_MAX || vocab >= INT32_MAX)
     return fail(GS_ERR_UNSUPPORTED, "gs_embedding_dot: more than 2^31 val tokens or ids");
+  if (embedding_dot_is_listed(n_val, T, vocab))
+    return embedding_dot_listed(ids, G, dtype, N, n_val, val_start, T, d, vocab, out_dot,
+                                workspace, workspace_bytes, static_cast<hipStream_t>(stream));
   Sizer sz;
   carve_embedding(sz, N, n_val, T, d, vocab);
   if (workspace == nullptr || workspace_bytes < sz.used)
@@ -1164,31 +969,6 @@ extern "C" int gs_embedding_dot(const int64_t* ids, const void* G, int dtype, in
   hipStream_t s = static_cast<hipStream_t>(stream);
   const RowMap va = val_rows(n_val, val_start, T);
   const RowMap tr = train_rows(N, n_val, val_start, T);
-  if (emb_sorted(n_val, T, vocab)) {
-    uint32_t* keys = cv.take<uint32_t>(n_vt);
-    float* S = cv.take<float>(n_vt * d);
-    float* part = cv.take<float>(n_t * chunks);
-    hipLaunchKernelGGL(emb_rank_kernel, dim3(static_cast<unsigned>(cdiv(n_vt, EMB_RK))),
-                       dim3(BW_THREADS), 0, s, ids, va, vocab, table, keys);
-    const dim3 gv(static_cast<unsigned>(n_vt));
-    const dim3 gt(static_cast<unsigned>(chunks), static_cast<unsigned>(n_t));
-    if (dtype == GS_DTYPE_BF16) {
-      const uint16_t* g = static_cast<const uint16_t*>(G);
-      hipLaunchKernelGGL(emb_segsum_kernel<uint16_t>, gv, dim3(128), 0, s, g, va, d, keys,
-                         table, S);
-      hipLaunchKernelGGL(emb_segdot_kernel<uint16_t>, gt, dim3(BW_THREADS), 0, s, ids, g, tr, va,
-                         d, vocab, keys, table, S, chunks, part);
-    } else {
-      const float* g = static_cast<const float*>(G);
-      hipLaunchKernelGGL(emb_segsum_kernel<float>, gv, dim3(128), 0, s, g, va, d, keys, table,
-                         S);
-      hipLaunchKernelGGL(emb_segdot_kernel<float>, gt, dim3(BW_THREADS), 0, s, ids, g, tr, va,
-                         d, vocab, keys, table, S, chunks, part);
-    }
-    hipLaunchKernelGGL(sum_chunks_kernel, dim3(static_cast<unsigned>(n_t)), dim3(BW_THREADS), 0,
-                       s, part, chunks, out_dot);
-    return check_launch("embedding kernels");
-  }
   unsigned* slots = cv.take<unsigned>(EMB_SLOTS);
   unsigned long long* fix = cv.take<unsigned long long>(n_vt * d);
   float* part = cv.take<float>(n_t * chunks);

@@ -167,4 +167,16 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return s;
 }
 
+// ---------------------------------------------------------------- embedding dots (gs_emb_grad.hip)
+// The val tokens' list and fp32 run sums up to these sizes; beyond, 64-bit fixed-point sums
+// (gs_bw.hip), which many more tokens of one id need.
+inline bool embedding_dot_is_listed(int64_t n_val, int64_t T, int64_t vocab) {
+  return n_val * T <= 8192 && vocab < (int64_t{1} << 19);
+}
+size_t embedding_dot_listed_workspace(int64_t N, int64_t n_val, int64_t T, int64_t d,
+                                      int64_t vocab);
+int embedding_dot_listed(const int64_t* ids, const void* G, int dtype, int64_t N, int64_t n_val,
+                         int64_t val_start, int64_t T, int64_t d, int64_t vocab, float* out_dot,
+                         void* workspace, size_t workspace_bytes, hipStream_t s);
+
 }  // namespace gs

@@ -1,4 +1,4 @@
-// Embedding train gradient, gfx950:
+// Embedding train gradient and dot products, gfx950.  The gradient:
 //
 //   grad[v] = scale * sum over the train tokens t with id_t = v of g_t        grad: [vocab, d]
 //
@@ -23,10 +23,18 @@
 //                           windows, by the 16 waves of a workgroup for a longer one, and by
 //                           the workgroups whose windows it covers, a share of the features
 //                           each, for a run of hundreds of tokens or more.
-// Token ids outside [0, vocab) take no part.  Measured on MI355X (GPT-2 wte, 16 train rows of
-// 1024 tokens, d = 768, bf16): list 11 us, windows 19.5 (102 MB written and read: the rate of a
-// copy), combine 6; a padded batch of 65536 train tokens with one id on 59k of them, d = 256:
-// list 52, windows 26, combine 33.
+// Token ids outside [0, vocab) take no part.
+//
+// The dots, dot_i = sum_t <g_it, V[x_it]> with V[v] the sum of the val rows of id v, for up to 8192
+// val tokens: the val tokens' list (with a table of runs per id) in launch 1, the sums of runs of
+// two tokens or more (eg_runs) in the launch of the windows, then
+//   eg_dot_kernel     -- each train token's row against its run's sum or its id's only val row.
+//   eg_dot_sum_kernel -- the parts of a train row added.
+// Either alone, or both in shared launches.  Measured on MI355X (GPT-2 wte, 16 + 4 rows of 1024
+// tokens, d = 768, bf16; 80 us before): lists 14.5 us, runs and windows 22.7 (102 MB written and
+// read: the rate of a copy), combine 6.4, dots 6.6 + 3.3; a padded batch of 65536 train tokens with
+// one id on 59k of them and 4096 val tokens likewise, d = 256: lists 57, windows 38, combine 34,
+// dots 14 + 4.6 (1870 before).
 
 #include <algorithm>
 
@@ -62,19 +70,36 @@ EgRows eg_rows(const RowMap& m) {
                 m.skip_n * m.seglen};
 }
 
-// An id's order in the token list.  Bucketed (shift >= 0): the list is ordered by (id % 256, id /
-// 256), whose number `(id % 256) << shift | id / 256` takes the id's place in the keys; presence
-// bits lie in whole words per bucket.  Otherwise (shift < 0): by the id itself.
+// An id's order in the token list.  Bucketed (shift >= 0): the list is ordered by (id % nb, id /
+// nb) for nb = 2^nbits buckets, whose number `(id % nb) << shift | id / nb` takes the id's place
+// in the keys; presence bits lie in whole words per bucket.  Otherwise (shift < 0): by the id.
 struct EgOrder {
-  int shift;
+  int shift, nbits;
+  __device__ int64_t of(int64_t v) const {
+    return shift < 0 ? v : (v & ((int64_t{1} << nbits) - 1)) << shift | v >> nbits;
+  }
   __device__ int64_t id(int64_t o) const {
-    return shift < 0 ? o : ((o & ((int64_t{1} << shift) - 1)) << 8) | (o >> shift);
+    return shift < 0 ? o : (o & ((int64_t{1} << shift) - 1)) << nbits | o >> shift;
   }
   __host__ __device__ int64_t bucket_words() const { return ((int64_t{1} << shift) + 31) / 32; }
   __device__ bool present(const uint32_t* __restrict__ bits, int64_t v) const {
     if (shift < 0) return (bits[v >> 5] >> (v & 31)) & 1u;
-    return (bits[(v & 255) * bucket_words() + (v >> 13)] >> ((v >> 8) & 31)) & 1u;
+    const int64_t b = v & ((int64_t{1} << nbits) - 1), l = v >> nbits;
+    return (bits[b * bucket_words() + (l >> 5)] >> (l & 31)) & 1u;
   }
+};
+
+// The token list of one row set and what is made from it.
+struct EgList {
+  EgRows rows;
+  EgOrder order;
+  int64_t chunks, windows;        // entries of cnt; windows of the list at its full length
+  unsigned long long* ck;         // the sorted chunks (not bucketed)
+  unsigned long long* sk;         // the list: order << 32 | token
+  int32_t* cnt;                   // in-range tokens, per chunk (bucketed: one number)
+  uint32_t* present;              // presence bits of the ids, or null
+  uint2* table;                   // null, or per id (in list order): its run's first place, length
+  float* part;                    // [windows][2][d] sums of runs that cross windows, or null
 };
 
 // Lane l's value of v, as a wave-uniform value (l a compile-time or uniform lane index).
@@ -376,11 +401,12 @@ __global__ void __launch_bounds__(EG_THREADS) eg_merge_kernel(
   }
 }
 
-// The token list of one row set in one launch (vocab of up to 256 << EG_BUCKET_SHIFT ids): bucket
-// b = blockIdx % 256 holds the ids congruent to b, and its workgroup reads every id of the set.
+// The token lists of one or two row sets (lists a and c, of one order) in one launch: bucket b of a
+// list holds the ids congruent to b modulo the number of buckets (256, or 1024 beyond 131072 ids),
+// and its workgroup reads every id of the set.
 // The tokens of lower buckets, counted in passing, are where the bucket's part of the list
-// begins, so no workgroup waits for another; taking ids modulo 256 spreads the frequent low ids
-// of a real vocabulary over the buckets.  Each of the 16 waves takes a contiguous share of the
+// begins, so no workgroup waits for another; taking ids by remainder spreads the frequent low ids
+// of a real vocabulary over the buckets.  Each of the 16 (8) waves takes a contiguous share of the
 // tokens and keeps the bucket's in LDS (a wave in whose share the bucket has more than
 // EG_BUCKET_KEEP, a padded batch, reads its ids a second time instead).  Counts per (wave, id) in
 // LDS, where tokens of one id among 64 are found by a ballot per bit of the id, become places by
@@ -391,24 +417,21 @@ __global__ void __launch_bounds__(EG_THREADS) eg_merge_kernel(
 // (whole gradient call, us): 16384 tokens of 50257 ids 53.9 -> 35.2 (11 in this kernel, 29 in
 // those two), with 90% of them one id 70.8 -> 53.9; 65536 tokens 101 -> 52.7, 90% one id 125 ->
 // 108; 131072 tokens 225 -> 86, 90% one id 240 -> 177; 192 tokens 40 -> 27.
-constexpr int EG_BUCKET_THREADS = 1024, EG_BUCKET_SHIFT = 9, EG_BUCKET_KEEP = 384;
-constexpr int64_t EG_BUCKET_TOKENS = int64_t{1} << 17;
-struct EgList {
-  EgRows rows;
-  unsigned long long* sk;
-  int32_t* cnt;
-  uint32_t* present;
-};
-
-__global__ void __launch_bounds__(EG_BUCKET_THREADS) eg_bucket_kernel(
-    const int64_t* __restrict__ ids, EgList list, int64_t vocab, EgOrder order) {
-  constexpr int NW = EG_BUCKET_THREADS / 64, U = 8, SHARE_BITS = 13;
-  static_assert(EG_BUCKET_TOKENS / NW <= 1 << SHARE_BITS, "a token's place in its share");
+constexpr int EG_BUCKET_SHIFT = 9, EG_BUCKET_KEEP = 384, EG_SHARE_BITS = 13;
+constexpr int64_t EG_BUCKET_TOKENS = int64_t{16} << EG_SHARE_BITS;
+template <int NW>
+__global__ void __launch_bounds__(64 * NW, 8) eg_bucket_kernel(
+    const int64_t* __restrict__ ids, EgList a, EgList c, int64_t vocab) {
+  constexpr int U = 8, SHARE_BITS = EG_SHARE_BITS;
+  static_assert(64 * NW >= 1 << EG_BUCKET_SHIFT, "a thread for every id of a bucket");
   extern __shared__ int eg_counts[];   // [NW][R]
   __shared__ uint32_t eg_kept[NW][EG_BUCKET_KEEP];   // id of the bucket << SHARE_BITS | place
   __shared__ int wbase[NW], wtot[NW];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int b = blockIdx.x, R = 1 << order.shift;
+  const EgOrder order = a.order;
+  const int nb = 1 << order.nbits, R = 1 << order.shift;
+  const EgList& list = static_cast<int>(blockIdx.x) < nb ? a : c;
+  const int b = blockIdx.x & (nb - 1);
   const int M = static_cast<int>(list.rows.M);
   const int share = ((M + NW - 1) / NW + 63) & ~63;
   const int q_begin = std::min(M, wv * share), q_end = std::min(M, q_begin + share);
@@ -454,11 +477,11 @@ __global__ void __launch_bounds__(EG_BUCKET_THREADS) eg_bucket_kernel(
   };
   int below = 0, n = 0;
   scan([&](unsigned v, int q) {
-    below += __popcll(__ballot(v < nv && static_cast<int>(v & 255u) < b));
-    const bool hit = v < nv && static_cast<int>(v & 255u) == b;
+    below += __popcll(__ballot(v < nv && static_cast<int>(v & (nb - 1)) < b));
+    const bool hit = v < nv && static_cast<int>(v & (nb - 1)) == b;
     const unsigned long long hits = __ballot(hit);
     if (hits == 0) return;
-    const int lid = static_cast<int>(v >> 8), n0 = n;
+    const int lid = static_cast<int>(v >> order.nbits), n0 = n;
     n += __popcll(hits);
     if (n <= EG_BUCKET_KEEP) {
       if (hit)
@@ -493,11 +516,14 @@ __global__ void __launch_bounds__(EG_BUCKET_THREADS) eg_bucket_kernel(
     place += wbase[w] + (w < wv ? wtot[w] : 0);
     all += wbase[w] + wtot[w];
   }
-  if (b == 255 && t == 0) list.cnt[0] = all;
+  if (b == nb - 1 && t == 0) list.cnt[0] = all;
   const unsigned long long present = __ballot(total > 0);
   const int words = static_cast<int>(order.bucket_words());
-  if ((lane & 31) == 0 && (t >> 5) < words)
+  if (list.present != nullptr && (lane & 31) == 0 && (t >> 5) < words)
     list.present[b * words + (t >> 5)] = static_cast<uint32_t>(present >> lane);
+  if (list.table != nullptr && t < R)
+    list.table[(b << order.shift) + t] =
+        make_uint2(static_cast<unsigned>(place), static_cast<unsigned>(total));
   if (t < R)
     for (int w = 0; w < NW; ++w) {
       const int x = eg_counts[w * R + t];
@@ -525,8 +551,8 @@ __global__ void __launch_bounds__(EG_BUCKET_THREADS) eg_bucket_kernel(
     }
   } else {
     scan([&](unsigned v, int q) {
-      const bool hit = v < nv && static_cast<int>(v & 255u) == b;
-      if (__ballot(hit) != 0) write(hit, hit ? static_cast<int>(v >> 8) : 0, q);
+      const bool hit = v < nv && static_cast<int>(v & (nb - 1)) == b;
+      if (__ballot(hit) != 0) write(hit, hit ? static_cast<int>(v >> order.nbits) : 0, q);
     });
   }
 }
@@ -604,21 +630,23 @@ __device__ __forceinline__ void eg_store(GE* __restrict__ out, int64_t f0, int64
 // Waves [windows, windows + zero_waves), overwrite mode: 16 table rows each; rows whose id is
 // absent from the list are written as zeros.
 template <class E, class GE>
-__global__ void __launch_bounds__(EG_THREADS) eg_window_kernel(
-    const E* __restrict__ G, EgRows tr, EgOrder order, int64_t d, int64_t vocab,
-    const unsigned long long* __restrict__ sk, const int32_t* __restrict__ cnt, int64_t chunks,
-    const uint32_t* __restrict__ present, int64_t windows, float scale, int accumulate, int vec,
-    float* __restrict__ part, GE* __restrict__ grad) {
+__device__ __forceinline__ void eg_window(const E* __restrict__ G, const EgList& list, int64_t d,
+                                          int64_t vocab, int64_t block, float scale,
+                                          int accumulate, int vec, GE* __restrict__ grad) {
   constexpr int VE = EgVec<E>::VE;
+  const unsigned long long* __restrict__ sk = list.sk;
+  float* __restrict__ part = list.part;
+  const EgOrder order = list.order;
+  const int64_t windows = list.windows;
   const int lane = threadIdx.x & 63;
-  const int64_t w = static_cast<int64_t>(blockIdx.x) * (EG_THREADS / 64) + (threadIdx.x >> 6);
+  const int64_t w = block * (EG_THREADS / 64) + (threadIdx.x >> 6);
   if (w >= windows) {
     // absent rows, overwrite mode only (the last workgroup's surplus waves land here in
     // both modes): 16 rows, lanes over chunks
     const int64_t v0 = (w - windows) * 16;
     if (accumulate || v0 >= vocab) return;
     const unsigned long long bits =
-        __ballot(lane < 16 && v0 + lane < vocab && order.present(present, v0 + lane));
+        __ballot(lane < 16 && v0 + lane < vocab && order.present(list.present, v0 + lane));
     for (int r = 0; r < 16 && v0 + r < vocab; ++r) {
       if ((bits >> r) & 1u) continue;
       GE* out = grad + (v0 + r) * d;
@@ -631,14 +659,14 @@ __global__ void __launch_bounds__(EG_THREADS) eg_window_kernel(
     }
     return;
   }
-  const int64_t n_list = list_length(cnt, chunks);
+  const int64_t n_list = list_length(list.cnt, list.chunks);
   const int64_t r0 = w * EG_WIN;
   if (r0 >= n_list) return;
   const int n = static_cast<int>(std::min<int64_t>(EG_WIN, n_list - r0));
   // lane i < n: the key at place r0 + i, its id and G row; read as wave-uniform values below
   const unsigned long long k = lane < n ? sk[r0 + lane] : EG_NONE;
   const int64_t my_id = key_id(k);
-  const int64_t my_row = lane < n ? tr(key_tok(k)) : 0;
+  const int64_t my_row = lane < n ? list.rows(key_tok(k)) : 0;
   const bool from_before = r0 > 0 && key_id(sk[r0 - 1]) == readlane_i64(my_id, 0);
   const bool into_next = r0 + n < n_list && key_id(sk[r0 + n]) == readlane_i64(my_id, n - 1);
   // two feature passes per round (lanes own chunks f0 and f0 + 64 VE); the window's rows in
@@ -709,6 +737,147 @@ __global__ void __launch_bounds__(EG_THREADS) eg_window_kernel(
   }
 }
 
+// Run sums of a list with a table: the sum of every run of two tokens or more, in fp32, goes to row
+// (first place) / 2 of S (the first places of two such runs differ by two or more).  Workgroup
+// `block` looks at four places, one a wave.  A run of at most EG_SHORT tokens is summed in list
+// order by the wave of its first place.  The workgroups that a longer run covers share its features,
+// 64 bytes of a row each: 64 groups of threads take every 64th token, and their sums are added in a
+// fixed order.  (90% of 4096 val tokens one id, d = 768, bf16: 56 us for a whole dot against 1.8 ms when
+// the workgroup of the first place walked the run; of 8192, d = 1024, fp32, 54 against 6.9 ms.)
+constexpr int EG_SHORT = 64;
+template <class E>
+struct EgRunsShared {
+  static constexpr int W = 64 / sizeof(E), NG = EG_THREADS / 4;   // features; groups of threads
+  float red[NG][W];
+  float red2[EG_THREADS];
+  int start[EG_THREADS / 64], count[EG_THREADS / 64];
+};
+
+template <class E>
+__device__ __forceinline__ void eg_runs(const E* __restrict__ G, const EgList& list, int64_t d,
+                                        int64_t block, int vec, EgRunsShared<E>& sh,
+                                        float* __restrict__ S) {
+  constexpr int VE = EgVec<E>::VE, B = 8, W = EgRunsShared<E>::W, NG = EgRunsShared<E>::NG;
+  const unsigned long long* __restrict__ sk = list.sk;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int64_t p = block * (EG_THREADS / 64) + wv;
+  int start = 0, count = 0;
+  if (p < list.cnt[0]) {
+    const uint2 e = list.table[key_id(sk[p])];
+    start = static_cast<int>(e.x);
+    count = static_cast<int>(e.y);
+  }
+  if (lane == 0) {
+    sh.start[wv] = start;
+    sh.count[wv] = count;
+  }
+  if (count >= 2 && count <= EG_SHORT && p == start) {
+    for (int64_t f_base = 0; f_base < d; f_base += 128 * VE) {   // every lane, for the rows below
+      const int64_t fb = f_base + static_cast<int64_t>(lane) * VE;
+      float acc[2][VE] = {};
+      for (int r0 = 0; r0 < count; r0 += B) {
+        const int n = std::min(B, count - r0);
+        const int64_t my_row =
+            (lane & (B - 1)) < n ? list.rows(key_tok(sk[start + r0 + (lane & (B - 1))])) : 0;
+        uint4 x[2][B];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int64_t f0 = fb + h * 64 * VE;
+#pragma unroll
+          for (int i = 0; i < B; ++i)
+            x[h][i] = i < n && f0 < d ? eg_load<E>(G + readlane_i64(my_row, i) * d, f0, d,
+                                                   vec && f0 + VE <= d)
+                                      : make_uint4(0u, 0u, 0u, 0u);
+        }
+#pragma unroll
+        for (int i = 0; i < B; ++i)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            typename EgVec<E>::U u;
+            u.u = x[h][i];
+#pragma unroll
+            for (int e = 0; e < VE; ++e)
+              if (i < n) acc[h][e] += to_f32<E>(u.e[e]);
+          }
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int64_t f0 = fb + h * 64 * VE;
+        if (f0 < d)
+          eg_store<float, VE>(S + (static_cast<int64_t>(start) >> 1) * d, f0, d, acc[h], 1.f, 0,
+                              vec && f0 + VE <= d);
+      }
+    }
+  }
+  __syncthreads();
+  for (int q = 0; q < EG_THREADS / 64; ++q) {
+    const int len = sh.count[q], first = sh.start[q];
+    // (the same for the whole workgroup, which may see the end of one run and another's start)
+    if (len <= EG_SHORT || (q > 0 && sh.start[q - 1] == first && sh.count[q - 1] == len)) continue;
+    const int b_lo = first / (EG_THREADS / 64), b_hi = (first + len - 1) / (EG_THREADS / 64);
+    const int64_t step = static_cast<int64_t>(b_hi - b_lo + 1) * W;
+    for (int64_t f0 = (block - b_lo) * W; f0 < d; f0 += step) {
+      const int col = t & 3, g = t >> 2;
+      const int64_t f = f0 + col * VE;
+      float acc[VE] = {};
+      if (f < d) {
+        unsigned tok[B];   // tokens of the next rows, loaded ahead of them
+        const auto tokens = [&](int r0) {
+#pragma unroll
+          for (int i = 0; i < B; ++i)
+            tok[i] = r0 + i * NG < len ? static_cast<unsigned>(sk[first + r0 + i * NG]) : 0u;
+        };
+        tokens(g);
+        for (int r0 = g; r0 < len; r0 += B * NG) {
+          uint4 x[B];
+#pragma unroll
+          for (int i = 0; i < B; ++i)
+            x[i] = r0 + i * NG < len
+                       ? eg_load<E>(G + list.rows(tok[i]) * d, f, d, vec && f + VE <= d)
+                       : make_uint4(0u, 0u, 0u, 0u);
+          tokens(r0 + B * NG);
+#pragma unroll
+          for (int i = 0; i < B; ++i) {
+            typename EgVec<E>::U u;
+            u.u = x[i];
+#pragma unroll
+            for (int e = 0; e < VE; ++e)
+              if (r0 + i * NG < len) acc[e] += to_f32<E>(u.e[e]);
+          }
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < VE; ++e) sh.red[g][col * VE + e] = acc[e];
+      __syncthreads();
+      constexpr int H = EG_THREADS / W, PER = NG / H;
+      const int e = t % W, h = t / W;
+      float a = sh.red[h * PER][e];
+      for (int x = 1; x < PER; ++x) a += sh.red[h * PER + x][e];
+      sh.red2[t] = a;
+      __syncthreads();
+      if (t < W && f0 + t < d) {
+        for (int x = 1; x < H; ++x) a += sh.red2[x * W + t];
+        S[(static_cast<int64_t>(first) >> 1) * d + f0 + t] = a;
+      }
+      __syncthreads();   // red is used again
+    }
+  }
+}
+
+// The first val_blocks workgroups: the run sums of the val list into S; the others: the train
+// gradient's rows.
+template <class E, class GE>
+__global__ void __launch_bounds__(EG_THREADS) eg_window_kernel(
+    const E* __restrict__ G, EgList val, EgList train, unsigned val_blocks, int64_t d,
+    int64_t vocab, float scale, int accumulate, int vec, float* __restrict__ S,
+    GE* __restrict__ grad) {
+  __shared__ EgRunsShared<E> sh;
+  if (blockIdx.x < val_blocks)
+    eg_runs<E>(G, val, d, blockIdx.x, vec, sh, S);
+  else
+    eg_window<E, GE>(G, train, d, vocab, blockIdx.x - val_blocks, scale, accumulate, vec, grad);
+}
+
 // Workgroup b looks at windows [16 b, 16 b + 16), one wave each.  A window whose last run
 // began in it and continues into the next window owns that run; its partials are part[w][1],
 // part[w + 1][0], ..., part[w_end][0] (w_end: the window of the run's last place).
@@ -724,7 +893,7 @@ __global__ void __launch_bounds__(EG_THREADS) eg_window_kernel(
 constexpr int EG_COMBINE_WAVES = 16;
 constexpr int EG_LIGHT = 8, EG_SPREAD = 2;
 
-// Features [j sw, (j + 1) sw) of row `id` for a long run, sw = the row split evenly over the
+// Features [j sw, (j + 1) sw) of row `out` for a long run, sw = the row split evenly over the
 // nb covering workgroups (whole float4s), but at least 16 features: 64-byte pieces of the
 // partial rows (measured at GPT-2 width, d = 768, and a 59k-token run: 34 us with 48
 // workgroups reading 64-byte pieces, 46 us with 192 reading 16-byte ones; a run covering few
@@ -734,14 +903,13 @@ constexpr int EG_LIGHT = 8, EG_SPREAD = 2;
 // at a time, then those results), and the row's features written.
 template <class GE>
 __device__ void eg_spread_sum(const float* __restrict__ part, int64_t ws, int64_t parts,
-                              int64_t d, int64_t id, int64_t j, int64_t nb, float scale,
-                              int accumulate, float* __restrict__ red, GE* __restrict__ grad) {
+                              int64_t d, GE* __restrict__ out, int64_t j, int64_t nb, float scale,
+                              int accumulate, float* __restrict__ red) {
   constexpr int NT = EG_COMBINE_WAVES * 64, B = 8, PASS = 4 * NT;
   const int t = threadIdx.x;
   const bool v4 = (d & 3) == 0;   // rows of whole float4s (part is 256-byte aligned)
   const int64_t sw = std::max<int64_t>(16, ((d + nb - 1) / nb + 3) & ~int64_t(3));
   const int64_t f_begin = j * sw, f_end = std::min(d, f_begin + sw);
-  GE* out = grad + id * d;
   float* red2 = red + PASS;   // the tree's first level: at most 4096 + 256 floats
   for (int64_t fp = f_begin; fp < f_end; fp += PASS) {
     const int width = static_cast<int>(std::min<int64_t>(PASS, f_end - fp));
@@ -799,24 +967,34 @@ __device__ void eg_spread_sum(const float* __restrict__ part, int64_t ws, int64_
   }
 }
 
+constexpr int EG_COMBINE_BLOCK = 1024;   // features per block
+struct EgCombineShared {
+  __attribute__((aligned(16))) float red[EG_COMBINE_WAVES][EG_COMBINE_BLOCK];
+  int64_t run_w[EG_COMBINE_WAVES], run_end[EG_COMBINE_WAVES], run_row[EG_COMBINE_WAVES];
+  int flags[EG_COMBINE_WAVES];
+  int n_runs;
+};
+
 template <class GE>
 __global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
-    const unsigned long long* __restrict__ sk, const int32_t* __restrict__ cnt, int64_t chunks,
-    const float* __restrict__ part, int64_t windows, EgOrder order, int64_t d, float scale,
-    int accumulate, GE* __restrict__ grad) {
-  constexpr int NW = EG_COMBINE_WAVES, CB = 1024;   // waves; features per block
+    EgList list, int64_t d, float scale, int accumulate, GE* __restrict__ grad) {
+  constexpr int NW = EG_COMBINE_WAVES, CB = EG_COMBINE_BLOCK;
+  __shared__ EgCombineShared sh;
+  const int64_t block = blockIdx.x;
   static_assert(NW * 64 == CB, "one feature of a block per thread");
-  __shared__ __attribute__((aligned(16))) float red[NW][CB];
-  __shared__ int64_t run_w[NW], run_end[NW], run_id[NW];
-  __shared__ int n_runs;
+  const unsigned long long* __restrict__ sk = list.sk;
+  const float* __restrict__ part = list.part;
+  const EgOrder order = list.order;
+  const int64_t windows = list.windows;
+  auto& red = sh.red;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int64_t n_list = list_length(cnt, chunks);
+  const int64_t n_list = list_length(list.cnt, list.chunks);
   {
     // A workgroup whose whole range of places lies inside one run that began before it and
     // continues after it (every thread decides alike): its share of that run if the run is
     // spread, else nothing (its windows own no run).
     constexpr int64_t SPAN = static_cast<int64_t>(NW) * EG_WIN;
-    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * SPAN;
+    const int64_t r0 = block * SPAN;
     if (r0 > 0 && r0 + SPAN < n_list) {
       const int64_t id0 = key_id(sk[r0]);
       if (key_id(sk[r0 - 1]) == id0 && key_id(sk[r0 + SPAN]) == id0) {
@@ -837,17 +1015,18 @@ __global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
         const int64_t ws = first / EG_WIN, w_end = (lo - 1) / EG_WIN;
         const int64_t b_lo = ws / NW + 1, nb = w_end / NW - 1 - b_lo + 1;
         if (nb >= EG_SPREAD)
-          eg_spread_sum<GE>(part, ws, w_end - ws + 1, d, order.id(id0), blockIdx.x - b_lo, nb, scale,
-                            accumulate, &red[0][0], grad);
+          eg_spread_sum<GE>(part, ws, w_end - ws + 1, d,
+                            grad + order.id(id0) * d, block - b_lo, nb, scale, accumulate,
+                            &red[0][0]);
         return;
       }
     }
   }
-  if (threadIdx.x == 0) n_runs = 0;
+  if (threadIdx.x == 0) sh.n_runs = 0;
   __syncthreads();
-  const int64_t w = static_cast<int64_t>(blockIdx.x) * NW + wid;
+  const int64_t w = block * NW + wid;
   bool found = false;
-  int64_t id = 0, end = 0;
+  int64_t id = 0, end = 0, row = 0;
   const int64_t r0 = w * EG_WIN;
   if (w < windows && r0 + EG_WIN < n_list) {   // a next window exists
     const int64_t r_last = r0 + EG_WIN - 1;
@@ -871,6 +1050,7 @@ __global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
         }
         end = lo;
       }
+      row = order.id(id);
       // a spread run is left to the workgroups it covers
       const int64_t w_end = (end - 1) / EG_WIN;
       found = (w_end / NW - 1) - (w / NW + 1) + 1 < EG_SPREAD;
@@ -881,7 +1061,7 @@ __global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
   // summed by the whole workgroup.
   const int64_t parts_found = found ? (end - 1) / EG_WIN - w + 1 : 0;
   if (found && parts_found <= EG_LIGHT) {
-    GE* out = grad + order.id(id) * d;
+    GE* out = grad + row * d;
     for (int64_t f = static_cast<int64_t>(lane) * 4; f < d; f += 256) {
       float4 x[EG_LIGHT];
 #pragma unroll
@@ -919,27 +1099,26 @@ __global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
     }
   }
   const bool heavy = found && parts_found > EG_LIGHT;
-  __shared__ int flags[NW];
-  if (lane == 0) flags[wid] = heavy ? 1 : 0;
+  if (lane == 0) sh.flags[wid] = heavy ? 1 : 0;
   __syncthreads();
   if (lane == 0 && heavy) {
     int slot = 0;
-    for (int v = 0; v < wid; ++v) slot += flags[v];
-    run_w[slot] = w;
-    run_end[slot] = end;
-    run_id[slot] = order.id(id);
-    atomicAdd(&n_runs, 1);
+    for (int v = 0; v < wid; ++v) slot += sh.flags[v];
+    sh.run_w[slot] = w;
+    sh.run_end[slot] = end;
+    sh.run_row[slot] = row;
+    atomicAdd(&sh.n_runs, 1);
   }
   __syncthreads();
-  const int runs = n_runs;
+  const int runs = sh.n_runs;
   for (int r = 0; r < runs; ++r) {
-    const int64_t ws = run_w[r], rid = run_id[r];
-    const int64_t w_end = (run_end[r] - 1) / EG_WIN;   // window of the run's last place
+    const int64_t ws = sh.run_w[r];
+    const int64_t w_end = (sh.run_end[r] - 1) / EG_WIN;   // window of the run's last place
     const int64_t parts = w_end - ws + 1;   // part[ws][1], then part[ws + 1 .. w_end][0]
     const int64_t share = (parts + NW - 1) / NW;
     const int64_t p_begin = std::min<int64_t>(parts, wid * share);
     const int64_t p_end = std::min<int64_t>(parts, p_begin + share);
-    GE* out = grad + rid * d;
+    GE* out = grad + sh.run_row[r] * d;
     const bool v4 = (d & 3) == 0;   // rows of whole float4s (part is 256-byte aligned)
     // feature blocks of CB = 4 x 256: lane l owns features 4 l + 256 j, j < 4, so a partial
     // row's block is one round of loads
@@ -986,58 +1165,298 @@ __global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
   }
 }
 
+// part[i * chunks + c] = sum over train row i's tokens in chunk c of <g_it, run sum of x_it>.  One
+// lane looks up each token; the tokens whose id the val rows have are taken by the half-waves in
+// turn, lanes over 16-byte feature chunks, all chunks of up to 1024 features (bf16) in flight.  A
+// run of two tokens or more is read from S, a single one straight from that val token's row of G.
+// (Letting a row's last workgroup add the parts in place of a launch: 15 us against 7 + 3.5, and 56
+// against 15 + 4.5 for 64 chunks a row; the release to the other XCDs costs every workgroup.)
+constexpr int EG_TOK = 32;   // tokens per workgroup
+template <class E>
+__global__ void __launch_bounds__(EG_THREADS) eg_dot_kernel(
+    const int64_t* __restrict__ ids, const E* __restrict__ G, EgRows train, int64_t T, EgList val,
+    int64_t d, int64_t vocab, const float* __restrict__ S, int vec, int64_t chunks,
+    float* __restrict__ part) {
+  constexpr int VE = EgVec<E>::VE, P = 4;
+  __shared__ float red[EG_THREADS / 64];
+  __shared__ int64_t rows[EG_TOK], src[EG_TOK];   // src: row of S, or -1 - row of G
+  __shared__ int hits;
+  const int64_t i = blockIdx.y, c = blockIdx.x;
+  if (threadIdx.x < 64) {
+    const int64_t t = c * EG_TOK + threadIdx.x;
+    const bool in = threadIdx.x < EG_TOK && t < T;
+    const int64_t row = in ? train(i * T + t) : 0;
+    const int64_t id = in ? ids[row] : -1;
+    const uint2 e = id >= 0 && id < vocab ? val.table[val.order.of(id)] : make_uint2(0u, 0u);
+    const unsigned long long found = __ballot(e.y != 0);
+    if (e.y != 0) {
+      const int h = __popcll(found & ((1ull << threadIdx.x) - 1ull));
+      rows[h] = row;
+      src[h] = e.y > 1 ? static_cast<int64_t>(e.x >> 1) : -1 - val.rows(key_tok(val.sk[e.x]));
+    }
+    if (threadIdx.x == 0) hits = __popcll(found);
+  }
+  __syncthreads();
+  const int hl = threadIdx.x & 31, n = hits;
+  float s = 0.f;
+  for (int h = threadIdx.x >> 5; h < n; h += EG_THREADS / 32) {
+    const E* g = G + rows[h] * d;
+    const int64_t sr = src[h];
+    for (int64_t fb = static_cast<int64_t>(hl) * VE; fb < d; fb += P * 32 * VE) {
+      typename EgVec<E>::U x[P];
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const int64_t f = fb + p * 32 * VE;
+        x[p].u = f < d ? eg_load<E>(g, f, d, vec && f + VE <= d) : make_uint4(0u, 0u, 0u, 0u);
+      }
+      if (sr >= 0) {
+        const float* v = S + sr * d;
+        float4 y[P][VE / 4];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          const int64_t f = fb + p * 32 * VE;
+#pragma unroll
+          for (int e = 0; e < VE / 4; ++e)
+            y[p][e] = f + 4 * e < d
+                          ? __builtin_bit_cast(float4, eg_load<float>(v, f + 4 * e, d,
+                                                                      vec && f + VE <= d))
+                          : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+          for (int e = 0; e < VE / 4; ++e)
+            s += to_f32<E>(x[p].e[4 * e]) * y[p][e].x + to_f32<E>(x[p].e[4 * e + 1]) * y[p][e].y +
+                 to_f32<E>(x[p].e[4 * e + 2]) * y[p][e].z + to_f32<E>(x[p].e[4 * e + 3]) * y[p][e].w;
+      } else {
+        const E* v = G + (-1 - sr) * d;
+        typename EgVec<E>::U y[P];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          const int64_t f = fb + p * 32 * VE;
+          y[p].u = f < d ? eg_load<E>(v, f, d, vec && f + VE <= d) : make_uint4(0u, 0u, 0u, 0u);
+        }
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+          for (int e = 0; e < VE; ++e) s += to_f32<E>(x[p].e[e]) * to_f32<E>(y[p].e[e]);
+      }
+    }
+  }
+  const float tot = block_sum(s, red);
+  if (threadIdx.x == 0) part[i * chunks + c] = tot;
+}
+
+__global__ void __launch_bounds__(EG_THREADS) eg_dot_sum_kernel(const float* __restrict__ part,
+                                                                int64_t chunks,
+                                                                float* __restrict__ out) {
+  __shared__ float red[EG_THREADS / 64];
+  const int64_t i = blockIdx.x;
+  float s = 0.f;
+  for (int64_t c = threadIdx.x; c < chunks; c += blockDim.x) s += part[i * chunks + c];
+  s = block_sum(s, red);
+  if (threadIdx.x == 0) out[i] = s;
+}
+
 int64_t eg_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-struct EgPlan {
-  int64_t M, chunks, windows, present_words;
-  EgOrder order;
+// One call: the dots (val list, its run sums S, parts of the dots), the train gradient (train
+// list), or both.
+struct EgCall {
+  int64_t N, n_val, val_start, T, d, vocab;
+  bool dot, grad;
+  EgList val, train;
+  float* S;
+  float* parts;
 };
 
-// The bucketed list where its counters and a wave's places fit (131072 tokens, 131072 ids): there it
-// was the faster one at every size measured (figures at eg_bucket_kernel).  Sort and merge beyond.
-EgPlan eg_plan(int64_t M, int64_t vocab) {
-  EgPlan p;
-  p.M = M;
-  p.windows = eg_cdiv(M, EG_WIN);
-  p.order.shift = -1;
-  if (M <= EG_BUCKET_TOKENS && vocab <= (int64_t{256} << EG_BUCKET_SHIFT)) {
-    p.order.shift = 0;
-    while ((int64_t{256} << p.order.shift) < vocab) ++p.order.shift;
-  }
-  p.chunks = p.order.shift < 0 ? eg_cdiv(M, EG_CHUNK) : 1;
-  p.present_words = p.order.shift < 0 ? eg_cdiv(vocab, 32) : 256 * p.order.bucket_words();
-  return p;
+// The bucketed list where its counters and a wave's places fit (131072 tokens, 524288 ids): there
+// it was the faster one at every size measured (figures at eg_bucket_kernel).  Sort and merge
+// beyond.
+EgOrder eg_order(int64_t M, int64_t vocab) {
+  EgOrder o{-1, 8};
+  if (M > EG_BUCKET_TOKENS || vocab > (int64_t{1024} << EG_BUCKET_SHIFT)) return o;
+  if (vocab > (int64_t{256} << EG_BUCKET_SHIFT)) o.nbits = 10;
+  o.shift = 0;
+  while ((int64_t{1} << (o.nbits + o.shift)) < vocab) ++o.shift;
+  return o;
 }
 
 template <class S>
-void carve_emb_grad(S& c, const EgPlan& p, int64_t d, unsigned long long** ck,
-                    unsigned long long** sk, int32_t** cnt, uint32_t** present, float** part) {
-  *ck = c.template take<unsigned long long>(p.order.shift < 0 ? p.chunks * EG_CHUNK : 0);
-  *sk = c.template take<unsigned long long>(p.M);
-  *cnt = c.template take<int32_t>(p.chunks);
-  *present = c.template take<uint32_t>(p.present_words);
-  *part = c.template take<float>(p.windows * 2 * d);
+void carve_list(S& c, EgList& l, const EgRows& rows, int64_t vocab) {
+  l = EgList{};
+  l.rows = rows;
+  l.order = eg_order(rows.M, vocab);
+  const bool bucketed = l.order.shift >= 0;
+  l.chunks = bucketed ? 1 : eg_cdiv(rows.M, EG_CHUNK);
+  l.windows = eg_cdiv(rows.M, EG_WIN);
+  if (!bucketed) l.ck = c.template take<unsigned long long>(l.chunks * EG_CHUNK);
+  l.sk = c.template take<unsigned long long>(rows.M);
+  l.cnt = c.template take<int32_t>(l.chunks);
+}
+
+template <class S>
+void carve_call(S& c, EgCall& e) {
+  if (e.dot) {   // always bucketed: at most 8192 tokens and 2^19 ids
+    carve_list(c, e.val, eg_rows(val_rows(e.n_val, e.val_start, e.T)), e.vocab);
+    e.val.table = c.template take<uint2>(size_t{1} << (e.val.order.nbits + e.val.order.shift));
+    e.S = c.template take<float>((e.n_val * e.T / 2 + 1) * e.d);
+    e.parts = c.template take<float>((e.N - e.n_val) * eg_cdiv(e.T, EG_TOK));
+  }
+  if (e.grad) {
+    EgList& l = e.train;
+    carve_list(c, l, eg_rows(train_rows(e.N, e.n_val, e.val_start, e.T)), e.vocab);
+    l.present = c.template take<uint32_t>(
+        l.order.shift >= 0 ? l.order.bucket_words() << l.order.nbits : eg_cdiv(e.vocab, 32));
+    l.part = c.template take<float>(l.windows * 2 * e.d);
+  }
+}
+
+int build_bucketed(const int64_t* ids, const EgList& a, const EgList* c, int64_t vocab,
+                   hipStream_t s) {
+  const dim3 grid((c != nullptr ? 2u : 1u) << a.order.nbits);
+  const int64_t M = std::max(a.rows.M, c != nullptr ? c->rows.M : 0);
+  const EgList& b = c != nullptr ? *c : a;
+  // Half the waves where a share is short anyway or the buckets are many (measured as the whole
+  // dot, us: 4096 val tokens of 50257 ids 22.1 -> 21.0, 2048 of 300000 27.8 -> 21.3).
+  if (M <= (int64_t{8} << EG_SHARE_BITS) && (a.order.nbits > 8 || M <= 8192))
+    hipLaunchKernelGGL(eg_bucket_kernel<8>, grid, dim3(512), 8 * sizeof(int) << a.order.shift, s,
+                       ids, a, b, vocab);
+  else
+    hipLaunchKernelGGL(eg_bucket_kernel<16>, grid, dim3(1024), 16 * sizeof(int) << a.order.shift,
+                       s, ids, a, b, vocab);
+  return check_launch("eg_bucket_kernel");
+}
+
+int build_list(const int64_t* ids, const EgList& l, int64_t vocab, hipStream_t s) {
+  if (l.order.shift >= 0) return build_bucketed(ids, l, nullptr, vocab, s);
+  const dim3 mgrid(static_cast<unsigned>(eg_cdiv(l.chunks * EG_CHUNK, EG_THREADS)));
+  const dim3 sgrid(static_cast<unsigned>(l.chunks));
+  const int64_t words = eg_cdiv(vocab, 32);
+  if (vocab <= EG_KEY32_VOCAB) {
+    uint32_t* ck32 = reinterpret_cast<uint32_t*>(l.ck);
+    hipLaunchKernelGGL(eg_sort_kernel<uint32_t>, sgrid, dim3(EG_SORT_THREADS), 0, s, ids, l.rows,
+                       vocab, ck32, l.cnt, l.present, words);
+    if (l.chunks <= EG_SAMP_CHUNKS)
+      hipLaunchKernelGGL((eg_merge_kernel<uint32_t, true>), mgrid, dim3(EG_THREADS),
+                         static_cast<unsigned>(l.chunks * EG_NSAMP * sizeof(uint32_t)), s, ck32,
+                         l.chunks, l.sk, l.present);
+    else
+      hipLaunchKernelGGL((eg_merge_kernel<uint32_t, false>), mgrid, dim3(EG_THREADS), 0, s, ck32,
+                         l.chunks, l.sk, l.present);
+  } else {
+    hipLaunchKernelGGL(eg_sort_kernel<unsigned long long>, sgrid, dim3(EG_SORT_THREADS), 0, s,
+                       ids, l.rows, vocab, l.ck, l.cnt, l.present, words);
+    hipLaunchKernelGGL((eg_merge_kernel<unsigned long long, false>), mgrid, dim3(EG_THREADS), 0,
+                       s, l.ck, l.chunks, l.sk, l.present);
+  }
+  return check_launch("eg_sort_kernel / eg_merge_kernel");
 }
 
 template <class E, class GE>
-int launch_rows(const void* G, const EgRows& tr, int64_t d, int64_t vocab, const EgPlan& pl,
-                const unsigned long long* sk, const int32_t* cnt, const uint32_t* present,
-                float* part, float scale, int accumulate, int vec, void* grad, hipStream_t s) {
-  const int64_t zero_waves = accumulate ? 0 : eg_cdiv(vocab, 16);
-  const int64_t waves = pl.windows + zero_waves;
-  hipLaunchKernelGGL((eg_window_kernel<E, GE>),
-                     dim3(static_cast<unsigned>(eg_cdiv(waves, EG_THREADS / 64))),
-                     dim3(EG_THREADS), 0, s, static_cast<const E*>(G), tr, pl.order, d, vocab, sk, cnt,
-                     pl.chunks, present, pl.windows, scale, accumulate, vec, part,
-                     static_cast<GE*>(grad));
-  hipLaunchKernelGGL((eg_combine_kernel<GE>),
-                     dim3(static_cast<unsigned>(eg_cdiv(pl.windows, EG_COMBINE_WAVES))),
-                     dim3(EG_COMBINE_WAVES * 64), 0, s, sk, cnt, pl.chunks, part, pl.windows,
-                     pl.order, d, scale, accumulate, static_cast<GE*>(grad));
-  return check_launch("eg_window_kernel / eg_combine_kernel");
+int run_call(const EgCall& c, const int64_t* ids, const void* Gv, float* out_dot, float scale,
+             int accumulate, int vec, void* gradv, hipStream_t s) {
+  const E* G = static_cast<const E*>(Gv);
+  GE* grad = static_cast<GE*>(gradv);
+  int rc = 0;
+  if (c.dot && c.grad && c.val.order.shift >= 0 && c.train.order.shift >= 0) {
+    rc = build_bucketed(ids, c.val, &c.train, c.vocab, s);
+  } else {
+    if (c.dot) rc = build_list(ids, c.val, c.vocab, s);
+    if (!rc && c.grad) rc = build_list(ids, c.train, c.vocab, s);
+  }
+  if (rc) return rc;
+  const auto blocks = [](int64_t waves, int64_t per) {
+    return static_cast<unsigned>(eg_cdiv(waves, per));
+  };
+  const int64_t zero_waves = accumulate ? 0 : eg_cdiv(c.vocab, 16);
+  const unsigned vw = c.dot ? blocks(c.n_val * c.T, EG_THREADS / 64) : 0;
+  const unsigned tw = c.grad ? blocks(c.train.windows + zero_waves, EG_THREADS / 64) : 0;
+  hipLaunchKernelGGL((eg_window_kernel<E, GE>), dim3(vw + tw), dim3(EG_THREADS), 0, s, G, c.val,
+                     c.train, vw, c.d, c.vocab, scale, accumulate, vec, c.S, grad);
+  if (c.grad)
+    hipLaunchKernelGGL((eg_combine_kernel<GE>), dim3(blocks(c.train.windows, EG_COMBINE_WAVES)),
+                       dim3(EG_COMBINE_WAVES * 64), 0, s, c.train, c.d, scale, accumulate, grad);
+  rc = check_launch("eg_window_kernel / eg_combine_kernel");
+  if (rc || !c.dot) return rc;
+  const int64_t n_t = c.N - c.n_val, chunks = eg_cdiv(c.T, EG_TOK);
+  hipLaunchKernelGGL(eg_dot_kernel<E>,
+                     dim3(static_cast<unsigned>(chunks), static_cast<unsigned>(n_t)),
+                     dim3(EG_THREADS), 0, s, ids, G,
+                     eg_rows(train_rows(c.N, c.n_val, c.val_start, c.T)), c.T, c.val, c.d, c.vocab,
+                     c.S, vec, chunks, c.parts);
+  hipLaunchKernelGGL(eg_dot_sum_kernel, dim3(static_cast<unsigned>(n_t)), dim3(EG_THREADS), 0, s,
+                     c.parts, chunks, out_dot);
+  return check_launch("eg_dot_kernel");
+}
+
+// grad_dtype: any when there is no gradient.
+int start_call(EgCall& c, const char* name, const int64_t* ids, const void* G, int dtype,
+               float* out_dot, float scale, void* grad, int grad_dtype, int accumulate,
+               void* workspace, size_t workspace_bytes, hipStream_t s) {
+  Sizer sz;
+  carve_call(sz, c);
+  if (workspace == nullptr || workspace_bytes < sz.used)
+    return fail(GS_ERR_WORKSPACE, std::string(name) + ": workspace too small");
+  Carver cv(workspace, workspace_bytes);
+  carve_call(cv, c);
+  const size_t esz = elem_size(dtype), gsz = c.grad ? elem_size(grad_dtype) : 4;
+  const int vec = (reinterpret_cast<uintptr_t>(G) % 16 == 0) &&
+                  (reinterpret_cast<uintptr_t>(grad) % 16 == 0) &&
+                  (c.d * static_cast<int64_t>(esz)) % 16 == 0 &&
+                  (c.d * static_cast<int64_t>(gsz)) % 16 == 0;
+  const bool half = c.grad && grad_dtype == GS_DTYPE_BF16;
+  const int acc = accumulate ? 1 : 0;
+  if (dtype == GS_DTYPE_BF16)
+    return half ? run_call<uint16_t, uint16_t>(c, ids, G, out_dot, scale, acc, vec, grad, s)
+                : run_call<uint16_t, float>(c, ids, G, out_dot, scale, acc, vec, grad, s);
+  return half ? run_call<float, uint16_t>(c, ids, G, out_dot, scale, acc, vec, grad, s)
+              : run_call<float, float>(c, ids, G, out_dot, scale, acc, vec, grad, s);
+}
+
+EgCall eg_call(int64_t N, int64_t n_val, int64_t val_start, int64_t T, int64_t d, int64_t vocab,
+               bool dot, bool grad) {
+  EgCall c{};
+  c.N = N, c.n_val = n_val, c.val_start = val_start, c.T = T, c.d = d, c.vocab = vocab;
+  c.dot = dot, c.grad = grad;
+  return c;
+}
+
+size_t call_workspace(EgCall c) {
+  Sizer sz;
+  carve_call(sz, c);
+  return sz.used + 256;
+}
+
+int grad_args_ok(const char* name, const int64_t* ids, const void* G, int dtype, int64_t N,
+                 int64_t n_val, int64_t val_start, int64_t T, int64_t d, int64_t vocab,
+                 const void* grad, int grad_dtype) {
+  if (dtype != GS_DTYPE_BF16 && dtype != GS_DTYPE_F32)
+    return fail(GS_ERR_DTYPE, std::string(name) + ": dtype must be bf16 or fp32");
+  if (grad_dtype != GS_DTYPE_BF16 && grad_dtype != GS_DTYPE_F32)
+    return fail(GS_ERR_DTYPE, std::string(name) + ": grad_dtype must be bf16 or fp32");
+  if (ids == nullptr || G == nullptr || grad == nullptr || N <= 0 || n_val < 0 || n_val >= N ||
+      val_start < 0 || val_start + n_val > N || T <= 0 || d <= 0 || vocab <= 0)
+    return fail(GS_ERR_INVALID, std::string(name) + ": invalid arguments");
+  if ((N - n_val) * T >= INT32_MAX || vocab >= INT32_MAX)
+    return fail(GS_ERR_UNSUPPORTED, std::string(name) + ": 2^31 or more tokens or ids");
+  return 0;
 }
 
 }  // namespace
+
+// The dots through the val tokens' list (gs_embedding_dot checks the arguments and the sizes).
+size_t embedding_dot_listed_workspace(int64_t N, int64_t n_val, int64_t T, int64_t d,
+                                      int64_t vocab) {
+  return call_workspace(eg_call(N, n_val, 0, T, d, vocab, true, false));
+}
+int embedding_dot_listed(const int64_t* ids, const void* G, int dtype, int64_t N, int64_t n_val,
+                         int64_t val_start, int64_t T, int64_t d, int64_t vocab, float* out_dot,
+                         void* workspace, size_t workspace_bytes, hipStream_t s) {
+  EgCall c = eg_call(N, n_val, val_start, T, d, vocab, true, false);
+  return start_call(c, "gs_embedding_dot", ids, G, dtype, out_dot, 0.f, nullptr, GS_DTYPE_F32, 0,
+                    workspace, workspace_bytes, s);
+}
 }  // namespace gs
 
 using namespace gs;
@@ -1045,14 +1464,7 @@ using namespace gs;
 extern "C" size_t gs_embedding_train_grad_workspace(int64_t N, int64_t n_val, int64_t T,
                                                     int64_t d, int64_t vocab) {
   if (N <= 0 || n_val < 0 || n_val >= N || T <= 0 || d <= 0 || vocab <= 0) return 0;
-  const EgPlan pl = eg_plan((N - n_val) * T, vocab);
-  Sizer sz;
-  unsigned long long *ck, *sk;
-  int32_t* cnt;
-  uint32_t* present;
-  float* part;
-  carve_emb_grad(sz, pl, d, &ck, &sk, &cnt, &present, &part);
-  return sz.used + 256;
+  return call_workspace(eg_call(N, n_val, 0, T, d, vocab, false, true));
 }
 
 extern "C" int gs_embedding_train_grad(const int64_t* ids, const void* G, int dtype, int64_t N,
@@ -1060,71 +1472,35 @@ extern "C" int gs_embedding_train_grad(const int64_t* ids, const void* G, int dt
                                        int64_t vocab, float scale, void* grad, int grad_dtype,
                                        int accumulate, void* workspace, size_t workspace_bytes,
                                        void* stream) {
-  if (dtype != GS_DTYPE_BF16 && dtype != GS_DTYPE_F32)
-    return fail(GS_ERR_DTYPE, "gs_embedding_train_grad: dtype must be bf16 or fp32");
-  if (grad_dtype != GS_DTYPE_BF16 && grad_dtype != GS_DTYPE_F32)
-    return fail(GS_ERR_DTYPE, "gs_embedding_train_grad: grad_dtype must be bf16 or fp32");
-  if (ids == nullptr || G == nullptr || grad == nullptr || N <= 0 || n_val < 0 || n_val >= N ||
-      val_start < 0 || val_start + n_val > N || T <= 0 || d <= 0 || vocab <= 0)
-    return fail(GS_ERR_INVALID, "gs_embedding_train_grad: invalid arguments");
-  const int64_t M = (N - n_val) * T;
-  if (M >= INT32_MAX || vocab >= INT32_MAX)
-    return fail(GS_ERR_UNSUPPORTED, "gs_embedding_train_grad: 2^31 or more tokens or ids");
-  const EgPlan pl = eg_plan(M, vocab);
-  Sizer sz;
-  unsigned long long *ck, *sk;
-  int32_t* cnt;
-  uint32_t* present;
-  float* part;
-  carve_emb_grad(sz, pl, d, &ck, &sk, &cnt, &present, &part);
-  if (workspace == nullptr || workspace_bytes < sz.used)
-    return fail(GS_ERR_WORKSPACE, "gs_embedding_train_grad: workspace too small");
-  Carver cv(workspace, workspace_bytes);
-  carve_emb_grad(cv, pl, d, &ck, &sk, &cnt, &present, &part);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const EgRows tr = eg_rows(train_rows(N, n_val, val_start, T));
-  const dim3 mgrid(static_cast<unsigned>(eg_cdiv(pl.chunks * EG_CHUNK, EG_THREADS)));
-  if (pl.order.shift >= 0) {
-    const EgList list{tr, sk, cnt, present};
-    hipLaunchKernelGGL(eg_bucket_kernel, dim3(256), dim3(EG_BUCKET_THREADS),
-                       (EG_BUCKET_THREADS / 64) * sizeof(int) << pl.order.shift, s, ids, list,
-                       vocab, pl.order);
-  } else if (vocab <= EG_KEY32_VOCAB) {
-    uint32_t* ck32 = reinterpret_cast<uint32_t*>(ck);
-    hipLaunchKernelGGL(eg_sort_kernel<uint32_t>, dim3(static_cast<unsigned>(pl.chunks)),
-                       dim3(EG_SORT_THREADS), 0, s, ids, tr, vocab, ck32, cnt, present,
-                       pl.present_words);
-    if (pl.chunks <= EG_SAMP_CHUNKS)
-      hipLaunchKernelGGL((eg_merge_kernel<uint32_t, true>), mgrid, dim3(EG_THREADS),
-                         static_cast<unsigned>(pl.chunks * EG_NSAMP * sizeof(uint32_t)), s,
-                         ck32, pl.chunks, sk, present);
-    else
-      hipLaunchKernelGGL((eg_merge_kernel<uint32_t, false>), mgrid, dim3(EG_THREADS), 0, s,
-                         ck32, pl.chunks, sk, present);
-  } else {
-    hipLaunchKernelGGL(eg_sort_kernel<unsigned long long>, dim3(static_cast<unsigned>(pl.chunks)),
-                       dim3(EG_SORT_THREADS), 0, s, ids, tr, vocab, ck, cnt, present,
-                       pl.present_words);
-    hipLaunchKernelGGL((eg_merge_kernel<unsigned long long, false>), mgrid, dim3(EG_THREADS),
-                       0, s, ck, pl.chunks, sk, present);
-  }
-  int rc = check_launch("eg_bucket_kernel / eg_sort_kernel / eg_merge_kernel");
-  if (rc) return rc;
-  const size_t esz = elem_size(dtype), gsz = elem_size(grad_dtype);
-  const int vec = (reinterpret_cast<uintptr_t>(G) % 16 == 0) &&
-                  (reinterpret_cast<uintptr_t>(grad) % 16 == 0) &&
-                  (d * static_cast<int64_t>(esz)) % 16 == 0 &&
-                  (d * static_cast<int64_t>(gsz)) % 16 == 0;
-  const int acc = accumulate ? 1 : 0;
-  if (dtype == GS_DTYPE_BF16)
-    return grad_dtype == GS_DTYPE_BF16
-               ? launch_rows<uint16_t, uint16_t>(G, tr, d, vocab, pl, sk, cnt, present, part,
-                                                 scale, acc, vec, grad, s)
-               : launch_rows<uint16_t, float>(G, tr, d, vocab, pl, sk, cnt, present, part,
-                                              scale, acc, vec, grad, s);
-  return grad_dtype == GS_DTYPE_BF16
-             ? launch_rows<float, uint16_t>(G, tr, d, vocab, pl, sk, cnt, present, part, scale,
-                                            acc, vec, grad, s)
-             : launch_rows<float, float>(G, tr, d, vocab, pl, sk, cnt, present, part, scale, acc,
-                                         vec, grad, s);
+  if (int rc = grad_args_ok("gs_embedding_train_grad", ids, G, dtype, N, n_val, val_start, T, d,
+                            vocab, grad, grad_dtype))
+    return rc;
+  EgCall c = eg_call(N, n_val, val_start, T, d, vocab, false, true);
+  return start_call(c, "gs_embedding_train_grad", ids, G, dtype, nullptr, scale, grad, grad_dtype,
+                    accumulate, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+extern "C" size_t gs_embedding_layer_pass_workspace(int64_t N, int64_t n_val, int64_t T, int64_t d,
+                                                    int64_t vocab) {
+  if (N <= 0 || n_val <= 0 || n_val >= N || T <= 0 || d <= 0 || vocab <= 0 ||
+      !embedding_dot_is_listed(n_val, T, vocab))
+    return 0;
+  return call_workspace(eg_call(N, n_val, 0, T, d, vocab, true, true));
+}
+
+extern "C" int gs_embedding_layer_pass(const int64_t* ids, const void* G, int dtype, int64_t N,
+                                       int64_t n_val, int64_t val_start, int64_t T, int64_t d,
+                                       int64_t vocab, float* out_dot, float scale, void* grad,
+                                       int grad_dtype, int accumulate, void* workspace,
+                                       size_t workspace_bytes, void* stream) {
+  if (int rc = grad_args_ok("gs_embedding_layer_pass", ids, G, dtype, N, n_val, val_start, T, d,
+                            vocab, grad, grad_dtype))
+    return rc;
+  if (n_val == 0 || out_dot == nullptr)
+    return fail(GS_ERR_INVALID, "gs_embedding_layer_pass: invalid arguments");
+  if (!embedding_dot_is_listed(n_val, T, vocab))
+    return fail(GS_ERR_UNSUPPORTED, "gs_embedding_layer_pass: more than 8192 val tokens or 2^19 ids");
+  EgCall c = eg_call(N, n_val, val_start, T, d, vocab, true, true);
+  return start_call(c, "gs_embedding_layer_pass", ids, G, dtype, out_dot, scale, grad, grad_dtype,
+                    accumulate, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }

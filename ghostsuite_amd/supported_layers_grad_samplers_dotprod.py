@@ -410,8 +410,6 @@ def _compute_embedding_dot_product(layer: nn.Embedding, A: torch.Tensor, B: torc
         B = B.float()
     elif B.dtype not in (torch.bfloat16, torch.float32):
         B = B.float()
-    layer.weight.grad_dot_prod = ops().embedding_dot(A, B, val_batch_size,
-                                                     vocab=layer.weight.shape[0])
     # With the train-grad scale announced, the train gradient is formed here as well (same
     # stream as the dot, no second hook-stage launch sequence) and parked for
     # _compute_embedding_train_grad.
@@ -422,8 +420,20 @@ def _compute_embedding_dot_product(layer: nn.Embedding, A: torch.Tensor, B: torc
         # its dot stage promoted to the backprops' dtype (:116-123), which may have rounded.
         ids = layer.__dict__.get("activations")
         ids = A if ids is None or ids.is_floating_point() else ids.detach()
-        layer.__dict__["_gs_weight_train_grad"] = _embedding_train_grad(
-            layer, ids, B, val_batch_size, scale)
+        out, grad, accumulate = _embedding_grad_out(layer)
+        layer_pass = getattr(ops(), "embedding_layer_pass", None)
+        dot = None
+        if layer_pass is not None and ids.data_ptr() == A.data_ptr() and \
+                ids.dtype == A.dtype and ids.stride() == A.stride():
+            dot = layer_pass(A, B, val_batch_size, scale, out, accumulate=accumulate)
+        if dot is None:
+            dot = ops().embedding_dot(A, B, val_batch_size, vocab=layer.weight.shape[0])
+            ops().embedding_train_grad(ids, B, val_batch_size, scale, out, accumulate=accumulate)
+        layer.weight.grad_dot_prod = dot
+        layer.__dict__["_gs_weight_train_grad"] = grad
+        return
+    layer.weight.grad_dot_prod = ops().embedding_dot(A, B, val_batch_size,
+                                                     vocab=layer.weight.shape[0])
 
 
 # Returned by a train-grad sampler that has already added its gradient into
@@ -455,14 +465,20 @@ def _embedding_train_grad(layer: nn.Embedding, A: torch.Tensor, B: torch.Tensor,
     B = B.detach()
     if B.dtype not in (torch.bfloat16, torch.float32):
         B = B.float()
+    out, grad, accumulate = _embedding_grad_out(layer)
+    ops().embedding_train_grad(A.detach(), B, val_batch_size, alpha, out, accumulate=accumulate)
+    return grad
+
+
+def _embedding_grad_out(layer: nn.Embedding):
+    """Where the layer's train gradient goes: (tensor, what the hook stage gets, whether it is
+    added to the tensor's contents)."""
     prev = getattr(layer.weight, "train_grad", None)
     if prev is not None and prev.shape == layer.weight.shape:
         _overlap.join(prev.device)   # prev may come from the other stream
-        ops().embedding_train_grad(A.detach(), B, val_batch_size, alpha, prev, accumulate=True)
-        return APPLIED
+        return prev, APPLIED, True
     grad = torch.empty_like(layer.weight)
-    ops().embedding_train_grad(A.detach(), B, val_batch_size, alpha, grad)
-    return grad
+    return grad, grad, False
 
 
 # LayerNorm Layer ###########################################################################

@@ -280,10 +280,11 @@ int gs_bias_dot(const void* G, int dtype, int64_t N, int64_t n_val, int64_t val_
 /* ---- Embedding dot product -----------------------------------------------------------
  * Replaces _compute_embedding_dot_product (:181-211):
  *   dot_i = sum_t <g_it, V[x_it]>,  V[v] = sum_{j in val, s : x_js = v} g_js
- * without a [vocab, d] table: val tokens with equal ids form one segment (keyed by the
- * first such val token through a [vocab] int32 index), segment sums are accumulated in
- * 64-bit fixed point (deterministic), and each train token looks its segment up by id.
- * ids: [N, T] int64 token ids in [0, vocab).  G: [N, T, d]. */
+ * without a [vocab, d] table: val tokens with equal ids form one segment, and each train
+ * token looks its segment up by id.  Up to 8192 val tokens and ids below 2^19: segments are
+ * runs of the val tokens' list by id, summed in fp32 in list order as the train gradient's
+ * (below).  Beyond: segment sums in 64-bit fixed point.  Both are deterministic.
+ * ids: [N, T] int64 token ids, those outside [0, vocab) take no part.  G: [N, T, d]. */
 size_t gs_embedding_dot_workspace(int64_t N, int64_t n_val, int64_t T, int64_t d,
                                   int64_t vocab);
 int gs_embedding_dot(const int64_t* ids, const void* G, int dtype, int64_t N, int64_t n_val,
@@ -294,9 +295,9 @@ int gs_embedding_dot(const int64_t* ids, const void* G, int dtype, int64_t N, in
  * Replaces _compute_embedding_train_grad (:214-235):
  *   grad[v] = scale * sum over the train tokens t with x_t = v of g_t     grad: [vocab, d]
  * (the reference: index_add_ of the N-scaled train rows into zeros_like(weight), then / n_t;
- * here scale = N / n_t carries both factors).  The train tokens are sorted by (id, token
- * index); each id's rows are summed in fp32 in token order over windows of 16 places of the
- * sorted list, a run that crosses windows by its window parts in window order, and written
+ * here scale = N / n_t carries both factors).  The train tokens are listed by id, equal ids
+ * in token order; each id's rows are summed in fp32 in token order over windows of 8 places of
+ * the list, a run that crosses windows by its window parts in window order, and written
  * once, rounded once to grad_dtype: the same bits on every run, and work linear in the
  * number of tokens however often an id repeats.
  * accumulate = 0: every row of grad is written (zeros where no train token has the id).
@@ -310,6 +311,18 @@ int gs_embedding_train_grad(const int64_t* ids, const void* G, int dtype, int64_
                             int64_t vocab, float scale, void* grad, int grad_dtype,
                             int accumulate, void* workspace, size_t workspace_bytes,
                             void* stream);
+
+/* Both of the above in shared launches (one token list kernel, one window pass, one pass over
+ * runs that cross windows, then the dots), with the same results.  For the sizes whose dots go
+ * through the val tokens' list; the workspace query answers 0 for others, which take the two
+ * calls (the call itself: GS_ERR_UNSUPPORTED). */
+size_t gs_embedding_layer_pass_workspace(int64_t N, int64_t n_val, int64_t T, int64_t d,
+                                         int64_t vocab);
+int gs_embedding_layer_pass(const int64_t* ids, const void* G, int dtype, int64_t N,
+                            int64_t n_val, int64_t val_start, int64_t T, int64_t d,
+                            int64_t vocab, float* out_dot, float scale, void* grad,
+                            int grad_dtype, int accumulate, void* workspace,
+                            size_t workspace_bytes, void* stream);
 
 /* ---- LayerNorm dot products and train gradients -------------------------------------
  * Replaces _compute_layernorm_dot_product (:242-300) and _compute_layernorm_train_grad

@@ -187,6 +187,45 @@ def test_embedding_train_grad_heavy_ids(gpu, shape, pad_frac):
     assert_close(got, prev.double() + want, 1e-2, "heavy ids, accumulate")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape,runs", [
+    # N, n_val, T, d, vocab; lengths of the first val tokens' runs
+    ((3, 1, 300, 8, 40), (64, 65, 66, 1, 2)),     # either side of the shared-run line
+    ((5, 2, 500, 1100, 3000), (400, 399, 7)),     # features past one pass, two long runs
+    ((4, 2, 300, 13, 524287), (65, 2)),           # most ids, rows of 13 features
+    ((4, 1, 8192, 24, 300), (7000,)),             # most val tokens
+])
+def test_embedding_layer_pass(gpu, dtype, shape, runs):
+    """Dots and train gradient in shared launches: the bits of the two calls, the dots within fp32
+    rounding of a sum in a fixed order of the float64 ones; absent beyond 8192 val tokens."""
+    N, n_val, T, d, vocab = shape
+    ids = torch.randint(-1, vocab + 1, (N, T), generator=gen(290 + T))
+    flat = ids[N - n_val:].view(-1)
+    at = 0
+    for k, n in enumerate(runs):
+        flat[at:at + n] = vocab - 1 - k
+        at += n
+    flat[:] = flat[torch.randperm(flat.numel(), generator=gen(291 + T))]
+    ids[0, :40] = vocab - 1 - torch.arange(40) % len(runs)
+    G = randn((N, T, d), 292 + T, 1e-2, dtype)
+    idd, Gd, ops = ids.to(gpu), G.to(gpu), _native.ops()
+    for acc in (False, True):
+        old = randn((vocab, d), 293, 1e-2, dtype).to(gpu)
+        new = old.clone()
+        dot = ops.embedding_layer_pass(idd, Gd, n_val, 1.5, new, accumulate=acc)
+        ops.embedding_train_grad(idd, Gd, n_val, 1.5, old, accumulate=acc)
+        assert torch.equal(new, old)
+        assert torch.equal(dot, ops.embedding_dot(idd, Gd, n_val, vocab))
+    ok = (ids >= 0) & (ids < vocab)
+    want = R.embedding_dot_exact(ids.clamp(0, vocab - 1), G * ok[..., None], n_val)
+    # chains of at most 128 + 16 rows in a run's sum, 4 d / 32 products a lane and 256 parts: fewer
+    # than 600 fp32 roundings of 2^-24, relative to the sum of magnitudes
+    mag = R.embedding_dot_exact(ids.clamp(0, vocab - 1), (G * ok[..., None]).abs(), n_val)
+    assert ((dot.cpu().double() - want).abs() <= 4e-5 * mag + 1e-30).all()
+    if n_val * T == 8192:
+        assert ops.embedding_layer_pass(idd, Gd, n_val + 1, 1.5, new) is None
+
+
 @pytest.mark.parametrize("shape,pad_frac", [
     # N, n_val, T, d, vocab
     ((3, 1, 500, 8, 256), 0.0),          # one id a bucket
