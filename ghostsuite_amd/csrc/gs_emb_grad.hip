@@ -28,13 +28,14 @@
 // The dots, dot_i = sum_t <g_it, V[x_it]> with V[v] the sum of the val rows of id v, for up to 8192
 // val tokens: the val tokens' list (with a table of runs per id) in launch 1, the sums of runs of
 // two tokens or more (eg_runs) in the launch of the windows, then
-//   eg_dot_kernel     -- each train token's row against its run's sum or its id's only val row.
+//   eg_dot_kernel     -- each train token's row against its run's sum or its id's only val row
+//                        (with a gradient: in launch 4, eg_combine_dot_kernel).
 //   eg_dot_sum_kernel -- the parts of a train row added.
 // Either alone, or both in shared launches.  Measured on MI355X (GPT-2 wte, 16 + 4 rows of 1024
-// tokens, d = 768, bf16; 80 us before): lists 14.5 us, runs and windows 22.7 (102 MB written and
-// read: the rate of a copy), combine 6.4, dots 6.6 + 3.3; a padded batch of 65536 train tokens with
-// one id on 59k of them and 4096 val tokens likewise, d = 256: lists 57, windows 38, combine 34,
-// dots 14 + 4.6 (1870 before).
+// tokens, d = 768, bf16; 80 us before): lists 14.9 us, runs and windows 23.0 (102 MB written and
+// read: the rate of a copy), combine and dots 7.5 + 3.9; a padded batch of 65536 train tokens with
+// one id on 59k of them and 4096 val tokens likewise, d = 256: lists 57, windows 38, combine
+// and dots 48 + 4.7 (1870 before).
 
 #include <algorithm>
 
@@ -976,11 +977,10 @@ struct EgCombineShared {
 };
 
 template <class GE>
-__global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
-    EgList list, int64_t d, float scale, int accumulate, GE* __restrict__ grad) {
+__device__ __forceinline__ void eg_combine(const EgList& list, int64_t d, float scale,
+                                           int accumulate, int64_t block, EgCombineShared& sh,
+                                           GE* __restrict__ grad) {
   constexpr int NW = EG_COMBINE_WAVES, CB = EG_COMBINE_BLOCK;
-  __shared__ EgCombineShared sh;
-  const int64_t block = blockIdx.x;
   static_assert(NW * 64 == CB, "one feature of a block per thread");
   const unsigned long long* __restrict__ sk = list.sk;
   const float* __restrict__ part = list.part;
@@ -1171,35 +1171,42 @@ __global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
 // run of two tokens or more is read from S, a single one straight from that val token's row of G.
 // (Letting a row's last workgroup add the parts in place of a launch: 15 us against 7 + 3.5, and 56
 // against 15 + 4.5 for 64 chunks a row; the release to the other XCDs costs every workgroup.)
-constexpr int EG_TOK = 32;   // tokens per workgroup
+constexpr int EG_TOK = 32;   // tokens per unit of EG_THREADS threads
+struct EgDotShared {
+  float red[EG_THREADS / 64];
+  int64_t rows[EG_TOK], src[EG_TOK];   // src: row of S, or -1 - row of G
+  int hits;
+};
+// Thread `tid` of unit i * chunks + c; units past n_t * chunks only keep the barriers.
 template <class E>
-__global__ void __launch_bounds__(EG_THREADS) eg_dot_kernel(
-    const int64_t* __restrict__ ids, const E* __restrict__ G, EgRows train, int64_t T, EgList val,
-    int64_t d, int64_t vocab, const float* __restrict__ S, int vec, int64_t chunks,
-    float* __restrict__ part) {
+__device__ __forceinline__ void eg_dot(const int64_t* __restrict__ ids, const E* __restrict__ G,
+                                       const EgRows& train, int64_t n_t, int64_t T,
+                                       const EgList& val, int64_t d, int64_t vocab,
+                                       const float* __restrict__ S, int vec, int64_t chunks,
+                                       int64_t unit, int tid, EgDotShared& sh,
+                                       float* __restrict__ part) {
   constexpr int VE = EgVec<E>::VE, P = 4;
-  __shared__ float red[EG_THREADS / 64];
-  __shared__ int64_t rows[EG_TOK], src[EG_TOK];   // src: row of S, or -1 - row of G
-  __shared__ int hits;
-  const int64_t i = blockIdx.y, c = blockIdx.x;
-  if (threadIdx.x < 64) {
-    const int64_t t = c * EG_TOK + threadIdx.x;
-    const bool in = threadIdx.x < EG_TOK && t < T;
+  auto& rows = sh.rows;
+  auto& src = sh.src;
+  const int64_t i = unit / chunks, c = unit - i * chunks;
+  if (tid < 64) {
+    const int64_t t = c * EG_TOK + tid;
+    const bool in = tid < EG_TOK && t < T && i < n_t;
     const int64_t row = in ? train(i * T + t) : 0;
     const int64_t id = in ? ids[row] : -1;
     const uint2 e = id >= 0 && id < vocab ? val.table[val.order.of(id)] : make_uint2(0u, 0u);
     const unsigned long long found = __ballot(e.y != 0);
     if (e.y != 0) {
-      const int h = __popcll(found & ((1ull << threadIdx.x) - 1ull));
+      const int h = __popcll(found & ((1ull << tid) - 1ull));
       rows[h] = row;
       src[h] = e.y > 1 ? static_cast<int64_t>(e.x >> 1) : -1 - val.rows(key_tok(val.sk[e.x]));
     }
-    if (threadIdx.x == 0) hits = __popcll(found);
+    if (tid == 0) sh.hits = __popcll(found);
   }
   __syncthreads();
-  const int hl = threadIdx.x & 31, n = hits;
+  const int hl = tid & 31, n = sh.hits;
   float s = 0.f;
-  for (int h = threadIdx.x >> 5; h < n; h += EG_THREADS / 32) {
+  for (int h = tid >> 5; h < n; h += EG_THREADS / 32) {
     const E* g = G + rows[h] * d;
     const int64_t sr = src[h];
     for (int64_t fb = static_cast<int64_t>(hl) * VE; fb < d; fb += P * 32 * VE) {
@@ -1243,8 +1250,64 @@ __global__ void __launch_bounds__(EG_THREADS) eg_dot_kernel(
       }
     }
   }
-  const float tot = block_sum(s, red);
-  if (threadIdx.x == 0) part[i * chunks + c] = tot;
+  s = wave_sum(s);
+  if ((tid & 63) == 0) sh.red[tid >> 6] = s;
+  __syncthreads();
+  if (tid == 0 && i < n_t) {
+    float tot = 0.f;
+    for (int w = 0; w < EG_THREADS / 64; ++w) tot += sh.red[w];
+    part[unit] = tot;
+  }
+}
+
+// What the train tokens' dots read.
+template <class E>
+struct EgDots {
+  const int64_t* ids;
+  const E* G;
+  EgRows train;
+  int64_t n_t, T, vocab, chunks;
+  const float* S;
+  int vec;
+  float* part;
+};
+
+template <class E>
+__global__ void __launch_bounds__(EG_THREADS) eg_dot_kernel(EgDots<E> q, EgList val, int64_t d) {
+  __shared__ EgDotShared sh;
+  eg_dot<E>(q.ids, q.G, q.train, q.n_t, q.T, val, d, q.vocab, q.S, q.vec, q.chunks, blockIdx.x,
+            threadIdx.x, sh, q.part);
+}
+
+template <class GE>
+__global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_kernel(
+    EgList list, int64_t d, float scale, int accumulate, GE* __restrict__ grad) {
+  __shared__ EgCombineShared sh;
+  eg_combine<GE>(list, d, scale, accumulate, blockIdx.x, sh, grad);
+}
+
+// Both need the window launch alone, and each leaves most of the chip waiting for its chains of
+// loads: the first dot_blocks workgroups take four units of dots each, the others combine.
+// GPT-2 wte, 16 + 4 rows of 1024 tokens, d = 768: 7.5 us against 6.4 + 6.6 apart, the hook 56.5 ->
+// 50.3; 8 + 4 rows of 2048, d = 2048: 128 -> 119; 2 + 2 rows of 64: 34.5 -> 31.5; 90% of 65536
+// tokens one id: 143.9 -> 143.5.
+constexpr int EG_DOT_UNITS = EG_COMBINE_WAVES * 64 / EG_THREADS;
+template <class E, class GE>
+__global__ void __launch_bounds__(EG_COMBINE_WAVES * 64) eg_combine_dot_kernel(
+    EgDots<E> q, EgList val, unsigned dot_blocks, EgList list, int64_t d, float scale,
+    int accumulate, GE* __restrict__ grad) {
+  __shared__ union {
+    EgCombineShared combine;
+    EgDotShared dot[EG_DOT_UNITS];
+  } sh;
+  if (blockIdx.x < dot_blocks) {
+    const int u = threadIdx.x / EG_THREADS;
+    eg_dot<E>(q.ids, q.G, q.train, q.n_t, q.T, val, d, q.vocab, q.S, q.vec, q.chunks,
+              static_cast<int64_t>(blockIdx.x) * EG_DOT_UNITS + u, threadIdx.x % EG_THREADS,
+              sh.dot[u], q.part);
+    return;
+  }
+  eg_combine<GE>(list, d, scale, accumulate, blockIdx.x - dot_blocks, sh.combine, grad);
 }
 
 __global__ void __launch_bounds__(EG_THREADS) eg_dot_sum_kernel(const float* __restrict__ part,
@@ -1374,20 +1437,26 @@ int run_call(const EgCall& c, const int64_t* ids, const void* Gv, float* out_dot
   const unsigned tw = c.grad ? blocks(c.train.windows + zero_waves, EG_THREADS / 64) : 0;
   hipLaunchKernelGGL((eg_window_kernel<E, GE>), dim3(vw + tw), dim3(EG_THREADS), 0, s, G, c.val,
                      c.train, vw, c.d, c.vocab, scale, accumulate, vec, c.S, grad);
-  if (c.grad)
-    hipLaunchKernelGGL((eg_combine_kernel<GE>), dim3(blocks(c.train.windows, EG_COMBINE_WAVES)),
-                       dim3(EG_COMBINE_WAVES * 64), 0, s, c.train, c.d, scale, accumulate, grad);
-  rc = check_launch("eg_window_kernel / eg_combine_kernel");
-  if (rc || !c.dot) return rc;
   const int64_t n_t = c.N - c.n_val, chunks = eg_cdiv(c.T, EG_TOK);
-  hipLaunchKernelGGL(eg_dot_kernel<E>,
-                     dim3(static_cast<unsigned>(chunks), static_cast<unsigned>(n_t)),
-                     dim3(EG_THREADS), 0, s, ids, G,
-                     eg_rows(train_rows(c.N, c.n_val, c.val_start, c.T)), c.T, c.val, c.d, c.vocab,
-                     c.S, vec, chunks, c.parts);
+  const unsigned cb = c.grad ? blocks(c.train.windows, EG_COMBINE_WAVES) : 0;
+  if (!c.dot) {
+    hipLaunchKernelGGL((eg_combine_kernel<GE>), dim3(cb), dim3(EG_COMBINE_WAVES * 64), 0, s,
+                       c.train, c.d, scale, accumulate, grad);
+    return check_launch("eg_window_kernel / eg_combine_kernel");
+  }
+  const EgDots<E> q{ids, G, eg_rows(train_rows(c.N, c.n_val, c.val_start, c.T)), n_t, c.T, c.vocab,
+                    chunks, c.S, vec, c.parts};
+  if (c.grad) {
+    const unsigned db = blocks(n_t * chunks, EG_DOT_UNITS);
+    hipLaunchKernelGGL((eg_combine_dot_kernel<E, GE>), dim3(db + cb), dim3(EG_COMBINE_WAVES * 64),
+                       0, s, q, c.val, db, c.train, c.d, scale, accumulate, grad);
+  } else {
+    hipLaunchKernelGGL(eg_dot_kernel<E>, dim3(static_cast<unsigned>(n_t * chunks)),
+                       dim3(EG_THREADS), 0, s, q, c.val, c.d);
+  }
   hipLaunchKernelGGL(eg_dot_sum_kernel, dim3(static_cast<unsigned>(n_t)), dim3(EG_THREADS), 0, s,
                      c.parts, chunks, out_dot);
-  return check_launch("eg_dot_kernel");
+  return check_launch("eg_window_kernel / eg_dot_kernel");
 }
 
 // grad_dtype: any when there is no gradient.

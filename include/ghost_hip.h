@@ -312,8 +312,8 @@ int gs_embedding_train_grad(const int64_t* ids, const void* G, int dtype, int64_
                             int accumulate, void* workspace, size_t workspace_bytes,
                             void* stream);
 
-/* Both of the above in shared launches (one token list kernel, one window pass, one pass over
- * runs that cross windows, then the dots), with the same results.  For the sizes whose dots go
+/* Both of the above in shared launches (one token list kernel, one window pass, then the
+ * runs that cross windows beside the dots, and the dots' parts added), with the same results.  For the sizes whose dots go
  * through the val tokens' list; the workspace query answers 0 for others, which take the two
  * calls (the call itself: GS_ERR_UNSUPPORTED). */
 size_t gs_embedding_layer_pass_workspace(int64_t N, int64_t n_val, int64_t T, int64_t d,

@@ -194,6 +194,7 @@ def test_embedding_train_grad_heavy_ids(gpu, shape, pad_frac):
     ((5, 2, 500, 1100, 3000), (400, 399, 7)),     # features past one pass, two long runs
     ((4, 2, 300, 13, 524287), (65, 2)),           # most ids, rows of 13 features
     ((4, 1, 8192, 24, 300), (7000,)),             # most val tokens
+    ((4, 1, 70, 8, 50), (64, 2)),                 # dot units past a whole workgroup of four
 ])
 def test_embedding_layer_pass(gpu, dtype, shape, runs):
     """Dots and train gradient in shared launches: the bits of the two calls, the dots within fp32
