@@ -2167,18 +2167,27 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tn_gemm_kernel(TnParams p
 // sum_t g_it^T V a_it = <V, G_i^T A_i>, and the train gradient is the sum over i of the same
 // G_i^T A_i, so a work item (split, mt, nt) accumulates G^T A over the k-rows of its split
 // (L = G's train rows, R = A's, logical k-rows with the val block skipped): at every sample
-// boundary (T k-rows, a multiple of the stage height) and at a split's end inside a sample,
-// each wave forms <acc, V tile> against the V tile it holds in registers and stores the
-// growth since the previous boundary as its share of that sample; acc runs on and ends as
-// the split's train-gradient partial.  RAG: T is not a multiple of the stage height, and every
-// sample's rows are padded with zeros to whole stages (nothing is read for them).  With CS the column sums of the L tile (G: the bias
-// terms) are taken per stage as well, after the stage's MFMAs, spread over the workgroups.
+// boundary and at a split's end inside a sample, each wave forms <acc, V tile> and stores it as
+// its share of that sample.
+//  - 64 x 64 wave tiles (HELD): acc is then added to the running train gradient, a second set of
+//    accumulators, and cleared, so that a dot holds nothing of the other samples: one sample's
+//    Inf or NaN, or a gradient of many times the others' size, stays in its own dot.  Each
+//    sample's rows are padded with zeros to whole stages (nothing is read for them): any T.
+//    (The adds and the registers cost 1%: GPT-2 fc 139.7 -> 141 us, 13 samples of T = 777,
+//    768 x 2304 80.5 -> 81.5.)
+//  - 128 x 64 wave tiles have no registers for a second set: acc runs on, and the share is the
+//    growth of <acc, V tile> since the previous boundary, which rounds at the running sum's size.
+//    T a multiple of the stage height only.  (Their place taken by 64 x 64 wave tiles: Pythia-1B
+//    fc 595 -> 702 us, 256 x 128 tiles of eight such waves 712, of four 128 x 64 waves with the
+//    registers of a whole SIMD 864; the sums kept in memory instead 930.)
+// With CS the column sums of the L tile (G: the bias terms) are taken per stage as well, after
+// the stage's MFMAs, spread over the workgroups.
 struct TgParams {
   TnParams tn;          // k-rows per split (kper) a multiple of the stage height, >= T;
                         // out: fp32 partials, or with one split the gradient (part_out 0)
   const uint4* V;       // V (bf16) in accumulator order of the same tiles (acc_store)
-  int64_t T, n_t;       // k-rows per sample (a multiple of the stage height), train samples
-  int64_t T_rows;       // with RAG: the rows a sample has (T counts them padded to whole stages)
+  int64_t T, n_t;       // k-rows per sample, padded to whole stages; train samples
+  int64_t T_rows;       // the rows a sample has
   float* pdot;          // [m_tiles * n_tiles][NW][2 slots][n_t] wave shares of the weight dots
   float* csum;          // with CS: [n_t][2 T / stage height][M] column sums of L (CS 1; of R,
                         // [..][N], with CS 2), two rows (halves of the stage's k-rows) per stage
@@ -2189,7 +2198,7 @@ struct TgParams {
                         //   dotted with vb
 };
 
-template <class C, class D, int CS, bool RAG = false>
+template <class C, class D, int CS>
 __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) {
   const TnParams& p = q.tn;
   __shared__ __attribute__((aligned(16))) unsigned char lds[D::STAGES * D::STAGE_BYTES];
@@ -2200,19 +2209,22 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: scalar
   const int wm = wid / C::WN, wn = wid % C::WN;
-  f32x16_t acc[C::MI][C::NI];
+  // HELD: 64 x 64 wave tiles, with registers for V and a second set of accumulators.
+  constexpr bool HELD = C::MI * C::NI <= 4;
+  f32x16_t acc[C::MI][C::NI];                                // of the current sample (HELD)
+  f32x16_t tot[HELD ? C::MI : 1][HELD ? C::NI : 1];          // of the ended ones
   zero_acc<TrBF16, C>(acc);
-  float s_prev = 0.f;  // <acc, V tile> of this wave at the previous boundary
+  if constexpr (HELD) zero_acc<TrBF16, C>(tot);
+  float s_prev = 0.f;  // not HELD: <acc, V tile> of this wave at the previous boundary
   // This lane's V entries: 16 bytes per half block.  With 64 x 64 wave tiles they are loaded
   // once and held for the work item (32 registers); wider wave tiles have no registers to spare
   // beside their accumulators, and load them again (from L2) at each boundary, a few per sample.
   // (In accumulator order: from a row-major V^T, 8 bytes of 32 rows per load, the eight boundaries
   // of a 2048 x 8192 gradient cost 52 of the hook's 663 us.)
-  constexpr bool VHELD = C::MI * C::NI <= 4;
   const int64_t tile = mt * p.n_tiles + nt;
   const uint4* vsrc = q.V + acc_base<C>(tile, wid);
-  uint4 vr[VHELD ? C::MI * C::NI * 2 : 1];
-  if constexpr (VHELD) {
+  uint4 vr[HELD ? C::MI * C::NI * 2 : 1];
+  if constexpr (HELD) {
 #pragma unroll
     for (int k = 0; k < C::MI * C::NI * 2; ++k) vr[k] = vsrc[k * 64];
   }
@@ -2262,17 +2274,25 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int k = (i * C::NI + j) * 2 + h;
-          acc_dot(acc[i][j], h, VHELD ? vr[VHELD ? k : 0] : vsrc[k * 64], d0, d1);
+          acc_dot(acc[i][j], h, HELD ? vr[HELD ? k : 0] : vsrc[k * 64], d0, d1);
         }
     const float d = wave_sum_dpp(d0 + d1);
     const int slot = started ? 0 : 1;
     const bool whole = started && ended;
     float* pd = q.pdot + (tile * (C::WM * C::WN) + wid) * 2 * q.n_t + sample;
     if (lane == 0) {
-      pd[slot * q.n_t] = d - s_prev;
+      pd[slot * q.n_t] = HELD ? d : d - s_prev;
       if (whole) pd[q.n_t] = 0.f;
     }
-    s_prev = d;
+    if constexpr (HELD) {
+#pragma unroll
+      for (int i = 0; i < C::MI; ++i)
+#pragma unroll
+        for (int j = 0; j < C::NI; ++j) tot[i][j] += acc[i][j];
+      zero_acc<TrBF16, C>(acc);
+    } else {
+      s_prev = d;
+    }
   };
   bf16x8_t keep[D::KSTEPS][F];  // with CS: the stage's L (R) fragments, kept by tn_compute
   auto hook = [&](int, const unsigned char*) {
@@ -2311,13 +2331,13 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
     auto cmp = [&](const unsigned char* stage, f32x16_t (&a)[C::MI][C::NI]) {
       tn_compute<C, D, CS>(stage, a, keep);
     };
-    if constexpr (RAG)
+    if constexpr (HELD)
       mainloop_tn_samples<C, D>(p, mt, nt, k_begin, k_end, q.T, static_cast<int>(q.T_rows), lds,
                                 acc, hook, cmp);
     else
       mainloop_tn<C, D>(p, mt, nt, k_begin, k_end, lds, acc, hook, cmp);
   } else {
-    if constexpr (RAG)
+    if constexpr (HELD)
       mainloop_tn_samples<C, D>(p, mt, nt, k_begin, k_end, q.T, static_cast<int>(q.T_rows), lds,
                                 acc, hook, TnPlainCompute<C, D>{});
     else
@@ -2328,16 +2348,22 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
   e.m_rows = p.M;
   e.n_cols = p.N;
   e.c_ld = p.N;
-  if (p.part_out) {
-    e.C = static_cast<float*>(p.out) + split * p.M * p.N;
-    store_epilogue<TrF32, C>(e, acc, mt, nt);
-  } else if (p.out != nullptr) {  // one split: the gradient itself
-    e.C = p.out;
-    if (p.out_f32)
-      store_epilogue<TrF32, C>(e, acc, mt, nt, p.alpha);
-    else
-      store_epilogue<TrBF16, C>(e, acc, mt, nt, p.alpha);
-  }
+  auto store = [&](f32x16_t (&sum)[C::MI][C::NI]) __attribute__((always_inline)) {
+    if (p.part_out) {
+      e.C = static_cast<float*>(p.out) + split * p.M * p.N;
+      store_epilogue<TrF32, C>(e, sum, mt, nt);
+    } else if (p.out != nullptr) {  // one split: the gradient itself
+      e.C = p.out;
+      if (p.out_f32)
+        store_epilogue<TrF32, C>(e, sum, mt, nt, p.alpha);
+      else
+        store_epilogue<TrBF16, C>(e, sum, mt, nt, p.alpha);
+    }
+  };
+  if constexpr (HELD)
+    store(tot);
+  else
+    store(acc);
 }
 
 // Per-pair weight dots <V_j, G_i^T A_i> (V_j = G_j^T A_j of val sample j) from one sample's
@@ -3830,9 +3856,11 @@ TgPlan plan_tg(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
   // CU), unsplit, when those tiles alone cover 7/8 of the CUs or more (the Pythia-1B MLP and
   // vocabulary head: 8-10% faster); in 128 x 128 tiles (two workgroups per CU) with split
   // k-rows otherwise: filling the CUs by splitting wide tiles costs their fp32 partials (7
-  // splits of a 768 x 3072 gradient write 66 MB, and measured slower).
+  // splits of a 768 x 3072 gradient write 66 MB, and measured slower).  Not for ragged T, whose
+  // dots would become differences of running sums there (tgdot_kernel): 8 + 2 samples of
+  // T = 1999, 2048 x 8192 take 675 us, 590 in wide tiles, 1110 by the separate passes.
   const int64_t wt = ceil_div(d_out, TnCW::BM) * ceil_div(d_in, TnCW::BN);
-  t.wide = wt >= 224 ? 1 : 0;
+  t.wide = wt >= 224 && T % TnDW::KB == 0 ? 1 : 0;
   if (t.wide) {
     t.m_tiles = ceil_div(d_out, TnCW::BM);
     t.n_tiles = ceil_div(d_in, TnCW::BN);
@@ -4123,25 +4151,21 @@ int dot_train_grad(const char* name, bool bias_a, bool any_T, const void* A, con
   if (items > INT32_MAX) return fail(GS_ERR_UNSUPPORTED, "GEMM grid too large");
   const dim3 tg_grid(static_cast<unsigned>(items));
   const int cs = q.csum == nullptr ? 0 : (t.bias_a ? 2 : 1);
-  auto go = [&](auto wide, auto csk, auto ragged) {
+  auto go = [&](auto wide, auto csk) {
     constexpr bool W = decltype(wide)::value;
     using C = std::conditional_t<W, TnCW, TnC>;
     using D = std::conditional_t<W, TnDW, TnD>;
-    hipLaunchKernelGGL((tgdot_kernel<C, D, decltype(csk)::value, decltype(ragged)::value>),
-                       tg_grid, dim3(C::NT), 0, s, q);
+    hipLaunchKernelGGL((tgdot_kernel<C, D, decltype(csk)::value>), tg_grid, dim3(C::NT), 0, s, q);
   };
-  auto go_cs = [&](auto wide, auto ragged) {
+  auto go_cs = [&](auto wide) {
     if (cs == 0)
-      go(wide, std::integral_constant<int, 0>{}, ragged);
+      go(wide, std::integral_constant<int, 0>{});
     else if (cs == 1)
-      go(wide, std::integral_constant<int, 1>{}, ragged);
+      go(wide, std::integral_constant<int, 1>{});
     else
-      go(wide, std::integral_constant<int, 2>{}, ragged);
+      go(wide, std::integral_constant<int, 2>{});
   };
-  if (t.wide)
-    rag ? go_cs(std::true_type{}, std::true_type{}) : go_cs(std::true_type{}, std::false_type{});
-  else
-    rag ? go_cs(std::false_type{}, std::true_type{}) : go_cs(std::false_type{}, std::false_type{});
+  t.wide ? go_cs(std::true_type{}) : go_cs(std::false_type{});
   rc = check_launch("tgdot_kernel");
   if (rc) return rc;
   const int64_t shares = t.m_tiles * t.n_tiles * (t.wm * t.wn) * 2;

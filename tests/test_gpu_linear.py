@@ -520,13 +520,15 @@ def test_linear_dot_train_grad_declines(gpu):
     (4, 1, 70, 2000, 7176, "pairwise", "mid", True, False),
     (4, 1, 70, 2000, 7176, "presum", "first", True, True),
     (6, 2, 128, 136, 264, "presum", "last", True, True),   # whole stages
+    (20, 4, 64, 768, 776, "pairwise", "mid", True, False),
 ])
 def test_linear_layer_pass_any_length(gpu, case):
     """gs_linear_layer_pass at any T, both weight layouts, fp32 and bf16 dots, against float64:
     the dots through the val-term form at the kernel's rounding points (beyond them the sums
     are fp32), the train gradients as closed forms; a bf16 dot is the fp32 one rounded once.
-    A NaN in one train sample stays in its own dot, though its rows follow another sample's
-    padded end."""
+    A train sample's NaN, Inf or gradient of 2^20 times the others' size leaves the bits of all
+    other dots as they are, before it and after it in its split (and a power of two scales the
+    sample's own dot exactly)."""
     N, n_val, T, d_in, d_out, sem, pos, bias, conv1d = case
     vs = {"last": N - n_val, "first": 0, "mid": 1}[pos]
     n_t = N - n_val
@@ -563,13 +565,19 @@ def test_linear_layer_pass_any_length(gpu, case):
     assert torch.equal(low[0], dot.bfloat16()) and torch.equal(low[1], grad)
     if bias:
         assert torch.equal(low[2], bdot.bfloat16())
-    # one train sample's NaN stays in its own dot (its first row follows another's last row)
-    if n_t > 1 and T > 1:
-        bad = A.clone()
-        rows = [i for i in range(N) if not vs <= i < vs + n_val]
-        bad[rows[1], 0] = float("nan")
-        dn = run(bad, torch.float32)[0].cpu()
-        assert torch.isnan(dn[1]) and torch.equal(dn[0], dot.cpu()[0])
+    rows = [i for i in range(N) if not vs <= i < vs + n_val]
+    for at in sorted({0, min(1, n_t - 1)}):
+        others = [i for i in range(n_t) if i != at]
+        for value in (float("nan"), float("inf"), None):
+            bad = A.clone()
+            if value is None:
+                bad[rows[at]] *= 2.0 ** 20
+            else:
+                bad[rows[at], 0] = value
+            dn = run(bad, torch.float32)[0].cpu()
+            assert torch.equal(dn[others], dot.cpu()[others]), (at, value)
+            assert torch.equal(dn[at], dot.cpu()[at] * 2.0 ** 20) if value is None else \
+                not torch.isfinite(dn[at])
 
 
 @pytest.mark.parametrize("case", [
