@@ -3057,29 +3057,15 @@ LinearPlan plan_linear(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_
   const double valgrad = vgemm + rowdot * (want_pair ? n_val : 1);
   pl.algo = algo;
   if (algo == GS_ALGO_AUTO) pl.algo = ghost <= valgrad ? GS_ALGO_GHOST : GS_ALGO_VALGRAD;
-  if (products) {
-    // Estimated times in us.  Sample products: whole 64-row stages of 128 x 128 tiles at
-    // 1 PF/s, the inner products at 0.13 ps per V_j entry and train sample, 12 us of launches
-    // and pipeline fill.  Ghost: rounds of 256 tiles of 256 x 256, each as long as its
-    // (d_in + d_out) / 64 stages however few tiles a round has.  Measured (products / ghost):
-    // 24 + 8 samples of 768 x 3072 at T = 64: 81 / 91, 256: 100 / 101, 512: 135 / 319, 1000:
-    // 211 / 1211; 2048 x 2048 at T = 64: 118 / 93, 512: 221 / 337; 8 + 2 of 512 x 512 at T = 16:
-    // 20 / 32.
-    const double area = static_cast<double>(pair_tiles(d_in, d_out)) * TnC::BM * TnC::BN;
-    const double prod = 12.0 + 2e-9 * N * ceil_div(T, TnD::KB) * TnD::KB * area +
-                        1.3e-7 * n_val * n_t * area;
-    const double tiles = static_cast<double>(nv_eff * ceil_div(T, GBM)) *
-                         ceil_div(n_t * T, static_cast<int64_t>(StashCfg::BN));
-    const double gtime = 6.0 + std::ceil(tiles / 256.0) * 0.024 * (d_in + d_out);
-    pl.pairs = algo == GS_ALGO_VALGRAD || prod <= gtime ? 1 : 0;
-    if (pl.pairs) {
-      pl.algo = GS_ALGO_VALGRAD;
-      pl.groups = n_val;
-      pl.p_rows = n_val * pair_tiles(d_in, d_out);
-      pl.p_ld = n_t;
-      pl.cols = 1;
-      return pl;
-    }
+  // The products are a form of the val-gradient algorithm: they do not take shapes whose flops
+  // choose the ghost kernel, whose dots round elsewhere (a Gram entry, not an entry of V_j).
+  if (products && pl.algo == GS_ALGO_VALGRAD) {
+    pl.pairs = 1;
+    pl.groups = n_val;
+    pl.p_rows = n_val * pair_tiles(d_in, d_out);
+    pl.p_ld = n_t;
+    pl.cols = 1;
+    return pl;
   }
   int64_t bn;
   if (pl.algo == GS_ALGO_GHOST) {
@@ -3113,16 +3099,13 @@ LinearPlan plan_any(int dtype, int64_t N, int64_t n_val, int64_t T, int64_t d_in
   return plan_linear<TrBF16>(N, n_val, T, d_in, d_out, semantics, algo, want_pair, products);
 }
 // The plan of a call on known operands, with at most `cap` bytes of scratch for the V_j's form.
-// AUTO with the reference's rounding keeps to the forms whose ghost side honours it.
 size_t linear_bytes(int dtype, const LinearPlan& pl, int64_t n_val, int64_t T, int64_t d_in,
                     int64_t d_out, int semantics, const void* A, const void* G);
 LinearPlan plan_call(int dtype, int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
-                     int semantics, int algo, int want_pair, int rounding, const void* A,
-                     const void* G, size_t cap = SIZE_MAX) {
-  const bool products = aligned16(A) && aligned16(G) &&
-                        !(algo == GS_ALGO_AUTO && rounding == GS_ROUND_REF_BF16);
+                     int semantics, int algo, int want_pair, const void* A, const void* G,
+                     size_t cap = SIZE_MAX) {
   const LinearPlan pl = plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair,
-                                 products);
+                                 aligned16(A) && aligned16(G));
   if (pl.pairs && linear_bytes(dtype, pl, n_val, T, d_in, d_out, semantics, A, G) > cap)
     return plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair, false);
   return pl;
@@ -3537,8 +3520,8 @@ extern "C" int gs_linear_dot(const void* A, const void* G, int dtype, int64_t N,
   int rc = check_linear_args("gs_linear_dot", A, G, dtype, N, n_val, val_start, T, d_in, d_out,
                              semantics, algo, rounding, out_dot, want_pair);
   if (rc) return rc;
-  const LinearPlan pl = plan_call(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair,
-                                  rounding, A, G);
+  const LinearPlan pl = plan_call(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair, A,
+                                  G);
   if (workspace == nullptr ||
       workspace_bytes < linear_bytes(dtype, pl, n_val, T, d_in, d_out, semantics, A, G))
     return fail(GS_ERR_WORKSPACE, "gs_linear_dot: workspace too small");
@@ -3555,8 +3538,8 @@ extern "C" size_t gs_linear_dot_noalloc_bytes(const void* A, const void* G, int 
                                               int64_t d_out, int semantics, int algo,
                                               int want_pair) {
   if (!linear_args_ok(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair)) return 0;
-  const LinearPlan pl = plan_call(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair,
-                                  GS_ROUND_FP32, A, G, GS_LINEAR_NOALLOC_SCRATCH_BYTES);
+  const LinearPlan pl = plan_call(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair, A,
+                                  G, GS_LINEAR_NOALLOC_SCRATCH_BYTES);
   return linear_bytes(dtype, pl, n_val, T, d_in, d_out, semantics, A, G);
 }
 
@@ -3568,8 +3551,8 @@ extern "C" int gs_linear_dot_noalloc(const void* A, const void* G, int dtype, in
   int rc = check_linear_args("gs_linear_dot_noalloc", A, G, dtype, N, n_val, val_start, T,
                              d_in, d_out, semantics, algo, rounding, out_dot, want_pair);
   if (rc) return rc;
-  const LinearPlan pl = plan_call(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair,
-                                  rounding, A, G, GS_LINEAR_NOALLOC_SCRATCH_BYTES);
+  const LinearPlan pl = plan_call(dtype, N, n_val, T, d_in, d_out, semantics, algo, want_pair, A,
+                                  G, GS_LINEAR_NOALLOC_SCRATCH_BYTES);
   const size_t need = linear_bytes(dtype, pl, n_val, T, d_in, d_out, semantics, A, G);
   if (need > GS_LINEAR_NOALLOC_SCRATCH_BYTES)
     return fail(GS_ERR_UNSUPPORTED,
@@ -3881,27 +3864,19 @@ TgPlan plan_tg(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
   return t;
 }
 // Whether the fused pass (V GEMM, the train rows' GEMM with each sample padded to whole stages)
-// beats the dots by `algo` and the train gradient apart.  Estimated times in us.  Measured, one
-// layer's hook with a bias, fused / apart: 16 + 4 samples of 768 x 3072 at T = 1: 57 / 106, 32:
+// beats the V GEMM, the row-dots and the train gradient apart: the padded rows cost less than a
+// second GEMM over the real ones and its launches.  Estimated times in us.  Measured, one layer's
+// hook with a bias, fused / apart: 16 + 4 samples of 768 x 3072 at T = 1: 57 / 106, 32:
 // 56 / 127, 129: 57 / 149, 500: 94 / 203; 200 + 16 samples of 1024 x 1024 at T = 1: 64 / 97 (64
-// padded rows to every real one); 13 + 3 of 768 x 2304 at T = 777: 86 / 162.
-bool layer_pass_pays(int algo, int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
-                     int semantics, int with_bias) {
-  const int64_t n_t = N - n_val, nv = semantics == GS_SEM_PRESUM ? 1 : n_val;
+// padded rows to every real one); 13 + 3 of 768 x 2304 at T = 777: 81 / 152.
+bool layer_pass_pays(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d_out,
+                     int with_bias) {
+  const int64_t n_t = N - n_val;
   const double area = static_cast<double>(pair_tiles(d_in, d_out)) * TnC::BM * TnC::BN;
   const int64_t Tp = ceil_div(T, static_cast<int64_t>(TnD::KB)) * TnD::KB;
   auto gemm = [&](double rows) { return 2e-6 * rows * area / 0.8e9; };
-  const double fused = 25.0 + gemm(static_cast<double>(nv) * T) + gemm(static_cast<double>(n_t) * Tp);
-  const double grad = 10.0 + gemm(static_cast<double>(n_t) * T) + (with_bias ? 15.0 : 0.0);
-  double dots;
-  if (algo == GS_ALGO_GHOST) {
-    const double tiles = static_cast<double>(ceil_div(nv * T, int64_t{StashCfg::BM})) *
-                         ceil_div(n_t * T, int64_t{StashCfg::BN});
-    dots = 6.0 + std::ceil(tiles / 256.0) * 0.024 * (d_in + d_out);
-  } else {
-    dots = 15.0 + gemm(static_cast<double>(nv) * T) + gemm(static_cast<double>(n_t) * T);
-  }
-  return fused <= dots + grad;
+  return gemm(static_cast<double>(n_t) * Tp) <=
+         2.0 * gemm(static_cast<double>(n_t) * T) + (with_bias ? 15.0 : 0.0);
 }
 struct TgBufs {
   uint16_t *abar, *gbar;
@@ -4394,8 +4369,10 @@ extern "C" size_t gs_linear_layer_pass_workspace(int dtype, int64_t N, int64_t n
                : 0;
   if (algo == GS_ALGO_GHOST || !tg_ok(dtype, N, n_val, T, d_in, d_out, semantics)) return 0;
   const LinearPlan pl = plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, 0);
-  if (pl.algo == GS_ALGO_GHOST && rounding == GS_ROUND_REF_BF16) return 0;
-  if (!layer_pass_pays(pl.algo, N, n_val, T, d_in, d_out, semantics, with_bias)) return 0;
+  // Shapes whose flops choose the ghost kernel keep its dots: the pass rounds elsewhere (an entry
+  // of V, not a Gram entry), 0.2-0.3% of the dots' norm apart.
+  if (pl.algo == GS_ALGO_GHOST) return 0;
+  if (!layer_pass_pays(N, n_val, T, d_in, d_out, with_bias)) return 0;
   return conv1d ? tg_workspace(dtype, N, n_val, T, d_out, d_in, semantics, with_bias != 0, true,
                                true)
                 : tg_workspace(dtype, N, n_val, T, d_in, d_out, semantics, with_bias != 0, false,

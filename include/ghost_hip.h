@@ -58,8 +58,7 @@ typedef enum { GS_SEM_PAIRWISE_SUM = 0, GS_SEM_PRESUM = 1 } gs_semantics;
  *            the epilogue of a second GEMM; per-sample gradients are never stored.  With a
  *            pair matrix and aligned bf16 operands: one V_j per val row, and each train row's
  *            gradient tile times every V_j as it leaves the accumulators.
- *   AUTO:    the one with fewer MFMA flops for the shape; where a pair matrix can come from the
- *            sample products above, the one with the shorter estimated time. */
+ *   AUTO:    the one with fewer MFMA flops for the shape. */
 typedef enum { GS_ALGO_AUTO = 0, GS_ALGO_GHOST = 1, GS_ALGO_VALGRAD = 2 } gs_algo;
 
 /* Rounding of the ghost Gram blocks.
@@ -184,9 +183,8 @@ int gs_conv1d_dot_train_grad(const void* A, const void* G, int dtype, int64_t N,
  * dots rounded once from fp32 to dot_dtype / bias_dot_dtype (GS_DTYPE_BF16 or GS_DTYPE_F32).
  * Where T is not a whole number of the kernel's stages each train sample is padded with zero rows inside the kernel
  * (nothing is read for them).  The workspace query returns 0 where the pass does not apply
- * (algo GHOST, or AUTO choosing GHOST with the
- * reference's rounding) and where, for `algo`, the dots and the train gradient apart are
- * estimated to be faster.  Reference: as for the two entry points above. */
+ * (algo GHOST, and bf16 operands for which AUTO chooses GHOST) and where the dots and the train
+ * gradient apart are estimated to be faster.  Reference: as for the two entry points above. */
 size_t gs_linear_layer_pass_workspace(int dtype, int64_t N, int64_t n_val, int64_t T,
                                       int64_t d_in, int64_t d_out, int semantics, int conv1d,
                                       int with_bias, int algo, int rounding);

@@ -625,9 +625,32 @@ def test_linear_layer_pass_fp32(gpu, case):
         assert torch.isnan(dn[1]) and torch.equal(dn[others], dot.cpu()[others])
 
 
+@pytest.mark.parametrize("shape", [
+    # N, n_val, T, d_in, d_out and whether a layer's flops choose the ghost kernel, as a pair
+    # matrix's do
+    (13, 7, 192, 320, 320, False), (8, 4, 512, 1280, 1280, False), (22, 8, 18, 320, 1280, True),
+    (10, 5, 128, 1024, 1024, True)])
+def test_automatic_choice_of_the_ghost_kernel_runs_it(gpu, shape):
+    """Where the automatic choice is the ghost kernel its dots are the ghost kernel's, bit for bit,
+    with a pair matrix and in a layer (which leaves the fused pass to others)."""
+    N, n_val, T, d_in, d_out, layer = shape
+    A, G = (x.to(gpu) for x in _inputs(N, T, d_in, d_out, 340 + T, torch.bfloat16))
+    ops = _native.ops()
+    for pair in (True, False) if layer else (True,):
+        assert ops.linear_algo(torch.bfloat16, N, n_val, T, d_in, d_out, 0, _native.ALGO_AUTO,
+                               pair) == _native.ALGO_GHOST
+        auto, ghost = (ops.linear_dot(A, G, n_val, algo=a, want_pair=pair)
+                       for a in (_native.ALGO_AUTO, _native.ALGO_GHOST))
+        assert torch.equal(auto[0], ghost[0]) and (not pair or torch.equal(auto[1], ghost[1]))
+    assert not layer or ops.linear_layer_pass(
+        A, G, n_val, semantics=_native.SEM_PAIRWISE_SUM, algo=_native.ALGO_AUTO,
+        rounding=_native.ROUND_FP32, conv1d=False, grad_scale=1.0, grad_dtype=torch.float32,
+        dot_dtype=torch.float32) is None
+
+
 def test_linear_layer_pass_declines(gpu):
     """Unaligned feature counts, the ghost algorithm, and the automatic choice of
-    the ghost kernel with the reference's rounding keep the separate passes."""
+    the ghost kernel keep the separate passes."""
     def taken(A, G, algo=_native.ALGO_AUTO, rounding=_native.ROUND_FP32):
         return _native.ops().linear_layer_pass(
             A.to(gpu), G.to(gpu), 2, semantics=_native.SEM_PAIRWISE_SUM, algo=algo,
@@ -643,7 +666,7 @@ def test_linear_layer_pass_declines(gpu):
     A, G = _inputs(6, 64, 2048, 2048, 8, torch.bfloat16)
     assert _native.ops().linear_algo(torch.bfloat16, 6, 2, 64, 2048, 2048, 0, 0,
                                      False) == _native.ALGO_GHOST
-    assert not taken(A, G, rounding=_native.ROUND_REF_BF16)
+    assert not taken(A, G) and not taken(A, G, rounding=_native.ROUND_REF_BF16)
 
 
 @pytest.mark.parametrize("case", [
