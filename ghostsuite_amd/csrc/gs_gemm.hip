@@ -4363,12 +4363,16 @@ extern "C" size_t gs_linear_layer_pass_workspace(int dtype, int64_t N, int64_t n
                                                  int conv1d, int with_bias, int algo,
                                                  int rounding) {
   if (!linear_args_ok(dtype, N, n_val, T, d_in, d_out, semantics, algo, 0)) return 0;
-  if (algo != GS_ALGO_GHOST && dtype == GS_DTYPE_F32)
+  if (algo == GS_ALGO_GHOST) return 0;
+  const LinearPlan pl = plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, 0);
+  if (dtype == GS_DTYPE_F32) {
+    // fp32 sums throughout, so only the reference's rounding of the Gram entries is another result
+    if (pl.algo == GS_ALGO_GHOST && rounding == GS_ROUND_REF_BF16) return 0;
     return tf_ok(dtype, N, n_val, T, d_in, d_out, semantics)
                ? tf_workspace(N, n_val, T, d_in, d_out, semantics, with_bias != 0, conv1d != 0)
                : 0;
-  if (algo == GS_ALGO_GHOST || !tg_ok(dtype, N, n_val, T, d_in, d_out, semantics)) return 0;
-  const LinearPlan pl = plan_any(dtype, N, n_val, T, d_in, d_out, semantics, algo, 0);
+  }
+  if (!tg_ok(dtype, N, n_val, T, d_in, d_out, semantics)) return 0;
   // Shapes whose flops choose the ghost kernel keep its dots: the pass rounds elsewhere (an entry
   // of V, not a Gram entry), 0.2-0.3% of the dots' norm apart.
   if (pl.algo == GS_ALGO_GHOST) return 0;

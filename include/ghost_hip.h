@@ -183,8 +183,9 @@ int gs_conv1d_dot_train_grad(const void* A, const void* G, int dtype, int64_t N,
  * dots rounded once from fp32 to dot_dtype / bias_dot_dtype (GS_DTYPE_BF16 or GS_DTYPE_F32).
  * Where T is not a whole number of the kernel's stages each train sample is padded with zero rows inside the kernel
  * (nothing is read for them).  The workspace query returns 0 where the pass does not apply
- * (algo GHOST, and bf16 operands for which AUTO chooses GHOST) and where the dots and the train
- * gradient apart are estimated to be faster.  Reference: as for the two entry points above. */
+ * (algo GHOST; AUTO choosing GHOST for bf16 operands, or for fp32 ones with the reference's
+ * rounding) and where the dots and the train gradient apart are estimated to be faster.
+ * Reference: as for the two entry points above. */
 size_t gs_linear_layer_pass_workspace(int dtype, int64_t N, int64_t n_val, int64_t T,
                                       int64_t d_in, int64_t d_out, int semantics, int conv1d,
                                       int with_bias, int algo, int rounding);

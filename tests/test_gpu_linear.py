@@ -667,6 +667,12 @@ def test_linear_layer_pass_declines(gpu):
     assert _native.ops().linear_algo(torch.bfloat16, 6, 2, 64, 2048, 2048, 0, 0,
                                      False) == _native.ALGO_GHOST
     assert not taken(A, G) and not taken(A, G, rounding=_native.ROUND_REF_BF16)
+    # fp32: the reference's rounding of the Gram entries is the ghost kernel's alone
+    A, G = _inputs(6, 16, 512, 768, 9, torch.float32)
+    assert _native.ops().linear_algo(torch.float32, 6, 2, 16, 512, 768, 0, 0,
+                                     False) == _native.ALGO_GHOST
+    assert taken(A, G) and not taken(A, G, rounding=_native.ROUND_REF_BF16)
+    assert taken(A, G, _native.ALGO_VALGRAD, _native.ROUND_REF_BF16)
 
 
 @pytest.mark.parametrize("case", [
