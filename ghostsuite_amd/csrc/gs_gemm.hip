@@ -2454,10 +2454,10 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tn_pair_kernel(TpParams q
 // one row per half-wave, no bank conflicts).  Bound by the fp32 matrix rate (a 128 x 128 tile's
 // 8-row stage is 1024 MFMA cycles per wave against 64 reads).  16 + 4 samples, T = 256, 768 x 768,
 // one layer's hook with a bias: 229 us as a transposed val GEMM on 64 x 64 tiles without splits,
-// row-dot, bias passes and hipBLASLt, 84 us so (6.0 GFLOP; the train launch 56 us, 79% MFMA busy
-// while its CUs are; a ring of 8 stages gives no more).  Measured against the separate passes at
-// T = 1 to 500 and 64 to 5120 features it is never behind (64 + 16 samples of a 1024 x 1024 2-D
-// layer 184 -> 53 us, 12 + 2 of 1280 x 5120 at T = 55 656 -> 147), so nothing else is estimated.
+// row-dot, bias passes and hipBLASLt, 79 us so (6.0 GFLOP; the train launch 56 us, 79% MFMA busy
+// while its CUs are; a ring of 8 stages gives no more).  64 + 16 samples of a 1024 x 1024 2-D
+// layer 184 -> 48 us, 12 + 2 of 1280 x 5120 at T = 55 656 -> 147; where many short samples cost
+// it more padded rows than it saves launches, the separate passes stay (tf_pays).
 //
 // Samples are padded with zero rows to whole stages (the buffer ends at the sample's last row).
 // At each sample's end the accumulators hold that sample's G_i^T A_i: its inner product with V
@@ -4238,6 +4238,41 @@ size_t tf_workspace(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t d
   carve_tf(sz, plan_tf(N, n_val, T, d_in, d_out, semantics, bias, conv1d), T, d_in, d_out);
   return sz.used + 256;
 }
+// Whether the pass beats the dots by `algo`, the bias pass and the train gradient apart.  Estimated
+// times in us of one layer's hook.  The pass: the split estimate's, with one more stage for the
+// inner product and the adds at each sample's end (as long as a stage: a 2-D layer of T = 1 pays
+// two stages, 16 rows, for one).  Apart: the gradient at 117 TF/s; the bias pass 72 ns a sample;
+// 65 ns a feature for every chain of 64 x 64 tiles, 1500 of them at a time, over the features
+// (ghost) or over the features and the val tokens (V unsplit, row-dots).  Fitted to 385 shapes of
+// 4 to 16384 samples, T = 1 to 512, 16 to 4800 features: within 15% of nearly all of both, and the
+// choice at most 30% behind the better one (fused / apart, us: 2048 + 64 samples of 1024 x 1024
+// at T = 1 535 / 396, 256 + 32 93 / 208; 8192 + 64 of 4096 x 4096 30400 / 3400, 64 + 8 307 / 668;
+// 2048 + 64 of 1024 x 1024 at T = 4 538 / 485, 8 535 / 723).
+bool tf_pays(const TfPlan& t, int algo, int64_t N, int64_t n_val, int64_t T, int64_t d_in,
+             int64_t d_out) {
+  const int64_t tiles = t.m_tiles * t.n_tiles, area = tiles * TfC::BM * TfC::BN;
+  auto launch = [&](int64_t sp, double rows, int64_t count) {
+    const int64_t items = tiles * sp;
+    return std::ceil(static_cast<double>(items) / 512.0) * 2.0 * TfC::BM * TfC::BN * rows /
+               (items <= 256 ? 0.33e6 : 0.27e6) +
+           8.0 * sp * count / 4e6;
+  };
+  const double fused =
+      25.0 + launch(t.vsp, static_cast<double>(t.vkper), area) +
+      launch(t.sp, static_cast<double>(t.kper) * (1.0 + static_cast<double>(TF_KB) / t.Tp), t.M * t.N);
+  constexpr int64_t TL = 64;
+  const double nvT = static_cast<double>(t.vrows), rows = static_cast<double>(t.n_t) * T;
+  auto rounds = [&](double a, double b, double at_once) {
+    return std::max(1.0, std::ceil(a / TL) * std::ceil(b / TL) / at_once);
+  };
+  double apart = 56.0 + (t.bias ? 0.072 * t.n_t : 0.0) + 2.0 * rows * d_in * d_out / 117e6;
+  if (algo == GS_ALGO_GHOST)
+    apart += 0.065 * (d_in + d_out) * rounds(nvT, rows, 1500.0);
+  else
+    apart += 0.062 * nvT * std::ceil(rounds(d_out, d_in, 256.0)) +
+             0.065 * d_in * rounds(rows, d_out, 1500.0) + 0.0054 * rows;
+  return fused <= apart;
+}
 template <bool VAL>
 void launch_tnf(const TfParams& p, int64_t items, int cs, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(items)), block(TfC::NT);
@@ -4368,9 +4403,11 @@ extern "C" size_t gs_linear_layer_pass_workspace(int dtype, int64_t N, int64_t n
   if (dtype == GS_DTYPE_F32) {
     // fp32 sums throughout, so only the reference's rounding of the Gram entries is another result
     if (pl.algo == GS_ALGO_GHOST && rounding == GS_ROUND_REF_BF16) return 0;
-    return tf_ok(dtype, N, n_val, T, d_in, d_out, semantics)
-               ? tf_workspace(N, n_val, T, d_in, d_out, semantics, with_bias != 0, conv1d != 0)
-               : 0;
+    if (!tf_ok(dtype, N, n_val, T, d_in, d_out, semantics) ||
+        !tf_pays(plan_tf(N, n_val, T, d_in, d_out, semantics, with_bias != 0, conv1d != 0),
+                 pl.algo, N, n_val, T, d_in, d_out))
+      return 0;
+    return tf_workspace(N, n_val, T, d_in, d_out, semantics, with_bias != 0, conv1d != 0);
   }
   if (!tg_ok(dtype, N, n_val, T, d_in, d_out, semantics)) return 0;
   // Shapes whose flops choose the ghost kernel keep its dots: the pass rounds elsewhere (an entry

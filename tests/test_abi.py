@@ -71,6 +71,23 @@ def test_auto_algorithm_choice_is_host_only():
     assert lib.gs_linear_dot_algo(0, 20, 4, 8, 1024, 4096, 0, 2, 0) == _native.ALGO_VALGRAD
 
 
+@pytest.mark.parametrize("shape,taken", [
+    # n_train, n_val, T, d_in, d_out (fp32): both sides of the line as measured, 2-D layers first
+    ((64, 16, 1, 1024, 1024), True), ((256, 32, 1, 1024, 1024), True),
+    ((1024, 64, 1, 2048, 2048), False), ((2048, 64, 1, 1024, 1024), False),
+    ((8192, 128, 1, 512, 1024), False), ((8192, 64, 1, 4096, 4096), False),
+    ((64, 8, 1, 4096, 4096), True), ((256, 32, 1, 4096, 4096), False),
+    ((2048, 64, 4, 1024, 4096), False), ((2048, 64, 8, 1024, 1024), True),
+    ((2048, 64, 9, 4096, 4096), False), ((16, 4, 256, 768, 768), True),
+    ((64, 8, 512, 4096, 4096), True)])
+def test_fp32_layer_pass_leaves_what_it_would_pad_to_the_separate_passes(shape, taken):
+    n_t, n_val, T, d_in, d_out = shape
+    for conv1d in (0, 1):
+        size = _native.load_library().gs_linear_layer_pass_workspace(
+            1, n_t + n_val, n_val, T, d_in, d_out, 0, conv1d, 1, 0, 0)
+        assert (size > 0) == taken
+
+
 def test_cpu_tensors_are_rejected_loudly():
     import torch
     with pytest.raises(_native.GhostHipError, match="ROCm GPU"):
