@@ -3059,7 +3059,19 @@ LinearPlan plan_linear(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_
   if (algo == GS_ALGO_AUTO) pl.algo = ghost <= valgrad ? GS_ALGO_GHOST : GS_ALGO_VALGRAD;
   // The products are a form of the val-gradient algorithm: they do not take shapes whose flops
   // choose the ghost kernel, whose dots round elsewhere (a Gram entry, not an entry of V_j).
-  if (products && pl.algo == GS_ALGO_VALGRAD) {
+  // And only where they beat a V GEMM and a row-dot GEMM per val sample.  Estimated times in us.
+  // Products: whole 64-row stages of 128 x 128 tiles at 1 PF/s, the inner products at 0.13 ps per
+  // V_j entry and train sample, 12 us of launches and pipeline fill.  Row-dots: 12 us, 13.5 ns a
+  // feature of fill and 1.5 PF/s per val sample.  Measured (products / row-dots, us): 24 + 8
+  // samples of T = 128, 768 x 3072 84 / 513, 24 + 1 38 / 67, of T = 1024 135 / 144; 200 + 1 of one
+  // token, 1024 x 1024 77 / 38, 200 + 4 117 / 143; 4000 + 1 of one token, 512 x 512 330 / 33;
+  // 48 + 1 of T = 200, 2048 x 2048 141 / 123; 8 + 1 of T = 2048, 2048 x 8192 604 / 536, 8 + 2
+  // 711 / 1053.
+  const double area = static_cast<double>(pair_tiles(d_in, d_out)) * TnC::BM * TnC::BN;
+  const double prod = 12.0 + 2e-9 * N * ceil_div(T, TnD::KB) * TnD::KB * area +
+                      1.3e-7 * n_val * n_t * area;
+  const double rows = n_val * (12.0 + 0.0135 * (d_in + d_out) + 1.3e-9 * n_t * T * d_in * d_out);
+  if (products && pl.algo == GS_ALGO_VALGRAD && prod <= rows) {
     pl.pairs = 1;
     pl.groups = n_val;
     pl.p_rows = n_val * pair_tiles(d_in, d_out);
