@@ -182,8 +182,11 @@ def _worth_overlapping(layer: nn.Module, acts, backprops) -> bool:
         return True
     if acts.numel() + backprops.numel() > _INLINE_ELEMENTS:
         return True
-    return not isinstance(layer, (nn.LayerNorm, nn.Embedding)) and \
-        2.0 * acts.numel() * backprops.shape[-1] > _INLINE_FLOPS
+    if isinstance(layer, (nn.LayerNorm, nn.Embedding)):
+        return False
+    if isinstance(layer, nn.Conv2d):   # channels first: every output element takes a filter's size
+        return 2.0 * backprops.numel() * layer.weight[0].numel() > _INLINE_FLOPS
+    return 2.0 * acts.numel() * backprops.shape[-1] > _INLINE_FLOPS
 
 
 def _train_grads_parked(layer: nn.Module) -> bool:

@@ -522,6 +522,21 @@ def test_gradient_stage_skips_side_stream_only_when_everything_is_parked():
     assert _train_grads_parked(emb)
 
 
+def test_conv2d_work_decides_its_stream():
+    """A convolution's output gradient is [N, C_out, H, W]: its work is every output element times
+    a filter's size, not times the output width."""
+    from ghostsuite_amd import autograd_grad_sample_dotprod as hooks
+    with torch.device("meta"):
+        conv = nn.Conv2d(256, 256, 3, padding=1)
+        x = torch.empty(80, 256, 14, 14)         # 8.03M elements in all, 18.5 GFLOP
+        assert 2 * x.numel() <= hooks._INLINE_ELEMENTS
+        assert hooks._worth_overlapping(conv, x, x)
+        assert hooks._worth_overlapping(nn.Conv2d(256, 256, 1), x, x)
+        assert not hooks._worth_overlapping(nn.Conv2d(3, 16, 3, padding=1),
+                                            torch.empty(16, 3, 32, 32),
+                                            torch.empty(16, 16, 32, 32))
+
+
 def test_dot_dtypes_follow_the_reference():
     """Each grad_dot_prod comes in the dtype the reference's sampler returns for a bf16
     layer: fp32 from a ghost branch (its fp32 sums, supported_layers_grad_samplers_dotprod.py
