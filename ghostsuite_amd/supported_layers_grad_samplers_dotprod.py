@@ -128,9 +128,10 @@ def _dot_dtype(x: torch.Tensor, pairwise: bool) -> torch.dtype:
 def _reference_dtypes(layer: nn.Module, weight_dtype: Optional[torch.dtype],
                       bias_dtype: Optional[torch.dtype]) -> None:
     """Casts the dots the sampler set to the dtypes the reference's sampler returns (a None
-    dtype: left fp32; nothing where the kernels already wrote them so).  Its materialised branches and bias dots are einsums over operands in
-    the layer's dtype (Linear :131-146 in the original dtype, Conv1D :445-471 and Conv2d
-    :552-559 in bf16); its ghost branches sum in fp32 (:129-130, :437, :550)."""
+    dtype: left fp32; nothing where the kernels already wrote them so).  Its materialised
+    branches and bias dots are einsums over operands in the layer's dtype (Linear :131-146 in
+    the original dtype, Conv1D :445-471 and Conv2d :552-559 in bf16); its ghost branches sum in
+    fp32 (:129-130, :437, :550)."""
     if options["dot_dtypes"] != "reference" or options["precision"] == "fp32":
         return
     for param, dt in ((_param(layer, "weight"), weight_dtype),
@@ -246,13 +247,14 @@ def _fused_dot_train_grad(layer: nn.Module, A: torch.Tensor, B: torch.Tensor,
     """Weight dot and weight train gradient (and with a bias its dot and train gradient) from
     one K-major pass over the train rows: per train row, sum_t g^T V a = <V, G_i^T A_i>, and
     the train gradient is the sum of the same G_i^T A_i (gs_linear_layer_pass).  Taken for
-    bf16 and fp32 layers whose weight trains, unless linear_algo is 'ghost' or the separate passes are
-    estimated to be faster; the train gradients are parked for _apply_train_grad.  Returns
-    False when the other paths must run.
+    bf16 and fp32 layers whose weight trains, unless the dots are the ghost kernel's (chosen or
+    asked for) or the separate passes are estimated to be faster; the train gradients are
+    parked for _apply_train_grad.  Returns False when the other paths must run.
 
-    With ``conv1d`` (HF Conv1D, weight [d_in, d_out]) the kernels run the same pass with the operands swapped: the dot <G_i^T A_i, V> equals <A_i^T G_i, V^T>, the train
-    gradient comes out as the sum of A_i^T G_i (the Conv1D layout), and the bias terms come
-    from the column sums of G as for a Linear layer."""
+    With ``conv1d`` (HF Conv1D, weight [d_in, d_out]) the kernels run the same pass with the
+    operands swapped: the dot <G_i^T A_i, V> equals <A_i^T G_i, V^T>, the train gradient comes
+    out as the sum of A_i^T G_i (the Conv1D layout), and the bias terms come from the column
+    sums of G as for a Linear layer."""
     d = layer.__dict__
     scale = d.get("_gs_bias_grad_scale")
     weight, bias_p = _param(layer, "weight"), _param(layer, "bias")
@@ -267,28 +269,13 @@ def _fused_dot_train_grad(layer: nn.Module, A: torch.Tensor, B: torch.Tensor,
         return False
     Bc = B.to(dtype) if B.dtype != dtype else B
     sem = _native.SEM_PAIRWISE_SUM if pairwise else _native.SEM_PRESUM
-    algo = _ALGOS[options["linear_algo"]]
-    layer_pass = getattr(ops(), "linear_layer_pass", None)
-    if layer_pass is not None:
-        weight_dt, bias_dt = _dot_result_dtypes(layer, A, B, conv1d)
-        res = layer_pass(A, Bc, val_batch_size, semantics=sem, algo=algo,
-                         rounding=_ROUNDINGS[options["rounding"]], conv1d=conv1d,
-                         grad_scale=scale, grad_dtype=weight.dtype, dot_dtype=weight_dt,
-                         bias_grad_dtype=bias_p.dtype if bias else None,
-                         bias_dot_dtype=bias_dt)
-    elif dtype != torch.bfloat16:
-        return False
-    else:   # a kernel layer without the whole-layer pass
-        N, d_in, d_out = A.shape[0], A.shape[-1], Bc.shape[-1]
-        T = A.numel() // (N * d_in)
-        if ops().linear_algo(dtype, N, val_batch_size, T, d_in, d_out, sem, algo,
-                             False) != _native.ALGO_VALGRAD:
-            return False
-        res = ops().linear_dot_train_grad(A, Bc, val_batch_size, semantics=sem,
-                                          grad_scale=scale, grad_dtype=weight.dtype,
-                                          bias=bias, bias_grad_scale=scale,
-                                          bias_grad_dtype=bias_p.dtype if bias else None,
-                                          conv1d=conv1d)
+    weight_dt, bias_dt = _dot_result_dtypes(layer, A, B, conv1d)
+    res = ops().linear_layer_pass(A, Bc, val_batch_size, semantics=sem,
+                                  algo=_ALGOS[options["linear_algo"]],
+                                  rounding=_ROUNDINGS[options["rounding"]], conv1d=conv1d,
+                                  grad_scale=scale, grad_dtype=weight.dtype, dot_dtype=weight_dt,
+                                  bias_grad_dtype=bias_p.dtype if bias else None,
+                                  bias_dot_dtype=bias_dt)
     if res is None:
         return False
     dot, grad, bias_dot, bias_grad = res
@@ -421,11 +408,11 @@ def _compute_embedding_dot_product(layer: nn.Embedding, A: torch.Tensor, B: torc
         ids = layer.__dict__.get("activations")
         ids = A if ids is None or ids.is_floating_point() else ids.detach()
         out, grad, accumulate = _embedding_grad_out(layer)
-        layer_pass = getattr(ops(), "embedding_layer_pass", None)
         dot = None
-        if layer_pass is not None and ids.data_ptr() == A.data_ptr() and \
-                ids.dtype == A.dtype and ids.stride() == A.stride():
-            dot = layer_pass(A, B, val_batch_size, scale, out, accumulate=accumulate)
+        if ids.data_ptr() == A.data_ptr() and ids.dtype == A.dtype and \
+                ids.stride() == A.stride():   # the same ids for both
+            dot = ops().embedding_layer_pass(A, B, val_batch_size, scale, out,
+                                             accumulate=accumulate)
         if dot is None:
             dot = ops().embedding_dot(A, B, val_batch_size, vocab=layer.weight.shape[0])
             ops().embedding_train_grad(ids, B, val_batch_size, scale, out, accumulate=accumulate)

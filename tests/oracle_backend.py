@@ -35,21 +35,32 @@ class OracleOps:
         bdot, grad = self.bias_dot(G, n_val, grad_scale=grad_scale, grad_dtype=grad_dtype)
         return dot, bdot, grad
 
-    def linear_dot_train_grad(self, A, G, n_val, *, val_start=None, semantics=0,
-                              grad_scale=None, grad_dtype=None, bias=False,
-                              bias_grad_scale=None, bias_grad_dtype=None):
-        """The fused weight dot + train gradient (+ bias dot and gradient), as closed forms."""
-        self.calls.append(("linear_dot_train_grad", tuple(A.shape), tuple(G.shape)))
+    def linear_layer_pass(self, A, G, n_val, *, semantics, algo, rounding, conv1d, grad_scale,
+                          grad_dtype, dot_dtype, bias_grad_dtype=None, bias_dot_dtype=None,
+                          val_start=None):
+        """The whole-layer pass as closed forms, or None where the kernels leave the layer to the
+        separate passes: the ghost algorithm (with fp32 operands, only asked for or with the
+        reference's rounding) and feature counts their loads do not take."""
+        N, d_in, d_out = A.shape[0], A.shape[-1], G.shape[-1]
+        T = A.numel() // (N * d_in)
+        chosen = self.linear_algo(A.dtype, N, n_val, T, d_in, d_out, semantics, algo, False)
+        fp32 = A.dtype == torch.float32
+        step = 4 if fp32 else 8
+        if algo == _native.ALGO_GHOST or d_in % step or d_out % step or \
+                (chosen == _native.ALGO_GHOST and
+                 (not fp32 or rounding == _native.ROUND_REF_BF16)):
+            self.calls.append(("linear_layer_pass declined", tuple(A.shape), tuple(G.shape)))
+            return None
+        self.calls.append(("linear_layer_pass", tuple(A.shape), tuple(G.shape)))
         dot, _ = self.linear_dot(A, G, n_val, val_start=val_start, semantics=semantics)
-        grad = None
-        if grad_scale is not None:
-            grad = self.linear_train_grad(A, G, n_val, grad_scale, val_start=val_start,
-                                          out_dtype=grad_dtype)
+        grad = self.linear_train_grad(A, G, n_val, grad_scale, val_start=val_start,
+                                      out_dtype=grad_dtype, conv1d=conv1d)
         bdot = bgrad = None
-        if bias:
-            bdot, bgrad = self.bias_dot(G, n_val, val_start=val_start,
-                                        grad_scale=bias_grad_scale, grad_dtype=bias_grad_dtype)
-        return dot, grad, bdot, bgrad
+        if bias_grad_dtype is not None:
+            bdot, bgrad = self.bias_dot(G, n_val, val_start=val_start, grad_scale=grad_scale,
+                                        grad_dtype=bias_grad_dtype)
+            bdot = bdot.to(bias_dot_dtype)
+        return dot.to(dot_dtype), grad, bdot, bgrad
 
     def linear_train_grad(self, A, G, n_val, scale, *, val_start=None, out_dtype=None,
                           conv1d=False):
@@ -90,6 +101,18 @@ class OracleOps:
             out[touched] = (out[touched].double() + g[touched]).to(out.dtype)
         else:
             out.copy_(g.to(out.dtype))
+
+    def embedding_layer_pass(self, ids, G, n_val, scale, out, *, accumulate=False,
+                             val_start=None):
+        """Both of the above, or None for the sizes the kernels leave to the two calls."""
+        if ids.numel() // ids.shape[0] * n_val > 8192 or out.shape[0] >= 1 << 19:
+            self.calls.append(("embedding_layer_pass declined", tuple(G.shape)))
+            return None
+        self.calls.append(("embedding_layer_pass", tuple(G.shape)))
+        dot = self.embedding_dot(ids, G, n_val, out.shape[0], val_start=val_start)
+        self.embedding_train_grad(ids, G, n_val, scale, out, accumulate=accumulate,
+                                  val_start=val_start)
+        return dot
 
     def layernorm_dot(self, X, G, n_val, eps, *, val_start=None, want_dot=True, want_bias=True,
                       grad_scale=None, grad_dtype=None):

@@ -630,7 +630,8 @@ def test_gradient_accumulation_over_backward_passes():
     """Several backward passes before prepare_gradients (the reference loop's gradient
     accumulation, Examples/GradDotProd_LM/training_loop.py:122-144, each on loss / k):
     grad_dot_prod is the last pass's (assigned), train_grad the sum of every pass's (added in
-    place, supported_layers_grad_samplers_dotprod.py:44-70)."""
+    place, supported_layers_grad_samplers_dotprod.py:44-70); through the whole-layer pass (the
+    first layer) and the separate passes (the second, whose width the pass declines)."""
     torch.manual_seed(4)
     dims = (32, 24, 10)
     model = MLP(dims)
@@ -638,13 +639,15 @@ def test_gradient_accumulation_over_backward_passes():
     n_t, n_v, k = 10, 3, 3
     X = torch.randn(n_t + n_v, dims[0], generator=gen(21))
     Y = torch.randint(0, 10, (n_t + n_v,), generator=gen(22))
-    with use_oracle_backend():
+    with use_oracle_backend() as ops:
         eng = GradDotProdEngine(model, val_batch_size=n_v, use_dummy_bias=False,
                                 precision="fp32")
         eng.attach(torch.optim.SGD(model.parameters(), lr=0.0))
         eng.attach_train_batch(X[:n_t], Y[:n_t], 0, 0)
         for _ in range(k):
             (F.cross_entropy(model(X), Y) / k).backward()
+        passes = [c[0] for c in ops.calls if c[0].startswith("linear_layer_pass")]
+        assert passes == ["linear_layer_pass declined", "linear_layer_pass"] * k
         dots = {n: p.grad_dot_prod.clone() for n, p in model.named_parameters()}
         eng.prepare_gradients()
         grads = {n: p.grad.clone() for n, p in model.named_parameters()}
