@@ -7,7 +7,7 @@
 // every run, and every step's work is linear in the number of tokens however often an id repeats.
 // Launches:
 //   1. eg_bucket_kernel  -- the list, its length and the presence bitmap of the ids, for up to
-//                           131072 tokens and 131072 ids; beyond that in two launches:
+//                           131072 tokens and 524288 ids; beyond that in two launches:
 //      eg_sort_kernel    -- chunks of EG_CHUNK tokens sorted in registers and LDS (bitonic);
 //                           per-chunk counts of in-range ids; the id-presence bitmap cleared.
 //   2. eg_merge_kernel   -- every key's place in the whole list = its place in its chunk plus

@@ -195,6 +195,7 @@ def test_embedding_train_grad_heavy_ids(gpu, shape, pad_frac):
     ((4, 2, 300, 13, 524287), (65, 2)),           # most ids, rows of 13 features
     ((4, 1, 8192, 24, 300), (7000,)),             # most val tokens
     ((4, 1, 70, 8, 50), (64, 2)),                 # dot units past a whole workgroup of four
+    ((66, 2, 2049, 8, 1000), (300, 2)),           # a bucketed val list beside sorted train chunks
 ])
 def test_embedding_layer_pass(gpu, dtype, shape, runs):
     """Dots and train gradient in shared launches: the bits of the two calls, the dots within fp32
@@ -231,10 +232,14 @@ def test_embedding_layer_pass(gpu, dtype, shape, runs):
     # N, n_val, T, d, vocab
     ((3, 1, 500, 8, 256), 0.0),          # one id a bucket
     ((3, 1, 1025, 8, 257), 0.5),         # two; a token past the waves' even shares
-    ((4, 1, 2100, 8, 131072), 0.93),     # most ids; shares that keep 384 tokens of a bucket or more
-    ((4, 1, 2100, 8, 131073), 0.93),     # one id too many: sorted chunks
+    ((4, 1, 2100, 8, 131072), 0.93),     # most ids of 256 buckets; shares that keep 384 or more
+    ((4, 1, 2100, 8, 131073), 0.93),     # 1024 buckets
+    ((4, 1, 2100, 8, 524288), 0.93),     # most ids
+    ((4, 1, 2100, 8, 524289), 0.5),      # one too many: sorted chunks, 32-bit keys
+    ((4, 1, 2100, 4, 1048577), 0.5),     # 64-bit keys
     ((65, 1, 2048, 8, 1000), 0.1),       # most tokens
-    ((66, 2, 2049, 8, 1000), 0.1),       # sorted chunks
+    ((66, 2, 2049, 8, 1000), 0.1),       # sorted chunks, merged by their samples
+    ((130, 2, 2049, 8, 1000), 0.1),      # more chunks than the merge samples
 ])
 def test_embedding_train_grad_list_edges(gpu, shape, pad_frac):
     """The token list at the edges of its two forms: float64 index_add within fp32 rounding of a
