@@ -14,7 +14,9 @@
 // reduced per sample in a fixed order.  Bound by HBM: 32 x 1024 tokens of 1024 + 4096
 // bf16 features at 16 x 16 projection rows take 67 us (5.0 TB/s, a 1 GiB copy 5.1; 75 us when
 // all waves loaded, multiplied and waited in step), of 1024 + 3072 at 39 x 13 54 us (113 us with
-// both sides padded to 64 rows and 133 KiB of LDS).
+// both sides padded to 64 rows and 133 KiB of LDS).  Rows off 16-byte boundaries are loaded 16
+// bytes at a time too: of 1023 + 4095 features at 20 x 20 221 us (element by element 435, in
+// chunks of 64 tokens 257), at 40 x 13 200 (452, 265).
 //
 // 16x16 MFMA layout: lane l supplies row (l % 16) of A and column (l % 16) of B with its
 // k-slice chosen by l / 16; result element e of lane l is C[4*(l/16) + e][l % 16].
@@ -69,7 +71,8 @@ struct PjF32 {
 // serves the PJ_TG row groups.  `rows` point at valid rows (a token past the end reads another
 // row and is dropped by the caller: an operand row reaches only its own result row), and rows of
 // P past kP repeat its last row (columns nobody reads).  VEC false: rows or projections are
-// not 16-byte aligned, elements are loaded one by one.
+// not 16-byte aligned; they are loaded 16 bytes at a time all the same, a row's last partial 16
+// element by element.
 template <class Tr, int NB, bool VEC>
 __device__ __forceinline__ void project_rows(const typename Tr::E* const (&rows)[PJ_TG],
                                              const typename Tr::E* P, int64_t n, int64_t kP,
@@ -93,8 +96,12 @@ __device__ __forceinline__ void project_rows(const typename Tr::E* const (&rows)
       return v;
     } else {
       union { uint4 v; E e[Tr::VEC]; } u;
+      if (whole || k + Tr::VEC <= n) {
+        __builtin_memcpy(&u.v, row + k, sizeof(u.v));
+      } else {
 #pragma unroll
-      for (int i = 0; i < Tr::VEC; ++i) u.e[i] = k + i < n ? row[k + i] : E(0);
+        for (int i = 0; i < Tr::VEC; ++i) u.e[i] = k + i < n ? row[k + i] : E(0);
+      }
       return u.v;
     }
   };
@@ -168,11 +175,10 @@ struct PjSlice {
 
 // GATHER: the input side is an embedding, whose "projected input" for token id x is column
 // x of P_i, i.e. row x of R = P_i^T ([vocab, ldr], this launch's kR columns); `ids` replaces A.
-// NL, NR: 16-row projection blocks of the two sides (kL <= 16 NL, kR <= 16 NR); VL, VR:
-// 16-byte aligned rows and projections of the G and A sides (element-wise loads need the
-// registers of two waves per SIMD).
-template <class Tr, bool GATHER, int NL, int NR, bool VL, bool VR>
-__global__ void __launch_bounds__(PJ_THREADS, VL && VR ? 4 : 2) kron_proj_kernel(
+// NL, NR: 16-row projection blocks of the two sides (kL <= 16 NL, kR <= 16 NR); VEC: 16-byte
+// aligned rows and projections on both sides.
+template <class Tr, bool GATHER, int NL, int NR, bool VEC>
+__global__ void __launch_bounds__(PJ_THREADS, 4) kron_proj_kernel(
     const typename Tr::E* __restrict__ A, const int64_t* __restrict__ ids, int64_t vocab,
     const typename Tr::E* __restrict__ G, int64_t T, int64_t n_a, int64_t n_g,
     const typename Tr::E* __restrict__ R, const typename Tr::E* __restrict__ L, int64_t kR,
@@ -200,7 +206,7 @@ __global__ void __launch_bounds__(PJ_THREADS, VL && VR ? 4 : 2) kron_proj_kernel
     }
     __syncthreads();
   };
-  auto side = [&](const E* X, int64_t n, const E* P, int64_t kP, int row0, auto nbc, auto vec) {
+  auto side = [&](const E* X, int64_t n, const E* P, int64_t kP, int row0, auto nbc) {
     constexpr int NB = decltype(nbc)::value;
     const E* rows[TG];
 #pragma unroll
@@ -215,7 +221,7 @@ __global__ void __launch_bounds__(PJ_THREADS, VL && VR ? 4 : 2) kron_proj_kernel
       for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[tg][nb][e] = 0.f;
-    project_rows<Tr, NB, decltype(vec)::value>(rows, P, n, kP, acc);
+    project_rows<Tr, NB, VEC>(rows, P, n, kP, acc);
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       f32x4_t one[TG];
@@ -224,7 +230,7 @@ __global__ void __launch_bounds__(PJ_THREADS, VL && VR ? 4 : 2) kron_proj_kernel
       combine(one, row0 + 16 * nb);
     }
   };
-  side(G, n_g, L, kL, 0, std::integral_constant<int, NL>{}, std::integral_constant<bool, VL>{});
+  side(G, n_g, L, kL, 0, std::integral_constant<int, NL>{});
   if constexpr (GATHER) {
     for (int x = threadIdx.x; x < 16 * NR * TOK; x += PJ_THREADS) {
       const int q = x % (16 * NR), tok = x / (16 * NR);
@@ -237,8 +243,7 @@ __global__ void __launch_bounds__(PJ_THREADS, VL && VR ? 4 : 2) kron_proj_kernel
     }
     __syncthreads();
   } else {
-    side(A, n_a, R, kR, 16 * NL, std::integral_constant<int, NR>{},
-         std::integral_constant<bool, VR>{});
+    side(A, n_a, R, kR, 16 * NL, std::integral_constant<int, NR>{});
   }
   // part[p][q] = sum over the tokens of fin[p][tok] fin[16 NL + q][tok]: 16 x 16 blocks by fp32
   // MFMAs, four tokens each.
@@ -298,10 +303,10 @@ int launch_pj_slice(const typename Tr::E* A, const int64_t* ids, int64_t vocab,
                     int64_t ldr, int va, int vg, int vr, int vl, int64_t chunks,
                     PjSlice sl, float* part, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(chunks), static_cast<unsigned>(B));
-  const bool vec_l = vg && vl, vec_r = GATHER || (va && vr);
-  auto go = [&](auto nl, auto nr, auto vecl, auto vecr) {
+  const bool vec = vg && vl && (GATHER || (va && vr));
+  auto go = [&](auto nl, auto nr, auto v) {
     auto k = kron_proj_kernel<Tr, GATHER, decltype(nl)::value, decltype(nr)::value,
-                              decltype(vecl)::value, decltype(vecr)::value>;
+                              decltype(v)::value>;
     hipLaunchKernelGGL(k, grid, dim3(PJ_THREADS), 0, s, A, ids, vocab, G, T, n_a, n_g, R, L, kr,
                        kl, ldr, chunks, sl, part);
   };
@@ -311,24 +316,10 @@ int launch_pj_slice(const typename Tr::E* A, const int64_t* ids, int64_t vocab,
     if (k <= 48) return f(std::integral_constant<int, 3>{});
     return f(std::integral_constant<int, 4>{});
   };
-  constexpr std::true_type yes{};
-  constexpr std::false_type no{};
-  if (vec_l && vec_r) {
-    blocks(kl, [&](auto nl) { blocks(kr, [&](auto nr) { go(nl, nr, yes, yes); }); });
-  } else {  // element-wise loads bound these: one or four blocks a side
-    auto some = [&](auto nb) {
-      if (vec_l)
-        go(nb, nb, yes, no);
-      else if (vec_r)
-        go(nb, nb, no, yes);
-      else
-        go(nb, nb, no, no);
-    };
-    if (std::max(kl, kr) <= 16)
-      some(std::integral_constant<int, 1>{});
-    else
-      some(std::integral_constant<int, 4>{});
-  }
+  auto with = [&](auto v) {
+    blocks(kl, [&](auto nl) { blocks(kr, [&](auto nr) { go(nl, nr, v); }); });
+  };
+  vec ? with(std::true_type{}) : with(std::false_type{});
   return check_launch(GATHER ? "kron_proj_kernel(gather)" : "kron_proj_kernel");
 }
 

@@ -301,8 +301,9 @@ def test_layernorm_dots_and_grads(gpu, dtype, shape, mid):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_kron_projection_edges(gpu, dtype, conf):
     """The chunk, piece and rank-block edges against float64 (fp32 sums of at most 2056 features
-    and 65 tokens: 1e-5 of the rms).  A token row of NaN reaches its own sample only, though the
-    next chunk's padded tokens read valid rows in its place."""
+    and 65 tokens: 1e-5 of the rms), the same bits from a tensor off its alignment.  A token row
+    of NaN reaches its own sample only, though the next chunk's padded tokens read valid rows in
+    its place."""
     B, T, n_i, n_o, k_i, k_o = conf
     print(f"kron edges conf={conf} {dtype}", flush=True)
     A = randn((B, T, n_i), 51 + T, 1.0, dtype)
@@ -315,6 +316,9 @@ def test_kron_projection_edges(gpu, dtype, conf):
     got = run(A)
     want = R.kron_proj_exact(A, G, P_i, P_o, 2.0)
     assert_close(got, want, 1e-5, "projection")
+    off = torch.zeros(A.numel() + 1, dtype=dtype, device=gpu)[1:].view(A.shape)
+    off.copy_(A)                                     # one element past a 16-byte boundary
+    assert torch.equal(run(off), got)
     if B > 1:
         bad = A.clone()
         bad[1, 0] = float("nan")
