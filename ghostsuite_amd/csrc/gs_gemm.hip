@@ -1373,8 +1373,27 @@ __device__ __forceinline__ float4 split_sum4(const float* __restrict__ part, int
   return s;
 }
 
+__device__ __forceinline__ void put_dot(void* out, int f32, int64_t at, float v) {
+  if (f32)
+    static_cast<float*>(out)[at] = v;
+  else
+    static_cast<uint16_t*>(out)[at] = f32_to_bf16(v);
+}
+
+// Whether a dot taken as the growth of running sums (tgdot_kernel) has lost more than bf16
+// rounding: growth2 is the sum of the wave shares' squares, size2 that of the running sums' products
+// with V, entry by entry.  A sum of T k-rows is rounded T / 16 times, each time by 2^-24 of its
+// size at most, independent in sign; that may be 2^-9 of the shares' size.  (Sums of Inf or NaN,
+// and squares that fp32 may have flushed, count as lost.)
+__device__ __forceinline__ bool growth_lost(double growth2, float size2, int64_t T) {
+  const double s = size2;
+  return !(s >= 1e-30 && s * static_cast<double>(T) <= growth2 * 0x1p34);
+}
+
 // After tgdot_kernel, three independent block ranges of one launch, fixed order throughout:
-// blocks b < n_t take weight dot b from its `shares` wave shares and, with pbias, bias dot b
+// blocks b < n_t take weight dot b from its `shares` wave shares (with redo: half as many, each
+// followed by the running sums' size; redo[b] says whether tg_redo_kernel must form the dot
+// again, redo[n_t + b] is its counter, cleared) and, with pbias, bias dot b
 // from its `bshares` shares; then (with bgrad) the bias train gradient, FINISH_GF features
 // per block, over the n_t * cs_rows column-sum rows of csum; then (with grad) the train
 // gradient: grad[i] = gscale * (the sum over the sp splits of part[s][i]), rounded once (or
@@ -1385,25 +1404,41 @@ __global__ void __launch_bounds__(256) tgdot_finish_kernel(
     int64_t bshares, const float* __restrict__ csum, int64_t cs_rows, int64_t M, void* out_dot,
     int dot_f32, void* out_bdot, int bdot_f32, GE* bgrad, float bscale, int64_t gblocks,
     const float* __restrict__ part, int64_t count, int sp, void* grad, float gscale,
-    int grad_f32) {
+    int grad_f32, int* __restrict__ redo, int64_t T) {
   __shared__ float red[4];
+  __shared__ double red2[256];
   int64_t b = blockIdx.x;
   if (b < n_t) {
     float s0 = 0.f, s1 = 0.f;
     int64_t r = threadIdx.x;
-    for (; r + 256 < shares; r += 512) {
-      s0 += pdot[r * n_t + b];
-      s1 += pdot[(r + 256) * n_t + b];
+    if (redo != nullptr) {
+      double g2 = 0.0;
+      for (; r < shares / 2; r += 256) {
+        const float d = pdot[2 * r * n_t + b];
+        s0 += d;
+        g2 += static_cast<double>(d) * d;
+        s1 += pdot[(2 * r + 1) * n_t + b];
+      }
+      red2[threadIdx.x] = g2;
+      const float size2 = block_sum(s1, red);
+      for (int off = 128; off > 0; off >>= 1) {
+        __syncthreads();
+        if (threadIdx.x < off) red2[threadIdx.x] += red2[threadIdx.x + off];
+      }
+      if (threadIdx.x == 0) {
+        redo[b] = growth_lost(red2[0], size2, T) ? 1 : 0;
+        redo[n_t + b] = 0;
+      }
+      s1 = 0.f;
+    } else {
+      for (; r + 256 < shares; r += 512) {
+        s0 += pdot[r * n_t + b];
+        s1 += pdot[(r + 256) * n_t + b];
+      }
+      if (r < shares) s0 += pdot[r * n_t + b];
     }
-    if (r < shares) s0 += pdot[r * n_t + b];
     const float s = block_sum(s0 + s1, red);
-    auto put = [](void* out, int f32, int64_t at, float v) {
-      if (f32)
-        static_cast<float*>(out)[at] = v;
-      else
-        static_cast<uint16_t*>(out)[at] = f32_to_bf16(v);
-    };
-    if (threadIdx.x == 0) put(out_dot, dot_f32, b, s);
+    if (threadIdx.x == 0) put_dot(out_dot, dot_f32, b, s);
     if (pbias == nullptr) return;
     const float* pb = pbias + b * bshares;
     float t0 = 0.f, t1 = 0.f;
@@ -1414,7 +1449,7 @@ __global__ void __launch_bounds__(256) tgdot_finish_kernel(
     }
     if (r < bshares) t0 += pb[r];
     const float t = block_sum(t0 + t1, red);
-    if (threadIdx.x == 0) put(out_bdot, bdot_f32, b, t);
+    if (threadIdx.x == 0) put_dot(out_bdot, bdot_f32, b, t);
     return;
   }
   b -= n_t;
@@ -2077,6 +2112,21 @@ __device__ __forceinline__ void acc_dot(const f32x16_t& a, int h, const uint4& w
   }
 }
 
+// acc_dot, and e += the sum of the products' squares.
+__device__ __forceinline__ void acc_dot_sq(const f32x16_t& a, int h, const uint4& w, float& d0,
+                                           float& d1, float& e) {
+  const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float x = a[8 * h + 2 * i] * __uint_as_float(u[i] << 16);
+    const float y = a[8 * h + 2 * i + 1] * __uint_as_float(u[i] & 0xFFFF0000u);
+    d0 += x;
+    d1 += y;
+    e += x * x;
+    e += y * y;
+  }
+}
+
 // One output tile per work item: bf16 out, or fp32 partials (several splits or an output
 // option) reduced by tn_reduce_kernel.
 template <class C, class D, int CSM>
@@ -2177,7 +2227,8 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tn_gemm_kernel(TnParams p
 //    768 x 2304 80.5 -> 81.5.)
 //  - 128 x 64 wave tiles have no registers for a second set: acc runs on, and the share is the
 //    growth of <acc, V tile> since the previous boundary, which rounds at the running sum's size.
-//    T a multiple of the stage height only.  (Their place taken by 64 x 64 wave tiles: Pythia-1B
+//    That size goes beside it, and tg_redo_kernel forms the dots again that lost too much to it.
+//    T a multiple of the stage height only, splits of whole samples.  (Their place taken by 64 x 64 wave tiles: Pythia-1B
 //    fc 595 -> 702 us, 256 x 128 tiles of eight such waves 712, of four 128 x 64 waves with the
 //    registers of a whole SIMD 864; the sums kept in memory instead 930.)
 // With CS the column sums of the L tile (G: the bias terms) are taken per stage as well, after
@@ -2188,7 +2239,8 @@ struct TgParams {
   const uint4* V;       // V (bf16) in accumulator order of the same tiles (acc_store)
   int64_t T, n_t;       // k-rows per sample, padded to whole stages; train samples
   int64_t T_rows;       // the rows a sample has
-  float* pdot;          // [m_tiles * n_tiles][NW][2 slots][n_t] wave shares of the weight dots
+  float* pdot;          // [m_tiles * n_tiles][NW][2 slots][n_t] wave shares of the weight dots; not
+                        //   HELD: the second slot is the sum of the products' squares
   float* csum;          // with CS: [n_t][2 T / stage height][M] column sums of L (CS 1; of R,
                         // [..][N], with CS 2), two rows (halves of the stage's k-rows) per stage
   const float* vb;      // with CS: [vb_rows][M] ([N]) the val rows' column sums of the same side
@@ -2266,7 +2318,7 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
   int left = static_cast<int>(((sample + 1) * q.T - k_begin) / D::KB);
   bool started = sample * q.T == k_begin;  // the current sample starts inside this split
   auto flush = [&](bool ended) __attribute__((always_inline)) {
-    float d0 = 0.f, d1 = 0.f;
+    float d0 = 0.f, d1 = 0.f, e = 0.f;
 #pragma unroll
     for (int i = 0; i < C::MI; ++i)
 #pragma unroll
@@ -2274,15 +2326,26 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int k = (i * C::NI + j) * 2 + h;
-          acc_dot(acc[i][j], h, HELD ? vr[HELD ? k : 0] : vsrc[k * 64], d0, d1);
+          if constexpr (HELD)
+            acc_dot(acc[i][j], h, vr[k], d0, d1);
+          else
+            acc_dot_sq(acc[i][j], h, vsrc[k * 64], d0, d1, e);
         }
     const float d = wave_sum_dpp(d0 + d1);
     const int slot = started ? 0 : 1;
     const bool whole = started && ended;
     float* pd = q.pdot + (tile * (C::WM * C::WN) + wid) * 2 * q.n_t + sample;
-    if (lane == 0) {
-      pd[slot * q.n_t] = HELD ? d : d - s_prev;
-      if (whole) pd[q.n_t] = 0.f;
+    if constexpr (HELD) {
+      if (lane == 0) {
+        pd[slot * q.n_t] = d;
+        if (whole) pd[q.n_t] = 0.f;
+      }
+    } else {
+      e = wave_sum_dpp(e);
+      if (lane == 0) {
+        pd[0] = d - s_prev;
+        pd[q.n_t] = e;
+      }
     }
     if constexpr (HELD) {
 #pragma unroll
@@ -2364,6 +2427,60 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tgdot_kernel(TgParams q) 
     store(tot);
   else
     store(acc);
+}
+
+// The dots of tgdot_kernel's running sums that lost too much (flag[i], growth_lost), each from its
+// sample's own product: a workgroup per tile of the same tile set, which forms the tile of every
+// flagged sample in turn; the last of a sample's workgroups adds their shares in tile order.  With
+// nothing flagged, the usual case, this launch and the squares above cost 2-15 us (the hooks of
+// Pythia-1B fc 612 -> 614 us and fc_out 605 -> 614, of a 768 x 50304 head 836 -> 851); a flagged
+// sample costs its share of the train GEMM once more.
+struct TgRedo {
+  const int* flag;  // [n_t]
+  int* done;        // [n_t] workgroups that have stored their share, 0
+  float* part;      // [m_tiles * n_tiles][n_t]
+  void* out_dot;
+  int dot_f32;
+};
+template <class C, class D>
+__global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tg_redo_kernel(TgParams q, TgRedo r) {
+  const TnParams& p = q.tn;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[D::STAGES * D::STAGE_BYTES];
+  __shared__ float red[C::WM * C::WN];
+  __shared__ int last;
+  const int64_t tile = xcd_order(blockIdx.x, gridDim.x);
+  const int64_t mt = tile / p.n_tiles, nt = tile - mt * p.n_tiles;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint4* vsrc = q.V + acc_base<C>(tile, wid);
+  for (int64_t s = 0; s < q.n_t; ++s) {
+    if (r.flag[s] == 0) continue;  // the same for every thread
+    f32x16_t acc[C::MI][C::NI];
+    zero_acc<TrBF16, C>(acc);
+    mainloop_tn<C, D>(p, mt, nt, s * q.T, (s + 1) * q.T, lds, acc);
+    float d0 = 0.f, d1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < C::MI; ++i)
+#pragma unroll
+      for (int j = 0; j < C::NI; ++j)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          acc_dot(acc[i][j], h, vsrc[((i * C::NI + j) * 2 + h) * 64], d0, d1);
+    const float d = block_sum(d0 + d1, red);
+    if (threadIdx.x == 0) {
+      r.part[tile * q.n_t + s] = d;
+      __threadfence();
+      last = atomicAdd(r.done + s, 1) == static_cast<int>(gridDim.x) - 1;
+    }
+    __syncthreads();
+    if (last) {
+      __threadfence();
+      float t = 0.f;
+      for (int64_t k = threadIdx.x; k < gridDim.x; k += C::NT) t += r.part[k * q.n_t + s];
+      t = block_sum(t, red);
+      if (threadIdx.x == 0) put_dot(r.out_dot, r.dot_f32, s, t);
+    }
+    __syncthreads();  // the stages, red and last are used again
+  }
 }
 
 // Per-pair weight dots <V_j, G_i^T A_i> (V_j = G_j^T A_j of val sample j) from one sample's
@@ -3893,7 +4010,8 @@ bool layer_pass_pays(int64_t N, int64_t n_val, int64_t T, int64_t d_in, int64_t 
 struct TgBufs {
   uint16_t *abar, *gbar;
   uint4* V;
-  float *vpart, *vp, *pdot, *csum, *pbias, *tgpart;
+  float *vpart, *vp, *pdot, *csum, *pbias, *tgpart, *rpart;
+  int* redo;
 };
 // The V GEMM of the pass: the train GEMM's orientation and tiles; wide tiles unsplit, narrow ones
 // by the split estimate.  With the presum and a bias its reduction launch also folds the presum
@@ -3925,6 +4043,8 @@ TgBufs carve_tg(S& c, const TgPlan& t, int64_t T, int64_t d_in, int64_t d_out) {
   const int64_t bw = t.bias_a ? t.n_tiles * t.wn : t.m_tiles * t.wm;
   b.pbias = t.bias ? c.template take<float>(t.n_t * (t.Tp / TnD::KB) * bw) : nullptr;
   b.tgpart = t.sp > 1 ? c.template take<float>(t.sp * d_out * d_in) : nullptr;
+  b.rpart = t.wide ? c.template take<float>(t.m_tiles * t.n_tiles * t.n_t) : nullptr;
+  b.redo = t.wide ? c.template take<int>(2 * t.n_t) : nullptr;
   return b;
 }
 }  // namespace
@@ -3969,7 +4089,8 @@ int launch_tgdot_finish(const float* pdot, int64_t shares, int64_t n_t, const fl
                         void* out_dot, int dot_dtype, void* out_bias_dot, int bias_dot_dtype,
                         void* out_bias_grad, int bias_grad_dtype, float bias_grad_scale,
                         const float* part, int64_t count, int64_t sp, void* out_grad,
-                        int grad_dtype, float grad_scale, hipStream_t s) {
+                        int grad_dtype, float grad_scale, hipStream_t s, int* redo = nullptr,
+                        int64_t T = 0) {
   const int64_t gblocks =
       out_bias_grad != nullptr ? ceil_div(bias_d, int64_t{FINISH_GF}) : 0;
   const dim3 grid(static_cast<unsigned>(n_t + gblocks + ceil_div(count / 4, int64_t{256})));
@@ -3979,12 +4100,12 @@ int launch_tgdot_finish(const float* pdot, int64_t shares, int64_t n_t, const fl
     hipLaunchKernelGGL(tgdot_finish_kernel<float>, grid, dim3(256), 0, s, pdot, shares, n_t, pbias,
                        bshares, csum, cs_rows, bias_d, out_dot, df32, out_bias_dot, bf32,
                        static_cast<float*>(out_bias_grad), bias_grad_scale, gblocks, part, count,
-                       static_cast<int>(sp), out_grad, grad_scale, gf32);
+                       static_cast<int>(sp), out_grad, grad_scale, gf32, redo, T);
   else
     hipLaunchKernelGGL(tgdot_finish_kernel<uint16_t>, grid, dim3(256), 0, s, pdot, shares, n_t,
                        pbias, bshares, csum, cs_rows, bias_d, out_dot, df32, out_bias_dot, bf32,
                        static_cast<uint16_t*>(out_bias_grad), bias_grad_scale, gblocks, part,
-                       count, static_cast<int>(sp), out_grad, grad_scale, gf32);
+                       count, static_cast<int>(sp), out_grad, grad_scale, gf32, redo, T);
   return check_launch("tgdot_finish_kernel");
 }
 
@@ -4158,11 +4279,17 @@ int dot_train_grad(const char* name, bool bias_a, bool any_T, const void* A, con
   const int64_t shares = t.m_tiles * t.n_tiles * (t.wm * t.wn) * 2;
   const int64_t sps = t.Tp / TnD::KB;
   const int64_t bshares = sps * (t.bias_a ? t.n_tiles * t.wn : t.m_tiles * t.wm);
-  return launch_tgdot_finish(b.pdot, shares, t.n_t, out_bias_dot != nullptr ? b.pbias : nullptr,
-                             bshares, b.csum, 2 * sps, t.bias_d, out_dot, dot_dtype,
-                             out_bias_dot, bias_dot_dtype, out_bias_grad, bias_grad_dtype,
-                             bias_grad_scale, b.tgpart,
-                             out_grad != nullptr && !direct ? d_out * d_in : 0, t.sp, out_grad, grad_dtype, grad_scale, s);
+  rc = launch_tgdot_finish(b.pdot, shares, t.n_t, out_bias_dot != nullptr ? b.pbias : nullptr,
+                           bshares, b.csum, 2 * sps, t.bias_d, out_dot, dot_dtype, out_bias_dot,
+                           bias_dot_dtype, out_bias_grad, bias_grad_dtype, bias_grad_scale,
+                           b.tgpart, out_grad != nullptr && !direct ? d_out * d_in : 0, t.sp,
+                           out_grad, grad_dtype, grad_scale, s, b.redo, T);
+  if (rc || !t.wide) return rc;
+  const TgRedo r{b.redo, b.redo + t.n_t, b.rpart, out_dot, dot_dtype == GS_DTYPE_F32 ? 1 : 0};
+  hipLaunchKernelGGL((tg_redo_kernel<TnCW, TnDW>),
+                     dim3(static_cast<unsigned>(t.m_tiles * t.n_tiles)), dim3(TnCW::NT), 0, s, q,
+                     r);
+  return check_launch("tg_redo_kernel");
 }
 }  // namespace
 }  // namespace gs

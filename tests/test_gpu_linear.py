@@ -4,6 +4,8 @@ Tolerances: bf16 operands 2e-2 normwise, fp32 operands 1e-4 normwise, both again
 float64 closed forms; the ghost kernel with reference rounding against the reference's
 own bf16 op sequence at 2e-3.
 """
+import math
+
 import pytest
 import torch
 
@@ -578,6 +580,54 @@ def test_linear_layer_pass_any_length(gpu, case):
             assert torch.equal(dn[others], dot.cpu()[others]), (at, value)
             assert torch.equal(dn[at], dot.cpu()[at] * 2.0 ** 20) if value is None else \
                 not torch.isfinite(dn[at])
+
+
+@pytest.mark.parametrize("case", [
+    # N, n_val, T, d_in, d_out, semantics, val position, bias, conv1d: whole 64-row stages and
+    # 256 x 256 tiles, whose dots are growths of running sums
+    (7, 2, 64, 2000, 7176, "pairwise", "mid", True, False),
+    (6, 1, 128, 7176, 2000, "presum", "first", True, True),
+    (9, 1, 64, 4096, 3600, "pairwise", "last", False, False),
+])
+def test_linear_layer_pass_wide_tiles_keep_samples_apart(gpu, case):
+    """One train sample's NaN, Inf or gradient of R times the others' size among the running sums:
+    the dots before it keep their bits, those after it stay within what a growth may lose before
+    it is formed again (an rms of 2^-9 of the shares' size; 1e-2 of the dots' is five times
+    that), for R on both sides of that line."""
+    N, n_val, T, d_in, d_out, sem, pos, bias, conv1d = case
+    vs = {"last": N - n_val, "first": 0, "mid": 1}[pos]
+    n_t = N - n_val
+    print(f"wide layer pass case={case}", flush=True)
+    A, G = (x.to(gpu) for x in _inputs(N, T, d_in, d_out, 220 + T, torch.bfloat16))
+    semantics = _native.SEM_PAIRWISE_SUM if sem == "pairwise" else _native.SEM_PRESUM
+
+    def run(a, dot_dtype=torch.float32):
+        return _native.ops().linear_layer_pass(
+            a, G, n_val, semantics=semantics, algo=_native.ALGO_VALGRAD,
+            rounding=_native.ROUND_FP32, conv1d=conv1d, grad_scale=1.0 / n_t,
+            grad_dtype=torch.bfloat16, dot_dtype=dot_dtype,
+            bias_grad_dtype=torch.float32 if bias else None, bias_dot_dtype=dot_dtype,
+            val_start=vs)
+    dot = run(A)[0].cpu()
+    want = R.linear_dot_valterm_exact(A, G, n_val, sem, val_start=vs,
+                                      round_dtype=torch.bfloat16).cpu()
+    assert_close(dot, want, 5e-3, "weight dot")
+    rows = [i for i in range(N) if not vs <= i < vs + n_val]
+    for at in (0, 2):
+        after = list(range(at + 1, n_t))
+        for r in (float("nan"), float("inf"), 2.0 ** 6, 2.0 ** 10, 2.0 ** 14, 2.0 ** 18, 2.0 ** 24):
+            bad = A.clone()
+            bad[rows[at]] *= r
+            dn = run(bad)[0].cpu()
+            assert torch.equal(dn[:at], dot[:at]), (at, r)
+            assert_close(dn[after], dot[after], 1e-2, f"dots after sample {at} times {r}")
+            if math.isfinite(r):
+                assert abs(dn[at] / r - dot[at]) <= 1e-3 * dot.square().mean().sqrt()
+            else:
+                assert not torch.isfinite(dn[at])
+            assert torch.equal(run(bad)[0].cpu().nan_to_num(0), dn.nan_to_num(0)), "not repeated"
+            low = run(bad, torch.bfloat16)[0].cpu()
+            assert torch.equal(low.nan_to_num(0), dn.bfloat16().nan_to_num(0))
 
 
 @pytest.mark.parametrize("case", [
