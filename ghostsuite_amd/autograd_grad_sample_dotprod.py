@@ -169,10 +169,14 @@ def _apply_train_grad(layer: nn.Module, val_batch_size: int, loss_reduction: str
 
 # Below this much work a layer's kernels run on the autograd stream: entering the side stream
 # costs the host 29 us a hook (an event recorded, waited for, and the stream switched; MI355X, one
-# hook), while such kernels take about 10 us and leave little to overlap.  Measured with everything
-# on the side stream / with this rule: an engine step of a 512-1024-1024-10 fp32 MLP of 80 rows
-# 1420 / 1160 us, of a four-layer GPT-2 of 10 rows x 512 tokens (its LayerNorms and embeddings are
-# below, its Linears above) 7113 / 6755 us.
+# hook), while such kernels take about 10 us and leave little to overlap.  Whole engine steps,
+# everything on the side stream / this rule / everything on the autograd stream (medians of 7, us):
+# a 512-1024-1024-10 fp32 MLP of 80 rows 1501 / 1241 / 1212; a four-layer GPT-2 of 10 rows x 256
+# tokens 11824 / 11250 / 7410, x 512 10738 / 10157 / 8809, 20 x 512 10955 / 11066 / 8850 (these
+# wait for the host, and spread by a third); the 12-layer GPT-2-small step of 20 x 1024, which waits
+# for the GPU, 29909 / 29776 / 31781.  A line of 64 Mi elements and 1e11 flops gives that step back
+# half of the overlap (30858), of 16 Mi elements or 1e10 flops nothing either way: it stays where
+# the steps that wait for the GPU lose nothing.
 _INLINE_ELEMENTS = 8 << 20     # of the layer's input and output gradient together
 _INLINE_FLOPS = 1e9            # of one product of the two
 
