@@ -1381,10 +1381,10 @@ __device__ __forceinline__ void put_dot(void* out, int f32, int64_t at, float v)
 }
 
 // Whether a dot taken as the growth of running sums (tgdot_kernel) has lost more than bf16
-// rounding: growth2 is the sum of the wave shares' squares, size2 that of the running sums' products
-// with V, entry by entry.  A sum of T k-rows is rounded T / 16 times, each time by 2^-24 of its
-// size at most, independent in sign; that may be 2^-9 of the shares' size.  (Sums of Inf or NaN,
-// and squares that fp32 may have flushed, count as lost.)
+// rounding: growth2 is the sum of the wave shares' squares, size2 that of the running sums'
+// products with V, entry by entry.  A sum of T k-rows is rounded T / 16 times, each time by 2^-24
+// of its size at most, independent in sign; that may be 2^-9 of the shares' size.  (Sums of Inf
+// or NaN, and squares that fp32 may have flushed, count as lost.)
 __device__ __forceinline__ bool growth_lost(double growth2, float size2, int64_t T) {
   const double s = size2;
   return !(s >= 1e-30 && s * static_cast<double>(T) <= growth2 * 0x1p34);
@@ -1393,11 +1393,11 @@ __device__ __forceinline__ bool growth_lost(double growth2, float size2, int64_t
 // After tgdot_kernel, three independent block ranges of one launch, fixed order throughout:
 // blocks b < n_t take weight dot b from its `shares` wave shares (with redo: half as many, each
 // followed by the running sums' size; redo[b] says whether tg_redo_kernel must form the dot
-// again, redo[n_t + b] is its counter, cleared) and, with pbias, bias dot b
-// from its `bshares` shares; then (with bgrad) the bias train gradient, FINISH_GF features
-// per block, over the n_t * cs_rows column-sum rows of csum; then (with grad) the train
-// gradient: grad[i] = gscale * (the sum over the sp splits of part[s][i]), rounded once (or
-// stored as fp32 with grad_f32), 4 elements per thread.
+// again, redo[n_t + b] is its counter, cleared) and, with pbias, bias dot b from its `bshares`
+// shares; then (with bgrad) the bias train gradient, FINISH_GF features per block, over the
+// n_t * cs_rows column-sum rows of csum; then (with grad) the train gradient: grad[i] = gscale *
+// (the sum over the sp splits of part[s][i]), rounded once (or stored as fp32 with grad_f32),
+// 4 elements per thread.
 template <class GE>
 __global__ void __launch_bounds__(256) tgdot_finish_kernel(
     const float* __restrict__ pdot, int64_t shares, int64_t n_t, const float* __restrict__ pbias,
@@ -2228,9 +2228,9 @@ __global__ void __launch_bounds__(C::NT, C::MIN_WAVES) tn_gemm_kernel(TnParams p
 //  - 128 x 64 wave tiles have no registers for a second set: acc runs on, and the share is the
 //    growth of <acc, V tile> since the previous boundary, which rounds at the running sum's size.
 //    That size goes beside it, and tg_redo_kernel forms the dots again that lost too much to it.
-//    T a multiple of the stage height only, splits of whole samples.  (Their place taken by 64 x 64 wave tiles: Pythia-1B
-//    fc 595 -> 702 us, 256 x 128 tiles of eight such waves 712, of four 128 x 64 waves with the
-//    registers of a whole SIMD 864; the sums kept in memory instead 930.)
+//    T a multiple of the stage height only, splits of whole samples.  (Their place taken by 64 x 64
+//    wave tiles: Pythia-1B fc 595 -> 702 us, 256 x 128 tiles of eight such waves 712, of four
+//    128 x 64 waves with the registers of a whole SIMD 864; the sums kept in memory instead 930.)
 // With CS the column sums of the L tile (G: the bias terms) are taken per stage as well, after
 // the stage's MFMAs, spread over the workgroups.
 struct TgParams {
@@ -4398,7 +4398,8 @@ bool tf_pays(const TfPlan& t, int algo, int64_t N, int64_t n_val, int64_t T, int
   };
   const double fused =
       25.0 + launch(t.vsp, static_cast<double>(t.vkper), area) +
-      launch(t.sp, static_cast<double>(t.kper) * (1.0 + static_cast<double>(TF_KB) / t.Tp), t.M * t.N);
+      launch(t.sp, static_cast<double>(t.kper) * (1.0 + static_cast<double>(TF_KB) / t.Tp),
+             t.M * t.N);
   constexpr int64_t TL = 64;
   const double nvT = static_cast<double>(t.vrows), rows = static_cast<double>(t.n_t) * T;
   auto rounds = [&](double a, double b, double at_once) {

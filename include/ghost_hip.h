@@ -56,8 +56,9 @@ typedef enum { GS_SEM_PAIRWISE_SUM = 0, GS_SEM_PRESUM = 1 } gs_semantics;
  *   GHOST:   fused dual-Gram MFMA kernel; the T x T Gram blocks live only in registers.
  *   VALGRAD: V = sum_val B^T A (one GEMM), then dot_i = sum_t <b_it, V a_it> fused into
  *            the epilogue of a second GEMM; per-sample gradients are never stored.  With a
- *            pair matrix and aligned bf16 operands: one V_j per val row, and each train row's
- *            gradient tile times every V_j as it leaves the accumulators.
+ *            pair matrix and aligned bf16 operands, where estimated to be faster: one V_j per
+ *            val row, and each train row's gradient tile times every V_j as it leaves the
+ *            accumulators.
  *   AUTO:    the one with fewer MFMA flops for the shape. */
 typedef enum { GS_ALGO_AUTO = 0, GS_ALGO_GHOST = 1, GS_ALGO_VALGRAD = 2 } gs_algo;
 
@@ -181,8 +182,8 @@ int gs_conv1d_dot_train_grad(const void* A, const void* G, int dtype, int64_t N,
  * aligned, feature counts multiples of 4, below 2 GiB; fp32 products throughout), any T, the weight layout by `conv1d` (0: out_grad
  * [d_out, d_in], gs_linear_dot_train_grad; 1: [d_in, d_out], gs_conv1d_dot_train_grad), and the
  * dots rounded once from fp32 to dot_dtype / bias_dot_dtype (GS_DTYPE_BF16 or GS_DTYPE_F32).
- * Where T is not a whole number of the kernel's stages each train sample is padded with zero rows inside the kernel
- * (nothing is read for them).  The workspace query returns 0 where the pass does not apply
+ * Where T is not a whole number of the kernel's stages each train sample is padded with zero rows
+ * inside the kernel (nothing is read for them).  The workspace query returns 0 where the pass does not apply
  * (algo GHOST; AUTO choosing GHOST for bf16 operands, or for fp32 ones with the reference's
  * rounding) and where the dots and the train gradient apart are estimated to be faster.
  * Reference: as for the two entry points above. */

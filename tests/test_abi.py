@@ -90,15 +90,16 @@ def test_fp32_layer_pass_leaves_what_it_would_pad_to_the_separate_passes(shape, 
 
 @pytest.mark.parametrize("shape,products", [
     # n_train, n_val, T, d_in, d_out: both sides of the line as measured
-    ((24, 8, 128, 768, 3072), True), ((24, 1, 128, 768, 3072), True), ((4, 1, 512, 1280, 1280), True),
-    ((200, 4, 1, 1024, 1024), True), ((200, 1, 1, 1024, 1024), False),
+    ((24, 8, 128, 768, 3072), True), ((24, 1, 128, 768, 3072), True),
+    ((4, 1, 512, 1280, 1280), True), ((200, 4, 1, 1024, 1024), True), ((200, 1, 1, 1024, 1024), False),
     ((4000, 1, 1, 512, 512), False), ((48, 1, 200, 2048, 2048), False)])
 def test_pair_matrix_by_row_dots_where_its_sample_products_would_be_slower(shape, products):
     n_t, n_val, T, d_in, d_out = shape
     aligned = ctypes.c_void_p(1 << 20)
     got = _native.load_library().gs_linear_dot_noalloc_bytes(
         aligned, aligned, 0, n_t + n_val, n_val, T, d_in, d_out, 0, _native.ALGO_VALGRAD, 1)
-    # the products' scratch: a V_j of 128 x 128 bf16 tiles per val sample, a partial per tile and pair
+    # the products' scratch: a V_j of 128 x 128 bf16 tiles per val sample and a partial per tile
+    # and pair
     tiles = n_val * -(-d_in // 128) * -(-d_out // 128)
     want = tiles * 128 * 128 * 2 + tiles * n_t * 4
     assert (want <= got < want + 512) == products
